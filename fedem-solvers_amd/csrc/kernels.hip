@@ -357,146 +357,249 @@ __device__ __forceinline__ double lane_bcast(double v, int src) {
   return __hiloint2double(hi, lo);
 }
 
+// 1/d to rounding: the hardware estimate r0 (relative error e below 2^-20)
+// and r0 (1 + e + e^2).
+__device__ __forceinline__ double recip64(double d) {
+  const double r = __builtin_amdgcn_rcp(d), e = __builtin_fma(-d, r, 1.0);
+  return __builtin_fma(__builtin_fma(e, e, e), r, r);
+}
+// a/d from r = recip64(d): the product corrected by its own residual (the
+// quotient's rounding), three dependent operations instead of a division's
+// scaling sequence.
+__device__ __forceinline__ double quot64(double a, double d, double r) {
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-d, q, a), r, q);
+}
+
+// a/d in the storage type
+__device__ __forceinline__ double div_pivot(double a, double d) { return quot64(a, d, recip64(d)); }
+__device__ __forceinline__ float div_pivot(float a, double d) { return a / (float)d; }
+
 // k_diag task: sn, k0 = first panel column.  Blocked LDL^T of the kb x kb
 // (kb <= 64) diagonal block in LDS by four waves, in 16-column steps:
-// (1) wave 0 factors the 16 x 16 diagonal sub-block with its rows in
-// registers and readlane broadcasts (L11 unit lower, D1, X11 = L11^-1);
-// (2) the rows below form L21 = A21 X11^T D1^-1 on FP64 MFMA, one 16-row
-// tile per wave; (3) the lower trailing block takes A22 -= (L21 D1) L21^T,
-// 16 x 16 MFMA tiles shared by the waves.  The off-diagonal tiles of
-// X = L^-1 then follow by distance from the diagonal:
-// X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj.  L and D go back into the front,
-// X into the diagonal tile of the pivot-block inverse pool.  The arithmetic
-// is FP64 for both storage types (the FP32 factor of the mixed-precision
-// path keeps its diagonal blocks' factorisation in FP64 and rounds only the
-// stored result).  Rows beyond kb are carried as identity rows.
+// (1) wave 0 factors the 16-column panel over all rows below its top, lane i
+// holding row i in registers with readlane broadcasts, so L11, D1 and L21
+// come out of one sweep; identity rows in the lanes that the panel leaves
+// free turn into X11 = L11^-1 in the same sweep; (2) the tiles of the next
+// panel's columns take A22 -= (L21 D1) L21^T on FP64 MFMA, one 16 x 16 tile
+// per wave.  While wave 0 sweeps the next panel, waves 1-3 update the
+// trailing tiles past it and form the off-diagonal tiles of X = L^-1,
+// X_ij = -X_ii T_ij with T_ij = sum_{k=j}^{i-1} L_ik X_kj (wave j + 1 owns
+// tile column j), so the chain of 64 pivots only waits for the sweeps and
+// one tile each.  D goes to the pivot array, X into the diagonal tile of the
+// pivot-block inverse pool.  The arithmetic is FP64 for both storage types
+// (the FP32 factor of the mixed-precision path keeps its diagonal blocks'
+// factorisation in FP64 and rounds only the stored result).  Rows beyond kb
+// are carried as identity rows.
+// Bound by the dependent chain over the pivots (a reciprocal, a quotient and
+// a broadcast each): it sets the pace of every panel of the top separators.
+// A k_diag_trsm launch takes 18-19 us (117 x 109 plate, 48 x 24 x 24 block)
+// where 16-row sweeps with a division per pivot, L21 through X11 and loads
+// under conditions (each waiting for the one before) took 37-39 us.
 //
-// diag_block: that factorisation in LDS; sA holds L (unit lower) with D on
-// its diagonal, sD = D, sX = L^-1, all in FP64.
+// diag_block: that factorisation in LDS; sA holds L (unit lower) below D,
+// sD = D, sX = L^-1 with zeros above it, all in FP64.
 template <class T>
 __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int k0, int kb, double (&sA)[64][65],
                                            double (&sX)[64][65], double (&sD)[64], double (&sT)[4][16][17],
                                            const DevSym& S, int colbase) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int lr = lane & 15, lk = lane >> 4;
-  // the singular-pivot test's |a_jj| of the block's columns, lane j of wave
-  // 0 holding column j: read once here, broadcast in the sweeps below (a
-  // load per pivot would put a memory latency on every step of the chain)
-  const double adv = (wv == 0 && lane < kb) ? S.adiag[colbase + lane] : 0.0;
-  for (int idx = tid; idx < 64 * 64; idx += 256) {
-    const int i = idx & 63, m = idx >> 6;
-    sA[i][m] = (i < kb && m <= i) ? (double)F[(int64_t)(k0 + i) + (int64_t)(k0 + m) * ld] : (i == m ? 1.0 : 0.0);
-    sX[i][m] = (i == m) ? 1.0 : 0.0;
+  // singular-pivot test: |a_jj| of the block's columns, lane j of wave 0
+  // holding column j, read once here
+  const double amax = wv == 0 ? *S.amax : 0.0;
+  const double adv = (wv == 0 && lane < kb) ? fabs(S.adiag[colbase + lane]) : 0.0;
+  {
+    // every load from inside the front and unconditional, the entries
+    // outside the block replaced afterwards: a load under a condition waits
+    // for the one before it
+    const T* row = F + (int64_t)k0 * (ld + 1) + min(lane, kb - 1);
+    T v[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) v[q] = row[(int64_t)min(wv + 4 * q, kb - 1) * ld];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int m = wv + 4 * q;
+      sA[lane][m] = (lane < kb && m <= lane) ? (double)v[q] : (lane == m ? 1.0 : 0.0);
+      sX[lane][m] = 0.0;
+    }
   }
   __syncthreads();
   const int nsb = (kb + 15) >> 4;
+  auto wave_fence = [&]() {  // this wave's LDS writes are visible to its own reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // A(ti, tj) -= (L(ti, p) D_p) L(tj, p)^T, 16 x 16 tiles, lower entries
+  auto update_tile = [&](int ti, int tj, int p) {
+    f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m0 = 0; m0 < 16; m0 += 4) {
+      const int m = 16 * p + m0 + lk;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[16 * tj + lr][m], sA[16 * ti + lr][m] * sD[m], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = 16 * ti + lr, j = 16 * tj + lk + 4 * r;
+      if (i >= j) sA[i][j] -= acc[r];
+    }
+  };
+  // X_00 = L_00^-1 where the sweep had no free lanes: lane c < 16 solves
+  // column c against the uniformly read L
+  auto invert_tile0 = [&]() {
+    if (lane < 16) {
+      double x[16];
+#pragma unroll
+      for (int m = 0; m < 16; m++) x[m] = m == lane ? 1.0 : 0.0;
+#pragma unroll
+      for (int k = 0; k < 15; k++)
+#pragma unroll
+        for (int i = k + 1; i < 16; i++) x[i] = __builtin_fma(-sA[i][k], x[k], x[i]);
+#pragma unroll
+      for (int m = 0; m < 16; m++) sX[m][lane] = x[m];
+    }
+  };
+  // T_ij into this wave's sT, then X_ij = -X_ii T_ij
+  auto sum_tile = [&](int i, int j) {
+    f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int kt = j; kt < i; kt++)
+#pragma unroll
+      for (int m0 = 0; m0 < 16; m0 += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sX[16 * kt + m0 + lk][16 * j + lr],
+                                                   sA[16 * i + lr][16 * kt + m0 + lk], acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; r++) sT[wv][lr][lk + 4 * r] = acc[r];
+    wave_fence();
+  };
+  auto finish_tile = [&](int i, int j) {
+    f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m0 = 0; m0 < 16; m0 += 4)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sT[wv][m0 + lk][lr], sX[16 * i + lr][16 * i + m0 + lk], acc, 0, 0,
+                                                 0);
+#pragma unroll
+    for (int r = 0; r < 4; r++) sX[16 * i + lr][16 * j + lk + 4 * r] = -acc[r];
+    wave_fence();
+  };
   for (int p = 0; p < nsb; p++) {
-    const int c0 = 16 * p;
-    // (1) the 16 x 16 diagonal sub-block: lane i < 16 holds row c0 + i
+    const int c0 = 16 * p, used = 16 * (nsb - p);  // lanes that hold panel rows
     if (wv == 0) {
-      double a[16], x[16];
+      // lane i holds row c0 + i of the panel; the sixteen lanes after the
+      // panel's rows (when there are any) the rows of the identity
+      const int row = min(c0 + lane, 63), unit = lane - used;
+      double a[16], u[16];  // u: column j before its division by the pivot
+      double d0;            // lane j: pivot c0 + j
+      const double ac = __shfl(adv, (c0 + lane) & 63), thr = S.tolf * ac, rep = ac != 0.0 ? ac : amax;
+      // TEST: a pivot below the limit is replaced (rare; the first pass only
+      // detects it, as a select in the chain would slow every pivot)
+      auto sweep = [&](auto test) {
+        constexpr bool TEST = decltype(test)::value;
 #pragma unroll
-      for (int m = 0; m < 16; m++) {
-        a[m] = (lane < 16 && m <= lane) ? sA[c0 + lane][c0 + m] : 0.0;
-        x[m] = (m == lane) ? 1.0 : 0.0;
+        for (int m = 0; m < 16; m++) a[m] = unit < 0 ? sA[row][c0 + m] : (unit == m ? 1.0 : 0.0);
+        auto pivot = [&](double v, int j) { return lane_bcast(TEST ? (fabs(v) > thr ? v : rep) : v, j); };
+        d0 = a[0];
+        double dj = pivot(a[0], 0), rj = recip64(dj);
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+          u[j] = a[j];
+          // the broadcasts of column j beside its quotient, then the next
+          // pivot and its reciprocal beside the column updates
+          double ub[16];
+#pragma unroll
+          for (int m = j + 1; m < 16; m++) ub[m] = lane_bcast(u[j], m);
+          const double l = quot64(u[j], dj, rj);
+          a[j] = lane > j ? l : (lane == j ? dj : a[j]);
+          if (j == 15) break;
+          __builtin_amdgcn_sched_barrier(0);
+          a[j + 1] = __builtin_fma(-l, ub[j + 1], a[j + 1]);
+          d0 = lane == j + 1 ? a[j + 1] : d0;
+          dj = pivot(a[j + 1], j + 1);
+          rj = recip64(dj);
+#pragma unroll
+          for (int m = j + 2; m < 16; m++) a[m] = __builtin_fma(-l, ub[m], a[m]);
+          __builtin_amdgcn_sched_barrier(0);  // the broadcasts stay in their step (few scalar registers)
+        }
+      };
+      sweep(std::false_type{});
+      const bool bad = lane < 16 && c0 + lane < kb && !(fabs(d0) > thr);
+      if (__any(bad)) {
+        sweep(std::true_type{});
+        // column flags of the replaced pivots: 1 a true zero, 2 reduced to near zero
+        if (lane < 16 && c0 + lane < kb && !(fabs(d0) > thr))
+          S.sing[colbase + c0 + lane] = ac == 0.0 || fabs(d0) <= 1.0e3 * 2.220446049250313e-16 * ac ? 1 : 2;
       }
+      if (unit < 0) {
+        // (the entries above the diagonal are not read again)
+        double dd = a[0];
 #pragma unroll
-      for (int j = 0; j < 16; j++) {
-        double dj = lane_bcast(a[j], j);
-        if (c0 + j < kb) {  // singular pivot: replaced, column flagged (same decision on every lane)
-          const int col = colbase + c0 + j;
-          const double aj = lane_bcast(adv, c0 + j);
-          if (!(fabs(dj) > S.tolf * fabs(aj))) {
-            const bool truez = aj == 0.0 || fabs(dj) <= 1.0e3 * 2.220446049250313e-16 * fabs(aj);
-            dj = aj != 0.0 ? fabs(aj) : *S.amax;
-            if (lane == j) a[j] = dj;
-            if (lane == 0) S.sing[col] = truez ? 1 : 2;
-          }
-        }
-        const bool below = lane > j && lane < 16;
-        const double l = below ? a[j] / dj : 0.0;
-        if (below) a[j] = l;
-        const double ldj = l * dj;
+        for (int m = 1; m < 16; m++) dd = m == lane ? a[m] : dd;
+        if (lane < 16) sD[c0 + lane] = dd;
 #pragma unroll
-        for (int m = j + 1; m < 16; m++) {
-          const double lm = lane_bcast(l, m);  // L[m][j]
-          if (m <= lane) a[m] -= ldj * lm;
-        }
+        for (int m = 0; m < 16; m++) sA[row][c0 + m] = a[m];
+      } else if (unit < 16) {
 #pragma unroll
-        for (int m = 0; m <= j; m++) x[m] -= l * lane_bcast(x[m], j);  // X[j][m]
+        for (int m = 0; m < 16; m++) sX[c0 + m][c0 + unit] = u[m];
       }
-      if (lane < 16) {
-        double dd = 0.0;
-#pragma unroll
-        for (int m = 0; m < 16; m++) {
-          if (m <= lane) {
-            sA[c0 + lane][c0 + m] = a[m];
-            sX[c0 + lane][c0 + m] = x[m];
-          }
-          dd = (m == lane) ? a[m] : dd;
-        }
-        sD[c0 + lane] = dd;
+    } else if (p > 0) {
+      // the work that the previous panel left: its row of X, T of this row if
+      // it is the last, the trailing tiles (ti, tj), p < tj <= ti
+      const int j = wv - 1, nt = nsb - p - 1;
+      if (p == 1 && nsb == 4 && wv == 1) {
+        invert_tile0();
+        wave_fence();
+      }
+      if (j < p - 1) {
+        sum_tile(p - 1, j);
+        finish_tile(p - 1, j);
+      }
+      if (p == nsb - 1 && j < p) sum_tile(p, j);
+      for (int q = (wv == 1 ? 2 : wv - 2); q < nt * (nt + 1) / 2; q += 3) {
+        const int ti = q == 0 ? 0 : (q < 3 ? 1 : 2), tj = q - ti * (ti + 1) / 2;
+        update_tile(p + 1 + ti, p + 1 + tj, p - 1);
       }
     }
     __syncthreads();
-    // (2) L21 = A21 X11^T D1^-1, wave w the row tile at c0 + 16 (w + 1)
-    const int rb0 = c0 + 16, nrt = nsb - p - 1;
-    if (wv < nrt) {
-      const int r0 = rb0 + 16 * wv;
-      f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int m0 = 0; m0 < 16; m0 += 4)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sX[c0 + lr][c0 + m0 + lk], sA[r0 + lr][c0 + m0 + lk], acc, 0, 0, 0);
-      // acc[r]: row r0 + lr, column c0 + lk + 4 r
-#pragma unroll
-      for (int r = 0; r < 4; r++) sA[r0 + lr][c0 + lk + 4 * r] = acc[r] / sD[c0 + lk + 4 * r];
+    if (p + 1 < nsb) {
+      if (p + 1 + wv < nsb) update_tile(p + 1 + wv, p + 1, p);
+      __syncthreads();
     }
-    __syncthreads();
-    // (3) A22 -= (L21 D1) L21^T over the lower 16 x 16 tiles (ti >= tj)
-    for (int q = wv; q < nrt * (nrt + 1) / 2; q += 4) {
-      const int ti = q == 0 ? 0 : (q < 3 ? 1 : (q < 6 ? 2 : 3));
-      const int tj = q - ti * (ti + 1) / 2;
-      const int ri = rb0 + 16 * ti, rj = rb0 + 16 * tj;
-      f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int m0 = 0; m0 < 16; m0 += 4) {
-        const int m = c0 + m0 + lk;
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[rj + lr][m], sA[ri + lr][m] * sD[m], acc, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = ri + lr, j = rj + lk + 4 * r;
-        if (i >= j) sA[i][j] -= acc[r];
-      }
-    }
-    __syncthreads();
   }
-  // off-diagonal 16 x 16 tiles of X = L^-1, by distance d from the diagonal
-  for (int d = 1; d < nsb; d++) {
-    const int j = wv, i = wv + d;
-    if (i < nsb) {
-      f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
-      for (int kt = j; kt < i; kt++)
+  if (wv > 0 && wv < nsb) finish_tile(nsb - 1, wv - 1);
+  __syncthreads();
+}
+
+// L_r = F_r L_kk^-T D^-1 for a 64-row tile at row R0: sF the rows, sL =
+// L_kk^-1 (lower, zeros above), C the panel's first column, d(j) its pivots.
+// Wave w takes rows 16 w .. 16 w + 15; column tile y only sums over the
+// column tiles m <= y, 40 MFMA steps a wave instead of 64.
+template <class T, class D>
+__device__ __forceinline__ void trsm_product(const T (*sF)[65], const T (*sL)[65], T* __restrict__ C, int ld, int R0,
+                                             int kb, D d) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4, nsb = (kb + 15) >> 4;
+  typename MF<T>::acc acc[4];
 #pragma unroll
-        for (int m0 = 0; m0 < 16; m0 += 4)
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sX[16 * kt + m0 + lk][16 * j + lr],
-                                                     sA[16 * i + lr][16 * kt + m0 + lk], acc, 0, 0, 0);
-      // T (rows of tile i, columns of tile j) through this wave's LDS tile
+  for (int y = 0; y < 4; y++) acc[y] = typename MF<T>::acc{};
 #pragma unroll
-      for (int r = 0; r < 4; r++) sT[wv][lr][lk + 4 * r] = acc[r];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      f64x4 acc2 = f64x4{0.0, 0.0, 0.0, 0.0};
+  for (int mt = 0; mt < 4; mt++) {
+    if (mt >= nsb) break;
 #pragma unroll
-      for (int m0 = 0; m0 < 16; m0 += 4)
-        acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(sT[wv][m0 + lk][lr], sX[16 * i + lr][16 * i + m0 + lk], acc2, 0,
-                                                    0, 0);
+    for (int m0 = 0; m0 < 16; m0 += 4) {
+      const int m = 16 * mt + m0 + lk;
+      const T aa = sF[16 * wv + lr][m];
 #pragma unroll
-      for (int r = 0; r < 4; r++) sX[16 * i + lr][16 * j + lk + 4 * r] = -acc2[r];
+      for (int y = mt; y < 4; y++) acc[y] = MF<T>::op(sL[16 * y + lr][m], aa, acc[y]);
     }
-    __syncthreads();
   }
+  const int i = R0 + 16 * wv + lr;
+  if (i >= ld) return;
+#pragma unroll
+  for (int y = 0; y < 4; y++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int j = 16 * y + MF<T>::col(lk, r);
+      if (j < kb) C[(int64_t)j * ld + i] = div_pivot(acc[y][r], d(j));
+    }
 }
 
 // X = L^-1 into the diagonal tile of the pivot-block inverse pool and D into
@@ -506,14 +609,14 @@ __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int 
 // workgroups of the same launch can still read it.
 template <class T>
 __device__ __forceinline__ void diag_store(T* __restrict__ Xg, double* __restrict__ dpiv, int nc, int k0, int kb,
-                                           int col0, const double (&sA)[64][65], const double (&sX)[64][65],
+                                           int col0, const double (&sD)[64], const double (&sX)[64][65],
                                            int* __restrict__ piv) {
   const int tid = threadIdx.x;
   for (int idx = tid; idx < 64 * 64; idx += 256) {
     const int i = idx & 63, m = idx >> 6;
     if (i < kb && m <= i) Xg[(int64_t)(k0 + i) + (int64_t)(k0 + m) * nc] = (T)sX[i][m];
   }
-  if (tid < kb) dpiv[col0 + k0 + tid] = sA[tid][tid];
+  if (tid < kb) dpiv[col0 + k0 + tid] = sD[tid];
   (void)piv;
 }
 
@@ -528,7 +631,7 @@ __global__ __launch_bounds__(256) void k_diag(const FTask* __restrict__ tasks, D
   T* F = pool + S.foff[sn];
   T* Xg = ipool + ioff[sn];
   diag_block<T>(F, ld, k0, kb, sA, sX, sD, sT, S, S.col0[sn] + k0);
-  diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sA, sX, piv);
+  diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sD, sX, piv);
 }
 
 // Diagonal block and triangular solve in one launch, for panels with few
@@ -554,49 +657,31 @@ __global__ __launch_bounds__(256) void k_diag_trsm(const FTask* __restrict__ tas
   const int R0 = k0 + kb + 64 * max(t.a, 0);
   T ra[16];
   if (t.a >= 0) {
+    // in-front addresses (rows past the front and columns past the panel
+    // repeat the last one; their products are not stored or meet a zero)
+    const T* row = F + (int64_t)k0 * ld + min(R0 + lane, ld - 1);
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-      ra[q] = (m < kb && R0 + i < ld) ? F[(int64_t)(R0 + i) + (int64_t)(k0 + m) * ld] : (T)0;
-    }
+    for (int q = 0; q < 16; q++) ra[q] = row[(int64_t)min(wv + 4 * q, kb - 1) * ld];
   }
   diag_block<T>(F, ld, k0, kb, sA, sX, sD, sT, S, S.col0[sn] + k0);
-  if (t.a <= 0) diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sA, sX, piv);
-  if (t.a < 0) return;
-  __syncthreads();  // every read of sA by the store is done
-  // operand tiles in the storage type: the row tile in sA's space, L^-1 in
-  // sX's space (in place for double: each thread rewrites only its entries)
+  if (t.a < 0) {
+    diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sD, sX, piv);
+    return;
+  }
+  // operand tiles in the storage type: the row tile in sA's space (every
+  // read of sA is behind diag_block's last barrier), L^-1 in sX itself or,
+  // rounded, behind the row tile
   T(*sF)[65] = reinterpret_cast<T(*)[65]>(&sA[0][0]);
-  T(*sL)[65] = reinterpret_cast<T(*)[65]>(&sX[0][0]);
-  T xv[16];
+  constexpr bool in_place = std::is_same<T, double>::value;
+  T(*sL)[65] = in_place ? reinterpret_cast<T(*)[65]>(&sX[0][0]) : sF + 64;
 #pragma unroll
   for (int q = 0; q < 16; q++) {
-    const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-    xv[q] = (m < kb && i < kb && i >= m) ? (T)sX[i][m] : (T)0;
+    sF[lane][wv + 4 * q] = wv + 4 * q < kb ? ra[q] : (T)0;
+    if (!in_place) sL[lane][wv + 4 * q] = (T)sX[lane][wv + 4 * q];
   }
   __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-    sF[i][m] = ra[q];
-    sL[i][m] = xv[q];
-  }
-  __syncthreads();
-  const int kbr = (kb + 3) & ~3;
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
-  typename MF<T>::acc acc[2][2];
-  zero_acc(acc);
-  mfma_tile<T>(sF, sL, kbr, acc, lane, wr, wc);
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = R0 + wr + 16 * x + lr;
-        const int j = wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ld && j < kb) F[(int64_t)i + (int64_t)(k0 + j) * ld] = acc[x][y][r] / (T)sD[j];
-      }
+  trsm_product<T>(sF, sL, F + (int64_t)k0 * ld, ld, R0, kb, [&](int j) { return sD[j]; });
+  if (t.a == 0) diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sD, sX, piv);
 }
 
 // k_trsm task: sn, a = 64-row tile below the diagonal block, k0 = panel.
@@ -615,38 +700,27 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
   T* F = pool + S.foff[sn];
   const T* Xg = ipool + ioff[sn];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int kbr = (kb + 3) & ~3;
   {
+    // unconditional in-bounds loads, as in k_diag_trsm; sB[j][m] = Linv_kk[j][m] (lower)
+    const T* row = F + (int64_t)k0 * ld + min(R0 + lane, ld - 1);
+    const T* xrow = Xg + (int64_t)k0 * (nc + 1) + min(lane, kb - 1);
     T ra[16], rb[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-      ra[q] = (m < kb && R0 + i < ld) ? F[(int64_t)(R0 + i) + (int64_t)(k0 + m) * ld] : (T)0;
-      // sB[j][m] = Linv_kk[j][m] (lower)
-      rb[q] = (m < kb && i < kb && i >= m) ? Xg[(int64_t)(k0 + i) + (int64_t)(k0 + m) * nc] : (T)0;
+      const int m = min(wv + 4 * q, kb - 1);
+      ra[q] = row[(int64_t)m * ld];
+      rb[q] = xrow[(int64_t)m * nc];
     }
 #pragma unroll
     for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-      sA[i][m] = ra[q];
-      sB[i][m] = rb[q];
+      const int m = wv + 4 * q;
+      sA[lane][m] = m < kb ? ra[q] : (T)0;
+      sB[lane][m] = (lane < kb && m <= lane) ? rb[q] : (T)0;
     }
   }
   __syncthreads();
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
-  typename MF<T>::acc acc[2][2];
-  zero_acc(acc);
-  mfma_tile<T>(sA, sB, kbr, acc, lane, wr, wc);
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = R0 + wr + 16 * x + lr;
-        const int j = wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ld && j < kb) F[(int64_t)i + (int64_t)(k0 + j) * ld] = acc[x][y][r] / (T)S.dpiv[S.col0[sn] + k0 + j];
-      }
+  const double* dp = S.dpiv + S.col0[sn] + k0;
+  trsm_product<T>(sA, sB, F + (int64_t)k0 * ld, ld, R0, kb, [&](int j) { return dp[j]; });
 }
 
 // ---------------------------------------------------------------- update
