@@ -17,13 +17,44 @@ struct FTask {
   int kb;      // trailing update: panel width (<= 128); the trailing block starts at k0 + kb
 };
 
-struct SolveTask {
-  int sn;
-  int r0, rn;  // target rows of the front work buffer
-  int k0, kn;  // source rows (K dimension); for reduce tasks: first slot, count
-  int j0;      // first right-hand side of this task
-  int slot;    // -1: apply to the target directly; >= 0: write a 64x64 partial
+// Elements that the solve-panel pools hold past their last front: k_panel's
+// 16-byte loads may run on past a column.
+constexpr int PANEL_PAD = 4;
+
+// A solve product task (solve.hip): target rows x right-hand sides j0 .. from
+// the operand at a (leading dimension ld) and kn source rows.
+struct MvTask {
+  int64_t a;   // offset of the operand's first element in the solve panels or (MV_FRONT) the fronts
+  int ld;
+  int rn, kn;  // target rows (<= 64) and source rows
+  int src;     // first source row, or (MV_BACK_ROWS) first entry of the fronts' row list
+  int ky;      // MV_BACK_ROWS: the first ky source rows are rows of Y, the others of X
+  int dst;     // first target row
+  int dst2;    // MV_Y: first row of V to keep the result in (-1: none); MV_YSUB: first row of Y
+  int flags;
+  int j0;
   int pad;
+};
+enum MvKind : int {
+  MV_FORWARD,    // operand rows contiguous
+  MV_BACK_ROWS,  // operand k contiguous, source rows through the fronts' row list
+  MV_BACK        // operand k contiguous, source rows contiguous in W
+};
+enum MvFlags : int {
+  MV_FRONT = 1,                  // operand in the fronts (L21), not the solve panels
+  MV_SRC_V = 2, MV_SRC_R = 4,    // source rows in V or R, not W
+  MV_APPLY = 0xf0,
+  MV_Y = 0x10,                   // Y = v / D (and V = v)
+  MV_SET = 0x20, MV_NEG = 0x30,  // W = v, W = -v
+  MV_ADD = 0x40, MV_SUB = 0x50,  // W += v, W -= v
+  MV_X = 0x60,                   // X = v
+  MV_YSUB = 0x70                 // W = Y - v (Y may be absent: zero)
+};
+
+// Forward initialisation of up to 64 work rows from w0 (k_fw_init).
+struct InitTask {
+  int w0, rn;
+  int np, r0;  // the first np rows are pivot rows, with right-hand side rows r0 ..
 };
 
 struct DevSym {
@@ -37,7 +68,7 @@ struct DevSym {
   const int* chlist;
   const int* relptr;
   const int* rel;
-  const int64_t* woff;  // per-front offsets of solve work buffers (rows)
+  const int* ild;       // per-front leading dimension of the solve panel (nrow in fused levels, else ncol)
   double* dpiv;         // pivots D of the LDL^T factor by pivot column (col0[front] + column)
   // singular pivots: a pivot d_j with |d_j| <= tolf |a_jj| (a_jj the
   // original diagonal, adiag) is replaced by |a_jj| (by amax when a_jj = 0)

@@ -1,6 +1,7 @@
 // gfx950 kernels of the part reducer: element matrices, pull assembly,
 // multifrontal LDL^T (panel factorisation on VALU, trailing updates on FP64
-// MFMA), front-based multi-RHS solves and the tall-skinny reductions.
+// MFMA) and the tall-skinny reductions; the triangular solves are in
+// solve.hip.
 //
 // Front storage: the front of supernode s is an nrow x nrow column-major
 // FP64 block at pool + foff[s]; only its lower triangle is meaningful.  After
@@ -608,13 +609,13 @@ __device__ __forceinline__ void trsm_product(const T (*sF)[65], const T (*sL)[65
 // pivot array, the solves L^-1 from the inverse pool), so that other
 // workgroups of the same launch can still read it.
 template <class T>
-__device__ __forceinline__ void diag_store(T* __restrict__ Xg, double* __restrict__ dpiv, int nc, int k0, int kb,
+__device__ __forceinline__ void diag_store(T* __restrict__ Xg, double* __restrict__ dpiv, int xld, int k0, int kb,
                                            int col0, const double (&sD)[64], const double (&sX)[64][65],
                                            int* __restrict__ piv) {
   const int tid = threadIdx.x;
   for (int idx = tid; idx < 64 * 64; idx += 256) {
     const int i = idx & 63, m = idx >> 6;
-    if (i < kb && m <= i) Xg[(int64_t)(k0 + i) + (int64_t)(k0 + m) * nc] = (T)sX[i][m];
+    if (i < kb && m < kb) Xg[(int64_t)(k0 + i) + (int64_t)(k0 + m) * xld] = (T)sX[i][m];
   }
   if (tid < kb) dpiv[col0 + k0 + tid] = sD[tid];
   (void)piv;
@@ -631,7 +632,7 @@ __global__ __launch_bounds__(256) void k_diag(const FTask* __restrict__ tasks, D
   T* F = pool + S.foff[sn];
   T* Xg = ipool + ioff[sn];
   diag_block<T>(F, ld, k0, kb, sA, sX, sD, sT, S, S.col0[sn] + k0);
-  diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sD, sX, piv);
+  diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX, piv);
 }
 
 // Diagonal block and triangular solve in one launch, for panels with few
@@ -665,7 +666,7 @@ __global__ __launch_bounds__(256) void k_diag_trsm(const FTask* __restrict__ tas
   }
   diag_block<T>(F, ld, k0, kb, sA, sX, sD, sT, S, S.col0[sn] + k0);
   if (t.a < 0) {
-    diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sD, sX, piv);
+    diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX, piv);
     return;
   }
   // operand tiles in the storage type: the row tile in sA's space (every
@@ -681,7 +682,7 @@ __global__ __launch_bounds__(256) void k_diag_trsm(const FTask* __restrict__ tas
   }
   __syncthreads();
   trsm_product<T>(sF, sL, F + (int64_t)k0 * ld, ld, R0, kb, [&](int j) { return sD[j]; });
-  if (t.a == 0) diag_store<T>(Xg, S.dpiv, nc, k0, kb, S.col0[sn], sD, sX, piv);
+  if (t.a == 0) diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX, piv);
 }
 
 // k_trsm task: sn, a = 64-row tile below the diagonal block, k0 = panel.
@@ -699,17 +700,18 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
   const int R0 = k0 + kb + 64 * t.a;
   T* F = pool + S.foff[sn];
   const T* Xg = ipool + ioff[sn];
+  const int xld = S.ild[sn];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   {
     // unconditional in-bounds loads, as in k_diag_trsm; sB[j][m] = Linv_kk[j][m] (lower)
     const T* row = F + (int64_t)k0 * ld + min(R0 + lane, ld - 1);
-    const T* xrow = Xg + (int64_t)k0 * (nc + 1) + min(lane, kb - 1);
+    const T* xrow = Xg + (int64_t)k0 * (xld + 1) + min(lane, kb - 1);
     T ra[16], rb[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) {
       const int m = min(wv + 4 * q, kb - 1);
       ra[q] = row[(int64_t)m * ld];
-      rb[q] = xrow[(int64_t)m * nc];
+      rb[q] = xrow[(int64_t)m * xld];
     }
 #pragma unroll
     for (int q = 0; q < 16; q++) {
@@ -843,6 +845,7 @@ __global__ __launch_bounds__(256) void k_inv_off(const FTask* __restrict__ tasks
   const int ri = 64 * t.b, ni = min(64, nc - ri);
   const T* F = pool + S.foff[sn];
   T* X = ipool + ioff[sn];
+  const int xld = S.ild[sn];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
   typename MF<T>::acc acc[2][2];
@@ -859,7 +862,7 @@ __global__ __launch_bounds__(256) void k_inv_off(const FTask* __restrict__ tasks
       // sB[c][m] = X[rk+m][rj+c]  (transposed, lower part only on the diagonal tile)
       const int c = idx >> 6, mm = idx & 63;
       const bool ok = c < nj && mm < nk && (kt > t.a || mm >= c);
-      rb[q] = ok ? X[(int64_t)(rk + mm) + (int64_t)(rj + c) * nc] : (T)0;
+      rb[q] = ok ? X[(int64_t)(rk + mm) + (int64_t)(rj + c) * xld] : (T)0;
     }
   };
   load(t.a);
@@ -885,7 +888,7 @@ __global__ __launch_bounds__(256) void k_inv_off(const FTask* __restrict__ tasks
       for (int r = 0; r < 4; r++) sB[wc + 16 * y + MF<T>::col(lk, r)][wr + 16 * x + lr] = acc[x][y][r];
   for (int idx = tid; idx < 64 * 64; idx += 256) {
     int r = idx & 63, m = idx >> 6;
-    sA[r][m] = (r < ni && m < ni && r >= m) ? X[(int64_t)(ri + r) + (int64_t)(ri + m) * nc] : (T)0;
+    sA[r][m] = (r < ni && m < ni && r >= m) ? X[(int64_t)(ri + r) + (int64_t)(ri + m) * xld] : (T)0;
   }
   __syncthreads();
   zero_acc(acc);
@@ -897,7 +900,7 @@ __global__ __launch_bounds__(256) void k_inv_off(const FTask* __restrict__ tasks
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int i = wr + 16 * x + lr, c = wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ni && c < nj) X[(int64_t)(ri + i) + (int64_t)(rj + c) * nc] = -acc[x][y][r];
+        if (i < ni && c < nj) X[(int64_t)(ri + i) + (int64_t)(rj + c) * xld] = -acc[x][y][r];
       }
 }
 
@@ -918,6 +921,7 @@ __global__ __launch_bounds__(256) void k_inv_part(const FTask* __restrict__ task
   const int ri = 64 * t.b, ni = min(64, nc - ri);
   const T* F = pool + S.foff[sn];
   const T* X = ipool + ioff[sn];
+  const int xld = S.ild[sn];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
   const int kend = min(t.k0 + INV_CHUNK, t.b);
@@ -932,7 +936,7 @@ __global__ __launch_bounds__(256) void k_inv_part(const FTask* __restrict__ task
       ra[q] = (r < ni && m < nk) ? F[(int64_t)(ri + r) + (int64_t)(rk + m) * ld] : (T)0;
       const int c = idx >> 6, mm = idx & 63;
       const bool ok = c < nj && mm < nk && (kt > t.a || mm >= c);
-      rb[q] = ok ? X[(int64_t)(rk + mm) + (int64_t)(rj + c) * nc] : (T)0;
+      rb[q] = ok ? X[(int64_t)(rk + mm) + (int64_t)(rj + c) * xld] : (T)0;
     }
   };
   load(t.k0);
@@ -968,6 +972,7 @@ __global__ __launch_bounds__(1024) void k_inv_fin(const FTask* __restrict__ task
   const int rj = 64 * t.a, nj = min(64, nc - rj);
   const int ri = 64 * t.b, ni = min(64, nc - ri);
   T* X = ipool + ioff[sn];
+  const int xld = S.ild[sn];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   // sum of the partials (slot order) for four entries per thread, every
   // slot's loads issued before the additions; X_ii lower -> sA
@@ -999,7 +1004,7 @@ __global__ __launch_bounds__(1024) void k_inv_fin(const FTask* __restrict__ task
       const int idx = tid + 1024 * e, m = idx >> 6, c = idx & 63;  // T[m][c] -> sB[c][m]
       sB[c][m] = v[e];
       const int r = idx & 63, mm = idx >> 6;  // X_ii lower -> sA[r][mm]
-      sA[r][mm] = (r < ni && mm < ni && r >= mm) ? X[(int64_t)(ri + r) + (int64_t)(ri + mm) * nc] : (T)0;
+      sA[r][mm] = (r < ni && mm < ni && r >= mm) ? X[(int64_t)(ri + r) + (int64_t)(ri + mm) * xld] : (T)0;
     }
   }
   __syncthreads();
@@ -1015,261 +1020,83 @@ __global__ __launch_bounds__(1024) void k_inv_fin(const FTask* __restrict__ task
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int i = wr + 16 * x + lr, c = wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ni && c < nj) X[(int64_t)(ri + i) + (int64_t)(rj + c) * nc] = -acc[x][y][r];
+        if (i < ni && c < nj) X[(int64_t)(ri + i) + (int64_t)(rj + c) * xld] = -acc[x][y][r];
       }
 }
 
-// ---------------------------------------------------------------- solves
-// Multi-vectors are row-major (rows x nrhs).  Work buffer W holds, for front
-// s, rows woff[s] .. woff[s]+nrow[s]-1; V holds the solved pivot rows before
-// D-scaling.  A k_mv task multiplies target rows r0..r0+rn-1 (rn <= 64) and
-// right-hand sides j0..j0+63 of front sn over the source slice k0..k0+kn-1:
-//   mode 0 FW_INV : V[r]      =  sum_{k<=r}   Linv[r][k]   W[k]
-//   mode 1 FW_UPD : W[nc+r]  -=  sum_{k<nc}   L[nc+r][k]   V[k]
-//   mode 2 BW_UPD : W[r]     -=  sum_{k<nu}   L[nc+k][r]   X[rows[nc+k]]
-//   mode 3 BW_INV : X[c0+r]   =  sum_{k>=r}   Linv[k][r]   W[k]
-// Long K ranges are split over several tasks (slot >= 0) whose 64x64
-// partials k_mv_red then sums in slot order (for the forward update rows
-// with at most 64 right-hand sides, the parent's k_fw_init does), so the
-// result does not depend on scheduling.
-__device__ __forceinline__ void mv_apply(int mode, const DevSym& S, int sn, int nc, int r, int j, int nrhs,
-                                         double v, double* Wf, double* Vf, double* X) {
-  switch (mode) {
-    case 0: Vf[(int64_t)r * nrhs + j] = v; break;
-    case 1: Wf[(int64_t)(nc + r) * nrhs + j] -= v; break;
-    case 2: Wf[(int64_t)r * nrhs + j] -= v; break;
-    default: X[(int64_t)(S.col0[sn] + r) * nrhs + j] = v; break;
-  }
-}
-
-template <int MODE, int NJ, class T>
-__global__ __launch_bounds__(256) void k_mv(const SolveTask* __restrict__ tasks, DevSym S,
-                                            const T* __restrict__ pool, const int64_t* __restrict__ ioff,
-                                            const T* __restrict__ ipool, double* __restrict__ W,
-                                            double* __restrict__ V, double* __restrict__ X,
-                                            double* __restrict__ part, int nrhs) {
-  constexpr int CH = 32;            // K chunk staged in LDS (small tiles: more workgroups per CU)
-  __shared__ double sA[64][CH + 1];
-  __shared__ double sB[NJ][CH + 1];  // B tile transposed: sB[j][k]
-  const SolveTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
-  const int sn = t.sn, ld = S.nrow[sn], nc = S.ncol[sn];
-  const T* F = pool + S.foff[sn];
-  const T* Xi = ipool + ioff[sn];
-  double* Wf = W + S.woff[sn] * (int64_t)nrhs;
-  double* Vf = V + S.woff[sn] * (int64_t)nrhs;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int nj = min(NJ, nrhs - t.j0);
-  const int r0 = t.r0, rn = t.rn;
-  // B rows: mode 1 the solved pivot rows V, mode 2 the final solution rows
-  // of the front's update rows (X[rows[nc + k]]), modes 0 and 3 W
-  const double* Bsrc = MODE == 1 ? Vf : Wf;
-  const int* urows = S.rows + S.rptr[sn] + nc;
-  constexpr bool rowmajorA = (MODE == 0 || MODE == 1);
-  constexpr int NT = NJ / 16;   // 16x16 MFMA result tiles per wave: rows 16 wv .. 16 wv + 15, all NJ columns
-  constexpr int BPT = NJ * CH / 256;  // B-tile values loaded per thread (CH x NJ tile)
-  f64x4 acc[NT];
-#pragma unroll
-  for (int y = 0; y < NT; y++) acc[y] = f64x4{0.0, 0.0, 0.0, 0.0};
-  const int kend = t.k0 + t.kn;
-  double ra[64 * CH / 256], rb[BPT];
-  // mode 2: the X row of each B value this thread loads, fetched one chunk
-  // ahead of the B loads that use them
-  int ur[BPT];
-  auto load_rows = [&](int kc) {
-#pragma unroll
-    for (int q = 0; q < BPT; q++) {
-      const int kb = (tid + 256 * q) / NJ;
-      ur[q] = kc + kb < kend ? urows[kc + kb] : 0;
-    }
-  };
-  if (MODE == 2) load_rows(t.k0);
-  // global loads of the CH-wide chunk starting at kc (zero outside the task)
-  auto load = [&](int kc) {
-    const int kn = min(CH, kend - kc);
-#pragma unroll
-    for (int q = 0; q < 64 * CH / 256; q++) {
-      const int idx = tid + 256 * q;
-      const int i = rowmajorA ? (idx & 63) : (idx / CH);
-      const int k = rowmajorA ? (idx >> 6) : (idx % CH);
-      const int r = r0 + i, kk = kc + k;
-      double v = 0.0;
-      if (i < rn && k < kn) {
-        if (MODE == 0) v = kk <= r ? (double)Xi[(int64_t)r + (int64_t)kk * nc] : 0.0;
-        else if (MODE == 1) v = F[(int64_t)(nc + r) + (int64_t)kk * ld];
-        else if (MODE == 2) v = F[(int64_t)(nc + kk) + (int64_t)r * ld];
-        else v = kk >= r ? (double)Xi[(int64_t)kk + (int64_t)r * nc] : 0.0;
-      }
-      ra[q] = v;
-    }
-#pragma unroll
-    for (int q = 0; q < BPT; q++) {
-      const int idx = tid + 256 * q, kb = idx / NJ, jb = idx % NJ;
-      if (MODE == 2) rb[q] = (kb < kn && jb < nj) ? X[(int64_t)ur[q] * nrhs + t.j0 + jb] : 0.0;
-      else rb[q] = (kb < kn && jb < nj) ? Bsrc[(int64_t)(kc + kb) * nrhs + t.j0 + jb] : 0.0;
-    }
-    if (MODE == 2) load_rows(kc + CH);
-  };
-  if (t.k0 < kend) load(t.k0);
-  for (int kc = t.k0; kc < kend; kc += CH) {
-    const int kn = min(CH, kend - kc);
-    __syncthreads();  // the previous chunk's products are done with the LDS tiles
-#pragma unroll
-    for (int q = 0; q < 64 * CH / 256; q++) {
-      const int idx = tid + 256 * q;
-      const int i = rowmajorA ? (idx & 63) : (idx / CH);
-      const int k = rowmajorA ? (idx >> 6) : (idx % CH);
-      sA[i][k] = ra[q];
-    }
-#pragma unroll
-    for (int q = 0; q < BPT; q++) {
-      const int idx = tid + 256 * q;
-      sB[idx % NJ][idx / NJ] = rb[q];
-    }
-    __syncthreads();
-    // the next chunk's loads are in flight while this one is multiplied
-    if (kc + CH < kend) load(kc + CH);
-    // v_mfma_f64_16x16x4f64 over k in steps of 4 (sA and sB are zero beyond
-    // kn and nj): the A operand takes the sB rows (columns j), the B operand
-    // the sA rows (target rows), as in mfma_tile
-    const int lr = lane & 15, lk = lane >> 4;
-    for (int m0 = 0; m0 < kn; m0 += 4) {
-      const double aa = sA[16 * wv + lr][m0 + lk];
-#pragma unroll
-      for (int y = 0; y < NT; y++)
-        acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[16 * y + lr][m0 + lk], aa, acc[y], 0, 0, 0);
-    }
-  }
-  // lane holds target row 16 wv + (lane & 15), columns 16 y + (lane >> 4) + 4 r
-  const int i = 16 * wv + (lane & 15), lk = lane >> 4;
-  if (t.slot >= 0) {
-    double* P = part + (int64_t)t.slot * 4096;
-#pragma unroll
-    for (int y = 0; y < NT; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) P[i * 64 + 16 * y + lk + 4 * r] = acc[y][r];
-    return;
-  }
-  if (i >= rn) return;
-#pragma unroll
-  for (int y = 0; y < NT; y++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int jj = 16 * y + lk + 4 * r;
-      if (jj < nj) mv_apply(MODE, S, sn, nc, r0 + i, t.j0 + jj, nrhs, acc[y][r], Wf, Vf, X);
-    }
-}
-
-// Reduce task: slots k0 .. k0+kn-1 hold the partials of rows r0.. (rn) and
-// right-hand sides j0.. of front sn; sum them in slot order and apply.
-__global__ __launch_bounds__(1024) void k_mv_red(const SolveTask* __restrict__ tasks, DevSym S,
-                                                double* __restrict__ W, double* __restrict__ V,
-                                                double* __restrict__ X, const double* __restrict__ part,
-                                                int nrhs, int mode) {
-  const SolveTask t = tasks[blockIdx.x];
-  const int sn = t.sn, nc = S.ncol[sn];
-  double* Wf = W + S.woff[sn] * (int64_t)nrhs;
-  double* Vf = V + S.woff[sn] * (int64_t)nrhs;
-  const int nj = min(64, nrhs - t.j0);
-  for (int idx = threadIdx.x; idx < t.rn * nj; idx += blockDim.x) {
-    const int i = idx / nj, jj = idx % nj;
-    const double* p = part + (int64_t)t.k0 * 4096 + i * 64 + jj;
-    // slots summed in order; the loads of four slots are issued together
-    double v = 0.0;
-    int q = 0;
-    for (; q + 3 < t.kn; q += 4) {
-      const double a0 = p[(int64_t)q * 4096], a1 = p[(int64_t)(q + 1) * 4096];
-      const double a2 = p[(int64_t)(q + 2) * 4096], a3 = p[(int64_t)(q + 3) * 4096];
-      v += a0;
-      v += a1;
-      v += a2;
-      v += a3;
-    }
-    for (; q < t.kn; q++) v += p[(int64_t)q * 4096];
-    mv_apply(mode, S, sn, nc, t.r0 + i, t.j0 + jj, nrhs, v, Wf, Vf, X);
-  }
-}
-
-// Forward-solve front initialisation, task = (front, 64-row chunk r0): pivot
-// rows from the global right-hand side R (row-major, perm rows; the Schur
-// front takes the boundary rows), update rows zero, plus the children's
-// update rows that land in each row.  Work row w adds the rows
-// gsrc[gptr[w]] .. gsrc[gptr[w+1]-1] of W in child order.  A gathered row
-// whose update product was split (ugrp[row] = g >= 0) is completed here:
-// W row minus the sum of its group's partials in slot order (group g:
-// first slot, slot count, first work row of the tile at ugroups[3 g ..]).
-__global__ __launch_bounds__(1024) void k_fw_init(const SolveTask* __restrict__ tasks, DevSym S,
-                                                 const int* __restrict__ gptr, const int* __restrict__ gsrc,
-                                                 const int* __restrict__ ugrp, const int* __restrict__ ugroups,
-                                                 const double* __restrict__ part, const double* __restrict__ R,
-                                                 double* __restrict__ W, int nrhs, int ndof1) {
-  const SolveTask t = tasks[blockIdx.x];
-  const int sn = t.sn, nc = S.ncol[sn], c0 = S.col0[sn];
-  const int64_t wo = S.woff[sn];
-  double* Wf = W + wo * nrhs;
-  const int base = nc > 0 ? c0 : ndof1;
-  for (int idx = threadIdx.x; idx < t.rn * nrhs; idx += blockDim.x) {
-    const int i = t.r0 + idx / nrhs, j = idx % nrhs;
-    double v = 0.0;
-    if (i < nc || nc == 0) v = R[(int64_t)(base + i) * nrhs + j];
-    const int e1 = gptr[wo + i + 1];
-    for (int e = gptr[wo + i]; e < e1; e++) {
-      const int w = gsrc[e];
-      double t = W[(int64_t)w * nrhs + j];
-      const int g = ugrp ? ugrp[w] : -1;
-      if (g >= 0) {
-        const int first = ugroups[3 * g], ns = ugroups[3 * g + 1], w0 = ugroups[3 * g + 2];
-        const double* p = part + (int64_t)first * 4096 + (w - w0) * 64 + j;
-        double sum = 0.0;
-        int q = 0;
-        for (; q + 3 < ns; q += 4) {
-          const double a0 = p[(int64_t)q * 4096], a1 = p[(int64_t)(q + 1) * 4096];
-          const double a2 = p[(int64_t)(q + 2) * 4096], a3 = p[(int64_t)(q + 3) * 4096];
-          sum += a0;
-          sum += a1;
-          sum += a2;
-          sum += a3;
-        }
-        for (; q < ns; q++) sum += p[(int64_t)q * 4096];
-        t -= sum;
-      }
-      v += t;
-    }
-    Wf[(int64_t)i * nrhs + j] = v;
-  }
-}
-
-// Copy solved rows out to Y, task = (front, 64-row chunk): internal fronts
-// give their pivot rows (V, optionally scaled by 1/D), the Schur front its
-// rows (W) to the boundary rows of Y.
+// Y21 = -L21 L11^-1 of a fused front, below L11^-1 in its solve panel, after
+// every inverse tile.  Task: sn, a = 64-column tile j, b = 64-row tile i of
+// the update rows: Y_ij = -sum_{k >= 64 j} L_ik X_kj.  Each wave forms a 32 x
+// 32 quarter with both operands straight from memory (rows of L contiguous;
+// X along k: each lane takes the VK neighbouring k of 16 bytes, step m of a
+// 4 VK-chunk multiplies k = VK (lane / 16) + m), one chunk ahead of its
+// products.
 template <class T>
-__global__ __launch_bounds__(256) void k_fw_out(const SolveTask* __restrict__ tasks, DevSym S,
-                                                const T* __restrict__ pool,
-                                                const double* __restrict__ W, const double* __restrict__ V,
-                                                double* __restrict__ Y, int nrhs, int scale, int ndof1) {
-  const SolveTask t = tasks[blockIdx.x];
-  const int sn = t.sn, nc = S.ncol[sn], c0 = S.col0[sn];
-  (void)pool;  // the storage type of the factor sets the rounding of the pivots
-  const double* Wf = (nc > 0 ? V : W) + S.woff[sn] * (int64_t)nrhs;
-  const int base = nc > 0 ? c0 : ndof1;
-  for (int idx = threadIdx.x; idx < t.rn * nrhs; idx += 256) {
-    const int i = t.r0 + idx / nrhs, j = idx % nrhs;
-    double v = Wf[(int64_t)i * nrhs + j];
-    if (scale && nc > 0) v /= (double)(T)S.dpiv[c0 + i];
-    Y[(int64_t)(base + i) * nrhs + j] = v;
+__global__ __launch_bounds__(256) void k_panel(const FTask* __restrict__ tasks, DevSym S, const T* __restrict__ pool,
+                                               const int64_t* __restrict__ ioff, T* __restrict__ ipool) {
+  const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const int sn = t.sn, ld = S.nrow[sn], nc = S.ncol[sn], nu = ld - nc;
+  const T* F = pool + S.foff[sn] + nc;
+  T* Z = ipool + ioff[sn];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int i0 = 64 * t.b + (wv >> 1) * 32, j0 = 64 * t.a + (wv & 1) * 32;
+  if (i0 >= nu || j0 >= nc) return;
+  const T *Fr[2], *Xc[2];
+#pragma unroll
+  for (int x = 0; x < 2; x++) {
+    Fr[x] = F + min(i0 + 16 * x + lr, nu - 1);
+    Xc[x] = Z + (int64_t)min(j0 + 16 * x + lr, nc - 1) * ld;
   }
-}
-
-// Backward-solve front initialisation, task = (front, 64-row chunk of the
-// pivot rows): pivot rows from Y (zero when Y is null).
-__global__ __launch_bounds__(256) void k_bw_init(const SolveTask* __restrict__ tasks, DevSym S,
-                                                 const double* __restrict__ Y, double* __restrict__ W, int nrhs) {
-  const SolveTask t = tasks[blockIdx.x];
-  const int sn = t.sn, c0 = S.col0[sn];
-  double* Wf = W + S.woff[sn] * (int64_t)nrhs;
-  for (int idx = threadIdx.x; idx < t.rn * nrhs; idx += 256) {
-    const int i = t.r0 + idx / nrhs, j = idx % nrhs;
-    Wf[(int64_t)i * nrhs + j] = Y ? Y[(int64_t)(c0 + i) * nrhs + j] : 0.0;
+  constexpr int VK = 16 / sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(VK), aligned(sizeof(T))));
+  struct Stage {
+    T a[4][2], b[4][2];
+  };
+  auto kof = [&](int kc, int s) { return kc + 4 * VK * (s / VK) + VK * lk + s % VK; };
+  auto load = [&](int kc, Stage& g) {
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+#pragma unroll
+      for (int s = 0; s < 4; s += VK) {
+        const vec v = *(const vec*)(Xc[x] + min(kof(kc, s), nc - 1));
+#pragma unroll
+        for (int m = 0; m < VK; m++) g.b[s + m][x] = v[m];
+      }
+#pragma unroll
+      for (int s = 0; s < 4; s++) g.a[s][x] = Fr[x][(int64_t)min(kof(kc, s), nc - 1) * ld];
+    }
+  };
+  typename MF<T>::acc acc[2][2];
+  zero_acc(acc);
+  auto multiply = [&](int kc, const Stage& g) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const bool in = kof(kc, s) < nc;
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int y = 0; y < 2; y++) acc[x][y] = MF<T>::op(in ? g.b[s][y] : (T)0, in ? g.a[s][x] : (T)0, acc[x][y]);
+    }
+  };
+  Stage g0, g1;
+  const int kb = 64 * t.a;
+  load(kb, g0);
+  for (int kc = kb; kc < nc; kc += 32) {
+    if (kc + 16 < nc) load(kc + 16, g1);
+    multiply(kc, g0);
+    if (kc + 16 >= nc) break;
+    if (kc + 32 < nc) load(kc + 32, g0);
+    multiply(kc + 16, g1);
   }
+#pragma unroll
+  for (int x = 0; x < 2; x++)
+#pragma unroll
+    for (int y = 0; y < 2; y++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int i = i0 + 16 * x + lr, j = j0 + 16 * y + MF<T>::col(lk, r);
+        if (i < nu && j < nc) Z[(int64_t)nc + i + (int64_t)j * ld] = -acc[x][y][r];
+      }
 }
 
 // ---------------------------------------------------------------- products
@@ -2035,42 +1862,13 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
                       T* ipool, const T* ipart) {                                                          \
     if (n > 0) k_inv_fin<T><<<n, 1024, 0, st>>>(t, S, ioff, ipool, ipart);                                    \
   }                                                                                                        \
-  void launch_mv(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const T* pool,                \
-                 const int64_t* ioff, const T* ipool, double* W, double* V, double* X, double* part,       \
-                 int nrhs, int mode) {                                                                     \
-    if (n <= 0) return;                                                                                    \
-    switch (mode * 2 + (nrhs <= 16 ? 0 : 1)) {                                                             \
-      case 0: k_mv<0, 16, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      case 1: k_mv<0, 64, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      case 2: k_mv<1, 16, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      case 3: k_mv<1, 64, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      case 4: k_mv<2, 16, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      case 5: k_mv<2, 64, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      case 6: k_mv<3, 16, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;      \
-      default: k_mv<3, 64, T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, W, V, X, part, nrhs); break;     \
-    }                                                                                                      \
-  }                                                                                                        \
-  void launch_fw_out(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const T* pool,            \
-                     const double* W, const double* V, double* Y, int nrhs, int scale, int ndof1) {        \
-    if (n > 0) k_fw_out<T><<<n, 256, 0, st>>>(t, S, pool, W, V, Y, nrhs, scale, ndof1);                      \
+  void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                 \
+                    const int64_t* ioff, T* ipool) {                                                       \
+    if (n > 0) k_panel<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                       \
   }
 FGPU_FACTOR_LAUNCHERS(double)
 FGPU_FACTOR_LAUNCHERS(float)
 #undef FGPU_FACTOR_LAUNCHERS
-void launch_mv_red(hipStream_t st, const SolveTask* t, int n, const DevSym& S, double* W, double* V, double* X,
-                   const double* part, int nrhs, int mode) {
-  if (n > 0) k_mv_red<<<n, nrhs <= 16 ? 64 * nrhs : 1024, 0, st>>>(t, S, W, V, X, part, nrhs, mode);
-}
-void launch_fw_init(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const int* gptr, const int* gsrc,
-                    const int* ugrp, const int* ugroups, const double* part, const double* R, double* W, int nrhs,
-                    int ndof1) {
-  if (n > 0)
-    k_fw_init<<<n, nrhs <= 16 ? 64 * nrhs : 1024, 0, st>>>(t, S, gptr, gsrc, ugrp, ugroups, part, R, W, nrhs, ndof1);
-}
-void launch_bw_init(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const double* Y, double* W,
-                    int nrhs) {
-  if (n > 0) k_bw_init<<<n, 256, 0, st>>>(t, S, Y, W, nrhs);
-}
 void launch_spmm(hipStream_t st, int n, int nrhs, const int* rowptr, const int* colind, const double* val,
                  const double* X, int ldx, double* Z, int ldz, bool skip_zeros) {
   if (n > 0 && nrhs > 0) {

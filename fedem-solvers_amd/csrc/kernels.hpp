@@ -80,22 +80,18 @@ constexpr int INV_CHUNK = 4;
                        const int64_t* ioff, const T* ipool, T* ipart);                                    \
   void launch_inv_fin(hipStream_t st, const FTask* t, int n, const DevSym& S, const int64_t* ioff,        \
                       T* ipool, const T* ipart);                                                          \
-  /* solve GEMM tasks, mode 0 FW_INV, 1 FW_UPD, 2 BW_UPD, 3 BW_INV */                                     \
-  void launch_mv(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const T* pool,               \
-                 const int64_t* ioff, const T* ipool, double* W, double* V, double* X, double* part,      \
-                 int nrhs, int mode);                                                                     \
-  void launch_fw_out(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const T* pool,           \
-                     const double* W, const double* V, double* Y, int nrhs, int scale, int ndof1);
+  /* Y21 = -L21 L11^-1 of the fused levels below L11^-1 (solve panels) */                               \
+  void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                \
+                    const int64_t* ioff, T* ipool);                                                       \
+  /* solve products (solve.hip): nt 16-column groups of right-hand sides per task, kw K parts */         \
+  void launch_mv(hipStream_t st, const MvTask* t, int n, int kind, int nt, int kw, const T* pool,         \
+                 const T* panel, const int* rows, const double* dpiv, double* W, double* V,               \
+                 const double* R, double* Y, double* X, int nrhs);
 FGPU_FACTOR_DECLS(double)
 FGPU_FACTOR_DECLS(float)
 #undef FGPU_FACTOR_DECLS
-void launch_mv_red(hipStream_t st, const SolveTask* t, int n, const DevSym& S, double* W, double* V, double* X,
-                   const double* part, int nrhs, int mode);
-void launch_fw_init(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const int* gptr, const int* gsrc,
-                    const int* ugrp, const int* ugroups, const double* part, const double* R, double* W, int nrhs,
-                    int ndof1);
-void launch_bw_init(hipStream_t st, const SolveTask* t, int n, const DevSym& S, const double* Y, double* W,
-                    int nrhs);
+void launch_fw_init(hipStream_t st, const InitTask* t, int n, const int* gptr, const int* gsrc, const double* R,
+                    double* W, int nrhs);
 void launch_spmm(hipStream_t st, int n, int nrhs, const int* rowptr, const int* colind, const double* val,
                  const double* X, int ldx, double* Z, int ldz,
                  bool skip_zeros = false);

@@ -110,34 +110,35 @@ struct HBuf {
 };
 
 enum OpKind {
-  EXTADD, DIAG, TRSM, DIAG_TRSM, UPDATE, INV_OFF, INV_PART, INV_FIN,
+  EXTADD, DIAG, TRSM, DIAG_TRSM, UPDATE, INV_OFF, INV_PART, INV_FIN, PANEL,
   UPDATE_SIDE, FORK, JOIN,  // lookahead: trailing tiles on the side stream, fork/join with the main one
-  FW_INIT, FW_INV, FW_UPD, FW_OUT, BW_INIT, BW_UPD, BW_INV,
-  FW_INV_R, FW_UPD_R, BW_UPD_R, BW_INV_R  // ordered reductions of split-K partials
+  FW_INIT, FW_MV, BW_ROWS, BW_MV  // solve plans
 };
 struct Op {
   int kind, off, n;
+  int kw = 1;  // solve products: K parts per workgroup
+};
+
+// Where the solve panels lie and which levels are fused (solve.hip).
+struct SolveLayout {
+  std::vector<char> fused;    // per level
+  std::vector<int64_t> ioff;  // per front (nsup + 1)
+  std::vector<int> ild;       // per front
+  bool unfused = false;       // some level with fronts is not fused (its solves need V)
 };
 
 struct SolvePlan {
   bool valid = false;  // built for the current structure
-  int nrhs = 0;
-  int nslots = 0;  // 64x64 partial buffers of the split-K solve tasks
-  std::vector<Op> fw_int, fw_all, bw;
-  DBuf<SolveTask> tasks;
-  DBuf<int> gptr, gsrc;  // forward init: the child update rows added to each work row, in child order
-  // Split-K update-row products of the forward pass (nrhs <= 64) are reduced
-  // by the parent's forward init as it gathers the rows: ugrp_int/ugrp_all
-  // (per work row, -1: none) index the groups (first slot, slots, first
-  // work row of the tile) of the internal-only and the full forward pass.
-  DBuf<int> ugrp_int, ugrp_all, ugroups;
-  DBuf<double> part;
+  int nrhs = 0, nt = 1;  // 16-column groups of right-hand sides per task
+  std::vector<Op> fw, bw, bw0;  // bw0: from a zero Y (displacement recovery matrix B)
+  DBuf<MvTask> tasks;
+  DBuf<InitTask> inits;
 };
 
 // Host lists of a solve plan before their upload.
 struct PlanHost {
-  std::vector<SolveTask> tasks;
-  std::vector<int> gptr, gsrc, ugrp[2], ugroups;
+  std::vector<MvTask> tasks;
+  std::vector<InitTask> inits;
 };
 
 // A captured launch sequence (HIP graph), replayed while the buffers it
@@ -187,7 +188,10 @@ struct DeviceReducer::Impl {
   DBuf<int64_t> eoff;
   // structure
   DBuf<int> col0, ncol, nrow, rptr, rows, chptr, chlist, relptr, rel, rowptr, colind, cptr, cidx;
-  DBuf<int64_t> foff, woff, fmap, ioff;
+  DBuf<int64_t> foff, fmap, ioff;
+  DBuf<int> ild;
+  SolveLayout lay;
+  DBuf<int> gptr, gsrc;  // forward init: the child update rows added to each work row, in child order
   // inputs of the device structure build: SAM arrays, element types, per
   // node first equation / equation count / neighbour lists (+ DOF offsets),
   // per row its node, per column its front
@@ -256,9 +260,41 @@ DeviceReducer::~DeviceReducer() {
   }
 }
 
-static void build_factor_schedule(const Symbolic& y, std::vector<FTask>& tasks, std::vector<Op>& ops,
-                                  std::vector<int>& xrange, double& flops, int panel, int& inv_slots,
-                                  bool lookahead) {
+// Solve panels of the fronts.  A level is fused (its Y21 = -L21 L11^-1
+// formed, one product per pass instead of two) when forming Y21 costs less
+// than the launches saved: sum nu nc^2 flops at about 40 TFLOP/s against
+// some 12 us for each pass pair, over the solves that the handle's options
+// let expect (block Lanczos 16, mixed-precision refinement 8, else B and one
+// load-case solve).
+static SolveLayout solve_layout(const Symbolic& y, const ReduceOptions& o) {
+  SolveLayout q;
+  const double nsolve = o.ngen > 0 ? 16 : o.mixed ? 8 : 2;
+  q.fused.assign(y.nlevels, 1);
+  q.ild.assign(y.nsup, 0);
+  q.ioff.assign(y.nsup + 1, 0);
+  for (int l = 0; l < y.nlevels; l++) {
+    double flops = 0.0;
+    bool any = false;
+    for (int k = y.lvptr[l]; k < y.lvptr[l + 1]; k++) {
+      const int s = y.lvsup[k];
+      const double nc = y.ncol[s], nu = y.nrow[s] - nc;
+      flops += nu * nc * nc;
+      any = any || nc > 0;
+    }
+    q.fused[l] = flops <= nsolve * 4.8e8;
+    if (any && !q.fused[l]) q.unfused = true;
+    for (int k = y.lvptr[l]; k < y.lvptr[l + 1]; k++) {
+      const int s = y.lvsup[k];
+      q.ild[s] = q.fused[l] ? y.nrow[s] : y.ncol[s];
+    }
+  }
+  for (int s = 0; s < y.nsup; s++) q.ioff[s + 1] = q.ioff[s] + (int64_t)q.ild[s] * y.ncol[s];
+  return q;
+}
+
+static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std::vector<FTask>& tasks,
+                                  std::vector<Op>& ops, std::vector<int>& xrange, double& flops, int panel,
+                                  int& inv_slots, bool lookahead) {
   xrange.clear();
   inv_slots = 0;
   flops = 0;
@@ -444,17 +480,34 @@ static void build_factor_schedule(const Symbolic& y, std::vector<FTask>& tasks, 
     }
     inv_slots = std::max(inv_slots, slot);
   }
+  // Y21 of the fused levels, long sums first
+  std::vector<FTask> pan;
+  for (int l = 0; l < y.nlevels; l++) {
+    if (!lay.fused[l]) continue;
+    for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++) {
+      const int s = y.lvsup[q], nu = y.nrow[s] - y.ncol[s];
+      for (int j = 0; 64 * j < y.ncol[s]; j++)
+        for (int i = 0; 64 * i < nu; i++) pan.push_back({s, j, i, y.ncol[s] - 64 * j, 0});
+    }
+  }
+  std::stable_sort(pan.begin(), pan.end(), [](const FTask& a, const FTask& b) { return a.k0 > b.k0; });
+  if (!pan.empty()) {
+    ops.push_back({PANEL, (int)tasks.size(), (int)pan.size()});
+    tasks.insert(tasks.end(), pan.begin(), pan.end());
+  }
 }
 
-static void build_solve_plan(const Symbolic& y, SolvePlan& sp, std::vector<SolveTask>& tasks,
-                             std::vector<int>& gptr, std::vector<int>& gsrc, std::vector<int> (&ugrp)[2],
-                             std::vector<int>& ugroups, int KSplit) {
-  const int nrhs = sp.nrhs, schur = y.nsup - 1;
-  // gather lists of the forward init: work row woff[s] + i of front s adds
-  // the update rows of s's children that land in its row i, child after
-  // child (a child adds at most one row to a parent row)
-  std::vector<int64_t> woff(y.nsup + 1, 0);
+// First work row of every front (nsup + 1 entries) and the gather lists of
+// the forward init: work row woff[s] + i of front s adds the update rows of
+// s's children that land in its row i, child after child (a child adds at
+// most one row to a parent row).
+static std::vector<int> work_rows(const Symbolic& y) {
+  std::vector<int> woff(y.nsup + 1, 0);
   for (int s = 0; s < y.nsup; s++) woff[s + 1] = woff[s] + y.nrow[s];
+  return woff;
+}
+static void build_gather(const Symbolic& y, std::vector<int>& gptr, std::vector<int>& gsrc) {
+  const std::vector<int> woff = work_rows(y);
   gptr.assign(woff[y.nsup] + 1, 0);
   for (int s = 0; s < y.nsup; s++)
     for (int q = y.chptr[s]; q < y.chptr[s + 1]; q++) {
@@ -463,121 +516,126 @@ static void build_solve_plan(const Symbolic& y, SolvePlan& sp, std::vector<Solve
       for (int k = 0; k < nu; k++) gptr[woff[s] + rel[k] + 1]++;
     }
   for (size_t i = 1; i < gptr.size(); i++) gptr[i] += gptr[i - 1];
-  gsrc.assign(gptr.back(), 0);
-  {
-    std::vector<int> fill(gptr.begin(), gptr.end() - 1);
-    for (int s = 0; s < y.nsup; s++)
-      for (int q = y.chptr[s]; q < y.chptr[s + 1]; q++) {
-        const int c = y.chlist[q], nu = y.nrow[c] - y.ncol[c];
-        const int* rel = y.rel.data() + y.relptr[c];
-        for (int k = 0; k < nu; k++) gsrc[fill[woff[s] + rel[k]]++] = (int)(woff[c] + y.ncol[c] + k);
+  gsrc.assign(std::max(1, gptr.back()), 0);
+  std::vector<int> fill(gptr.begin(), gptr.end() - 1);
+  for (int s = 0; s < y.nsup; s++)
+    for (int q = y.chptr[s]; q < y.chptr[s + 1]; q++) {
+      const int c = y.chlist[q], nu = y.nrow[c] - y.ncol[c];
+      const int* rel = y.rel.data() + y.relptr[c];
+      for (int k = 0; k < nu; k++) gsrc[fill[woff[s] + rel[k]]++] = woff[c] + y.ncol[c] + k;
+    }
+}
+
+// Solve plan for sp.nrhs right-hand sides: per level a forward init (fronts
+// with children), one product in a fused level and two in another, then the
+// levels top-down.  zero_start: also the backward pass from Y = 0.
+//
+// Right-hand sides go in groups of up to 96 columns, as even as 16-column
+// tiles allow.  A task's K range is split over the 4 waves of a workgroup
+// (the fastest split from 60 to 5544 pivot columns, see k_fw); over 16 (8
+// for wide groups) where there is at most one 4-wave workgroup per CU and a
+// wave would have more than ksplit of it; and not at all where it is short
+// or, forward, where a level of short ranges (K <= ksplit) has enough rows
+// to fill the device with 64-row tasks (24 against 28 us for 306 fronts of
+// 700 rows and 60 pivot columns).
+static void build_solve_plan(const Symbolic& y, const SolveLayout& lay, SolvePlan& sp, PlanHost& h, int ksplit,
+                             bool zero_start) {
+  const int nrhs = sp.nrhs, schur = y.nsup - 1;
+  const int ngrp = (nrhs + 95) / 96;
+  sp.nt = ((nrhs + ngrp - 1) / ngrp + 15) / 16;
+  const std::vector<int> woff = work_rows(y);
+  // one launch: (task with its whole row range, rows) pieces, cut into row tiles
+  struct Piece {
+    MvTask t;      // rn = all rows
+    int64_t da;    // operand step per target row
+    int tri;       // 1: row tile r0 takes K up to r0 + rn (lower triangle), 2: K from r0 on, 0: all
+  };
+  auto cut = [&](std::vector<Op>& ops, int kind, const std::vector<Piece>& ps) {
+    int64_t t16 = 0;
+    int kmax = 0;
+    for (const Piece& p : ps) {
+      t16 += (p.t.rn + 15) / 16 * ngrp;
+      kmax = std::max(kmax, p.t.kn);
+    }
+    const bool wide = kind == FW_MV && t16 >= 4096 && kmax <= ksplit;
+    Op op{kind, (int)h.tasks.size(), 0, 4};
+    if (wide || kmax <= 32) op.kw = 1;
+    else if (t16 <= 256 && kmax > 4 * ksplit) op.kw = 16;
+    const int rt = op.kw == 1 && kind == FW_MV ? 64 : 16;
+    for (const Piece& p : ps)
+      for (int r0 = 0; r0 < p.t.rn; r0 += rt) {
+        MvTask t = p.t;
+        t.rn = std::min(rt, p.t.rn - r0);
+        t.a += p.da * r0;
+        t.dst += r0;
+        if (t.dst2 >= 0) t.dst2 += r0;
+        if (p.tri == 1) t.kn = std::min(t.kn, r0 + t.rn);
+        if (p.tri == 2) {
+          const int step = std::min(r0, t.kn);
+          t.a += step;
+          t.src += step;
+          t.ky -= std::min(step, t.ky);
+          t.kn -= step;
+        }
+        for (int g = 0; g < ngrp; g++) {
+          t.j0 = 16 * sp.nt * g;
+          if (t.j0 < nrhs) h.tasks.push_back(t);
+        }
       }
+    op.n = (int)h.tasks.size() - op.off;
+    if (op.n > 0) ops.push_back(op);
+  };
+  for (int l = 0; l < y.nlevels; l++) {
+    const int i0 = (int)h.inits.size();
+    std::vector<Piece> first, second;
+    for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++) {
+      const int s = y.lvsup[q];
+      if (s == schur) continue;
+      const int nc = y.ncol[s], nu = y.nrow[s] - nc, ld = lay.ild[s];
+      const bool leaf = y.chptr[s + 1] == y.chptr[s], up = y.parent[s] != schur && y.parent[s] >= 0;
+      // rows that only the boundary would take are not formed
+      const int rows = up ? y.nrow[s] : nc;
+      if (!leaf)
+        for (int r0 = 0; r0 < rows; r0 += 64)
+          h.inits.push_back({woff[s] + r0, std::min(64, rows - r0), std::max(0, std::min(64, nc - r0)), y.col0[s] + r0});
+      const int from = leaf ? y.col0[s] : woff[s], ff = leaf ? MV_SRC_R : 0;
+      if (lay.fused[l]) {
+        if (up)
+          first.push_back({{lay.ioff[s] + nc, ld, nu, nc, from, 0, woff[s] + nc, -1, ff | (leaf ? MV_SET : MV_ADD), 0, 0}, 1, 0});
+        first.push_back({{lay.ioff[s], ld, nc, nc, from, 0, y.col0[s], -1, ff | MV_Y, 0, 0}, 1, 1});
+      } else {
+        first.push_back({{lay.ioff[s], ld, nc, nc, from, 0, y.col0[s], up ? woff[s] : -1, ff | MV_Y, 0, 0}, 1, 1});
+        if (up)
+          second.push_back({{y.foff[s] + nc, y.nrow[s], nu, nc, woff[s], 0, woff[s] + nc, -1,
+                             MV_FRONT | MV_SRC_V | (leaf ? MV_NEG : MV_SUB), 0, 0}, 1, 0});
+      }
+    }
+    if ((int)h.inits.size() > i0) sp.fw.push_back({FW_INIT, i0, (int)h.inits.size() - i0});
+    cut(sp.fw, FW_MV, first);
+    cut(sp.fw, FW_MV, second);
   }
-  // (front, 64-row chunk) tasks over all rows (forward init), the solved
-  // rows (forward output, the Schur front: all its rows) or the pivot rows
-  // (backward init)
-  auto add_sns = [&](std::vector<Op>& ops, int kind, const std::vector<int>& list) {
-    int off = (int)tasks.size();
-    for (int s : list) {
-      const bool piv = (kind == FW_OUT && s != schur) || kind == BW_INIT;
-      const int nr = piv ? y.ncol[s] : y.nrow[s];
-      for (int r0 = 0; r0 < nr; r0 += 64) tasks.push_back({s, r0, std::min(64, nr - r0), 0, 0, 0, -1, 0});
-    }
-    if ((int)tasks.size() > off) ops.push_back({kind, off, (int)tasks.size() - off});
-  };
-  // GEMM tasks over the row tiles of a front and all right-hand-side tiles;
-  // K ranges longer than KS are split and reduced in slot order
-  const bool fuse_upd = nrhs <= 64;
-  ugroups.clear();
-  for (auto& u : ugrp) u.assign(woff[y.nsup], -1);
-  int pass = 0;  // forward pass being built (0: internal fronts only, 1: all)
-  auto add_tiles = [&](std::vector<Op>& ops, int kind, const std::vector<int>& list, bool upd_rows) {
-    const int mode = kind == FW_INV ? 0 : kind == FW_UPD ? 1 : kind == BW_UPD ? 2 : 3;
-    // an op with enough unsplit tasks to fill the device is not split
-    int64_t ntask = 0;
-    for (int s : list) {
-      const int nc = y.ncol[s], nu = y.nrow[s] - nc;
-      if (kind == BW_UPD && nu == 0) continue;
-      ntask += (int64_t)((upd_rows ? nu : nc) + 63) / 64 * ((nrhs + 63) / 64);
-    }
-    const int KS = ntask >= 1024 ? INT_MAX : KSplit;
-    const int rkind = kind == FW_INV ? FW_INV_R : kind == FW_UPD ? FW_UPD_R : kind == BW_UPD ? BW_UPD_R : BW_INV_R;
-    std::vector<SolveTask> red;
-    int off = (int)tasks.size();
-    for (int s : list) {
-      const int nc = y.ncol[s], nu = y.nrow[s] - nc;
-      int nr = upd_rows ? nu : nc;
-      if (kind == BW_UPD && nu == 0) continue;
-      for (int r0 = 0; r0 < nr; r0 += 64) {
-        const int rn = std::min(64, nr - r0);
-        int kb = 0, ke = 0;
-        switch (mode) {
-          case 0: kb = 0; ke = r0 + rn; break;
-          case 1: kb = 0; ke = nc; break;
-          case 2: kb = 0; ke = nu; break;
-          default: kb = r0; ke = nc; break;
-        }
-        for (int j0 = 0; j0 < nrhs; j0 += 64) {
-          if (ke - kb <= KS) {
-            tasks.push_back({s, r0, rn, kb, ke - kb, j0, -1, 0});
-            continue;
-          }
-          int first = sp.nslots;
-          for (int k = kb; k < ke; k += KS) tasks.push_back({s, r0, rn, k, std::min(KS, ke - k), j0, sp.nslots++, 0});
-          if (mode == 1 && fuse_upd && pass < 2) {
-            const int w0 = (int)(woff[s] + nc + r0), g = (int)ugroups.size() / 3;
-            ugroups.insert(ugroups.end(), {first, sp.nslots - first, w0});
-            for (int i = 0; i < rn; i++) ugrp[pass][w0 + i] = g;
-            continue;
-          }
-          red.push_back({s, r0, rn, first, sp.nslots - first, j0, -2, 0});
-        }
-      }
-    }
-    if ((int)tasks.size() > off) ops.push_back({kind, off, (int)tasks.size() - off});
-    if (!red.empty()) {
-      off = (int)tasks.size();
-      tasks.insert(tasks.end(), red.begin(), red.end());
-      ops.push_back({rkind, off, (int)red.size()});
-    }
-  };
-  // forward: levels bottom-up; fw_all also carries the Schur front.  The
-  // solved pivot rows of a front stay in V, so one output launch after the
-  // last level copies them all.
-  for (pass = 0; pass < 2; pass++) {
-    std::vector<Op>& ops = pass == 0 ? sp.fw_int : sp.fw_all;
-    std::vector<int> all;
-    for (int l = 0; l < y.nlevels; l++) {
-      std::vector<int> list, ilist;
+  for (int z = 0; z < (zero_start ? 2 : 1); z++) {
+    std::vector<Op>& ops = z ? sp.bw0 : sp.bw;
+    for (int l = y.nlevels - 1; l >= 0; l--) {
+      std::vector<Piece> first, second;
       for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++) {
-        int s = y.lvsup[q];
-        if (s == schur && pass == 0) continue;
-        list.push_back(s);
-        if (s != schur) ilist.push_back(s);
+        const int s = y.lvsup[q];
+        if (s == schur) continue;
+        const int nc = y.ncol[s], nu = y.nrow[s] - nc, ld = lay.ild[s];
+        if (lay.fused[l]) {
+          if (z)
+            first.push_back({{lay.ioff[s] + nc, ld, nc, nu, y.rptr[s] + nc, 0, y.col0[s], -1, MV_X, 0, 0}, ld, 0});
+          else
+            first.push_back({{lay.ioff[s], ld, nc, nc + nu, y.rptr[s], nc, y.col0[s], -1, MV_X, 0, 0}, ld, 2});
+        } else {
+          first.push_back({{y.foff[s] + nc, y.nrow[s], nc, nu, y.rptr[s] + nc, 0, woff[s], y.col0[s],
+                            MV_FRONT | MV_YSUB, 0, 0}, y.nrow[s], 0});
+          second.push_back({{lay.ioff[s], ld, nc, nc, woff[s], 0, y.col0[s], -1, MV_X, 0, 0}, ld, 2});
+        }
       }
-      add_sns(ops, FW_INIT, list);
-      add_tiles(ops, FW_INV, ilist, false);
-      add_tiles(ops, FW_UPD, ilist, true);
-      all.insert(all.end(), list.begin(), list.end());
+      cut(ops, BW_ROWS, first);
+      cut(ops, BW_MV, second);
     }
-    add_sns(ops, FW_OUT, all);
-  }
-  // backward: the pivot rows of every internal front from Y in one launch,
-  // then levels top-down (the update-row products read the final rows of X
-  // directly)
-  {
-    std::vector<int> all;
-    for (int s = 0; s < y.nsup; s++)
-      if (s != schur) all.push_back(s);
-    add_sns(sp.bw, BW_INIT, all);
-  }
-  for (int l = y.nlevels - 1; l >= 0; l--) {
-    std::vector<int> list;
-    for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++)
-      if (y.lvsup[q] != schur) list.push_back(y.lvsup[q]);
-    if (list.empty()) continue;
-    add_tiles(sp.bw, BW_UPD, list, false);
-    add_tiles(sp.bw, BW_INV, list, false);
   }
 }
 
@@ -701,7 +759,7 @@ int DeviceReducer::build_structure(std::string& err) {
 // Device upload of the part and of every structure array the kernels read.
 static void lanczos_sizes(int n1, int nev, const ReduceOptions& o, int& bs, int& mcap);
 static SolvePlan* plan_slot(DeviceReducer::Impl& d, int nrhs);
-static void plan_host(const Symbolic& y, SolvePlan& sp, PlanHost& h, int split);
+static void plan_host(const Symbolic& y, const DeviceReducer::Impl& d, SolvePlan& sp, PlanHost& h);
 static int plan_upload(SolvePlan& sp, const PlanHost& h, std::string& err);
 
 int DeviceReducer::upload(std::string& err) {
@@ -746,29 +804,27 @@ int DeviceReducer::upload(std::string& err) {
   HIPCHK(d.relptr.upload(y.relptr));
   HIPCHK(d.rel.upload(y.rel));
   HIPCHK(d.foff.upload(y.foff));
-  std::vector<int64_t> woff(y.nsup + 1, 0);
-  for (int s = 0; s < y.nsup; s++) woff[s + 1] = woff[s] + y.nrow[s];
-  d.wrows = woff[y.nsup];
-  HIPCHK(d.woff.upload(woff));
-  std::vector<int64_t> ioff(y.nsup + 1, 0);
-  for (int s = 0; s < y.nsup; s++) ioff[s + 1] = ioff[s] + (int64_t)y.ncol[s] * y.ncol[s];
+  d.wrows = work_rows(y)[y.nsup];
+  d.lay = solve_layout(y, opt_);
+  const std::vector<int64_t>& ioff = d.lay.ioff;
   HIPCHK(d.ioff.upload(ioff));
+  HIPCHK(d.ild.upload(d.lay.ild));
   d.mixed = opt_.mixed;
   d.m_lumped = d.hexl.empty() && d.bml.empty();
   d.solve_split = std::max(64, (opt_.solve_split / 64) * 64);
   if (d.mixed) {
     d.ipool.release();
-    HIPCHK(d.ipool32.alloc(ioff[y.nsup]));
+    HIPCHK(d.ipool32.alloc(ioff[y.nsup] + PANEL_PAD));
   } else {
     d.ipool32.release();
-    HIPCHK(d.ipool.alloc(ioff[y.nsup]));
+    HIPCHK(d.ipool.alloc(ioff[y.nsup] + PANEL_PAD));
   }
   HIPCHK(d.dpiv.alloc((size_t)std::max(1, y.ndof1)));
   HIPCHK(d.adiag.alloc((size_t)std::max(1, y.ndof1)));
   HIPCHK(d.amax.alloc(1));
   HIPCHK(d.sing.alloc((size_t)std::max(1, y.ndof1)));
   d.S = DevSym{d.col0.p, d.ncol.p, d.nrow.p, d.foff.p, d.rptr.p, d.rows.p, d.chptr.p,
-               d.chlist.p, d.relptr.p, d.rel.p, d.woff.p, d.dpiv.p,
+               d.chlist.p, d.relptr.p, d.rel.p, d.ild.p, d.dpiv.p,
                d.adiag.p, d.amax.p, d.sing.p, std::max(opt_.tol_factorize, 1e-20)};
   // The host-side schedules (the factorisation's and the solve plans the
   // reduction uses) are built on host threads while the device builds the
@@ -797,14 +853,18 @@ int DeviceReducer::upload(std::string& err) {
   const int panel = std::min(256, std::max(64, (opt_.factor_panel / 64) * 64));
   std::vector<std::future<void>> host_jobs;
   host_jobs.push_back(std::async(std::launch::async, [&]() {
-    build_factor_schedule(y, ft, d.fops, xr, upd_flops_, panel, inv_slots, opt_.factor_lookahead);
+    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_slots, opt_.factor_lookahead);
   }));
+  std::vector<int> gptr, gsrc;
+  host_jobs.push_back(std::async(std::launch::async, [&]() { build_gather(y, gptr, gsrc); }));
   for (size_t i = 0; i < sps.size(); i++)
-    host_jobs.push_back(std::async(std::launch::async, [&, i]() { plan_host(y, *sps[i], phs[i], d.solve_split); }));
+    host_jobs.push_back(std::async(std::launch::async, [&, i]() { plan_host(y, d, *sps[i], phs[i]); }));
   const int src = build_structure(err);
   for (auto& f : host_jobs) f.get();
   if (src) return src;
   mark("structure built");
+  HIPCHK(d.gptr.upload(gptr));
+  HIPCHK(d.gsrc.upload(gsrc));
   for (size_t i = 0; i < sps.size(); i++)
     if (int rc = plan_upload(*sps[i], phs[i], err)) return rc;
   HIPCHK(ensure_side(d));
@@ -866,10 +926,9 @@ static SolvePlan* plan_slot(DeviceReducer::Impl& d, int nrhs) {
   SolvePlan* sp = nullptr;
   if (it != d.plans.end()) {
     sp = it->second.get();
-    sp->nslots = 0;
-    sp->fw_int.clear();
-    sp->fw_all.clear();
+    sp->fw.clear();
     sp->bw.clear();
+    sp->bw0.clear();
   } else {
     auto fresh = std::make_unique<SolvePlan>();
     sp = fresh.get();
@@ -880,19 +939,16 @@ static SolvePlan* plan_slot(DeviceReducer::Impl& d, int nrhs) {
   return sp;
 }
 
-// Host part of a plan (pure host work, safe on another thread).
-static void plan_host(const Symbolic& y, SolvePlan& sp, PlanHost& h, int split) {
-  build_solve_plan(y, sp, h.tasks, h.gptr, h.gsrc, h.ugrp, h.ugroups, split);
+// Host part of a plan (pure host work, safe on another thread).  B has as
+// many right-hand sides as boundary equations, so their plan gets the
+// backward pass from zero too.
+static void plan_host(const Symbolic& y, const DeviceReducer::Impl& d, SolvePlan& sp, PlanHost& h) {
+  build_solve_plan(y, d.lay, sp, h, d.solve_split, sp.nrhs == y.ndof2);
 }
 
 static int plan_upload(SolvePlan& sp, const PlanHost& h, std::string& err) {
   HIPCHK(sp.tasks.upload(h.tasks));
-  HIPCHK(sp.gptr.upload(h.gptr));
-  HIPCHK(sp.gsrc.upload(h.gsrc.empty() ? std::vector<int>(1, 0) : h.gsrc));
-  HIPCHK(sp.ugrp_int.upload(h.ugrp[0]));
-  HIPCHK(sp.ugrp_all.upload(h.ugrp[1]));
-  HIPCHK(sp.ugroups.upload(h.ugroups.empty() ? std::vector<int>(3, 0) : h.ugroups));
-  HIPCHK(sp.part.alloc((size_t)std::max(1, sp.nslots) * 4096));
+  HIPCHK(sp.inits.upload(h.inits));
   sp.valid = true;
   return 0;
 }
@@ -902,7 +958,7 @@ static int get_plan(const Symbolic& y, DeviceReducer::Impl& d, int nrhs, SolvePl
   if (it != d.plans.end() && it->second->valid) { out = it->second.get(); return 0; }
   SolvePlan* sp = plan_slot(d, nrhs);
   PlanHost h;
-  plan_host(y, *sp, h, d.solve_split);
+  plan_host(y, d, *sp, h);
   if (int rc = plan_upload(*sp, h, err)) return rc;
   out = sp;
   return 0;
@@ -910,7 +966,7 @@ static int get_plan(const Symbolic& y, DeviceReducer::Impl& d, int nrhs, SolvePl
 
 static int ensure_work(DeviceReducer::Impl& d, int nrhs, std::string& err) {
   HIPCHK(d.W.alloc((size_t)d.wrows * nrhs));
-  HIPCHK(d.V.alloc((size_t)d.wrows * nrhs));
+  if (d.lay.unfused) HIPCHK(d.V.alloc((size_t)d.wrows * nrhs));
   return 0;
 }
 
@@ -965,55 +1021,31 @@ int DeviceReducer::prepare_solves(std::string& err) {
   return 0;
 }
 
-static void run_mv_op(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const Op& op, double* X) {
-  static const int mode_of[] = {0, 1, 2, 3};
-  const SolveTask* t = sp.tasks.p + op.off;
-  switch (op.kind) {
-    case FW_INV: case FW_UPD: case BW_UPD: case BW_INV: {
-      int mode = op.kind == FW_INV ? 0 : op.kind == FW_UPD ? 1 : op.kind == BW_UPD ? 2 : 3;
-      if (d.mixed)
-        launch_mv(st, t, op.n, d.S, d.pool32.p, d.ioff.p, d.ipool32.p, d.W.p, d.V.p, X, sp.part.p, sp.nrhs,
-                  mode_of[mode]);
-      else
-        launch_mv(st, t, op.n, d.S, d.pool.p, d.ioff.p, d.ipool.p, d.W.p, d.V.p, X, sp.part.p, sp.nrhs,
-                  mode_of[mode]);
-      break;
-    }
-    case FW_INV_R: case FW_UPD_R: case BW_UPD_R: case BW_INV_R: {
-      int mode = op.kind == FW_INV_R ? 0 : op.kind == FW_UPD_R ? 1 : op.kind == BW_UPD_R ? 2 : 3;
-      launch_mv_red(st, t, op.n, d.S, d.W.p, d.V.p, X, sp.part.p, sp.nrhs, mode);
-      break;
-    }
+static void run_mv(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const Op& op, const double* R,
+                   double* Y, double* X) {
+  const MvTask* t = sp.tasks.p + op.off;
+  const int kind = op.kind == FW_MV ? MV_FORWARD : op.kind == BW_ROWS ? MV_BACK_ROWS : MV_BACK;
+  if (d.mixed)
+    launch_mv(st, t, op.n, kind, sp.nt, op.kw, d.pool32.p, d.ipool32.p, d.S.rows, d.S.dpiv, d.W.p, d.V.p, R, Y, X,
+              sp.nrhs);
+  else
+    launch_mv(st, t, op.n, kind, sp.nt, op.kw, d.pool.p, d.ipool.p, d.S.rows, d.S.dpiv, d.W.p, d.V.p, R, Y, X, sp.nrhs);
+}
+
+// Y = D^{-1} L^{-1} R on the internal rows
+static void run_forward(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const double* R, double* Y) {
+  for (const Op& op : sp.fw) {
+    if (op.kind == FW_INIT)
+      launch_fw_init(st, sp.inits.p + op.off, op.n, d.gptr.p, d.gsrc.p, R, d.W.p, sp.nrhs);
+    else
+      run_mv(st, d, sp, op, R, Y, nullptr);
   }
 }
 
-// Y = L^{-1} R (scale: D^{-1} L^{-1} R); all: also the Schur front (reduced RHS rows)
-static void run_forward(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const double* R, double* Yout,
-                        int ndof1, bool scale, bool all) {
-  const std::vector<Op>& ops = all ? sp.fw_all : sp.fw_int;
-  for (const Op& op : ops) {
-    switch (op.kind) {
-      case FW_INIT:
-        launch_fw_init(st, sp.tasks.p + op.off, op.n, d.S, sp.gptr.p, sp.gsrc.p, all ? sp.ugrp_all.p : sp.ugrp_int.p,
-                       sp.ugroups.p, sp.part.p, R, d.W.p, sp.nrhs, ndof1);
-        break;
-      case FW_OUT:
-        if (d.mixed)
-          launch_fw_out(st, sp.tasks.p + op.off, op.n, d.S, d.pool32.p, d.W.p, d.V.p, Yout, sp.nrhs, scale, ndof1);
-        else
-          launch_fw_out(st, sp.tasks.p + op.off, op.n, d.S, d.pool.p, d.W.p, d.V.p, Yout, sp.nrhs, scale, ndof1);
-        break;
-      default: run_mv_op(st, d, sp, op, nullptr); break;
-    }
-  }
-}
-
-// X = L^{-T} Y on the internal rows; X's boundary rows must be set by the caller
-static void run_backward(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const double* Yin, double* X) {
-  for (const Op& op : sp.bw) {
-    if (op.kind == BW_INIT) launch_bw_init(st, sp.tasks.p + op.off, op.n, d.S, Yin, d.W.p, sp.nrhs);
-    else run_mv_op(st, d, sp, op, X);
-  }
+// X = L^{-T} Y on the internal rows (Y null: zero); X's boundary rows must
+// be set by the caller
+static void run_backward(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, double* Y, double* X) {
+  for (const Op& op : Y ? sp.bw : sp.bw0) run_mv(st, d, sp, op, nullptr, Y, X);
 }
 
 // Relative size ||D|| / ||X|| of a correction D against the solution X
@@ -1061,7 +1093,7 @@ static int refine_state(double rel, double prev, int steps, const ReduceOptions&
 static void approx_solve(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, int neq, int ndof1,
                          double* Rin, double* Yw, double* D) {
   launch_scale_rc(st, ndof1, sp.nrhs, d.dscale.p, nullptr, Rin);
-  run_forward(st, d, sp, Rin, Yw, ndof1, true, false);
+  run_forward(st, d, sp, Rin, Yw);
   launch_fill(st, D + (size_t)ndof1 * sp.nrhs, (int64_t)(neq - ndof1) * sp.nrhs, 0.0);  // boundary rows
   run_backward(st, d, sp, Yw, D);
   launch_scale_rc(st, ndof1, sp.nrhs, d.dscale.p, nullptr, D);
@@ -1183,7 +1215,7 @@ static int solve_int(hipStream_t st, DeviceReducer::Impl& d, const Symbolic& y, 
   const int neq = y.neq, n1 = y.ndof1, nr = sp.nrhs;
   const int64_t nall = (int64_t)neq * nr, nint = (int64_t)n1 * nr;
   if (!d.mixed) {
-    run_forward(st, d, sp, R, Yw, n1, true, false);
+    run_forward(st, d, sp, R, Yw);
     launch_fill(st, X + nint, nall - nint, 0.0);  // boundary rows; the backward pass writes the others
     run_backward(st, d, sp, Yw, X);
     if (steps) *steps = 0;
@@ -1315,6 +1347,7 @@ int DeviceReducer::reduce(std::string& err) {
           launch_inv_part(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool,
                           reinterpret_cast<decltype(pool)>(d.ipart.p));
           break;
+        case PANEL: launch_panel(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
         case INV_FIN:
           launch_inv_fin(st, d.ftasks.p + op.off, op.n, d.S, d.ioff.p, ipool,
                          reinterpret_cast<decltype(pool)>(d.ipart.p));
@@ -1588,7 +1621,7 @@ int DeviceReducer::reduce(std::string& err) {
       HIPCHK(hipMemcpy2DAsync(d.Tmp.p, sizeof(double) * bs, d.P.p + (size_t)j * bs, sizeof(double) * mcap,
                               sizeof(double) * bs, neq, hipMemcpyDeviceToDevice, st));
       auto solve_step = [&]() {
-        run_forward(st, d, *pl, d.Tmp.p, d.Yl.p, n1, true, false);
+        run_forward(st, d, *pl, d.Tmp.p, d.Yl.p);
         launch_fill(st, d.Wl.p + (size_t)n1 * bs, (int64_t)(neq - n1) * bs, 0.0);  // boundary rows stay zero
         run_backward(st, d, *pl, d.Yl.p, d.Wl.p);
       };
@@ -1596,8 +1629,8 @@ int DeviceReducer::reduce(std::string& err) {
         if (int rc2 = solve_int(st, d, y, opt_, *pl, d.Tmp.p, d.Yl.p, d.Wl.p, nullptr, err)) return rc2;
       } else if (!opt_.use_graphs) solve_step();
       else HIPCHK(run_graph(st, d.g_lanczos,
-                       {pl, pl->tasks.p, pl->part.p, d.Tmp.p, d.Yl.p, d.Wl.p, d.W.p, d.V.p, d.pool.p, d.ipool.p,
-                        d.S.foff, d.S.woff, d.S.dpiv}, solve_step));
+                       {pl, pl->tasks.p, pl->inits.p, d.gptr.p, d.Tmp.p, d.Yl.p, d.Wl.p, d.W.p, d.V.p, d.pool.p, d.ipool.p,
+                        d.S.rows, d.S.dpiv}, solve_step));
       for (int pass = 0; pass < 2; pass++) {
         // coefficients of the pass into Cc, their running sum into Cacc
         launch_xty(st, neq, mj, bs, d.P.p, mcap, d.Wl.p, bs, d.part.p, d.Cc.p, d.Cacc.p, pass > 0);
@@ -2058,7 +2091,7 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
     std::vector<int> xr;
     d.fops.clear();
     int inv_slots = 0;
-    build_factor_schedule(sym_, ft, d.fops, xr, upd_flops_, P, inv_slots, opt_.factor_lookahead);
+    build_factor_schedule(sym_, d.lay, ft, d.fops, xr, upd_flops_, P, inv_slots, opt_.factor_lookahead);
     HIPCHK(ensure_side(d));
     HIPCHK(d.ipart.alloc((size_t)std::max(1, inv_slots) * 4096));
     HIPCHK(d.ftasks.upload(ft));
@@ -2105,11 +2138,9 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
 size_t DeviceReducer::footprint_bytes() const {
   const Symbolic& y = sym_;
   const size_t nnz = y.rowptr.empty() ? 0 : (size_t)y.rowptr.back();
-  size_t ipool = 0, wrows = 0;
-  for (int s = 0; s < y.nsup; s++) {
-    ipool += (size_t)y.ncol[s] * y.ncol[s];
-    wrows += y.nrow[s];
-  }
+  size_t wrows = 0;
+  for (int s = 0; s < y.nsup; s++) wrows += y.nrow[s];
+  const size_t ipool = y.nsup > 0 ? (size_t)solve_layout(y, opt_).ioff[y.nsup] : 0;
   const int nev = opt_.ngen > 0 ? std::max(opt_.neval, opt_.ngen) : 0;
   const int bs = opt_.lanczos_block;
   const size_t mcap = nev > 0 ? (size_t)std::max(10 * nev + 40, 16 * bs) : 0;
