@@ -14,7 +14,8 @@ struct FTask {
   int sn;      // supernode
   int a, b;    // meaning depends on the kernel (row chunk, tile indices)
   int k0;      // first pivot column of the panel
-  int kb;      // trailing update: panel width (<= 128); the trailing block starts at k0 + kb
+  int kb;      // trailing update: panel width (<= 256); the trailing block starts at k0 + kb
+  int je;      // trailing update: columns from je on are left alone (0: none)
 };
 
 // Elements that the solve-panel pools hold past their last front: k_panel's

@@ -727,95 +727,123 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
 
 // ---------------------------------------------------------------- update
 // Task: sn, a = ti, b = tj (64x64 tiles of the trailing lower triangle),
-// k0 = panel, kb = panel width (<= 128).  F[I,J] -= (L_I D) L_J^T over the
-// panel, staged through LDS in UCH-column chunks whose products accumulate
-// in the MFMA registers, so a 128-wide panel reads and writes the trailing
-// tile once for both halves.  FP64: the accumulators start from the tile's
-// current values (loaded with the first chunk, so the two latencies
-// overlap) and the staged L_I D is negated, so the MFMA chain forms
-// F - sum (L_I D) L_J^T directly and the tile is only stored at the end.
-// FP32 (mixed precision) sums the products from zero and subtracts them
-// from the tile at the end: accumulating onto the tile through the FP32
-// MFMA left the factor too inexact for the FP64 refinement of a thin
-// 200x200 plate to converge.
-template <class T>
-__global__ __launch_bounds__(256) void k_update(const FTask* __restrict__ tasks, DevSym S,
-                                                T* __restrict__ pool) {
-  constexpr int UCH = 16, UQ = 64 * UCH / 256;  // chunk width, loads per thread per operand
-  // two LDS buffers: chunk c is multiplied from buffer c & 1 while chunk
-  // c + 1 is staged into the other, one barrier per chunk
-  __shared__ T sI[2][64][UCH + 1];
-  __shared__ T sJ[2][64][UCH + 1];
+// k0 = panel, kb = panel width (<= 256), je = column limit.  F[I,J] -= (L_I
+// D) L_J^T over the panel.  A wave holds 16 XA x 32 of the tile in its MFMA accumulators and
+// reads both operands straight from the panel (128 contiguous bytes per
+// column and 16 rows), eight columns ahead of their products: a 16x16x4 FP64
+// step keeps the matrix core for 64 cycles, so the first-level cache feeds
+// it without staging, barriers or staging arithmetic.  FP64: the
+// accumulators start from the tile's current values and the A operand is
+// negated, so the chain forms F - sum (L_I D) L_J^T and the tile is only
+// stored at the end.  FP32 (mixed precision) sums the products from zero and
+// subtracts them from the tile at the end: accumulating onto the tile
+// through the FP32 MFMA left the factor too inexact for the FP64 refinement
+// of a thin 200x200 plate to converge.
+// Bound by the matrix cores and, at 128 columns a panel, by the tile's read
+// and write (16 flop per byte of it).  Measured at 128 columns: one front of
+// 6000 rows 45 TFLOP/s (four waves of 32x32: 42; staged through LDS: 37),
+// 16 fronts of 1500 rows 44 (41; 36), one of 1900 rows 17 (24; 21): the wide
+// waves where a launch has UPD_WIDE or more tiles, else the four.
+constexpr int UPD_WIDE = 2048;
+
+template <int XA, class T>
+__global__ __launch_bounds__(XA == 2 ? 256 : 128, XA == 2 ? 4 : 3) void k_update(const FTask* __restrict__ tasks, DevSym S,
+                                                                T* __restrict__ pool) {
+  constexpr int YB = 2, CH = 8, ST = CH / 4;
   const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
-  const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn];
-  const int kb = t.kb;
-  const int t0 = k0 + kb;
-  const int I0 = t0 + 64 * t.a, J0 = t0 + 64 * t.b;
+  const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn], kb = t.kb;
   T* F = pool + S.foff[sn];
-  const int c0s = S.col0[sn];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wv = tid >> 6;
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
-  const int lr = lane & 15, lk = lane >> 4;
-  T ri[UQ], rj[UQ], rd[UQ];
-  // global loads of the chunk at c0 (zero beyond the panel)
-  auto load = [&](int c0) {
-    const int kc = min(UCH, kb - c0), p0 = k0 + c0;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int I0 = k0 + kb + 64 * t.a + 16 * XA * (wv >> 1), J0 = k0 + kb + 64 * t.b + 32 * (wv & 1);
+  const int je = t.je > 0 ? t.je : ld;
+  if (I0 >= ld || J0 >= je || J0 >= I0 + 16 * XA) return;  // nothing of this part is stored
+  // rows past the front repeat its last one and are not stored
+  const T* base = F + (int64_t)(k0 + lk) * ld;
+  const T *Ip[XA], *Jp[YB];
 #pragma unroll
-    for (int q = 0; q < UQ; q++) {
-      const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-      const bool okm = m < kc;
-      rd[q] = okm ? (T)S.dpiv[c0s + p0 + m] : (T)0;
-      ri[q] = (okm && I0 + i < ld) ? F[(int64_t)(I0 + i) + (int64_t)(p0 + m) * ld] : (T)0;
-      rj[q] = (okm && J0 + i < ld) ? F[(int64_t)(J0 + i) + (int64_t)(p0 + m) * ld] : (T)0;
+  for (int x = 0; x < XA; x++) Ip[x] = base + min(I0 + 16 * x + lr, ld - 1);
+#pragma unroll
+  for (int y = 0; y < YB; y++) Jp[y] = base + min(J0 + 16 * y + lr, ld - 1);
+  const double* Dp = S.dpiv + S.col0[sn] + k0;
+  struct Stage {
+    T a[ST][XA], b[ST][YB], d[ST];
+  };
+  // the next whole chunk, the pointers moving on (an address product per
+  // load costs as much as the matrix step: 23 TFLOP/s)
+  const int64_t step = (int64_t)4 * ld;
+  const double* Dq = Dp + lk;
+  auto load = [&](Stage& g) {
+#pragma unroll
+    for (int s = 0; s < ST; s++) {
+#pragma unroll
+      for (int x = 0; x < XA; x++) g.a[s][x] = Ip[x][s * step];
+#pragma unroll
+      for (int y = 0; y < YB; y++) g.b[s][y] = Jp[y][s * step];
+      g.d[s] = (T)Dq[4 * s];
+    }
+#pragma unroll
+    for (int x = 0; x < XA; x++) Ip[x] += ST * step;
+#pragma unroll
+    for (int y = 0; y < YB; y++) Jp[y] += ST * step;
+    Dq += CH;
+  };
+  const int kf = kb & ~(2 * CH - 1);
+  // a chunk from column c on, after the whole pairs of chunks; the columns
+  // past the panel repeat the last one with a zero pivot
+  auto load_tail = [&](int c, Stage& g) {
+#pragma unroll
+    for (int s = 0; s < ST; s++) {
+      const int k = c + 4 * s + lk, kc = min(k, kb - 1);
+      const int64_t o = (int64_t)(kc - kf - lk) * ld;
+#pragma unroll
+      for (int x = 0; x < XA; x++) g.a[s][x] = Ip[x][o];
+#pragma unroll
+      for (int y = 0; y < YB; y++) g.b[s][y] = Jp[y][o];
+      const T d = (T)Dp[kc];
+      g.d[s] = k < kb ? d : (T)0;
     }
   };
-  load(0);
-  // FP64: the stored elements of the tile (lower triangle inside the
-  // front) seed the accumulators; the others start at zero, never stored
   constexpr bool seed = std::is_same<T, double>::value;
-  typename MF<T>::acc acc[2][2];
+  typename MF<T>::acc acc[XA][YB];
+  auto multiply = [&](const Stage& g) {
 #pragma unroll
-  for (int x = 0; x < 2; x++)
+    for (int s = 0; s < ST; s++)
 #pragma unroll
-    for (int y = 0; y < 2; y++)
+      for (int x = 0; x < XA; x++) {
+        const T a = seed ? -(g.a[s][x] * g.d[s]) : g.a[s][x] * g.d[s];
+#pragma unroll
+        for (int y = 0; y < YB; y++) acc[x][y] = MF<T>::op(g.b[s][y], a, acc[x][y]);
+      }
+  };
+  Stage g0, g1;
+  if (kf > 0) load(g0);
+#pragma unroll
+  for (int x = 0; x < XA; x++)
+#pragma unroll
+    for (int y = 0; y < YB; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = I0 + wr + 16 * x + lr;
-        const int j = J0 + wc + 16 * y + MF<T>::col(lk, r);
-        acc[x][y][r] = (seed && i < ld && j < ld && i >= j) ? F[(int64_t)i + (int64_t)j * ld] : (T)0;
+        const int i = min(I0 + 16 * x + lr, ld - 1), j = min(J0 + 16 * y + MF<T>::col(lk, r), ld - 1);
+        acc[x][y][r] = seed ? F[(int64_t)i + (int64_t)j * ld] : (T)0;
       }
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < UQ; q++) {
-      const int idx = tid + 256 * q, i = idx & 63, m = idx >> 6;
-      sI[buf][i][m] = seed ? -(ri[q] * rd[q]) : ri[q] * rd[q];
-      sJ[buf][i][m] = rj[q];
-    }
-  };
-  stage(0);
-  __syncthreads();
-  for (int c0 = 0, buf = 0; c0 < kb; c0 += UCH, buf ^= 1) {
-    const int kc = min(UCH, kb - c0);
-    const bool more = c0 + UCH < kb;
-    if (more) load(c0 + UCH);  // the next chunk's loads are in flight during the products
-    mfma_tile<T>(sI[buf], sJ[buf], (kc + 3) & ~3, acc, lane, wr, wc);
-    // the other buffer was last read by the products of the chunk before
-    // this one, which every wave finished before the previous barrier
-    if (more) {
-      stage(buf ^ 1);
-      __syncthreads();
-    }
+  for (int c = 0; c < kf; c += 2 * CH) {
+    load(g1);
+    multiply(g0);
+    if (c + 2 * CH < kf) load(g0);
+    multiply(g1);
+  }
+  for (int c = kf; c < kb; c += CH) {
+    load_tail(c, g0);
+    multiply(g0);
   }
 #pragma unroll
-  for (int x = 0; x < 2; x++)
+  for (int x = 0; x < XA; x++)
 #pragma unroll
-    for (int y = 0; y < 2; y++)
+    for (int y = 0; y < YB; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = I0 + wr + 16 * x + lr;
-        const int j = J0 + wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ld && j < ld && i >= j) {
+        const int i = I0 + 16 * x + lr, j = J0 + 16 * y + MF<T>::col(lk, r);
+        if (i < ld && j < je && i >= j) {
           if (seed) F[(int64_t)i + (int64_t)j * ld] = acc[x][y][r];
           else F[(int64_t)i + (int64_t)j * ld] -= acc[x][y][r];
         }
@@ -1848,7 +1876,8 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
     if (n > 0) k_trsm<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                        \
   }                                                                                                        \
   void launch_update(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {                    \
-    if (n > 0) k_update<T><<<n, 256, 0, st>>>(t, S, pool);                                                   \
+    if (n >= UPD_WIDE) k_update<4, T><<<n, 128, 0, st>>>(t, S, pool);                                       \
+    else if (n > 0) k_update<2, T><<<n, 256, 0, st>>>(t, S, pool);                                          \
   }                                                                                                        \
   void launch_inv_off(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,               \
                       const int64_t* ioff, T* ipool) {                                                     \

@@ -309,7 +309,7 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
       // end) ranges of child update columns landing in the block, in child
       // order, at xrange[3 b ..], kb of them
       for (int j0 = 0; j0 < y.nrow[s]; j0 += 16) {
-        FTask t{s, j0, (int)xrange.size() / 3, 0, 0};
+        FTask t{s, j0, (int)xrange.size() / 3, 0, 0, 0};
         for (int q = y.chptr[s]; q < y.chptr[s + 1]; q++) {
           const int c = y.chlist[q], nu = y.nrow[c] - y.ncol[c];
           const int* rel = y.rel.data() + y.relptr[c];
@@ -328,12 +328,13 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
     if ((int)tasks.size() > off) ops.push_back({EXTADD, off, (int)tasks.size() - off});
     int maxnc = 0;
     for (int q = 0; q < ns; q++) maxnc = std::max(maxnc, y.ncol[sups[q]]);
-    // Pivot columns go in panels of P = 64 h columns (h sub-panels of 64):
-    // for each sub-panel the diagonal block and the triangular solve, then
-    // its update of the panel's remaining columns only; after the last
-    // sub-panel one trailing update over the whole panel, so the trailing
-    // block is read and written once per panel.  A front with fewer than P
-    // pivot columns left takes plain 64-column panels.
+    // Pivot columns go in panels of up to P columns (sub-panels of 64): for
+    // each sub-panel the diagonal block and the triangular solve, then its
+    // update of the panel's remaining columns only; after the last sub-panel
+    // one trailing update over the whole panel, so the trailing block is
+    // read and written once per panel, and ceil(ncol / P) times per front
+    // (factor of the 45x41x43 block: P = 64, 128, 192, 256 take 81, 62, 55,
+    // 53 ms; of the 48x24x24 block 12.7, 11.4, 11.0, 11.0).
     // Panels with at most FUSE_TRSM row tiles below their diagonal blocks
     // (summed over the level) take one fused launch instead.
     constexpr int FUSE_TRSM = 256;
@@ -349,8 +350,8 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
           int s = sups[q];
           if (y.ncol[s] <= k0) continue;
           int kb = std::min(64, y.ncol[s] - k0), rem = y.nrow[s] - k0 - kb;
-          if (rem <= 0) tasks.push_back({s, -1, 0, k0, 0});
-          for (int a = 0; 64 * a < rem; a++) tasks.push_back({s, a, 0, k0, 0});
+          if (rem <= 0) tasks.push_back({s, -1, 0, k0, 0, 0});
+          for (int a = 0; 64 * a < rem; a++) tasks.push_back({s, a, 0, k0, 0, 0});
         }
         if ((int)tasks.size() > off) ops.push_back({DIAG_TRSM, off, (int)tasks.size() - off});
         return;
@@ -358,7 +359,7 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
       int off = (int)tasks.size();
       for (int q = 0; q < ns; q++) {
         int s = sups[q];
-        if (y.ncol[s] > k0) tasks.push_back({s, 0, 0, k0, 0});
+        if (y.ncol[s] > k0) tasks.push_back({s, 0, 0, k0, 0, 0});
       }
       if ((int)tasks.size() > off) ops.push_back({DIAG, off, (int)tasks.size() - off});
       off = (int)tasks.size();
@@ -366,24 +367,24 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
         int s = sups[q];
         if (y.ncol[s] <= k0) continue;
         int kb = std::min(64, y.ncol[s] - k0), rem = y.nrow[s] - k0 - kb;
-        for (int a = 0; 64 * a < rem; a++) tasks.push_back({s, a, 0, k0, 0});
+        for (int a = 0; 64 * a < rem; a++) tasks.push_back({s, a, 0, k0, 0, 0});
       }
       if ((int)tasks.size() > off) ops.push_back({TRSM, off, (int)tasks.size() - off});
     };
     // 64x64 lower tiles of the trailing block from k0 + kb, tile columns in
-    // [tlo, thi) (thi < 0: all), appended to `out`
-    auto add_update_to = [&](std::vector<FTask>& out, int s, int k0, int kb, int tlo, int thi) {
+    // [tlo, thi) (thi < 0: all), columns before je (0: all), appended to `out`
+    auto add_update_to = [&](std::vector<FTask>& out, int s, int k0, int kb, int tlo, int thi, int je) {
       const int rem = y.nrow[s] - k0 - kb;
       if (rem <= 0) return;
       const int T = (rem + 63) / 64;
       for (int ti = 0; ti < T; ti++)
-        for (int tj = tlo; tj <= ti && (thi < 0 || tj < thi); tj++) out.push_back({s, ti, tj, k0, kb});
+        for (int tj = tlo; tj <= ti && (thi < 0 || tj < thi); tj++) out.push_back({s, ti, tj, k0, kb, je});
       // lower-triangle entries (incl. diagonal) of the updated columns c in
       // [clo, chi), rem - c each, 2 flops per FMA
-      const double clo = std::min(rem, 64 * tlo), chi = thi < 0 ? rem : std::min(rem, 64 * thi);
+      double clo = std::min(rem, 64 * tlo), chi = thi < 0 ? rem : std::min(rem, 64 * thi);
+      if (je > 0) chi = std::min(chi, (double)(je - k0 - kb));
       if (chi > clo) flops += 2.0 * kb * ((chi - clo) * rem - (chi * (chi - 1) - clo * (clo - 1)) / 2);
     };
-    auto add_update = [&](int s, int k0, int kb, int ntc) { add_update_to(tasks, s, k0, kb, 0, ntc); };
     const int P = panel, NA = P / 64;
     // Lookahead on the levels of few large fronts (those that take the fused
     // diagonal/TRSM launch): the trailing update after a panel is split into
@@ -408,21 +409,17 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
         bool past = false;  // some task updates columns past the next panel
         for (int q = 0; q < ns; q++) {
           int s = sups[q];
-          const int rc = y.ncol[s] - k0;
+          const int rc = y.ncol[s] - k0, w = std::min(P, rc);  // this front's panel
           if (rc <= 64 * h) continue;
-          if (rc >= P) {
-            if (h + 1 < P / 64) {
-              add_update(s, kh, 64, P / 64 - h - 1);  // the panel's remaining columns
-            } else if (look) {                        // the trailing block, whole panel: split
-              add_update_to(tasks, s, k0, P, 0, NA);
-              add_update_to(side, s, k0, P, NA, -1);
-              past = true;
+          if (64 * (h + 1) < w) {  // the panel's remaining columns
+            add_update_to(tasks, s, kh, 64, 0, (w - 64 * (h + 1) + 63) / 64, k0 + w);
+          } else {  // the trailing block, whole panel
+            if (look && rc > P) {
+              add_update_to(tasks, s, k0, w, 0, NA, 0);
+              add_update_to(side, s, k0, w, NA, -1, 0);
             } else {
-              add_update(s, k0, P, -1);
-              past = true;
+              add_update_to(tasks, s, k0, w, 0, -1, 0);
             }
-          } else {
-            add_update(s, kh, std::min(64, rc - 64 * h), -1);
             past = true;
           }
         }
@@ -461,12 +458,12 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
       const int T = (y.ncol[s] + 63) / 64;
       for (int j = 0; j + dist < T; j++) {
         if (dist <= INV_CHUNK) {
-          tasks.push_back({s, j, j + dist, 0, 0});
+          tasks.push_back({s, j, j + dist, 0, 0, 0});
           continue;
         }
         const int first = slot;
-        for (int k = j; k < j + dist; k += INV_CHUNK) part.push_back({s, j, j + dist, k, slot++});
-        fin.push_back({s, j, j + dist, first, slot - first});
+        for (int k = j; k < j + dist; k += INV_CHUNK) part.push_back({s, j, j + dist, k, slot++, 0});
+        fin.push_back({s, j, j + dist, first, slot - first, 0});
       }
     }
     if ((int)tasks.size() > off) ops.push_back({INV_OFF, off, (int)tasks.size() - off});
@@ -487,7 +484,7 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
     for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++) {
       const int s = y.lvsup[q], nu = y.nrow[s] - y.ncol[s];
       for (int j = 0; 64 * j < y.ncol[s]; j++)
-        for (int i = 0; 64 * i < nu; i++) pan.push_back({s, j, i, y.ncol[s] - 64 * j, 0});
+        for (int i = 0; 64 * i < nu; i++) pan.push_back({s, j, i, y.ncol[s] - 64 * j, 0, 0});
     }
   }
   std::stable_sort(pan.begin(), pan.end(), [](const FTask& a, const FTask& b) { return a.k0 > b.k0; });

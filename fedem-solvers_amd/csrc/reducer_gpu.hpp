@@ -28,7 +28,7 @@ struct ReduceOptions {
   // and Schur updates, FP64 diagonal-block factorisation), every solve with
   // K_ii refined against the FP64 matrix until the correction falls below
   // ir_tol relative (at most ir_maxit steps; no convergence is an error).
-  int factor_panel = 128;   // pivot columns per trailing update (64..256, multiple of 64)
+  int factor_panel = 256;   // most pivot columns per trailing update (64..256, multiple of 64)
   // top levels: trailing tiles past the next panel on a side stream (off by
   // default: on the 48x24x24 block the side updates take the CUs that the
   // critical-path diagonal launches need, 12.8 -> 13.1 ms)
