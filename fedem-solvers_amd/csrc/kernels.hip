@@ -1,7 +1,7 @@
 // gfx950 kernels of the part reducer: element matrices, pull assembly,
 // multifrontal LDL^T (panel factorisation on VALU, trailing updates on FP64
-// MFMA) and the tall-skinny reductions; the triangular solves are in
-// solve.hip.
+// MFMA) and sparse products; the triangular solves are in solve.hip, the
+// tall-skinny products in dense.hip.
 //
 // Front storage: the front of supernode s is an nrow x nrow column-major
 // FP64 block at pool + foff[s]; only its lower triangle is meaningful.  After
@@ -1264,161 +1264,6 @@ __global__ __launch_bounds__(256) void k_spmm4(int n, int nrhs, const int* __res
   for (int c = 0; c < 4; c++) z[c] = (s[c][0] + s[c][1]) + (s[c][2] + s[c][3]);
 }
 
-// Partial C = X^T Y: blockIdx.x = chunk of crows rows, blockIdx.y = 64
-// columns of X (a), blockIdx.z = 64 columns of Y (b); lane -> a, wave -> b
-// (b = 16*wave + u).  part[chunk][a][b] (na x nb row-major per chunk).
-#define XTY_ROWS 128
-__global__ __launch_bounds__(256) void k_xty_part(int n, int crows, int na, int nb, const double* __restrict__ X,
-                                                  int ldx, const double* __restrict__ Y, int ldy,
-                                                  double* __restrict__ part) {
-  __shared__ double sX[32][64];
-  __shared__ double sY[32][64];
-  const int r0 = blockIdx.x * crows, a0 = blockIdx.y * 64, b0 = blockIdx.z * 64;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int nbt = min(64, nb - b0), nat = min(64, na - a0);
-  const bool narrow = nb <= 16;
-  double acc[16];
-#pragma unroll
-  for (int q = 0; q < 16; q++) acc[q] = 0.0;
-  const int rend = min(n, r0 + crows);
-  for (int rc = r0; rc < rend; rc += 32) {
-    double rx[8], ry[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int idx = tid + 256 * q, rr = idx >> 6, c = idx & 63, r = rc + rr;
-      const bool ok = r < rend;
-      rx[q] = (ok && c < nat) ? X[(int64_t)r * ldx + a0 + c] : 0.0;
-      ry[q] = (ok && c < nbt) ? Y[(int64_t)r * ldy + b0 + c] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int idx = tid + 256 * q;
-      sX[idx >> 6][idx & 63] = rx[q];
-      sY[idx >> 6][idx & 63] = ry[q];
-    }
-    __syncthreads();
-    // sY is zero beyond nbt: same unguarded loop in every thread.  Up to 16
-    // columns of Y (the Lanczos block) the four waves split the rows of the
-    // chunk instead of the columns, so none of them multiplies zeros.
-    if (narrow) {
-#pragma unroll 2
-      for (int rr = wv; rr < 32; rr += 4) {
-        const double xv = sX[rr][lane];
-#pragma unroll
-        for (int q = 0; q < 16; q++) acc[q] += xv * sY[rr][q];
-      }
-    } else {
-#pragma unroll 4
-      for (int rr = 0; rr < 32; rr++) {
-        const double xv = sX[rr][lane];
-#pragma unroll
-        for (int q = 0; q < 16; q++) acc[q] += xv * sY[rr][wv * 16 + q];
-      }
-    }
-  }
-  double* P = part + (int64_t)blockIdx.x * na * nb;
-  if (narrow) {
-    // the waves' partial sums, added in wave order by wave 0: waves 1 and 2
-    // leave theirs in rows 0-15 and 16-31 of sX, wave 3 in rows 0-15 of sY
-    __syncthreads();
-    if (wv == 1 || wv == 2) {
-#pragma unroll
-      for (int q = 0; q < 16; q++) sX[(wv - 1) * 16 + q][lane] = acc[q];
-    } else if (wv == 3) {
-#pragma unroll
-      for (int q = 0; q < 16; q++) sY[q][lane] = acc[q];
-    }
-    __syncthreads();
-    if (wv == 0 && lane < nat) {
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const double v = ((acc[q] + sX[q][lane]) + sX[16 + q][lane]) + sY[q][lane];
-        if (q < nbt) P[(int64_t)(a0 + lane) * nb + b0 + q] = v;
-      }
-    }
-    return;
-  }
-  if (lane < nat) {
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      int b = wv * 16 + q;
-      if (b < nbt) P[(int64_t)(a0 + lane) * nb + b0 + b] = acc[q];
-    }
-  }
-}
-
-// Partial C = X^T Y for wide products (both sides >= 64 columns), on FP64
-// MFMA: the workgroup's 64 x 64 output tile accumulates over its chunk of
-// crows rows in steps of 32; X and Y rows are read along their columns
-// (coalesced) and stored transposed in LDS (sA[a][r], sB[b][r]) for
-// mfma_tile.  Same grid and partial layout as k_xty_part.
-__global__ __launch_bounds__(256) void k_xty_mfma(int n, int crows, int na, int nb, const double* __restrict__ X,
-                                                  int ldx, const double* __restrict__ Y, int ldy,
-                                                  double* __restrict__ part) {
-  __shared__ double sA[64][33];
-  __shared__ double sB[64][33];
-  const int r0 = blockIdx.x * crows, a0 = blockIdx.y * 64, b0 = blockIdx.z * 64;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int nbt = min(64, nb - b0), nat = min(64, na - a0);
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
-  f64x4 acc[2][2];
-  zero_acc(acc);
-  const int rend = min(n, r0 + crows);
-  double rx[8], ry[8];
-  auto load = [&](int rc) {
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int idx = tid + 256 * q, rr = idx >> 6, c = idx & 63, r = rc + rr;
-      const bool ok = r < rend;
-      rx[q] = (ok && c < nat) ? X[(int64_t)r * ldx + a0 + c] : 0.0;
-      ry[q] = (ok && c < nbt) ? Y[(int64_t)r * ldy + b0 + c] : 0.0;
-    }
-  };
-  if (r0 < rend) load(r0);
-  for (int rc = r0; rc < rend; rc += 32) {
-    if (rc > r0) __syncthreads();  // the previous rows' products are done with the tiles
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int idx = tid + 256 * q;
-      sA[idx & 63][idx >> 6] = rx[q];
-      sB[idx & 63][idx >> 6] = ry[q];
-    }
-    __syncthreads();
-    if (rc + 32 < rend) load(rc + 32);
-    mfma_tile<double, 33>(sA, sB, 32, acc, lane, wr, wc);
-  }
-  double* P = part + (int64_t)blockIdx.x * na * nb;
-  const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int a = wr + 16 * x + lr, b = wc + 16 * y + lk + 4 * r;
-        if (a < nat && b < nbt) P[(int64_t)(a0 + a) * nb + b0 + b] = acc[x][y][r];
-      }
-}
-
-// One wave per output element: lane l sums chunks l, l+64, ... then a fixed
-// butterfly combines the lanes (same order on every run).
-// C = the sum of the chunk partials; acc (optional) = C, or acc + C with
-// acc_add.
-__global__ __launch_bounds__(256) void k_xty_sum(int nchunk, int nab, const double* __restrict__ part,
-                                                 double* __restrict__ C, double* __restrict__ acc, int acc_add) {
-  const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (e >= nab) return;
-  double s = 0.0;
-  for (int c = lane; c < nchunk; c += 64) s += part[(int64_t)c * nab + e];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (lane == 0) {
-    C[e] = s;
-    if (acc) acc[e] = acc_add ? acc[e] + s : s;
-  }
-}
-
 // Sign convention of the component modes: for column i of Phi (rows in
 // permuted order, ld columns), the component of largest magnitude over the
 // internal equations taken in equation order (q -> row p1[q]; the first
@@ -1483,85 +1328,6 @@ __global__ void k_scale_cols(int64_t n, int nc, const double* __restrict__ sign,
   if (g < n * nc) X[g] *= sign[g % nc];
 }
 
-// Y[r][j] = alpha*Y[r][j] + beta * sum_a X[r][a] S[a][j]; S is (na x nb) row-major.
-__global__ __launch_bounds__(256) void k_gemm_small(int n, int na, int nb, const double* __restrict__ X,
-                                                    int ldx, const double* __restrict__ Sm,
-                                                    double* __restrict__ Y, int ldy, double alpha,
-                                                    double beta) {
-  extern __shared__ double sS[];
-  for (int i = threadIdx.x; i < na * nb; i += blockDim.x) sS[i] = Sm[i];
-  __syncthreads();
-  int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int r = (int)(g / nb), j = (int)(g % nb);
-  if (r >= n) return;
-  double s = 0.0;
-  for (int a = 0; a < na; a++) s += X[(int64_t)r * ldx + a] * sS[a * nb + j];
-  double y = (alpha == 0.0) ? 0.0 : alpha * Y[(int64_t)r * ldy + j];
-  Y[(int64_t)r * ldy + j] = y + beta * s;
-}
-
-// Y = alpha Y + beta X S for S with at most 16 columns, on FP64 MFMA: a
-// workgroup takes 64 rows of X, staged through LDS in 32-column chunks read
-// in row order (coalesced), the next chunk's loads in flight during the
-// current chunk's products; wave w accumulates rows 16 w .. 16 w + 15.
-// blockIdx.y = 1 takes the second pair (X2, Y2) with the same S.  S rows
-// are lds apart (the nb columns may be a slice of a wider S).  Y may be X
-// (in place: a workgroup has read its rows of X before it writes them).
-__global__ __launch_bounds__(256) void k_gemm_rows16(int n, int na, int nb, const double* X1, int ldx1,
-                                                     const double* __restrict__ Sm, int lds, double* Y1, int ldy1,
-                                                     double alpha, double beta, const double* X2, int ldx2,
-                                                     double* Y2, int ldy2) {
-  const double* X = blockIdx.y ? X2 : X1;
-  double* Y = blockIdx.y ? Y2 : Y1;
-  const int ldx = blockIdx.y ? ldx2 : ldx1, ldy = blockIdx.y ? ldy2 : ldy1;
-  __shared__ double sX[64][33];
-  __shared__ double sS[16][33];  // S chunk transposed: sS[j][k]
-  const int r0 = blockIdx.x * 64;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
-  f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
-  double rx[8], rs[2];
-  auto load = [&](int kc) {
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int idx = tid + 256 * q, k = idx & 31, r = r0 + (idx >> 5);
-      rx[q] = (r < n && kc + k < na) ? X[(int64_t)r * ldx + kc + k] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int idx = tid + 256 * q, k = idx >> 4, j = idx & 15;
-      rs[q] = (kc + k < na && j < nb) ? Sm[(int64_t)(kc + k) * lds + j] : 0.0;
-    }
-  };
-  if (na > 0) load(0);
-  for (int kc = 0; kc < na; kc += 32) {
-    __syncthreads();  // the previous chunk's products are done with the LDS tiles
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int idx = tid + 256 * q;
-      sX[idx >> 5][idx & 31] = rx[q];
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int idx = tid + 256 * q;
-      sS[idx & 15][idx >> 4] = rs[q];
-    }
-    __syncthreads();
-    if (kc + 32 < na) load(kc + 32);
-#pragma unroll
-    for (int m0 = 0; m0 < 32; m0 += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sS[lr][m0 + lk], sX[16 * wv + lr][m0 + lk], acc, 0, 0, 0);
-  }
-  // acc[q]: row r0 + 16 wv + lr, column lk + 4 q
-  const int r = r0 + 16 * wv + lr;
-  if (r >= n) return;
-  double* y = Y + (int64_t)r * ldy;
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int j = lk + 4 * q;
-    if (j < nb) y[j] = ((alpha == 0.0) ? 0.0 : alpha * y[j]) + beta * acc[q];
-  }
-}
-
 // X[(ndof1 + b) * nrhs + b] = 1, all other entries 0 (the [B; I] identity rows)
 __global__ void k_identity_rows(double* __restrict__ X, int64_t nrows, int nrhs, int ndof1) {
   int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1602,108 +1368,21 @@ __global__ __launch_bounds__(256) void k_sum_fixed(int n, const double* __restri
   if (threadIdx.x == 0) out[0] = red[0];
 }
 
-// ---------------------------------------------------------------- Lanczos block orthonormalisation
-// Cholesky factor of the symmetrised n x n Gram matrix G = R^T R (R upper,
-// row-major) and R^{-1}, by one workgroup (n <= 64): at step j every thread
-// forms the pivot (same value in each), thread i > j the entry R[j][i]; the
-// inverse is solved column by column, thread t owning column t.  A
-// non-positive pivot sets *bad (the block has broken down).
-__global__ __launch_bounds__(64) void k_chol_inv(int n, const double* __restrict__ G, double* __restrict__ R,
-                                                 double* __restrict__ Ri, int* __restrict__ bad) {
-  __shared__ double A[64][65], U[64][65], V[64][65];
-  const int t = threadIdx.x;
-  if (t < n)
-    for (int i = 0; i < n; i++) {
-      A[i][t] = i == t ? G[i * n + t] : 0.5 * (G[i * n + t] + G[t * n + i]);
-      U[i][t] = 0.0;
-      V[i][t] = 0.0;
-    }
-  __syncthreads();
-  for (int j = 0; j < n; j++) {
-    double s = A[j][j];
-    for (int k = 0; k < j; k++) s -= U[k][j] * U[k][j];
-    if (!(s > 0.0)) {
-      if (t == 0) *bad = 1;
-      s = 1.0;
-    }
-    const double d = sqrt(s);
-    if (t == j) U[j][j] = d;
-    if (t > j && t < n) {
-      double v = A[j][t];
-      for (int k = 0; k < j; k++) v -= U[k][j] * U[k][t];
-      U[j][t] = v / d;
-    }
-    __syncthreads();
-  }
-  if (t < n) {
-    V[t][t] = 1.0 / U[t][t];
-    for (int i = t - 1; i >= 0; i--) {
-      double v = 0.0;
-      for (int k = i + 1; k <= t; k++) v += U[i][k] * V[k][t];
-      V[i][t] = -v / U[i][i];
-    }
-    for (int i = 0; i < n; i++) {
-      R[i * n + t] = U[i][t];
-      Ri[i * n + t] = V[i][t];
-    }
-  }
-}
-
-// k_chol_inv for n <= 16 in one wave with the rows in registers (lane i <
-// 16 holds row i): the LDL^T readlane sweep of k_diag gives the unit lower
-// L1, D and X1 = L1^-1, then G = R^T R with R = D^1/2 L1^T and
-// R^-1 = X1^T D^-1/2.  Rows and columns beyond n are identity.
-__global__ __launch_bounds__(64) void k_chol16(int n, const double* __restrict__ G, double* __restrict__ R,
-                                               double* __restrict__ Ri, int* __restrict__ bad) {
-  const int lane = threadIdx.x;
-  double a[16], x[16];
-#pragma unroll
-  for (int m = 0; m < 16; m++) {
-    double v = lane == m ? 1.0 : 0.0;
-    if (lane < n && m < n) v = lane == m ? G[lane * n + m] : 0.5 * (G[lane * n + m] + G[m * n + lane]);
-    a[m] = m <= lane ? v : 0.0;
-    x[m] = lane == m ? 1.0 : 0.0;
-  }
-  bool nonpos = false;
-#pragma unroll
-  for (int j = 0; j < 16; j++) {
-    double dj = lane_bcast(a[j], j);
-    if (!(dj > 0.0)) {
-      nonpos = true;
-      dj = 1.0;
-    }
-    const bool below = lane > j && lane < 16;
-    const double l = below ? a[j] / dj : 0.0;
-    if (below) a[j] = l;
-    if (lane == j) a[j] = dj;
-    const double ldj = l * dj;
-#pragma unroll
-    for (int m = j + 1; m < 16; m++) {
-      const double lm = lane_bcast(l, m);  // L1[m][j]
-      if (m <= lane) a[m] -= ldj * lm;
-    }
-#pragma unroll
-    for (int m = 0; m <= j; m++) x[m] -= l * lane_bcast(x[m], j);  // X1[j][m]
-  }
-  if (nonpos && lane == 0) *bad = 1;
-  // lane i: D_i = a[i]; L1[i][m] = a[m] (m < i), X1[i][m] = x[m] (m <= i)
-  double sq[16];
-#pragma unroll
-  for (int m = 0; m < 16; m++) sq[m] = sqrt(lane_bcast(a[m], m));
-  if (lane >= n) return;
-  double si = 1.0;
-#pragma unroll
-  for (int m = 0; m < 16; m++) si = m == lane ? sq[m] : si;
-  const double ri = 1.0 / si;
-#pragma unroll
-  for (int m = 0; m < 16; m++) {
-    if (m >= n) break;
-    const double sm = sq[m];
-    // R[m][i] = sqrt(D_m) L1[i][m] (m < i), sqrt(D_i) on the diagonal, 0 above
-    R[m * n + lane] = m < lane ? sm * a[m] : (m == lane ? si : 0.0);
-    // R^-1[m][i] = X1[i][m] / sqrt(D_i) (m <= i)
-    Ri[m * n + lane] = m <= lane ? x[m] * ri : 0.0;
-  }
+// ---------------------------------------------------------------- Lanczos start block
+// Deterministic pseudo-random values in (-1/2, 1/2) on the first n1 rows of
+// the row-major neq x bs block, zeros below: entry g of the rows takes the
+// (g + 1)-th output of the SplitMix64 sequence of the seed (Steele, Lea and
+// Flood 2014), whose state is a plain multiple of the step, so every entry
+// stands alone.  Made here because the host took 3 ms and its copy 1.5 ms
+// for a 91,839 x 16 block, with the device idle (now 3 us).
+__global__ void k_start_block(int64_t n, int64_t n1, uint64_t seed, double* __restrict__ W) {
+  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= n) return;
+  uint64_t z = seed + (uint64_t)(g + 1) * 0x9E3779B97F4A7C15ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  W[g] = g < n1 ? (double)(z >> 11) * (1.0 / 9007199254740992.0) - 0.5 : 0.0;
 }
 
 // ---------------------------------------------------------------- mixed precision
@@ -1914,56 +1593,6 @@ void launch_spmm(hipStream_t st, int n, int nrhs, const int* rowptr, const int* 
     }
   }
 }
-int xty_chunks(int n) { return (n + XTY_ROWS - 1) / XTY_ROWS; }
-void launch_xty(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Y, int ldy,
-                double* part, double* C, double* acc, bool acc_add) {
-  if (na <= 0 || nb <= 0) return;
-  // wide products (many 64x64 output tiles) take longer row chunks: fewer
-  // partial matrices to write and add, still thousands of workgroups
-  const int tiles = ((na + 63) / 64) * ((nb + 63) / 64);
-  const int crows = tiles >= 16 ? 8 * XTY_ROWS : XTY_ROWS;
-  const int nch = (n + crows - 1) / crows;
-  if (nch == 0) {
-    launch_fill(st, C, (int64_t)na * nb, 0.0);
-    if (acc && !acc_add) launch_fill(st, acc, (int64_t)na * nb, 0.0);
-    return;
-  }
-  dim3 g(nch, (na + 63) / 64, (nb + 63) / 64);
-  if (tiles >= 16) k_xty_mfma<<<g, 256, 0, st>>>(n, crows, na, nb, X, ldx, Y, ldy, part);
-  else k_xty_part<<<g, 256, 0, st>>>(n, crows, na, nb, X, ldx, Y, ldy, part);
-  k_xty_sum<<<nblk((int64_t)na * nb, 4), 256, 0, st>>>(nch, na * nb, part, C, acc, acc_add ? 1 : 0);
-}
-void launch_gemm_small2(hipStream_t st, int n, int na, int nb, const double* X1, int ldx1, double* Y1, int ldy1,
-                        const double* X2, int ldx2, double* Y2, int ldy2, const double* Sm, double alpha,
-                        double beta) {
-  if (n <= 0 || nb <= 0) return;
-  if (nb > 16) {
-    launch_gemm_small(st, n, na, nb, X1, ldx1, Sm, Y1, ldy1, alpha, beta);
-    launch_gemm_small(st, n, na, nb, X2, ldx2, Sm, Y2, ldy2, alpha, beta);
-    return;
-  }
-  k_gemm_rows16<<<dim3((unsigned)((n + 63) / 64), 2), 256, 0, st>>>(n, na, nb, X1, ldx1, Sm, nb, Y1, ldy1, alpha,
-                                                                     beta, X2, ldx2, Y2, ldy2);
-}
-void launch_gemm_small(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Sm,
-                       double* Y, int ldy, double alpha, double beta) {
-  if (n <= 0 || nb <= 0) return;
-  if (nb <= 64) {  // MFMA over 64-row tiles, 16 columns of S per launch
-    for (int c0 = 0; c0 < nb; c0 += 16)
-      k_gemm_rows16<<<(unsigned)((n + 63) / 64), 256, 0, st>>>(n, na, std::min(16, nb - c0), X, ldx, Sm + c0, nb,
-                                                               Y + c0, ldy, alpha, beta, nullptr, 0, nullptr, 0);
-    return;
-  }
-  // S is staged in LDS in row chunks of at most 64 KiB; chunk k adds
-  // beta X_k S_k to the result of the chunks before it (fixed order)
-  const int rows = std::max(1, (int)(65536 / (sizeof(double) * nb)));
-  for (int a0 = 0; a0 < na || a0 == 0; a0 += rows) {
-    const int ka = std::min(rows, na - a0);
-    k_gemm_small<<<nblk((int64_t)n * nb, 256), 256, sizeof(double) * std::max(ka, 1) * nb, st>>>(
-        n, ka, nb, X + a0, ldx, Sm + (size_t)a0 * nb, Y, ldy, a0 == 0 ? alpha : 1.0, beta);
-    if (na <= 0) break;
-  }
-}
 void launch_mode_signs(hipStream_t st, int n1, const int* p1, double* Phi, int64_t nrows, int nev, double* sign) {
   if (nev <= 0) return;
   // sign[0 .. nev) is the result; the groups' bests follow it
@@ -1981,9 +1610,9 @@ void launch_emass(hipStream_t st, int n, const int* elist, int nen, int d, const
 void launch_sum_fixed(hipStream_t st, int n, const double* x, double* out) {
   k_sum_fixed<<<1, 256, 0, st>>>(n, x, out);
 }
-void launch_chol_inv(hipStream_t st, int n, const double* G, double* R, double* Ri, int* bad) {
-  if (n <= 16) k_chol16<<<1, 64, 0, st>>>(n, G, R, Ri, bad);
-  else k_chol_inv<<<1, 64, 0, st>>>(n, G, R, Ri, bad);
+void launch_start_block(hipStream_t st, int neq, int n1, int bs, uint64_t seed, double* W) {
+  const int64_t n = (int64_t)neq * bs;
+  if (n > 0) k_start_block<<<nblk(n, 256), 256, 0, st>>>(n, (int64_t)n1 * bs, seed, W);
 }
 void launch_diag_scale(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val, double* s) {
   if (n > 0) k_diag_scale<<<nblk(n, 256), 256, 0, st>>>(n, rowptr, colind, val, s);

@@ -101,24 +101,28 @@ int xty_chunks(int n);
 void launch_xty(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Y, int ldy,
                 double* part, double* C, double* acc = nullptr, bool acc_add = false);
 // Y = alpha Y + beta X S (X n x na, S na x nb, row-major); up to 64 columns
-// on FP64 MFMA, 16 columns of S per launch.  For nb <= 16, Y may be X itself
-// (same leading dimension): each row tile reads its rows before it writes
-// them.
+// on FP64 MFMA, where Y may be X itself (same leading dimension).
 void launch_gemm_small(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Sm,
                        double* Y, int ldy, double alpha, double beta);
-// the same for two pairs (X1 -> Y1, X2 -> Y2) with one S, in one launch
+// Y1 = X1 S and Y2 = X2 S in one launch (nb <= 64); dup (optional, leading
+// dimension ldd): a copy of Y2
 void launch_gemm_small2(hipStream_t st, int n, int na, int nb, const double* X1, int ldx1, double* Y1, int ldy1,
-                        const double* X2, int ldx2, double* Y2, int ldy2, const double* Sm, double alpha,
-                        double beta);
+                        const double* X2, int ldx2, double* Y2, int ldy2, const double* Sm, double* dup = nullptr,
+                        int ldd = 0);
 // sign convention of the modes Phi (nrows x nev row-major): largest-magnitude
 // internal component (rows p1[0..n1-1], equation order) made positive;
 // sign: nev * (1 + 3 * MODE_SIGN_GROUPS) doubles of scratch
 constexpr int MODE_SIGN_GROUPS = 256;
 void launch_mode_signs(hipStream_t st, int n1, const int* p1, double* Phi, int64_t nrows, int nev, double* sign);
 void launch_identity_rows(hipStream_t st, double* X, int64_t nrows, int nrhs, int ndof1);
-// Lanczos: G (n x n, n <= 64) = R^T R, R and R^-1 row-major; *bad = 1 if
-// G is not positive definite
-void launch_chol_inv(hipStream_t st, int n, const double* G, double* R, double* Ri, int* bad);
+// Lanczos start block: pseudo-random values on the first n1 of neq rows
+// (row-major, bs columns), zeros below
+void launch_start_block(hipStream_t st, int neq, int n1, int bs, uint64_t seed, double* W);
+// Lanczos: the Gram matrix G = X^T Y (bs x bs, bs <= 64, X and Y n x bs)
+// = R^T R, R and R^-1 row-major; *bad = 1 if G is not positive definite
+// (first: else 0)
+void launch_gram_inv(hipStream_t st, int n, int bs, const double* X, const double* Y, double* part, double* G,
+                     double* R, double* Ri, bool first, int* bad);
 // mixed precision: s = 1/sqrt(diag K) per perm row; equilibrated lower
 // entries of K into the FP32 fronts; X = diag(rs) X diag(cs) (cs may be
 // null); Y = a X + b Y; partial sums of squares of x and y over

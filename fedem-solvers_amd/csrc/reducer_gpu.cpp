@@ -228,10 +228,11 @@ struct DeviceReducer::Impl {
   std::vector<double> s22;  // mixed: Schur complement from the refined B (n2 x n2, column-major)
   // component modes
   DBuf<double> Q, P, Wl, Zl, Yl, Cc, Phi, Tmp;
-  DBuf<double> Cacc, Rdev;  // reorthogonalisation coefficients of a step; the two CholQR factors
-  DBuf<int> lzbad;
-  HBuf<double> hC, hR;  // two slots each (step parity)
-  HBuf<int> hbad;
+  // a Lanczos step's record for the host: the breakdown flag (an int in the
+  // first entry), the two CholQR factors, the reorthogonalisation
+  // coefficients; two pinned copies (step parity)
+  DBuf<double> lzrec;
+  HBuf<double> hrec;
   hipEvent_t lz_ev[2]{};
   hipStream_t side = nullptr;  // lookahead stream of the factorisation
   hipEvent_t fj[2]{};          // its fork and join events
@@ -1010,8 +1011,7 @@ int DeviceReducer::prepare_solves(std::string& err) {
     HIPCHK(d.Cc.alloc((size_t)mcap * std::max(bs, nev) + 64));
     HIPCHK(d.part.alloc((size_t)xty_chunks(neq) * mcap * std::max(bs, nev)));
     HIPCHK(d.small.alloc((size_t)mcap * mcap + 64));
-    HIPCHK(d.Cacc.alloc((size_t)mcap * bs));
-    HIPCHK(d.Rdev.alloc((size_t)2 * bs * bs));
+    HIPCHK(d.lzrec.alloc(1 + (size_t)2 * bs * bs + (size_t)mcap * bs));
     HIPCHK(d.signs.alloc((size_t)nev * (1 + 3 * MODE_SIGN_GROUPS)));
   }
   if (opt_.want_vgi && get_plan(y, d, 3, p, err)) return -3;
@@ -1480,64 +1480,45 @@ int DeviceReducer::reduce(std::string& err) {
     HIPCHK(d.Cc.alloc((size_t)mcap * std::max(bs, nev) + 64));
     HIPCHK(d.part.alloc((size_t)xty_chunks(neq) * mcap * std::max(bs, nev)));
     HIPCHK(d.small.alloc((size_t)mcap * mcap + 64));
-    HIPCHK(d.Cacc.alloc((size_t)mcap * bs));
-    HIPCHK(d.Rdev.alloc((size_t)2 * bs * bs));
-    HIPCHK(d.lzbad.alloc(1));
-    HIPCHK(d.hC.alloc((size_t)2 * mcap * bs));
-    HIPCHK(d.hR.alloc((size_t)4 * bs * bs));
-    HIPCHK(d.hbad.alloc(2));
+    const size_t nrec = 1 + (size_t)2 * bs * bs, slot = nrec + (size_t)mcap * bs;
+    HIPCHK(d.lzrec.alloc(slot));
+    HIPCHK(d.hrec.alloc(2 * slot));
+    double *const Rdev = d.lzrec.p + 1, *const Cacc = d.lzrec.p + nrec;
+    int* const lzbad = reinterpret_cast<int*>(d.lzrec.p);
     for (auto& e : d.lz_ev)
       if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    // start block: deterministic pseudo-random values on the internal rows
-    {
-      std::vector<double> q0((size_t)neq * bs, 0.0);
-      uint64_t s = opt_.seed;
-      for (int r = 0; r < n1; r++)
-        for (int j = 0; j < bs; j++) {
-          s += 0x9E3779B97F4A7C15ull;
-          uint64_t z = s;
-          z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-          z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-          z ^= z >> 31;
-          q0[(size_t)r * bs + j] = (double)(z >> 11) * (1.0 / 9007199254740992.0) - 0.5;
-        }
-      HIPCHK(hipMemcpyAsync(d.Wl.p, q0.data(), q0.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    }
-    std::vector<double> Cfull;
+    // start block: pseudo-random values on the internal rows, zero boundary
+    // rows, which every step leaves alone
+    launch_start_block(st, neq, n1, bs, opt_.seed, d.Wl.p);
     std::vector<double> H((size_t)mcap * mcap, 0.0);
-    // M-orthonormalise W into block j of Q (and M W into P); returns R with W = Q_j R
     // Block M-orthonormalisation of W (CholQR twice): G = W^T M W = R^T R on
-    // the device, W <- W R^-1, M W <- (M W) R^-1, then Q_j = W and P_j = M W.
-    // orth_issue queues the work and the copies of both R factors and the
-    // breakdown flag to host slot `par`; orth_finish (after the stream has
-    // passed them) forms R_tot = R_2 R_1.
-    auto orth_issue = [&](int j, int par) -> int {
-      HIPCHK(hipMemsetAsync(d.lzbad.p, 0, sizeof(int), st));
+    // the device, W <- W R^-1, M W <- (M W) R^-1, then Q_j = W and P_j = M W
+    // (also in Tmp, the next solve's right-hand side).  orth_issue queues the
+    // work, copy_rec the copy of the step's record with its first nc
+    // coefficients to host slot `par`; orth_finish (after the stream has
+    // passed it) forms R_tot = R_2 R_1, W = Q_j R_tot.
+    auto orth_issue = [&](int j) {
       // M W is formed once: the second pass's M (W R_1^-1) is (M W) R_1^-1
       launch_spmm(st, neq, bs, d.rowptr.p, d.colind.p, d.Mv.p, d.Wl.p, bs, d.Zl.p, bs, d.m_lumped);
-      // the first pass rescales W and M W (in place for blocks of up to 16
-      // columns), the second writes block j of Q and P
-      const bool inplace = bs <= 16;
       for (int pass = 0; pass < 2; pass++) {
-        launch_xty(st, neq, bs, bs, d.Wl.p, bs, d.Zl.p, bs, d.part.p, d.Cc.p);
-        launch_chol_inv(st, bs, d.Cc.p, d.Rdev.p + (size_t)pass * bs * bs, d.small.p, d.lzbad.p);
-        double* qo = pass ? d.Q.p + (size_t)j * bs : (inplace ? d.Wl.p : d.Tmp.p);
-        double* po = pass ? d.P.p + (size_t)j * bs : (inplace ? d.Zl.p : d.Yl.p);
-        const int ldo = pass ? mcap : bs;
-        launch_gemm_small2(st, neq, bs, bs, d.Wl.p, bs, qo, ldo, d.Zl.p, bs, po, ldo, d.small.p, 0.0, 1.0);
-        if (pass == 0 && !inplace) {
-          HIPCHK(hipMemcpyAsync(d.Wl.p, d.Tmp.p, sizeof(double) * neq * bs, hipMemcpyDeviceToDevice, st));
-          HIPCHK(hipMemcpyAsync(d.Zl.p, d.Yl.p, sizeof(double) * neq * bs, hipMemcpyDeviceToDevice, st));
-        }
+        launch_gram_inv(st, neq, bs, d.Wl.p, d.Zl.p, d.part.p, d.Cc.p, Rdev + (size_t)pass * bs * bs, d.small.p,
+                        pass == 0, lzbad);
+        // the first pass rescales in place, the second writes block j
+        if (pass == 0) launch_gemm_small2(st, neq, bs, bs, d.Wl.p, bs, d.Wl.p, bs, d.Zl.p, bs, d.Zl.p, bs, d.small.p);
+        else
+          launch_gemm_small2(st, neq, bs, bs, d.Wl.p, bs, d.Q.p + (size_t)j * bs, mcap, d.Zl.p, bs,
+                             d.P.p + (size_t)j * bs, mcap, d.small.p, d.Tmp.p, bs);
       }
-      HIPCHK(hipMemcpyAsync(d.hR.p + (size_t)par * 2 * bs * bs, d.Rdev.p, sizeof(double) * 2 * bs * bs,
-                            hipMemcpyDeviceToHost, st));
-      HIPCHK(hipMemcpyAsync(d.hbad.p + par, d.lzbad.p, sizeof(int), hipMemcpyDeviceToHost, st));
-      return 0;
+    };
+    auto copy_rec = [&](int par, size_t nc) {
+      return hipMemcpyAsync(d.hrec.p + par * slot, d.lzrec.p, sizeof(double) * (nrec + nc), hipMemcpyDeviceToHost, st);
     };
     auto orth_finish = [&](int par, std::vector<double>& Rtot) -> int {
-      if (d.hbad.p[par]) { err = "Lanczos: block breakdown (Gram matrix not positive definite)"; return -6; }
-      const double* R1 = d.hR.p + (size_t)par * 2 * bs * bs;
+      if (*reinterpret_cast<const int*>(d.hrec.p + par * slot)) {
+        err = "Lanczos: block breakdown (Gram matrix not positive definite)";
+        return -6;
+      }
+      const double* R1 = d.hrec.p + par * slot + 1;
       const double* R2 = R1 + (size_t)bs * bs;
       Rtot.assign((size_t)bs * bs, 0.0);
       for (int a = 0; a < bs; a++)
@@ -1549,7 +1530,8 @@ int DeviceReducer::reduce(std::string& err) {
       return 0;
     };
     std::vector<double> R0;
-    if ((rc = orth_issue(0, 0))) return rc;
+    orth_issue(0);
+    HIPCHK(copy_rec(0, 0));
     HIPCHK(hipStreamSynchronize(st));
     if ((rc = orth_finish(0, R0))) return rc;
     int nb = 0;  // number of completed blocks in H
@@ -1615,11 +1597,8 @@ int DeviceReducer::reduce(std::string& err) {
     // never waits for the host between blocks.
     auto issue_step = [&](int j) -> int {
       const int mj = (j + 1) * bs, par = j & 1;
-      HIPCHK(hipMemcpy2DAsync(d.Tmp.p, sizeof(double) * bs, d.P.p + (size_t)j * bs, sizeof(double) * mcap,
-                              sizeof(double) * bs, neq, hipMemcpyDeviceToDevice, st));
       auto solve_step = [&]() {
         run_forward(st, d, *pl, d.Tmp.p, d.Yl.p);
-        launch_fill(st, d.Wl.p + (size_t)n1 * bs, (int64_t)(neq - n1) * bs, 0.0);  // boundary rows stay zero
         run_backward(st, d, *pl, d.Yl.p, d.Wl.p);
       };
       if (d.mixed) {
@@ -1630,13 +1609,11 @@ int DeviceReducer::reduce(std::string& err) {
                         d.S.rows, d.S.dpiv}, solve_step));
       for (int pass = 0; pass < 2; pass++) {
         // coefficients of the pass into Cc, their running sum into Cacc
-        launch_xty(st, neq, mj, bs, d.P.p, mcap, d.Wl.p, bs, d.part.p, d.Cc.p, d.Cacc.p, pass > 0);
+        launch_xty(st, neq, mj, bs, d.P.p, mcap, d.Wl.p, bs, d.part.p, d.Cc.p, Cacc, pass > 0);
         launch_gemm_small(st, neq, mj, bs, d.Q.p, mcap, d.Cc.p, d.Wl.p, bs, 1.0, -1.0);
       }
-      HIPCHK(hipMemcpyAsync(d.hC.p + (size_t)par * mcap * bs, d.Cacc.p, sizeof(double) * mj * bs,
-                            hipMemcpyDeviceToHost, st));
-      if (mj + bs <= mcap)
-        if (int rc2 = orth_issue(j + 1, par)) return rc2;
+      if (mj + bs <= mcap) orth_issue(j + 1);
+      HIPCHK(copy_rec(par, (size_t)mj * bs));
       HIPCHK(hipEventRecord(d.lz_ev[par], st));
       return 0;
     };
@@ -1646,7 +1623,7 @@ int DeviceReducer::reduce(std::string& err) {
       const bool last = mj + bs > mcap;
       if (!last && (rc = issue_step(j + 1))) return rc;
       HIPCHK(hipEventSynchronize(d.lz_ev[par]));
-      const double* hc = d.hC.p + (size_t)par * mcap * bs;
+      const double* hc = d.hrec.p + par * slot + nrec;
       for (int a = 0; a < mj; a++)
         for (int b = 0; b < bs; b++) H[(size_t)a * mcap + j * bs + b] = hc[(size_t)a * bs + b];
       nb = j + 1;
