@@ -233,64 +233,120 @@ __global__ void k_fill(double* __restrict__ p, int64_t n, double v) {
   for (; i < n; i += stride) p[i] = v;
 }
 
-// ---------------------------------------------------------------- extend-add
-#define XADD_REL 4096
-// Task: sn = parent front, a = first parent column of a 16-column block.  The
-// workgroup adds, child after child, every child update-matrix column whose
-// parent column falls in its block; the task's b/kb index the (child,
-// first, end) column ranges in xrange, found when the schedule was built.
-// Blocks are disjoint, so no two workgroups touch the same parent entry;
-// children are added in list order.
+// ---------------------------------------------------------------- front values
+// The part of a front that no extend-add writes is cleared before the original
+// entries are scattered into it: its own columns (the first ncol, which hold
+// every original entry of a front but the Schur front's), and all of it where
+// the front has no children or is the Schur front.  Task: sn, a = first of 16
+// columns, k0 = end of the own columns; rows from the column block down (only
+// the lower triangle has a meaning).
+// Bound by HBM writes.  Clearing the whole pool took 3.0 ms for the 45x41x43
+// block, this 0.8 ms.
+template <class T>
+__global__ __launch_bounds__(256) void k_front_zero(const FTask* __restrict__ tasks, DevSym S, T* __restrict__ pool) {
+  const FTask t = tasks[blockIdx.x];
+  const int ld = S.nrow[t.sn], lane = threadIdx.x & 63;
+  T* F = pool + S.foff[t.sn];
+  for (int j = t.a + (threadIdx.x >> 6); j < min(t.a + 16, t.k0); j += 4) {
+    T* col = F + (int64_t)j * ld;
+#pragma unroll 4
+    for (int i = t.a + lane; i < ld; i += 64) col[i] = (T)0;
+  }
+}
+
+// Task: sn = parent front, a = first parent column of a 16-column block, k0 =
+// end of the own columns (above); blockIdx.y takes 512 of its rows from
+// column a down.  The front's entries are gathered: the workgroup finds, child
+// after child, which child row and column lands on each of its rows and
+// columns (b/kb index the (child, first, end) column ranges in xrange, found
+// when the schedule was built; the rows by a search in the child's sorted
+// parent positions), adds the child's entries in registers and stores the
+// block once.  Only own columns are read, the others start at zero, so the
+// update part of a front is neither cleared nor read and written once per
+// child.  Children are added in list order.
+// Bound by HBM: one read of the children's update matrices and one write of
+// the front.  Scattering each child into a cleared front took 7.1 + 3.0 ms
+// for the 45x41x43 block, this 4.6 + 0.8 (18 GB: 4.0 TB/s), for the 48x24x24
+// block 1.5 + 0.6 and 1.1 + 0.2.
+constexpr int XADD_ROWS = 512;
+
 template <class T>
 __global__ __launch_bounds__(256) void k_extend_add(const FTask* __restrict__ tasks, DevSym S,
                                                     const int* __restrict__ xrange, T* __restrict__ pool) {
-  // the child's parent positions rel[a..nu) staged in LDS (when they fit),
-  // so that the parent loads of a batch wait on one memory round, not two
-  __shared__ int srel[XADD_REL];
+  __shared__ int srow[2][XADD_ROWS], scol[2][16];
   const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
-  const int sn = t.sn;
-  const int ldp = S.nrow[sn];
+  const int sn = t.sn, ld = S.nrow[sn], own = t.k0, c0 = t.a, tid = threadIdx.x, lane = tid & 63;
+  const int r0 = c0 + XADD_ROWS * blockIdx.y;
+  if (r0 >= ld || (t.kb == 0 && c0 + 16 <= own)) return;
   T* P = pool + S.foff[sn];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int halves = ld - r0 > 256 ? 2 : 1;  // 256 rows each
+  T acc[2][16];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int r = r0 + 256 * h + tid;
+#pragma unroll
+    for (int c = 0; c < 16; c++) acc[h][c] = (T)0;
+    if (c0 < own && h < halves) {
+      const T* p = P + min(r, ld - 1);
+#pragma unroll
+      for (int c = 0; c < 16; c++) acc[h][c] = p[(int64_t)min(c0 + c, own - 1) * ld];
+#pragma unroll
+      for (int c = 0; c < 16; c++) acc[h][c] = c0 + c < own ? acc[h][c] : (T)0;
+    }
+  }
   for (int q = 0; q < t.kb; q++) {
     const int* xr = xrange + 3 * (t.b + q);
-    const int c = xr[0], a = xr[1], b = xr[2];
-    const int nc = S.ncol[c], ldc = S.nrow[c], nu = ldc - nc;
-    const int* rel = S.rel + S.relptr[c];
-    const T* C = pool + S.foff[c] + (int64_t)nc * ldc + nc;
-    const bool staged = nu - a <= XADD_REL;
-    if (staged) {
-      for (int i = a + (int)threadIdx.x; i < nu; i += 256) srel[i - a] = rel[i];
-      __syncthreads();
+    const int ch = xr[0], a = xr[1], b = xr[2];
+    const int nc = S.ncol[ch], ldc = S.nrow[ch], nu = ldc - nc;
+    const int* rel = S.rel + S.relptr[ch];
+    int* row = srow[q & 1];
+    int* col = scol[q & 1];
+    // a buffer is free once every thread has passed the barrier after the
+    // next child's maps were made
+    row[tid] = -1;
+    row[tid + 256] = -1;
+    if (tid < 16) col[tid] = -1;
+    // first child row at or past r0: 64 probes a round, every wave for itself
+    int lo = a, hi = blockIdx.y == 0 ? a : nu;
+    while (lo < hi) {
+      const int step = (hi - lo + 63) >> 6, at = lo + lane * step;
+      const int less = __popcll(__ballot(at < hi && rel[min(at, hi - 1)] < r0));
+      if (less == 0) break;
+      hi = min(hi, lo + less * step);
+      lo += (less - 1) * step + 1;
     }
-    // rl(i) = rel[i] for i >= a, from LDS or from memory
-    auto columns = [&](auto rl) {
-      for (int jj = a + w; jj < b; jj += 4) {
-        const int pc = rl(jj);
-        T* dst = P + (int64_t)pc * ldp;
-        const T* src = C + (int64_t)jj * ldc;
-        // the rows of one child column land in distinct parent rows, so
-        // eight iterations' loads go out before their stores
-        for (int i0 = jj + lane; i0 < nu; i0 += 64 * 8) {
-          int pr[8];
-          T v[8], o[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) {
-            const int ii = i0 + 64 * u;
-            pr[u] = ii < nu ? rl(ii) : -1;
-            v[u] = ii < nu ? src[ii] : (T)0;
-          }
-#pragma unroll
-          for (int u = 0; u < 8; u++) o[u] = pr[u] >= 0 ? dst[pr[u]] : (T)0;
-#pragma unroll
-          for (int u = 0; u < 8; u++)
-            if (pr[u] >= 0) dst[pr[u]] = o[u] + v[u];
-        }
-      }
-    };
-    if (staged) columns([&](int i) { return srel[i - a]; });
-    else columns([&](int i) { return rel[i]; });
     __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int i = lo + 256 * h + tid;
+      const int p = rel[min(i, nu - 1)] - r0;
+      if (i < nu && p < XADD_ROWS) row[p] = i;
+    }
+    if (tid < b - a) col[rel[a + tid] - c0] = a + tid;
+    __syncthreads();
+    const T* C = pool + S.foff[ch] + (int64_t)nc * ldc + nc;
+    int jj[16];
+#pragma unroll
+    for (int c = 0; c < 16; c++) jj[c] = __builtin_amdgcn_readfirstlane(col[c]);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int i = row[256 * h + tid];
+      if (h >= halves || !__any(i >= 0)) continue;
+      const T* src = C + max(i, a);  // unmatched rows and columns read another entry and drop it
+      T v[16];
+#pragma unroll
+      for (int c = 0; c < 16; c++) v[c] = src[(int64_t)max(jj[c], a) * ldc];
+#pragma unroll
+      for (int c = 0; c < 16; c++) acc[h][c] = jj[c] >= 0 && i >= jj[c] ? acc[h][c] + v[c] : acc[h][c];
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int r = r0 + 256 * h + tid;
+    if (r >= ld) continue;
+#pragma unroll
+    for (int c = 0; c < 16; c++)
+      if (r >= c0 + c) P[r + (int64_t)(c0 + c) * ld] = acc[h][c];
   }
 }
 
@@ -1538,9 +1594,12 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
   if (n > 0) k_fill<<<(unsigned)std::min<int64_t>(nblk(n, 256), 16384), 256, 0, st>>>(p, n, v);
 }
 #define FGPU_FACTOR_LAUNCHERS(T)                                                                           \
-  void launch_extend_add(hipStream_t st, const FTask* t, int n, const DevSym& S, const int* xrange,        \
-                         T* pool) {                                                                        \
-    if (n > 0) k_extend_add<T><<<n, 256, 0, st>>>(t, S, xrange, pool);                                       \
+  void launch_front_zero(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {                \
+    if (n > 0) k_front_zero<T><<<n, 256, 0, st>>>(t, S, pool);                                               \
+  }                                                                                                        \
+  void launch_extend_add(hipStream_t st, const FTask* t, int n, int rows, const DevSym& S,                 \
+                         const int* xrange, T* pool) {                                                     \
+    if (n > 0) k_extend_add<T><<<dim3(n, nblk(rows, XADD_ROWS)), 256, 0, st>>>(t, S, xrange, pool);          \
   }                                                                                                        \
   void launch_diag(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,   \
                    T* ipool, int* piv) {                                                                   \

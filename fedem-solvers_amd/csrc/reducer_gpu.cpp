@@ -110,13 +110,14 @@ struct HBuf {
 };
 
 enum OpKind {
+  FRONT_ZERO,  // the first of the factor schedule, issued before the assembly
   EXTADD, DIAG, TRSM, DIAG_TRSM, UPDATE, INV_OFF, INV_PART, INV_FIN, PANEL,
   UPDATE_SIDE, FORK, JOIN,  // lookahead: trailing tiles on the side stream, fork/join with the main one
   FW_INIT, FW_MV, BW_ROWS, BW_MV  // solve plans
 };
 struct Op {
   int kind, off, n;
-  int kw = 1;  // solve products: K parts per workgroup
+  int kw = 1;  // solve products: K parts per workgroup; extend-add: rows of the largest front
 };
 
 // Where the solve panels lie and which levels are fused (solve.hip).
@@ -299,18 +300,25 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
   xrange.clear();
   inv_slots = 0;
   flops = 0;
+  // columns of a front cleared before the original entries go in (k_front_zero),
+  // the largest fronts first
+  auto own = [&](int s) { return y.chptr[s + 1] == y.chptr[s] || s == y.nsup - 1 ? y.nrow[s] : y.ncol[s]; };
+  for (int s = y.nsup - 1; s >= 0; s--)
+    for (int j0 = 0; j0 < own(s); j0 += 16) tasks.push_back({s, j0, 0, own(s), 0, 0});
+  ops.push_back({FRONT_ZERO, 0, (int)tasks.size()});
   for (int l = 0; l < y.nlevels; l++) {
     const int* sups = &y.lvsup[y.lvptr[l]];
     const int ns = y.lvptr[l + 1] - y.lvptr[l];
-    int off = (int)tasks.size();
+    int off = (int)tasks.size(), rows = 0;
     for (int q = 0; q < ns; q++) {
       int s = sups[q];
       if (y.chptr[s + 1] == y.chptr[s]) continue;
+      rows = std::max(rows, y.nrow[s]);
       // extend-add task (front s, 16-column block j0): the (child, first,
       // end) ranges of child update columns landing in the block, in child
       // order, at xrange[3 b ..], kb of them
       for (int j0 = 0; j0 < y.nrow[s]; j0 += 16) {
-        FTask t{s, j0, (int)xrange.size() / 3, 0, 0, 0};
+        FTask t{s, j0, (int)xrange.size() / 3, own(s), 0, 0};
         for (int q = y.chptr[s]; q < y.chptr[s + 1]; q++) {
           const int c = y.chlist[q], nu = y.nrow[c] - y.ncol[c];
           const int* rel = y.rel.data() + y.relptr[c];
@@ -326,7 +334,7 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
         tasks.push_back(t);
       }
     }
-    if ((int)tasks.size() > off) ops.push_back({EXTADD, off, (int)tasks.size() - off});
+    if ((int)tasks.size() > off) ops.push_back({EXTADD, off, (int)tasks.size() - off, rows});
     int maxnc = 0;
     for (int q = 0; q < ns; q++) maxnc = std::max(maxnc, y.ncol[sups[q]]);
     // Pivot columns go in panels of up to P columns (sub-panels of 64): for
@@ -1278,9 +1286,9 @@ int DeviceReducer::reduce(std::string& err) {
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(d.ev[1], st));
   // ---- assembly (CSR K, M and the K entries of the fronts)
-  // fronts start at zero (eager, outside any graph capture)
-  if (d.mixed) HIPCHK(hipMemsetAsync(d.pool32.p, 0, sizeof(float) * y.fpool, st));
-  else HIPCHK(hipMemsetAsync(d.pool.p, 0, sizeof(double) * y.fpool, st));
+  const Op& fz = d.fops.front();
+  if (d.mixed) launch_front_zero(st, d.ftasks.p + fz.off, fz.n, d.S, d.pool32.p);
+  else launch_front_zero(st, d.ftasks.p + fz.off, fz.n, d.S, d.pool.p);
   launch_assemble(st, nnz, d.cptr.p, d.cidx.p, y.has_rigid ? d.ccoef.p : nullptr, d.Kp.p, d.Mp.p, d.Kv.p, d.Mv.p,
                   d.fmap.p, d.mixed ? nullptr : d.pool.p);
   if (d.mixed) {  // equilibrated stiffness into the FP32 fronts
@@ -1313,7 +1321,7 @@ int DeviceReducer::reduce(std::string& err) {
   auto factor_with = [&](auto* pool, auto* ipool) {
     for (const Op& op : d.fops) {
       switch (op.kind) {
-        case EXTADD: launch_extend_add(st, d.ftasks.p + op.off, op.n, d.S, d.xrange.p, pool); break;
+        case EXTADD: launch_extend_add(st, d.ftasks.p + op.off, op.n, op.kw, d.S, d.xrange.p, pool); break;
         case DIAG: launch_diag(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool, d.piv.p); break;
         case TRSM: launch_trsm(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
         case DIAG_TRSM: launch_diag_trsm(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool, d.piv.p); break;
