@@ -181,7 +181,7 @@ static hipError_t run_graph(hipStream_t st, GraphCache& gc, const std::vector<co
 }
 
 struct DeviceReducer::Impl {
-  GraphCache g_factor, g_lanczos;
+  GraphCache g_factor;
   int factor_runs = 0;  // factorisations since the last upload
   // part
   DBuf<double> xyz, eprop;
@@ -884,7 +884,6 @@ int DeviceReducer::upload(std::string& err) {
   // a new structure: every captured launch sequence is stale
   d.g_factor.reset();
   d.factor_runs = 0;
-  d.g_lanczos.reset();
   // value buffers
   const int64_t nnz = y.rowptr[y.neq];
   HIPCHK(d.Kp.alloc(y.elem_pool));
@@ -1605,16 +1604,15 @@ int DeviceReducer::reduce(std::string& err) {
     // never waits for the host between blocks.
     auto issue_step = [&](int j) -> int {
       const int mj = (j + 1) * bs, par = j & 1;
-      auto solve_step = [&]() {
-        run_forward(st, d, *pl, d.Tmp.p, d.Yl.p);
-        run_backward(st, d, *pl, d.Yl.p, d.Wl.p);
-      };
       if (d.mixed) {
         if (int rc2 = solve_int(st, d, y, opt_, *pl, d.Tmp.p, d.Yl.p, d.Wl.p, nullptr, err)) return rc2;
-      } else if (!opt_.use_graphs) solve_step();
-      else HIPCHK(run_graph(st, d.g_lanczos,
-                       {pl, pl->tasks.p, pl->inits.p, d.gptr.p, d.Tmp.p, d.Yl.p, d.Wl.p, d.W.p, d.V.p, d.pool.p, d.ipool.p,
-                        d.S.rows, d.S.dpiv}, solve_step));
+      } else {
+        // launch by launch: a captured graph of the two passes costs more to
+        // start and to join than it saves (17x13x11 block 5.61 against 5.50 ms,
+        // 450-element frame 4.40 / 4.30, 48x24x24 block 66.4 / 66.0)
+        run_forward(st, d, *pl, d.Tmp.p, d.Yl.p);
+        run_backward(st, d, *pl, d.Yl.p, d.Wl.p);
+      }
       for (int pass = 0; pass < 2; pass++) {
         // coefficients of the pass into Cc, their running sum into Cacc
         launch_xty(st, neq, mj, bs, d.P.p, mcap, d.Wl.p, bs, d.part.p, d.Cc.p, Cacc, pass > 0);
@@ -2089,8 +2087,7 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
     d.solve_split = KS;
     opt_.solve_split = KS;
     d.plans.clear();
-    d.g_lanczos.reset();
-  };
+    };
   // warm-up (allocations, first captures), then one timed reduction per candidate
   if (int rc = reduce(err)) return rc;
   double best = INFINITY;

@@ -23,7 +23,7 @@ struct ReduceOptions {
   bool want_vgi = false;   // K_ii^{-1} g_i (dispfile)
   bool no_mass = false;
   bool time_updates = false;  // bracket every trailing-update launch with HIP events
-  bool use_graphs = true;     // replay the factorisation and Lanczos solve steps as HIP graphs
+  bool use_graphs = true;     // replay the factorisation as a HIP graph
   // Mixed precision: FP32 fronts of the equilibrated K (FP32 MFMA trailing
   // and Schur updates, FP64 diagonal-block factorisation), every solve with
   // K_ii refined against the FP64 matrix until the correction falls below
