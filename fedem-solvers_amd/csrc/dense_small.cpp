@@ -150,15 +150,16 @@ namespace {
 
 // Householder tridiagonalisation of A (row-major, destroyed); reflector k is
 // stored in R row k (entries k+1..n-1, unit 2-norm), beta[k] = 0 when skipped.
+template <class Stop>
 void tridiag(int n, std::vector<double>& A, std::vector<double>& R, std::vector<char>& used, std::vector<double>& d,
-             std::vector<double>& e) {
+             std::vector<double>& e, Stop&& stopped) {
   // Householder reduction working on the lower triangle only (row-major
   // storage, A[i*n + j] with j <= i): p = A v as a symmetric product, then
   // the rank-2 update A -= v q^T + q v^T on the lower triangle.
   R.assign((size_t)n * n, 0.0);
   used.assign(n, 0);
   std::vector<double> p(n), q(n);
-  for (int k = 0; k + 2 < n; k++) {
+  for (int k = 0; k + 2 < n && !stopped(); k++) {
     double nrm = 0.0;
     for (int i = k + 1; i < n; i++) nrm += A[(size_t)i * n + k] * A[(size_t)i * n + k];
     nrm = std::sqrt(nrm);
@@ -219,8 +220,9 @@ void tridiag(int n, std::vector<double>& A, std::vector<double>& R, std::vector<
 }
 
 // eigenvalues of the symmetric tridiagonal (d, e) by implicit QL (no vectors)
-void tql_values(int n, std::vector<double> d, std::vector<double> e, std::vector<double>& w) {
-  for (int l = 0; l < n; l++) {
+template <class Stop>
+void tql_values(int n, std::vector<double> d, std::vector<double> e, std::vector<double>& w, Stop&& stopped) {
+  for (int l = 0; l < n && !stopped(); l++) {
     int iter = 0;
     while (true) {
       int m = l;
@@ -302,17 +304,19 @@ void trisolve(int n, const std::vector<double>& d, const std::vector<double>& e,
 
 }  // namespace
 
-void sym_eig_top(int n, const std::vector<double>& Ain, int k, std::vector<double>& w, std::vector<double>& V) {
+bool sym_eig_top(int n, const std::vector<double>& Ain, int k, std::vector<double>& w, std::vector<double>& V,
+                 const std::atomic<bool>* stop) {
+  auto stopped = [stop]() { return stop && stop->load(std::memory_order_relaxed); };
   std::vector<double> A(Ain), R, d, e;
   std::vector<char> used;
-  tridiag(n, A, R, used, d, e);
-  tql_values(n, d, e, w);
+  tridiag(n, A, R, used, d, e, stopped);
+  tql_values(n, d, e, w, stopped);
   k = std::min(k, n);
   V.assign((size_t)n * k, 0.0);
   double scale = 0.0;
   for (int i = 0; i < n; i++) scale = std::max(scale, std::fabs(w[i]));
   std::vector<std::vector<double>> Z;  // tridiagonal eigenvectors
-  for (int c = 0; c < k; c++) {
+  for (int c = 0; c < k && !stopped(); c++) {
     const double lam = w[n - 1 - c];
     std::vector<double> x(n);
     for (int i = 0; i < n; i++) x[i] = 1.0 + 0.01 * ((i * 7919) % 101);
@@ -343,6 +347,7 @@ void sym_eig_top(int n, const std::vector<double>& Ain, int k, std::vector<doubl
     }
     for (int i = 0; i < n; i++) V[(size_t)i * k + c] = x[i];
   }
+  return !stopped();
 }
 
 int sym_gen_eig_lowest(int n, const double* A, const double* B, int nval, double* lambda) {

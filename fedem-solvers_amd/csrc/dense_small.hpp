@@ -2,6 +2,7 @@
 // Gram matrices of the Lanczos process and its projected eigenproblem).
 // Sizes are at most a few hundred; everything is row-major.
 #pragma once
+#include <atomic>
 #include <vector>
 
 namespace fgpu {
@@ -18,8 +19,10 @@ void sym_eig(int n, const std::vector<double>& A, std::vector<double>& w, std::v
 // V (n x k row-major, column c belongs to w[n-1-c]): Householder
 // tridiagonalisation with stored reflectors, implicit QL for the
 // eigenvalues, inverse iteration on the tridiagonal (clusters kept
-// orthogonal), back-transformation by the reflectors.
-void sym_eig_top(int n, const std::vector<double>& A, int k, std::vector<double>& w, std::vector<double>& V);
+// orthogonal), back-transformation by the reflectors.  False, with w and V
+// unspecified, if *stop (optional) became true on the way.
+bool sym_eig_top(int n, const std::vector<double>& A, int k, std::vector<double>& w, std::vector<double>& V,
+                 const std::atomic<bool>* stop = nullptr);
 
 // Lowest nval eigenvalues (ascending) of the generalized problem A z = l B z
 // with A symmetric and B symmetric positive definite (the task of LAPACK
