@@ -109,6 +109,7 @@ struct Symbolic {
   // built on the device from the arrays below (structure.hip)
   std::vector<int> rowptr;
   std::vector<int> nfirst, neqd;      // per node: first perm equation (-1: none), equation count
+  std::vector<int> nrow0;             // first row of every node with equations, in row order, then neq
   std::vector<int> nbptr, nbl;        // per node: neighbour nodes through elements, itself included
   std::vector<int> rnode;             // per perm row: its node
   std::vector<int> colsn;             // per perm column: the front that eliminates it (Schur front last)

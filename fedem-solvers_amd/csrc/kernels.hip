@@ -197,18 +197,26 @@ __global__ __launch_bounds__(256) void k_assemble(int64_t nnz, const int* __rest
 
 // original diagonal a_jj of the first n permuted equations (times rs_j^2 when
 // rs is given: the equilibrated matrix) and the largest |a_jj| in *amax
-// (non-negative doubles order as their bit patterns; *amax starts at 0)
-__global__ void k_diag_extract(int n, const int* __restrict__ rowptr, const int* __restrict__ colind,
-                               const double* __restrict__ val, const double* __restrict__ rs,
-                               double* __restrict__ adiag, unsigned long long* __restrict__ amax) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  double a = 0.0;
-  for (int k = rowptr[r]; k < rowptr[r + 1]; k++)
-    if (colind[k] == r) a = val[k];
-  if (rs) a *= rs[r] * rs[r];
-  adiag[r] = a;
-  atomicMax(amax, (unsigned long long)__double_as_longlong(fabs(a)));
+// (non-negative doubles order as their bit patterns; *amax starts at 0).  One
+// atomic per workgroup: one per thread on the one address, and a walk along
+// the row to its diagonal, took 14 us for 354 rows and 48 for 77,496 (now 4 and 6).
+__global__ __launch_bounds__(256) void k_diag_extract(int n, const int* __restrict__ dpos,
+                                                      const double* __restrict__ val, const double* __restrict__ rs,
+                                                      double* __restrict__ adiag, unsigned long long* __restrict__ amax) {
+  __shared__ double top[4];
+  double big = 0.0;
+  for (int r = blockIdx.x * 256 + threadIdx.x; r < n; r += gridDim.x * 256) {
+    double a = val[dpos[r]];
+    if (rs) a *= rs[r] * rs[r];
+    adiag[r] = a;
+    big = fabs(a) > big ? fabs(a) : big;
+  }
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) big = fmax(big, __shfl_xor(big, off));
+  if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = big;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    atomicMax(amax, (unsigned long long)__double_as_longlong(fmax(fmax(top[0], top[1]), fmax(top[2], top[3]))));
 }
 
 // pivot statistics of the factor: out[0] negative pivots, out[1] true-zero
@@ -1185,139 +1193,116 @@ __global__ __launch_bounds__(256) void k_panel(const FTask* __restrict__ tasks, 
 
 // ---------------------------------------------------------------- products
 // Z = A X for the full symmetric CSR matrix A (perm space), X, Z row-major.
-template <bool SKIP>
-__global__ __launch_bounds__(256) void k_spmm(int n, int nrhs, const int* __restrict__ rowptr,
-                                              const int* __restrict__ colind,
-                                              const double* __restrict__ val,
-                                              const double* __restrict__ X, int ldx,
+// The rows of a node are neighbours and share their column list (the CSR rows
+// are built from the node neighbours), so a wave takes the rows of one node,
+// RB at a time, and gathers each row of X once for all of them.  It brings 64
+// entries of the list and their values into its own LDS by loads of
+// neighbouring places, the next 64 under the products, and its groups of W
+// lanes take every (64 / W)-th entry: a lane gathers VEC neighbouring columns,
+// NC times W VEC apart.  The groups' sums are added at the end; blockIdx.y
+// takes the next W VEC NC columns.
+// Bound by the load instructions of the gather (values and indices read by
+// each group from memory: 2.5 times the time).  48x24x24 block (7.0 million
+// entries) by 16 columns 92 -> 39 us, 45x41x43 194 -> 94, 90x84 plate by 66
+// 142 -> 62, where a thread had a row and four columns.
+template <int W, int VEC, int RB, int NC>
+__global__ __launch_bounds__(256) void k_spmm(int nnode, int nrhs, const int* __restrict__ nrow0,
+                                              const int* __restrict__ rowptr, const int* __restrict__ colind,
+                                              const double* __restrict__ val, const double* __restrict__ X, int ldx,
                                               double* __restrict__ Z, int ldz) {
-  // threads sweep all rows for one block of columns (all of them up to 128,
-  // else 64) before the next block, so the rows of X that a sweep gathers
-  // stay in cache
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int wcol = nrhs <= 128 ? nrhs : 64;
-  const int64_t per = (int64_t)n * wcol;
-  const int jb = (int)(g / per);
-  const int64_t rem = g - (int64_t)jb * per;
-  const int r = (int)(rem / wcol), j = jb * wcol + (int)(rem % wcol);
-  if (r >= n || j >= nrhs) return;
-  const int kb = rowptr[r], ke = rowptr[r + 1];
-  // SKIP: entries that are zero in value (the off-diagonal pattern of a
-  // lumped mass) skip their gather of X
-  // entry k goes to sum k mod 4 (relative to kb), each sum in entry order;
-  // sixteen entries' index, value and gather loads are issued together
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  int k = kb;
-  for (; k + 16 <= ke; k += 16) {
-    int c[16];
-    double v[16], x[16];
+  constexpr int P = 64 / W, U = NC * VEC >= 4 ? 2 : 4;  // groups; gathers in flight of each
+  typedef double vec __attribute__((ext_vector_type(VEC), aligned(8)));
+  __shared__ double sv[4][RB][64];
+  __shared__ int sc[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, j = lane % W, ph = lane / W;
+  const int node = 4 * xcd_task(blockIdx.x, gridDim.x) + wv;
+  if (node >= nnode) return;
+  const int r0 = nrow0[node], dn = nrow0[node + 1] - r0;
+  const int kb = rowptr[r0], len = rowptr[r0 + 1] - kb;
+  // VEC columns from col(c) on (VEC divides nrhs), past the last ones these again
+  auto col = [&](int c) { return (int)blockIdx.y * W * VEC * NC + VEC * (j + W * c); };
+  const double* xb[NC];
 #pragma unroll
-    for (int u = 0; u < 16; u++) {
-      c[u] = colind[k + u];
-      v[u] = val[k + u];
+  for (int c = 0; c < NC; c++) xb[c] = X + min(col(c), nrhs - VEC);
+  for (int rb = 0; rb < dn; rb += RB) {
+    double acc[RB][NC][VEC];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int m = 0; m < VEC; m++) acc[i][c][m] = 0.0;
+    int ci;
+    double cv[RB];
+    // entries past the list repeat its last one with a zero value
+    auto load = [&](int k0) {
+      const int k = min(k0 + lane, len - 1);
+      ci = colind[kb + k];
+#pragma unroll
+      for (int i = 0; i < RB; i++) cv[i] = val[(int64_t)kb + (int64_t)min(rb + i, dn - 1) * len + k];
+    };
+    load(0);
+    for (int k0 = 0; k0 < len; k0 += 64) {
+      __builtin_amdgcn_wave_barrier();  // this wave's LDS keeps its order
+      sc[wv][lane] = ci;
+#pragma unroll
+      for (int i = 0; i < RB; i++) sv[wv][i][lane] = k0 + lane < len ? cv[i] : 0.0;
+      __builtin_amdgcn_wave_barrier();
+      if (k0 + 64 < len) load(k0 + 64);
+      const int n = min(64, len - k0);
+      for (int e0 = 0; e0 < n; e0 += P * U) {
+        vec x[U][NC];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int64_t o = (int64_t)sc[wv][(e0 + u * P + ph) & 63] * ldx;
+#pragma unroll
+          for (int c = 0; c < NC; c++) x[u][c] = *(const vec*)(xb[c] + o);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int i = 0; i < RB; i++) {
+            const double v = sv[wv][i][(e0 + u * P + ph) & 63];
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+              for (int m = 0; m < VEC; m++) acc[i][c][m] = __builtin_fma(v, x[u][c][m], acc[i][c][m]);
+          }
+      }
     }
 #pragma unroll
-    for (int u = 0; u < 16; u++) x[u] = (!SKIP || v[u] != 0.0) ? X[(int64_t)c[u] * ldx + j] : 0.0;
+    for (int i = 0; i < RB; i++)
 #pragma unroll
-    for (int u = 0; u < 16; u += 4) {
-      if (!SKIP || v[u] != 0.0) s0 += v[u] * x[u];
-      if (!SKIP || v[u + 1] != 0.0) s1 += v[u + 1] * x[u + 1];
-      if (!SKIP || v[u + 2] != 0.0) s2 += v[u + 2] * x[u + 2];
-      if (!SKIP || v[u + 3] != 0.0) s3 += v[u + 3] * x[u + 3];
-    }
+      for (int c = 0; c < NC; c++) {
+        vec s;
+#pragma unroll
+        for (int m = 0; m < VEC; m++) {
+          double t = acc[i][c][m];
+#pragma unroll
+          for (int off = W; off < 64; off <<= 1) t += __shfl_xor(t, off);
+          s[m] = t;
+        }
+        if (rb + i < dn && ph == (i * NC + c) % P && col(c) < nrhs) *(vec*)(Z + (int64_t)(r0 + rb + i) * ldz + col(c)) = s;
+      }
   }
-  for (; k + 4 <= ke; k += 4) {
-    const int c0 = colind[k], c1 = colind[k + 1], c2 = colind[k + 2], c3 = colind[k + 3];
-    const double v0 = val[k], v1 = val[k + 1], v2 = val[k + 2], v3 = val[k + 3];
-    if (!SKIP || v0 != 0.0) s0 += v0 * X[(int64_t)c0 * ldx + j];
-    if (!SKIP || v1 != 0.0) s1 += v1 * X[(int64_t)c1 * ldx + j];
-    if (!SKIP || v2 != 0.0) s2 += v2 * X[(int64_t)c2 * ldx + j];
-    if (!SKIP || v3 != 0.0) s3 += v3 * X[(int64_t)c3 * ldx + j];
-  }
-  for (; k < ke; k++) {
-    const double v = val[k];
-    if (!SKIP || v != 0.0) s0 += v * X[(int64_t)colind[k] * ldx + j];
-  }
-  Z[(int64_t)r * ldz + j] = (s0 + s1) + (s2 + s3);
 }
 
-// k_spmm with four columns per thread (nrhs, ldx and ldz multiples of 4):
-// each entry's gather is two 16-byte loads and its index and value are
-// loaded once for the four columns; every column keeps k_spmm's four sums
-// (entry k to sum k mod 4 relative to kb, in entry order), so the results
-// are the same bits.
-template <bool SKIP>
-__global__ __launch_bounds__(256) void k_spmm4(int n, int nrhs, const int* __restrict__ rowptr,
-                                               const int* __restrict__ colind, const double* __restrict__ val,
-                                               const double* __restrict__ X, int ldx, double* __restrict__ Z, int ldz) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int wcol = nrhs <= 128 ? nrhs : 64, q4 = wcol / 4;
-  const int64_t per = (int64_t)n * q4;
-  const int jb = (int)(g / per);
-  const int64_t rem = g - (int64_t)jb * per;
-  const int r = (int)(rem / q4), j0 = jb * wcol + 4 * (int)(rem % q4);
-  if (r >= n || j0 >= nrhs) return;
-  const int kb = rowptr[r], ke = rowptr[r + 1];
-  double s[4][4];
-#pragma unroll
-  for (int c = 0; c < 4; c++)
-#pragma unroll
-    for (int m = 0; m < 4; m++) s[c][m] = 0.0;
-  auto gather = [&](int c, double2& a, double2& b) {
-    const double2* p = reinterpret_cast<const double2*>(X + (int64_t)c * ldx + j0);
-    a = p[0];
-    b = p[1];
-  };
-  int k = kb;
-  for (; k + 8 <= ke; k += 8) {
-    int cc[8];
-    double v[8];
-    double2 xa[8], xb[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      cc[u] = colind[k + u];
-      v[u] = val[k + u];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      if (!SKIP || v[u] != 0.0) gather(cc[u], xa[u], xb[u]);
-      else xa[u] = xb[u] = double2{0.0, 0.0};
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      if (SKIP && v[u] == 0.0) continue;
-      s[0][u & 3] += v[u] * xa[u].x;
-      s[1][u & 3] += v[u] * xa[u].y;
-      s[2][u & 3] += v[u] * xb[u].x;
-      s[3][u & 3] += v[u] * xb[u].y;
-    }
+// Z = diag(A) X where A has no other value (the lumped mass of the shell
+// elements in the stiffness' pattern, without constraints), dpos the diagonal's
+// places.  A zero of the diagonal gives a zero row.  One pass over X and Z:
+// 117x109 plate by 384 columns 325 -> 85 us.
+constexpr int DIAG_ROWS = 2048;  // entries of Z per workgroup, whole rows
+
+__global__ __launch_bounds__(256) void k_diag_mm(int n, int nrhs, int rows, const int* __restrict__ dpos,
+                                                 const double* __restrict__ val, const double* __restrict__ X, int ldx,
+                                                 double* __restrict__ Z, int ldz) {
+  const int r0 = blockIdx.x * rows, end = min(rows, n - r0) * nrhs;
+#pragma unroll 4
+  for (int e = threadIdx.x; e < end; e += 256) {
+    const int r = r0 + e / nrhs, j = e % nrhs;
+    const double v = val[dpos[r]], x = X[(int64_t)r * ldx + j];
+    Z[(int64_t)r * ldz + j] = v != 0.0 ? v * x : 0.0;
   }
-  for (; k + 4 <= ke; k += 4) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const double vv = val[k + u];
-      if (SKIP && vv == 0.0) continue;
-      double2 a, b;
-      gather(colind[k + u], a, b);
-      s[0][u] += vv * a.x;
-      s[1][u] += vv * a.y;
-      s[2][u] += vv * b.x;
-      s[3][u] += vv * b.y;
-    }
-  }
-  for (; k < ke; k++) {
-    const double vv = val[k];
-    if (SKIP && vv == 0.0) continue;
-    double2 a, b;
-    gather(colind[k], a, b);
-    s[0][0] += vv * a.x;
-    s[1][0] += vv * a.y;
-    s[2][0] += vv * b.x;
-    s[3][0] += vv * b.y;
-  }
-  double* z = Z + (int64_t)r * ldz + j0;
-#pragma unroll
-  for (int c = 0; c < 4; c++) z[c] = (s[c][0] + s[c][1]) + (s[c][2] + s[c][3]);
 }
 
 // Sign convention of the component modes: for column i of Phi (rows in
@@ -1445,13 +1430,11 @@ __global__ void k_start_block(int64_t n, int64_t n1, uint64_t seed, double* __re
 // Symmetric diagonal equilibration of the stiffness matrix for the FP32
 // factor: s[r] = 1/sqrt(K[r][r]) for every perm row r of the CSR matrix
 // (1 for a non-positive diagonal, which the factorisation then reports).
-__global__ void k_diag_scale(int n, const int* __restrict__ rowptr, const int* __restrict__ colind,
-                             const double* __restrict__ val, double* __restrict__ s) {
+__global__ void k_diag_scale(int n, const int* __restrict__ dpos, const double* __restrict__ val,
+                             double* __restrict__ s) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
-  double d = 0.0;
-  for (int k = rowptr[r]; k < rowptr[r + 1]; k++)
-    if (colind[k] == r) d = val[k];
+  const double d = val[dpos[r]];
   s[r] = d != 0.0 ? 1.0 / sqrt(fabs(d)) : 1.0;
 }
 
@@ -1581,11 +1564,11 @@ void launch_assemble(hipStream_t st, int64_t nnz, const int* cptr, const int* ci
   if (ccoef) k_assemble<true><<<nblk(nnz, 256), 256, 0, st>>>(nnz, cptr, cidx, ccoef, Kp, Mp, Kv, Mv, fmap, pool);
   else k_assemble<false><<<nblk(nnz, 256), 256, 0, st>>>(nnz, cptr, cidx, ccoef, Kp, Mp, Kv, Mv, fmap, pool);
 }
-void launch_diag_extract(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val,
-                         const double* rs, double* adiag, double* amax) {
+void launch_diag_extract(hipStream_t st, int n, const int* dpos, const double* val, const double* rs, double* adiag,
+                         double* amax) {
   if (n > 0)
-    k_diag_extract<<<nblk(n, 256), 256, 0, st>>>(n, rowptr, colind, val, rs, adiag,
-                                                 reinterpret_cast<unsigned long long*>(amax));
+    k_diag_extract<<<std::min(256u, nblk(n, 256)), 256, 0, st>>>(n, dpos, val, rs, adiag,
+                                                                 reinterpret_cast<unsigned long long*>(amax));
 }
 void launch_pivot_stats(hipStream_t st, int n, const double* dpiv, const int* sing, int* out) {
   if (n > 0) k_pivot_stats<<<std::min(1024u, nblk(n, 256)), 256, 0, st>>>(n, dpiv, sing, out);
@@ -1636,21 +1619,39 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
 FGPU_FACTOR_LAUNCHERS(double)
 FGPU_FACTOR_LAUNCHERS(float)
 #undef FGPU_FACTOR_LAUNCHERS
-void launch_spmm(hipStream_t st, int n, int nrhs, const int* rowptr, const int* colind, const double* val,
-                 const double* X, int ldx, double* Z, int ldz, bool skip_zeros) {
-  if (n > 0 && nrhs > 0) {
-    const int wcol = nrhs <= 128 ? nrhs : 64;
-    const int64_t threads = (int64_t)n * wcol * ((nrhs + wcol - 1) / wcol);
-    if (nrhs % 4 == 0 && ldx % 4 == 0 && ldz % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 31) == 0) {
-      const int64_t t4 = threads / 4;
-      if (skip_zeros) k_spmm4<true><<<nblk(t4, 256), 256, 0, st>>>(n, nrhs, rowptr, colind, val, X, ldx, Z, ldz);
-      else k_spmm4<false><<<nblk(t4, 256), 256, 0, st>>>(n, nrhs, rowptr, colind, val, X, ldx, Z, ldz);
-    } else if (skip_zeros) {
-      k_spmm<true><<<nblk(threads, 256), 256, 0, st>>>(n, nrhs, rowptr, colind, val, X, ldx, Z, ldz);
-    } else {
-      k_spmm<false><<<nblk(threads, 256), 256, 0, st>>>(n, nrhs, rowptr, colind, val, X, ldx, Z, ldz);
-    }
-  }
+void launch_spmm(hipStream_t st, const NodeRows& nr, int nrhs, const int* rowptr, const int* colind, const double* val,
+                 const double* X, int ldx, double* Z, int ldz) {
+  if (nr.nnode <= 0 || nrhs <= 0) return;
+  // columns in as even groups as tiles of 16 allow, up to 64 a wave, in pairs
+  // where they are even; three rows at a time where most nodes have no more
+  // (solids), else six
+  const int groups = (nrhs + 63) / 64, nc = (nrhs + 16 * groups - 1) / (16 * groups);
+  using std::integral_constant;
+  auto go = [&](auto w, auto vec, auto rb, auto c) {
+    constexpr int W = decltype(w)::value, VEC = decltype(vec)::value, NC = decltype(c)::value;
+    k_spmm<W, VEC, decltype(rb)::value, NC><<<dim3(nblk(nr.nnode, 4), nblk(nrhs, W * VEC * NC)), 256, 0, st>>>(
+        nr.nnode, nrhs, nr.row0, rowptr, colind, val, X, ldx, Z, ldz);
+  };
+  auto by_cols = [&](auto rb) {
+    using W4 = integral_constant<int, 4>;
+    using W8 = integral_constant<int, 8>;
+    using W16 = integral_constant<int, 16>;
+    using C1 = integral_constant<int, 1>;
+    using C2 = integral_constant<int, 2>;
+    if (nrhs <= 4) go(W4{}, C1{}, rb, C1{});
+    else if (nrhs % 2) nc == 1 ? go(W16{}, C1{}, rb, C1{}) : go(W16{}, C1{}, rb, C2{});
+    else if (nc == 1) go(W8{}, C2{}, rb, C1{});
+    else if (nc == 2) go(W8{}, C2{}, rb, C2{});
+    else if (nc == 3) go(W8{}, C2{}, rb, integral_constant<int, 3>{});
+    else go(W8{}, C2{}, rb, integral_constant<int, 4>{});
+  };
+  if (2 * nr.nrow < 9 * nr.nnode) by_cols(integral_constant<int, 3>{});
+  else by_cols(integral_constant<int, 6>{});
+}
+void launch_diag_mm(hipStream_t st, int n, int nrhs, const int* dpos, const double* val, const double* X, int ldx,
+                    double* Z, int ldz) {
+  const int rows = std::max(1, DIAG_ROWS / std::max(1, nrhs));
+  if (n > 0 && nrhs > 0) k_diag_mm<<<nblk(n, rows), 256, 0, st>>>(n, nrhs, rows, dpos, val, X, ldx, Z, ldz);
 }
 void launch_mode_signs(hipStream_t st, int n1, const int* p1, double* Phi, int64_t nrows, int nev, double* sign) {
   if (nev <= 0) return;
@@ -1673,8 +1674,8 @@ void launch_start_block(hipStream_t st, int neq, int n1, int bs, uint64_t seed, 
   const int64_t n = (int64_t)neq * bs;
   if (n > 0) k_start_block<<<nblk(n, 256), 256, 0, st>>>(n, (int64_t)n1 * bs, seed, W);
 }
-void launch_diag_scale(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val, double* s) {
-  if (n > 0) k_diag_scale<<<nblk(n, 256), 256, 0, st>>>(n, rowptr, colind, val, s);
+void launch_diag_scale(hipStream_t st, int n, const int* dpos, const double* val, double* s) {
+  if (n > 0) k_diag_scale<<<nblk(n, 256), 256, 0, st>>>(n, dpos, val, s);
 }
 void launch_front_scatter32(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val,
                             const double* s, const int64_t* fmap, float* pool) {

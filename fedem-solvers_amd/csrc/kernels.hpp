@@ -38,7 +38,7 @@ void launch_contrib(hipStream_t st, int pass, int nel, const int* etype, const i
                     const int* cptr, int* cidx, double* ccoef, int* bad);
 void launch_seg_sort(hipStream_t st, int nnz, const int* cptr, int* cidx, double* ccoef);
 void launch_fmap(hipStream_t st, int neq, const int* rowptr, const int* colind, const int* colsn, const DevSym& S,
-                 int64_t* fmap, int* bad);
+                 int64_t* fmap, int* dpos, int* bad);
 int scan_tiles(int n);
 void launch_exclusive_scan(hipStream_t st, int n, const int* in, int* out, int* tsum);
 void launch_fill(hipStream_t st, double* p, int64_t n, double v);
@@ -54,8 +54,8 @@ void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, 
 // magnitude (amax must start at 0); the pivot statistics
 // out[0..5] = negative, true-zero, reduced-to-zero pivots, first column of
 // each (out must start at {0, 0, 0, INT_MAX, INT_MAX, INT_MAX})
-void launch_diag_extract(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val,
-                         const double* rs, double* adiag, double* amax);
+void launch_diag_extract(hipStream_t st, int n, const int* dpos, const double* val, const double* rs, double* adiag,
+                         double* amax);
 void launch_pivot_stats(hipStream_t st, int n, const double* dpiv, const int* sing, int* out);
 // Pivot-block inverse tiles whose sum X_ij = -X_ii sum_k L_ik X_kj has more
 // than INV_CHUNK terms are summed in INV_CHUNK-tile chunks in parallel.
@@ -93,9 +93,17 @@ FGPU_FACTOR_DECLS(float)
 #undef FGPU_FACTOR_DECLS
 void launch_fw_init(hipStream_t st, const InitTask* t, int n, const int* gptr, const int* gsrc, const double* R,
                     double* W, int nrhs);
-void launch_spmm(hipStream_t st, int n, int nrhs, const int* rowptr, const int* colind, const double* val,
-                 const double* X, int ldx, double* Z, int ldz,
-                 bool skip_zeros = false);
+// rows of the CSR matrix by node: node q has rows row0[q] .. row0[q + 1], which
+// share one column list; nrow rows in all
+struct NodeRows {
+  const int* row0;
+  int nnode, nrow;
+};
+// Z = A X, and Z = diag(A) X with the diagonal's places dpos
+void launch_spmm(hipStream_t st, const NodeRows& nr, int nrhs, const int* rowptr, const int* colind, const double* val,
+                 const double* X, int ldx, double* Z, int ldz);
+void launch_diag_mm(hipStream_t st, int n, int nrhs, const int* dpos, const double* val, const double* X, int ldx,
+                    double* Z, int ldz);
 int xty_chunks(int n);
 // C = X^T Y (X n x na, Y n x nb, row-major; C na x nb row-major); acc
 // (optional) = C, or acc + C with acc_add
@@ -129,7 +137,7 @@ void launch_gram_inv(hipStream_t st, int n, int bs, const double* X, const doubl
 // null); Y = a X + b Y; partial sums of squares of x and y over
 // SUMSQ_BLOCKS blocks (2 doubles each, summed on the host in block order)
 constexpr int SUMSQ_BLOCKS = 512;
-void launch_diag_scale(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val, double* s);
+void launch_diag_scale(hipStream_t st, int n, const int* dpos, const double* val, double* s);
 void launch_front_scatter32(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val,
                             const double* s, const int64_t* fmap, float* pool);
 void launch_scale_rc(hipStream_t st, int64_t nrows, int nrhs, const double* rs, const double* cs, double* X);

@@ -222,7 +222,10 @@ struct DeviceReducer::Impl {
   // mixed precision: FP32 fronts and pivot-block inverses, equilibration
   // scale, refinement residual and norm partials
   bool mixed = false;
-  bool m_lumped = false;  // only lumped-mass (ANDES4) elements: M is diagonal in a K-shaped pattern
+  bool m_diag = false;  // only lumped-mass (ANDES4) elements and no constraints: M is diagonal in a K-shaped pattern
+  DBuf<int> row0, dpos;  // first row of every node (in row order), place of every row's diagonal
+  int nnode = 0;
+  NodeRows node_rows(int nrow) const { return {row0.p, nnode, nrow}; }
   int solve_split = 128;
   DBuf<float> pool32, ipool32;
   DBuf<double> dscale, dcs, Rr, irpart;
@@ -724,6 +727,8 @@ int DeviceReducer::build_structure(std::string& err) {
   HIPCHK(d.rnode.upload(y.rnode));
   HIPCHK(d.colsn.upload(y.colsn));
   HIPCHK(d.rowptr.upload(y.rowptr));
+  HIPCHK(d.row0.upload(y.nrow0));
+  d.nnode = (int)y.nrow0.size() - 1;
   HIPCHK(d.nbo.alloc(std::max<size_t>(1, y.nbl.size())));
   HIPCHK(d.colind.alloc(nnz));
   HIPCHK(d.cptr.alloc((size_t)nnz + 1));
@@ -731,6 +736,7 @@ int DeviceReducer::build_structure(std::string& err) {
   if (y.has_rigid) HIPCHK(d.ccoef.alloc(y.ncontrib));
   else d.ccoef.release();
   HIPCHK(d.fmap.alloc(nnz));
+  HIPCHK(d.dpos.alloc(y.neq));
   DBuf<int> cnt, tsum, bad;
   HIPCHK(cnt.alloc((size_t)nnz));
   HIPCHK(tsum.alloc((size_t)scan_tiles(nnz) + 1));
@@ -748,7 +754,7 @@ int DeviceReducer::build_structure(std::string& err) {
     if (pass == 0) launch_exclusive_scan(st, nnz, cnt.p, d.cptr.p, tsum.p);
   }
   launch_seg_sort(st, nnz, d.cptr.p, d.cidx.p, ccoef);
-  launch_fmap(st, y.neq, d.rowptr.p, d.colind.p, d.colsn.p, d.S, d.fmap.p, bad.p);
+  launch_fmap(st, y.neq, d.rowptr.p, d.colind.p, d.colsn.p, d.S, d.fmap.p, d.dpos.p, bad.p);
   HIPCHK(hipGetLastError());
   int hb = 0, total = 0;
   HIPCHK(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -817,7 +823,7 @@ int DeviceReducer::upload(std::string& err) {
   HIPCHK(d.ioff.upload(ioff));
   HIPCHK(d.ild.upload(d.lay.ild));
   d.mixed = opt_.mixed;
-  d.m_lumped = d.hexl.empty() && d.bml.empty();
+  d.m_diag = d.hexl.empty() && d.bml.empty() && !y.has_rigid;
   d.solve_split = std::max(64, (opt_.solve_split / 64) * 64);
   if (d.mixed) {
     d.ipool.release();
@@ -1038,6 +1044,13 @@ static void run_mv(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, 
 }
 
 // Y = D^{-1} L^{-1} R on the internal rows
+// Z = M X
+static void mass_mm(hipStream_t st, int neq, const DeviceReducer::Impl& d, int nrhs, const double* X, int ldx, double* Z,
+                    int ldz) {
+  if (d.m_diag) launch_diag_mm(st, neq, nrhs, d.dpos.p, d.Mv.p, X, ldx, Z, ldz);
+  else launch_spmm(st, d.node_rows(neq), nrhs, d.rowptr.p, d.colind.p, d.Mv.p, X, ldx, Z, ldz);
+}
+
 static void run_forward(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const double* R, double* Y) {
   for (const Op& op : sp.fw) {
     if (op.kind == FW_INIT)
@@ -1158,11 +1171,11 @@ static int pcg_int(hipStream_t st, DeviceReducer::Impl& d, const Symbolic& y, co
     if (stationary) {
       // X += z; r = b - K_ii X = r - K_ii z
       launch_axpby(st, nint, 1.0, d.cg_z.p, 1.0, X);
-      launch_spmm(st, neq, nr, d.rowptr.p, d.colind.p, d.Kv.p, d.cg_z.p, nr, d.cg_q.p, nr);
+      launch_spmm(st, d.node_rows(neq), nr, d.rowptr.p, d.colind.p, d.Kv.p, d.cg_z.p, nr, d.cg_q.p, nr);
       launch_axpby(st, nint, -1.0, d.cg_q.p, 1.0, R);
       if (rel_correction(st, d, nint, d.cg_z.p, X, rel, err)) return -3;
     } else {
-      launch_spmm(st, neq, nr, d.rowptr.p, d.colind.p, d.Kv.p, d.cg_p.p, nr, d.cg_q.p, nr);
+      launch_spmm(st, d.node_rows(neq), nr, d.rowptr.p, d.colind.p, d.Kv.p, d.cg_p.p, nr, d.cg_q.p, nr);
       if (int rc = dots(3, d.cg_p.p, d.cg_q.p, d.cg_p.p, d.cg_p.p, d.cg_p.p, X)) return rc;
       double num = 0.0, den = 0.0;
       for (int c = 0; c < nr; c++) {
@@ -1292,14 +1305,14 @@ int DeviceReducer::reduce(std::string& err) {
   launch_assemble(st, nnz, d.cptr.p, d.cidx.p, y.has_rigid ? d.ccoef.p : nullptr, d.Kp.p, d.Mp.p, d.Kv.p, d.Mv.p,
                   d.fmap.p, d.mixed ? nullptr : d.pool.p);
   if (d.mixed) {  // equilibrated stiffness into the FP32 fronts
-    launch_diag_scale(st, neq, d.rowptr.p, d.colind.p, d.Kv.p, d.dscale.p);
+    launch_diag_scale(st, neq, d.dpos.p, d.Kv.p, d.dscale.p);
     launch_front_scatter32(st, neq, d.rowptr.p, d.colind.p, d.Kv.p, d.dscale.p, d.fmap.p, d.pool32.p);
   }
   // original diagonal of K_ii for the singular-pivot test (equilibrated for
   // the mixed-precision factor), no pivot flagged yet
   HIPCHK(hipMemsetAsync(d.amax.p, 0, sizeof(double), st));
   HIPCHK(hipMemsetAsync(d.sing.p, 0, sizeof(int) * (size_t)std::max(1, n1), st));
-  launch_diag_extract(st, n1, d.rowptr.p, d.colind.p, d.Kv.p, d.mixed ? d.dscale.p : nullptr, d.adiag.p, d.amax.p);
+  launch_diag_extract(st, n1, d.dpos.p, d.Kv.p, d.mixed ? d.dscale.p : nullptr, d.adiag.p, d.amax.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(d.ev[2], st));
   mark("elements and assembly issued");
@@ -1401,7 +1414,7 @@ int DeviceReducer::reduce(std::string& err) {
     run_backward(st, d, *pb, nullptr, d.X.p);
     HIPCHK(hipEventRecord(d.ev[9], st));
     if (defer_z) {
-      launch_spmm(st, neq, n2, d.rowptr.p, d.colind.p, d.Mv.p, d.X.p, n2, d.Z.p, n2, d.m_lumped);
+      mass_mm(st, neq, d, n2, d.X.p, n2, d.Z.p, n2);
       HIPCHK(hipEventRecord(d.ev[11], st));
     }
     return 0;
@@ -1419,11 +1432,11 @@ int DeviceReducer::reduce(std::string& err) {
       // conjugate gradients on K_ii B = -K_ib from this B: the internal
       // rows of K [B; I] are -(the residual), its boundary rows K_bb + K_bi B
       // (the Schur complement once B has converged)
-      launch_spmm(st, neq, n2, d.rowptr.p, d.colind.p, d.Kv.p, d.X.p, n2, d.Z.p, n2);
+      launch_spmm(st, d.node_rows(neq), n2, d.rowptr.p, d.colind.p, d.Kv.p, d.X.p, n2, d.Z.p, n2);
       launch_axpby(st, (int64_t)n1 * n2, -1.0, d.Z.p, 0.0, d.Z.p);
       int steps = 0;
       if (int rc = pcg_int(st, d, y, opt_, *pb, d.X.p, d.Z.p, d.Y.p, &steps, "B", err)) return rc;
-      launch_spmm(st, neq, n2, d.rowptr.p, d.colind.p, d.Kv.p, d.X.p, n2, d.Z.p, n2);
+      launch_spmm(st, d.node_rows(neq), n2, d.rowptr.p, d.colind.p, d.Kv.p, d.X.p, n2, d.Z.p, n2);
       times_.refine_steps = steps;
       std::vector<double> zb((size_t)n2 * n2);
       HIPCHK(hipMemcpyAsync(zb.data(), d.Z.p + (size_t)n1 * n2, sizeof(double) * zb.size(), hipMemcpyDeviceToHost,
@@ -1507,7 +1520,7 @@ int DeviceReducer::reduce(std::string& err) {
     // passed it) forms R_tot = R_2 R_1, W = Q_j R_tot.
     auto orth_issue = [&](int j) {
       // M W is formed once: the second pass's M (W R_1^-1) is (M W) R_1^-1
-      launch_spmm(st, neq, bs, d.rowptr.p, d.colind.p, d.Mv.p, d.Wl.p, bs, d.Zl.p, bs, d.m_lumped);
+      mass_mm(st, neq, d, bs, d.Wl.p, bs, d.Zl.p, bs);
       for (int pass = 0; pass < 2; pass++) {
         launch_gram_inv(st, neq, bs, d.Wl.p, d.Zl.p, d.part.p, d.Cc.p, Rdev + (size_t)pass * bs * bs, d.small.p,
                         pass == 0, lzbad);
@@ -1714,7 +1727,7 @@ int DeviceReducer::reduce(std::string& err) {
     // without a converged test the Ritz pairs come from the full basis; the
     // M-Gram matrix of the last (reorthogonalised) block gives their residuals
     if (!conv) {
-      launch_spmm(st, neq, bs, d.rowptr.p, d.colind.p, d.Mv.p, d.Wl.p, bs, d.Zl.p, bs, d.m_lumped);
+      mass_mm(st, neq, d, bs, d.Wl.p, bs, d.Zl.p, bs);
       launch_xty(st, neq, bs, bs, d.Wl.p, bs, d.Zl.p, bs, d.part.p, d.Cc.p);
       std::vector<double> Gl((size_t)bs * bs);
       HIPCHK(hipMemcpyAsync(Gl.data(), d.Cc.p, sizeof(double) * bs * bs, hipMemcpyDeviceToHost, st));
@@ -1778,15 +1791,15 @@ int DeviceReducer::reduce(std::string& err) {
     return 0;
   };
   if (!opt_.no_mass && n2 > 0) {
-    if (!defer_z) launch_spmm(st, neq, n2, d.rowptr.p, d.colind.p, d.Mv.p, d.X.p, n2, d.Z.p, n2, d.m_lumped);
+    if (!defer_z) mass_mm(st, neq, d, n2, d.X.p, n2, d.Z.p, n2);
     if (xty_host(n2, n2, d.X.p, n2, d.Z.p, n2, M22)) return -3;
   }
   if (ngen > 0) {
     HIPCHK(d.Yl.alloc((size_t)neq * std::max(ngen, opt_.lanczos_block)));
-    launch_spmm(st, neq, ngen, d.rowptr.p, d.colind.p, d.Kv.p, d.Phi.p, nev, d.Yl.p, ngen);
+    launch_spmm(st, d.node_rows(neq), ngen, d.rowptr.p, d.colind.p, d.Kv.p, d.Phi.p, nev, d.Yl.p, ngen);
     if (xty_host(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, K11)) return -3;
     if (!opt_.no_mass) {
-      launch_spmm(st, neq, ngen, d.rowptr.p, d.colind.p, d.Mv.p, d.Phi.p, nev, d.Yl.p, ngen, d.m_lumped);
+      mass_mm(st, neq, d, ngen, d.Phi.p, nev, d.Yl.p, ngen);
       if (xty_host(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, M11)) return -3;
       if (n2 > 0 && xty_host(ngen, n2, d.Phi.p, nev, d.Z.p, n2, M12)) return -3;
     }
@@ -1795,7 +1808,7 @@ int DeviceReducer::reduce(std::string& err) {
   // ---- gravity: g = M a ; G_e = [B; I]^T g ; G_g = Phi^T g
   if (!opt_.no_mass) {
     HIPCHK(d.Tmp.alloc((size_t)neq * std::max(3, std::max(opt_.lanczos_block, nev))));
-    launch_spmm(st, neq, 3, d.rowptr.p, d.colind.p, d.Mv.p, d.grav.p, 3, d.Tmp.p, 3, d.m_lumped);
+    mass_mm(st, neq, d, 3, d.grav.p, 3, d.Tmp.p, 3);
     if (n2 > 0 && xty_host(n2, 3, d.X.p, n2, d.Tmp.p, 3, Ge)) return -3;
     if (ngen > 0 && xty_host(ngen, 3, d.Phi.p, nev, d.Tmp.p, 3, Gg)) return -3;
     if (opt_.want_vgi && n1 > 0) {
@@ -1986,7 +1999,7 @@ int DeviceReducer::gravity_internal(std::vector<double>& gi, std::string& err) {
   if (opt_.no_mass) { err = "gravity forces need the mass matrix"; return -1; }
   DBuf<double>& g = d.gi_g;
   HIPCHK(g.alloc((size_t)neq * 3));
-  launch_spmm(st_, neq, 3, d.rowptr.p, d.colind.p, d.Mv.p, d.grav.p, 3, g.p, 3, d.m_lumped);
+  mass_mm(st_, neq, d, 3, d.grav.p, 3, g.p, 3);
   std::vector<double> h((size_t)neq * 3);
   HIPCHK(hipMemcpyAsync(h.data(), g.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st_));
   HIPCHK(hipStreamSynchronize(st_));
@@ -2171,6 +2184,7 @@ size_t DeviceReducer::footprint_bytes() const {
   const size_t fb = opt_.mixed ? 4 : 8;  // bytes per factor entry
   size_t b = fb * ((size_t)y.fpool + ipool) + 8 * (2 * nnz + 2 * (size_t)y.elem_pool);  // fronts, inverses, K, M, elements
   b += (y.has_rigid ? 12 : 4) * (size_t)y.ncontrib + 4 * (nnz + 1) + 8 * nnz + 4 * nnz;  // contributions, fmap, colind
+  b += 4 * (2 * (size_t)y.neq + 1);  // node rows and diagonal places
   b += 8 * nnz;                                                                     // structure-build counts
   b += 20 * sam_.ceq_dof.size() + 4 * sam_.ceq_ptr.size();                          // constraint equations
   b += 8 * (size_t)y.neq * (3 * (size_t)y.ndof2 + 2 * mcap + 8 * (size_t)bs);     // B solves and Lanczos basis

@@ -168,9 +168,11 @@ __global__ void k_seg_sort(int nnz, const int* __restrict__ cptr, int* __restric
 }
 
 // ---------------------------------------------------------------- front map
-// front position of every lower entry (c <= r) of row r, -1 for the others
+// front position of every lower entry (c <= r) of row r, -1 for the others;
+// dpos[r] = the diagonal's entry
 __global__ void k_fmap(int neq, const int* __restrict__ rowptr, const int* __restrict__ colind,
-                       const int* __restrict__ colsn, DevSym S, int64_t* __restrict__ fmap, int* __restrict__ bad) {
+                       const int* __restrict__ colsn, DevSym S, int64_t* __restrict__ fmap, int* __restrict__ dpos,
+                       int* __restrict__ bad) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= neq) return;
   int last = -1;
@@ -181,6 +183,7 @@ __global__ void k_fmap(int neq, const int* __restrict__ rowptr, const int* __res
       fmap[k] = -1;
       continue;
     }
+    if (c == r) dpos[r] = k;
     const int sn = colsn[c];
     if (sn != last) {
       const int* rw = S.rows + S.rptr[sn];
@@ -301,8 +304,8 @@ void launch_seg_sort(hipStream_t st, int nnz, const int* cptr, int* cidx, double
 }
 
 void launch_fmap(hipStream_t st, int neq, const int* rowptr, const int* colind, const int* colsn, const DevSym& S,
-                 int64_t* fmap, int* bad) {
-  if (neq > 0) k_fmap<<<(neq + 255) / 256, 256, 0, st>>>(neq, rowptr, colind, colsn, S, fmap, bad);
+                 int64_t* fmap, int* dpos, int* bad) {
+  if (neq > 0) k_fmap<<<(neq + 255) / 256, 256, 0, st>>>(neq, rowptr, colind, colsn, S, fmap, dpos, bad);
 }
 
 int scan_tiles(int n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }

@@ -352,13 +352,16 @@ int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,
     y.nbptr[u + 1] = (int)y.nbl.size();
   }
   y.rnode.assign(s.neq, -1);
+  y.nrow0.reserve(pos + 1);
   for (int q = 0; q < pos; q++) {
     const int i = node_at[q];
+    y.nrow0.push_back(nfirst[i]);
     for (int j = 0; j < neqd[i]; j++) {
       y.rnode[nfirst[i] + j] = i;
       y.rowptr[nfirst[i] + j + 1] = rowlen[i];
     }
   }
+  y.nrow0.push_back(s.neq);
   for (int r = 0; r < s.neq; r++) y.rowptr[r + 1] += y.rowptr[r];
   y.colsn.swap(colsn);
   y.drank.assign(s.ndof, -1);

@@ -72,3 +72,19 @@ def test_row_counts(dims):
     # square of the vectors'
     q = np.sum(phi * (K @ phi), axis=0) / np.sum(phi * (M @ phi), axis=0)
     assert np.max(np.abs(lam - q) / q) <= 1e-9
+
+
+# six equations a node: the consistent mass of beams (sparse product) and the
+# lumped one of shells (its diagonal)
+@pytest.mark.parametrize("kind", ["beams", "shells"])
+@pytest.mark.parametrize("bs", [2, 5, 24, 33, 40, 64])
+def test_six_equation_nodes(kind, bs):
+    print(kind, "block", bs, flush=True)
+    if kind == "beams":
+        p = parts.beam_frame(n_el=90, seed=1, n_ext=4)
+    else:
+        p = parts.plate(9, 7, 0.18, 0.14, ext_nodes=[0, 9, 79])
+    lam, SM, ref, K, M, phi = reduced(p, 4, lanczosBlock=bs)
+    check_mass(SM, ref)
+    q = np.sum(phi * (K @ phi), axis=0) / np.sum(phi * (M @ phi), axis=0)
+    assert np.max(np.abs(lam - q) / q) <= 1e-7  # K phi cancels: eps |K| / lambda of a thin part
