@@ -13,38 +13,80 @@
 // reducer sees.  The ordering does not change the reduced matrices, only the
 // rounding.
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
+#include <future>
 #include <numeric>
+#include <system_error>
+#include <thread>
 #include "fgpu.hpp"
 
 namespace fgpu {
 namespace {
 
-struct NDBuilder {
-  const Part& p;
-  const std::vector<int>& adjptr;
-  const std::vector<int>& adj;
-  int leaf;
-  std::vector<char> mark;            // scratch: 1 = in current set, 2 = in L
-  std::vector<std::vector<int>> sn;  // node lists of the supernodes (postorder)
-  std::vector<int> parent;
+// f(thread, begin, end) over blocks of [0, n), the next block to the next
+// free thread; without threads (n small or threads = 1) f(0, 0, n).
+template <class F>
+void par_for(int threads, int n, int block, F&& f) {
+  threads = std::min(threads, (n + block - 1) / block);
+  if (threads <= 1) {
+    if (n > 0) f(0, 0, n);
+    return;
+  }
+  std::atomic<int> next{0};
+  auto run = [&](int t) {
+    for (int b; (b = next.fetch_add(block)) < n;) f(t, b, std::min(n, b + block));
+  };
+  std::vector<std::future<void>> jobs;
+  try {
+    for (int t = 1; t < threads; t++) jobs.push_back(std::async(std::launch::async, run, t));
+  } catch (const std::system_error&) {
+    // no further thread to be had: the ones there do the work
+  }
+  run(0);
+  for (auto& j : jobs) j.get();
+}
 
-  NDBuilder(const Part& part, const std::vector<int>& ap, const std::vector<int>& a, int lf)
-      : p(part), adjptr(ap), adj(a), leaf(lf), mark(part.nnod, 0) {}
+// Supernodes of a part of the dissection, in postorder.
+struct Forest {
+  std::vector<std::vector<int>> sn;  // node lists
+  std::vector<int> parent;           // -1: a root
+  std::vector<int> roots;
 
   int make(std::vector<int>&& nodes) {
     sn.push_back(std::move(nodes));
     parent.push_back(-1);
     return (int)sn.size() - 1;
   }
+  void append(Forest&& o) {
+    const int base = (int)sn.size();
+    for (size_t i = 0; i < o.sn.size(); i++) {
+      sn.push_back(std::move(o.sn[i]));
+      parent.push_back(o.parent[i] < 0 ? -1 : base + o.parent[i]);
+    }
+    for (int r : o.roots) roots.push_back(base + r);
+  }
+};
 
-  // returns the roots of the supernode forest spanning S
-  std::vector<int> nd(std::vector<int> S) {
-    std::vector<int> roots;
-    if (S.empty()) return roots;
+struct NDBuilder {
+  const Part& p;
+  const std::vector<int>& adjptr;
+  const std::vector<int>& adj;
+  int leaf;
+  std::vector<char> mark;  // scratch: 1 = in current set, 2 = in L; 0 outside of every set
+
+  NDBuilder(const Part& part, const std::vector<int>& ap, const std::vector<int>& a, int lf)
+      : p(part), adjptr(ap), adj(a), leaf(lf), mark(part.nnod, 0) {}
+
+  // Adds the supernode forest spanning S to `out`.  The halves of the first
+  // `fork` dissections are taken by threads of their own: they have no node
+  // in common and no edge between them, so neither reads a mark of the other.
+  void nd(std::vector<int> S, Forest& out, int fork) {
+    if (S.empty()) return;
+    const size_t r0 = out.roots.size();
     if ((int)S.size() <= leaf) {
-      roots.push_back(make(std::move(S)));
-      return roots;
+      out.roots.push_back(out.make(std::move(S)));
+      return;
     }
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
     for (int v : S)
@@ -55,36 +97,59 @@ struct NDBuilder {
     int ax = 0;
     for (int d = 1; d < 3; d++)
       if (hi[d] - lo[d] > hi[ax] - lo[ax]) ax = d;
-    std::stable_sort(S.begin(), S.end(), [&](int a, int b) {
-      return p.xyz[3 * a + ax] < p.xyz[3 * b + ax];
-    });
     int n = (int)S.size();
+    // sorted with the coordinates beside the nodes: the sort reads no
+    // coordinate through the node number
+    struct Key {
+      double x;
+      int v;
+    };
+    std::vector<Key> key(n);
+    for (int i = 0; i < n; i++) key[i] = {p.xyz[3 * S[i] + ax], S[i]};
+    std::stable_sort(key.begin(), key.end(), [](const Key& a, const Key& b) { return a.x < b.x; });
     // split at the widest coordinate gap near the median
     int k0 = std::max(1, (int)(0.4 * n)), k1 = std::min(n - 1, (int)(0.6 * n));
     if (k1 < k0) k1 = k0;
     int ks = n / 2;
     double best = -1.0;
     for (int k = k0; k <= k1; k++) {
-      double g = p.xyz[3 * S[k] + ax] - p.xyz[3 * S[k - 1] + ax];
+      double g = key[k].x - key[k - 1].x;
       if (g > best * (1.0 + 1e-9)) { best = g; ks = k; }
     }
-    for (int i = 0; i < n; i++) mark[S[i]] = (i < ks) ? 2 : 1;
-    std::vector<int> L(S.begin(), S.begin() + ks), R, sep;
+    std::vector<int> L(ks), R, sep;
+    for (int i = 0; i < ks; i++) mark[L[i] = key[i].v] = 2;
+    for (int i = ks; i < n; i++) mark[key[i].v] = 1;
+    R.reserve(n - ks);
     for (int i = ks; i < n; i++) {
-      int v = S[i];
+      int v = key[i].v;
       bool touch = false;
       for (int k = adjptr[v]; k < adjptr[v + 1] && !touch; k++) touch = mark[adj[k]] == 2;
       (touch ? sep : R).push_back(v);
     }
-    for (int v : S) mark[v] = 0;
-    std::vector<int> rl = nd(std::move(L));
-    std::vector<int> rr = nd(std::move(R));
-    rl.insert(rl.end(), rr.begin(), rr.end());
-    if (sep.empty()) return rl;
-    int s = make(std::move(sep));
-    for (int c : rl) parent[c] = s;
-    roots.push_back(s);
-    return roots;
+    for (int i = 0; i < n; i++) mark[key[i].v] = 0;
+    std::vector<Key>().swap(key);
+    std::vector<int>().swap(S);
+    if (fork > 0) {
+      Forest right;
+      std::future<void> job;
+      auto rest = [&]() { nd(std::move(R), right, fork - 1); };
+      try {
+        job = std::async(std::launch::async, rest);
+      } catch (const std::system_error&) {  // no further thread to be had
+      }
+      nd(std::move(L), out, fork - 1);
+      if (job.valid()) job.get();
+      else rest();
+      out.append(std::move(right));
+    } else {
+      nd(std::move(L), out, 0);
+      nd(std::move(R), out, 0);
+    }
+    if (sep.empty()) return;
+    const int s = out.make(std::move(sep));
+    for (size_t r = r0; r < out.roots.size(); r++) out.parent[out.roots[r]] = s;
+    out.roots.resize(r0);
+    out.roots.push_back(s);
   }
 };
 
@@ -146,47 +211,57 @@ int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,
     for (int e = 0; e < p.nel; e++)
       for (int k = ecptr[e]; k < ecptr[e + 1]; k++) elist[fill[ecn[k]]++] = e;
   }
+  // The lists that follow are made by several threads where the part is large
+  // enough to pay for them (a thread starts in 20 us, 1000 nodes take 0.6 ms
+  // in all); they do not depend on the number.  48x24x24 block: 25 ms with one
+  // thread, indirect sort keys, a search per update row and a second graph
+  // without boundary nodes, 13 now (61x47 plate, one thread: 1.07 and 0.91).
+  const int threads = nnod < 4000 ? 1 : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
   std::vector<int> adjptr(nnod + 1, 0), adj;
   {
-    std::vector<int> stamp(nnod, -1), tmp;
-    adj.reserve((size_t)nnod * 16);
-    for (int u = 0; u < nnod; u++) {
-      tmp.clear();
-      if (ncls[u]) {
-        for (int k = nel_of[u]; k < nel_of[u + 1]; k++) {
-          int e = elist[k];
-          for (int q = ecptr[e]; q < ecptr[e + 1]; q++) {
-            int v = ecn[q];
-            if (v != u && ncls[v] && stamp[v] != u) { stamp[v] = u; tmp.push_back(v); }
+    constexpr int BLOCK = 1024;  // nodes of one list
+    std::vector<std::vector<int>> stamps(std::max(1, threads)), list((nnod + BLOCK - 1) / BLOCK);
+    par_for(threads, nnod, BLOCK, [&](int t, int ub, int ue) {
+      std::vector<int>& stamp = stamps[t];
+      if (stamp.empty()) stamp.assign(nnod, -1);
+      for (int u = ub; u < ue; u++) {
+        std::vector<int>& out = list[u / BLOCK];
+        const size_t first = out.size();
+        if (ncls[u]) {
+          for (int k = nel_of[u]; k < nel_of[u + 1]; k++) {
+            int e = elist[k];
+            for (int q = ecptr[e]; q < ecptr[e + 1]; q++) {
+              int v = ecn[q];
+              if (v != u && ncls[v] && stamp[v] != u) { stamp[v] = u; out.push_back(v); }
+            }
           }
         }
+        std::sort(out.begin() + first, out.end());
+        adjptr[u + 1] = (int)(out.size() - first);
       }
-      std::sort(tmp.begin(), tmp.end());
-      adj.insert(adj.end(), tmp.begin(), tmp.end());
-      adjptr[u + 1] = (int)adj.size();
-    }
+    });
+    for (int u = 0; u < nnod; u++) adjptr[u + 1] += adjptr[u];
+    adj.resize(adjptr[nnod]);
+    par_for(threads, (int)list.size(), 1, [&](int, int b, int e) {
+      for (int i = b; i < e; i++) std::copy(list[i].begin(), list[i].end(), adj.begin() + adjptr[i * BLOCK]);
+    });
   }
-  // internal-node graph (boundary nodes removed) for the dissection
-  std::vector<int> iadjptr(nnod + 1, 0), iadj;
-  iadj.reserve(adj.size());
-  for (int u = 0; u < nnod; u++) {
-    if (ncls[u] == 1)
-      for (int k = adjptr[u]; k < adjptr[u + 1]; k++)
-        if (ncls[adj[k]] == 1) iadj.push_back(adj[k]);
-    iadjptr[u + 1] = (int)iadj.size();
+  // dissection of the internal nodes (boundary nodes are in no set of it)
+  NDBuilder nb(p, adjptr, adj, std::max(1, o.leaf_nodes));
+  Forest forest;
+  {
+    std::vector<int> inodes;
+    for (int i = 0; i < nnod; i++)
+      if (ncls[i] == 1) inodes.push_back(i);
+    nb.nd(std::move(inodes), forest, threads >= 8 ? 3 : threads >= 4 ? 2 : threads >= 2 ? 1 : 0);
   }
-  NDBuilder nb(p, iadjptr, iadj, std::max(1, o.leaf_nodes));
-  std::vector<int> inodes;
-  for (int i = 0; i < nnod; i++)
-    if (ncls[i] == 1) inodes.push_back(i);
-  std::vector<int> roots = nb.nd(inodes);
-  const int nsi = (int)nb.sn.size();  // internal supernodes
-  y.nsup = nsi + 1;                   // + Schur front
+  const int nsi = (int)forest.sn.size();  // internal supernodes
+  y.nsup = nsi + 1;                       // + Schur front
   // node positions
   std::vector<int> npos(nnod, -1);
   int pos = 0;
   for (int sidx = 0; sidx < nsi; sidx++)
-    for (int v : nb.sn[sidx]) npos[v] = pos++;
+    for (int v : forest.sn[sidx]) npos[v] = pos++;
   for (int i = 0; i < nnod; i++)
     if (ncls[i] == 2) npos[i] = pos++;
   std::vector<int> node_at(pos);
@@ -212,83 +287,11 @@ int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,
   if (pp != s.neq) { err = "symbolic: equation count mismatch"; return -1; }
   // supernode parents
   y.parent.assign(y.nsup, -1);
-  for (int sidx = 0; sidx < nsi; sidx++) y.parent[sidx] = nb.parent[sidx] >= 0 ? nb.parent[sidx] : nsi;
+  for (int sidx = 0; sidx < nsi; sidx++) y.parent[sidx] = forest.parent[sidx] >= 0 ? forest.parent[sidx] : nsi;
   // node-level update structures (children are complete before parents)
   std::vector<std::vector<int>> ust(nsi);
   std::vector<std::vector<int>> kids(y.nsup);
   for (int sidx = 0; sidx < nsi; sidx++) kids[y.parent[sidx]].push_back(sidx);
-  {
-    std::vector<int> stamp(pos, -1);
-    for (int sidx = 0; sidx < nsi; sidx++) {
-      int maxp = -1;
-      for (int v : nb.sn[sidx]) maxp = std::max(maxp, npos[v]);
-      std::vector<int>& u = ust[sidx];
-      u.clear();
-      for (int v : nb.sn[sidx])
-        for (int k = adjptr[v]; k < adjptr[v + 1]; k++) {
-          int w = npos[adj[k]];
-          if (w > maxp && stamp[w] != sidx) { stamp[w] = sidx; u.push_back(w); }
-        }
-      for (int c : kids[sidx])
-        for (int w : ust[c])
-          if (w > maxp && stamp[w] != sidx) { stamp[w] = sidx; u.push_back(w); }
-      std::sort(u.begin(), u.end());
-    }
-  }
-  // DOF-level rows
-  y.col0.assign(y.nsup, 0);
-  y.ncol.assign(y.nsup, 0);
-  y.nrow.assign(y.nsup, 0);
-  y.rptr.assign(y.nsup + 1, 0);
-  for (int sidx = 0; sidx < nsi; sidx++) {
-    int c0 = nfirst[nb.sn[sidx][0]], nc = 0;
-    for (int v : nb.sn[sidx]) nc += neqd[v];
-    y.col0[sidx] = c0;
-    y.ncol[sidx] = nc;
-    int nr = nc;
-    for (int w : ust[sidx]) nr += neqd[node_at[w]];
-    y.nrow[sidx] = nr;
-    y.rptr[sidx + 1] = y.rptr[sidx] + nr;
-  }
-  y.col0[nsi] = s.ndof1;
-  y.ncol[nsi] = 0;
-  y.nrow[nsi] = s.ndof2;
-  y.rptr[nsi + 1] = y.rptr[nsi] + s.ndof2;
-  y.rows.resize(y.rptr[y.nsup]);
-  for (int sidx = 0; sidx < nsi; sidx++) {
-    int* r = &y.rows[y.rptr[sidx]];
-    int k = 0;
-    for (int j = 0; j < y.ncol[sidx]; j++) r[k++] = y.col0[sidx] + j;
-    for (int w : ust[sidx]) {
-      int i = node_at[w];
-      for (int j = 0; j < neqd[i]; j++) r[k++] = nfirst[i] + j;
-    }
-  }
-  for (int j = 0; j < s.ndof2; j++) y.rows[y.rptr[nsi] + j] = s.ndof1 + j;
-  std::vector<std::vector<int>>().swap(ust);
-  // children, relative maps, levels
-  y.chptr.assign(y.nsup + 1, 0);
-  for (int sidx = 0; sidx < y.nsup; sidx++) y.chptr[sidx + 1] = y.chptr[sidx] + (int)kids[sidx].size();
-  y.chlist.resize(y.chptr[y.nsup]);
-  for (int sidx = 0; sidx < y.nsup; sidx++)
-    std::copy(kids[sidx].begin(), kids[sidx].end(), y.chlist.begin() + y.chptr[sidx]);
-  y.relptr.assign(y.nsup + 1, 0);
-  for (int sidx = 0; sidx < y.nsup; sidx++)
-    y.relptr[sidx + 1] = y.relptr[sidx] + (y.nrow[sidx] - y.ncol[sidx]) * (sidx < nsi ? 1 : 0);
-  y.rel.resize(y.relptr[y.nsup]);
-  for (int sidx = 0; sidx < nsi; sidx++) {
-    int par = y.parent[sidx];
-    const int* pr = &y.rows[y.rptr[par]];
-    const int* pe = pr + y.nrow[par];
-    int* rr = &y.rel[y.relptr[sidx]];
-    const int* cr = &y.rows[y.rptr[sidx]];
-    const int* it = pr;
-    for (int k = y.ncol[sidx]; k < y.nrow[sidx]; k++) {
-      it = std::lower_bound(it, pe, cr[k]);
-      if (it == pe || *it != cr[k]) { err = "symbolic: update row missing in parent front"; return -1; }
-      rr[k - y.ncol[sidx]] = (int)(it - pr);
-    }
-  }
   y.level.assign(y.nsup, 0);
   for (int sidx = 0; sidx < y.nsup; sidx++)
     for (int c : kids[sidx]) y.level[sidx] = std::max(y.level[sidx], y.level[c] + 1);
@@ -301,6 +304,108 @@ int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,
     std::vector<int> fill(y.lvptr.begin(), y.lvptr.end() - 1);
     for (int sidx = 0; sidx < y.nsup; sidx++) y.lvsup[fill[y.level[sidx]]++] = sidx;
   }
+  {
+    // level by level: a supernode waits for its children, which were taken
+    // before it
+    std::vector<std::vector<int>> stamps(std::max(1, threads));
+    std::vector<std::atomic<char>> ready(nsi);
+    std::atomic<bool> failed{false};
+    auto block = [&](int t, int qb, int qe) {
+      std::vector<int>& stamp = stamps[t];
+      if (stamp.empty()) stamp.assign(pos, -1);
+      for (int q = qb; q < qe; q++) {
+        const int sidx = y.lvsup[q];
+        if (sidx == nsi) continue;
+        for (int c : kids[sidx])
+          while (!ready[c].load(std::memory_order_acquire)) {
+            if (failed) return;
+            std::this_thread::yield();
+          }
+        int maxp = -1;
+        for (int v : forest.sn[sidx]) maxp = std::max(maxp, npos[v]);
+        std::vector<int>& u = ust[sidx];
+        u.clear();
+        for (int v : forest.sn[sidx])
+          for (int k = adjptr[v]; k < adjptr[v + 1]; k++) {
+            int w = npos[adj[k]];
+            if (w > maxp && stamp[w] != sidx) { stamp[w] = sidx; u.push_back(w); }
+          }
+        for (int c : kids[sidx])
+          for (int w : ust[c])
+            if (w > maxp && stamp[w] != sidx) { stamp[w] = sidx; u.push_back(w); }
+        std::sort(u.begin(), u.end());
+        ready[sidx].store(1, std::memory_order_release);
+      }
+    };
+    par_for(threads, y.nsup, 1, [&](int t, int qb, int qe) {
+      try {
+        block(t, qb, qe);
+      } catch (...) {  // out of memory: nobody waits for this one any more
+        failed = true;
+        throw;
+      }
+    });
+  }
+  // DOF-level rows
+  y.col0.assign(y.nsup, 0);
+  y.ncol.assign(y.nsup, 0);
+  y.nrow.assign(y.nsup, 0);
+  y.rptr.assign(y.nsup + 1, 0);
+  for (int sidx = 0; sidx < nsi; sidx++) {
+    int c0 = nfirst[forest.sn[sidx][0]], nc = 0;
+    for (int v : forest.sn[sidx]) nc += neqd[v];
+    y.col0[sidx] = c0;
+    y.ncol[sidx] = nc;
+    int nr = nc;
+    for (int w : ust[sidx]) nr += neqd[node_at[w]];
+    y.nrow[sidx] = nr;
+    y.rptr[sidx + 1] = y.rptr[sidx] + nr;
+  }
+  y.col0[nsi] = s.ndof1;
+  y.ncol[nsi] = 0;
+  y.nrow[nsi] = s.ndof2;
+  y.rptr[nsi + 1] = y.rptr[nsi] + s.ndof2;
+  y.rows.resize(y.rptr[y.nsup]);
+  par_for(threads, nsi, 16, [&](int, int sb, int se) {
+    for (int sidx = sb; sidx < se; sidx++) {
+      int* r = &y.rows[y.rptr[sidx]];
+      int k = 0;
+      for (int j = 0; j < y.ncol[sidx]; j++) r[k++] = y.col0[sidx] + j;
+      for (int w : ust[sidx]) {
+        int i = node_at[w];
+        for (int j = 0; j < neqd[i]; j++) r[k++] = nfirst[i] + j;
+      }
+    }
+  });
+  for (int j = 0; j < s.ndof2; j++) y.rows[y.rptr[nsi] + j] = s.ndof1 + j;
+  std::vector<std::vector<int>>().swap(ust);
+  // children, relative maps, levels
+  y.chptr.assign(y.nsup + 1, 0);
+  for (int sidx = 0; sidx < y.nsup; sidx++) y.chptr[sidx + 1] = y.chptr[sidx] + (int)kids[sidx].size();
+  y.chlist.resize(y.chptr[y.nsup]);
+  for (int sidx = 0; sidx < y.nsup; sidx++)
+    std::copy(kids[sidx].begin(), kids[sidx].end(), y.chlist.begin() + y.chptr[sidx]);
+  y.relptr.assign(y.nsup + 1, 0);
+  for (int sidx = 0; sidx < y.nsup; sidx++)
+    y.relptr[sidx + 1] = y.relptr[sidx] + (y.nrow[sidx] - y.ncol[sidx]) * (sidx < nsi ? 1 : 0);
+  y.rel.resize(y.relptr[y.nsup]);
+  std::atomic<bool> missing{false};
+  par_for(threads, nsi, 16, [&](int, int sb, int se) {
+    for (int sidx = sb; sidx < se; sidx++) {
+      int par = y.parent[sidx];
+      const int* pr = &y.rows[y.rptr[par]];
+      const int* pe = pr + y.nrow[par];
+      int* rr = &y.rel[y.relptr[sidx]];
+      const int* cr = &y.rows[y.rptr[sidx]];
+      const int* it = pr;
+      for (int k = y.ncol[sidx]; k < y.nrow[sidx]; k++) {
+        while (it != pe && *it < cr[k]) it++;  // both lists ascend
+        if (it == pe || *it != cr[k]) { missing = true; return; }
+        rr[k - y.ncol[sidx]] = (int)(it - pr);
+      }
+    }
+  });
+  if (missing) { err = "symbolic: update row missing in parent front"; return -1; }
   // fronts, work
   y.foff.assign(y.nsup + 1, 0);
   for (int sidx = 0; sidx < y.nsup; sidx++) {
@@ -384,7 +489,6 @@ int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,
     err = "symbolic: the part's matrix is too large for 32-bit contribution indices";
     return -1;
   }
-  (void)roots;
   return 0;
 }
 
