@@ -46,6 +46,11 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v);
 // (address and size), the permuted-row gather of column-major load vectors
 // and the scatter of the reduced rows into Fred
 int noalloc_scratch(double** ptr, size_t* bytes, std::string& err);
+// order changes (order.hip): rows of a column-major array into row-major rows
+// map[q], and the sum of up to two row-major arrays' rows map[q] back
+void launch_rows_in(hipStream_t st, int n, int nc, const int* map, const double* in, int64_t ldi, double* out, int ldo);
+void launch_rows_out(hipStream_t st, int n, int nc, const int* map, const double* A, int lda, const double* B, int ldb,
+                     double* out, int64_t ldo);
 void launch_perm_rows(hipStream_t st, int neq, int nrhs, const int* p2e, const double* F, double* Fp);
 void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, const int* pos2, const double* r2,
                             const double* r1, double* Fred);

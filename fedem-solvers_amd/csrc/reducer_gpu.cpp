@@ -1895,32 +1895,30 @@ hipError_t DeviceReducer::d2h(void* dst, const void* src, size_t bytes) const {
   return e == hipSuccess ? hipStreamSynchronize(st_) : e;
 }
 
-int DeviceReducer::get_B(std::vector<double>& B) {
-  const Symbolic& y = sym_;
-  const int n1 = y.ndof1, n2 = y.ndof2;
-  std::vector<double> x((size_t)y.neq * n2);
-  if (n2 == 0) { B.clear(); return 0; }
-  if (d2h(x.data(), d_->X.p, sizeof(double) * x.size()) != hipSuccess) return -3;
-  B.assign((size_t)n1 * n2, 0.0);
-  for (int q = 0; q < n1; q++) {
-    int r = y.eq_to_perm[sam_.meqn1[q] - 1];
-    for (int c = 0; c < n2; c++) B[q + (size_t)c * n1] = x[(size_t)r * n2 + c];
+// Internal rows of the row-major neq x nc array A, in equation order and
+// column-major, to the host: ordered on the device, at most 2^23 values (64
+// MiB of device memory) at a time.
+int DeviceReducer::internal_to_host(const double* A, int nc, double* out) const {
+  Impl& d = *d_;
+  std::string err;
+  const int n1 = sym_.ndof1, step = std::max(1, std::min(nc, (1 << 23) / std::max(1, n1)));
+  HIPCHK(d.sk_t.alloc((size_t)n1 * step));
+  for (int c0 = 0; c0 < nc; c0 += step) {
+    const int k = std::min(step, nc - c0);
+    launch_rows_out(st_, n1, k, d.p1.p, A + c0, nc, nullptr, 0, d.sk_t.p, n1);
+    HIPCHK(d2h(out + (size_t)c0 * n1, d.sk_t.p, sizeof(double) * (size_t)n1 * k));
   }
   return 0;
 }
 
+int DeviceReducer::get_B(std::vector<double>& B) {
+  B.resize((size_t)sym_.ndof1 * sym_.ndof2);
+  return B.empty() ? 0 : internal_to_host(d_->X.p, sym_.ndof2, B.data());
+}
+
 int DeviceReducer::get_phi(std::vector<double>& P) {
-  const Symbolic& y = sym_;
-  const int n1 = y.ndof1, nev = res_.nev;
-  P.assign((size_t)n1 * nev, 0.0);
-  if (nev == 0) return 0;
-  std::vector<double> x((size_t)y.neq * nev);
-  if (d2h(x.data(), d_->Phi.p, sizeof(double) * x.size()) != hipSuccess) return -3;
-  for (int q = 0; q < n1; q++) {
-    int r = y.eq_to_perm[sam_.meqn1[q] - 1];
-    for (int c = 0; c < nev; c++) P[q + (size_t)c * n1] = x[(size_t)r * nev + c];
-  }
-  return 0;
+  P.resize((size_t)sym_.ndof1 * res_.nev);
+  return P.empty() ? 0 : internal_to_host(d_->Phi.p, res_.nev, P.data());
 }
 
 int DeviceReducer::get_schur(std::vector<double>& S) {
@@ -1962,32 +1960,38 @@ int DeviceReducer::get_element_matrices(std::vector<double>& Kp, std::vector<dou
   return 0;
 }
 
-int DeviceReducer::solve_kii(int nrhs, const double* R_eq, double* X_eq, std::string& err) {
-  StreamScope scope(st_);
+// K_ii^-1 R into row-major x = d.sk_x (rows in elimination order), R as the
+// caller's column-major n1 x nrhs.  The caller's array is read by an
+// asynchronous copy: the stream has to pass it before the call returns.
+int DeviceReducer::solve_rows(int nrhs, const double* R_eq, std::string& err) {
   Impl& d = *d_;
   const Symbolic& y = sym_;
   const int neq = y.neq, n1 = y.ndof1;
   SolvePlan* p = nullptr;
   if (get_plan(y, d, nrhs, p, err)) return -3;
   if (ensure_work(d, std::max(nrhs, std::max(y.ndof2, opt_.lanczos_block)), err)) return -3;
-  DBuf<double>& r = d.sk_r;
-  DBuf<double>& t = d.sk_t;
-  DBuf<double>& x = d.sk_x;
-  std::vector<double> h((size_t)neq * nrhs, 0.0);
-  for (int q = 0; q < n1; q++) {
-    int rr = y.eq_to_perm[sam_.meqn1[q] - 1];
-    for (int c = 0; c < nrhs; c++) h[(size_t)rr * nrhs + c] = R_eq[q + (size_t)c * n1];
+  const size_t n = (size_t)neq * nrhs;
+  HIPCHK(d.sk_r.alloc(n));
+  HIPCHK(d.sk_t.alloc(n));
+  HIPCHK(d.sk_x.alloc(n));
+  // the caller's order arrives in the solve's work array
+  HIPCHK(hipMemcpyAsync(d.sk_t.p, R_eq, sizeof(double) * (size_t)n1 * nrhs, hipMemcpyHostToDevice, st_));
+  launch_rows_in(st_, n1, nrhs, d.p1.p, d.sk_t.p, n1, d.sk_r.p, nrhs);
+  launch_fill(st_, d.sk_r.p + (size_t)n1 * nrhs, (int64_t)(neq - n1) * nrhs, 0.0);
+  return solve_int(st_, d, y, opt_, *p, d.sk_r.p, d.sk_t.p, d.sk_x.p, nullptr, err);
+}
+
+int DeviceReducer::solve_kii(int nrhs, const double* R_eq, double* X_eq, std::string& err) {
+  StreamScope scope(st_);
+  Impl& d = *d_;
+  const int n1 = sym_.ndof1;
+  if (n1 == 0) return 0;
+  if (int rc = solve_rows(nrhs, R_eq, err)) {
+    (void)hipStreamSynchronize(st_);
+    return rc;
   }
-  HIPCHK(r.upload(h));
-  HIPCHK(t.alloc(h.size()));
-  HIPCHK(x.alloc(h.size()));
-  if (int rc = solve_int(st_, d, y, opt_, *p, r.p, t.p, x.p, nullptr, err)) return rc;
-  HIPCHK(hipMemcpyAsync(h.data(), x.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st_));
-  HIPCHK(hipStreamSynchronize(st_));
-  for (int q = 0; q < n1; q++) {
-    int rr = y.eq_to_perm[sam_.meqn1[q] - 1];
-    for (int c = 0; c < nrhs; c++) X_eq[q + (size_t)c * n1] = h[(size_t)rr * nrhs + c];
-  }
+  launch_rows_out(st_, n1, nrhs, d.p1.p, d.sk_x.p, nrhs, nullptr, 0, d.sk_t.p, n1);
+  HIPCHK(d2h(X_eq, d.sk_t.p, sizeof(double) * (size_t)n1 * nrhs));
   return 0;
 }
 
@@ -2000,15 +2004,8 @@ int DeviceReducer::gravity_internal(std::vector<double>& gi, std::string& err) {
   DBuf<double>& g = d.gi_g;
   HIPCHK(g.alloc((size_t)neq * 3));
   mass_mm(st_, neq, d, 3, d.grav.p, 3, g.p, 3);
-  std::vector<double> h((size_t)neq * 3);
-  HIPCHK(hipMemcpyAsync(h.data(), g.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st_));
-  HIPCHK(hipStreamSynchronize(st_));
-  gi.assign((size_t)n1 * 3, 0.0);
-  for (int q = 0; q < n1; q++) {
-    int rr = y.eq_to_perm[sam_.meqn1[q] - 1];
-    for (int c = 0; c < 3; c++) gi[q + (size_t)c * n1] = h[(size_t)rr * 3 + c];
-  }
-  return 0;
+  gi.resize((size_t)n1 * 3);
+  return gi.empty() ? 0 : internal_to_host(g.p, 3, gi.data());
 }
 
 int DeviceReducer::reduce_loads(int nrhs, const double* F_eq, std::vector<double>& out, std::string& err) {
@@ -2018,32 +2015,23 @@ int DeviceReducer::reduce_loads(int nrhs, const double* F_eq, std::vector<double
   const int neq = y.neq, n2 = y.ndof2, ngen = res_.ngen, nev = res_.nev, nd = res_.ndim;
   out.assign((size_t)nd * std::max(nrhs, 0), 0.0);
   if (nrhs <= 0) return 0;
-  std::vector<double> h((size_t)neq * nrhs);
-  for (int e = 0; e < neq; e++) {
-    int rr = y.eq_to_perm[e];
-    for (int c = 0; c < nrhs; c++) h[(size_t)rr * nrhs + c] = F_eq[e + (size_t)c * neq];
-  }
-  DBuf<double>& f = d.rl_f;
-  HIPCHK(f.upload(h));
-  const int maxab = std::max(std::max(n2, ngen), nrhs);
-  HIPCHK(d.part.alloc((size_t)xty_chunks(neq) * maxab * maxab));
-  HIPCHK(d.acc.alloc((size_t)maxab * maxab));
-  std::vector<double> r2((size_t)n2 * nrhs), r1((size_t)ngen * nrhs);
-  if (n2 > 0) {  // rhs2 = f_e + B^T f_i = [B; I]^T f
-    launch_xty(st_, neq, n2, nrhs, d.X.p, n2, f.p, nrhs, d.part.p, d.acc.p);
-    HIPCHK(hipMemcpyAsync(r2.data(), d.acc.p, sizeof(double) * r2.size(), hipMemcpyDeviceToHost, st_));
-    HIPCHK(hipStreamSynchronize(st_));
-  }
-  if (ngen > 0) {  // rhs1 = Phi^T f_i
-    launch_xty(st_, neq, ngen, nrhs, d.Phi.p, nev, f.p, nrhs, d.part.p, d.acc.p);
-    HIPCHK(hipMemcpyAsync(r1.data(), d.acc.p, sizeof(double) * r1.size(), hipMemcpyDeviceToHost, st_));
-    HIPCHK(hipStreamSynchronize(st_));
-  }
-  const std::vector<int>& pos2 = sam_.dofPosIn2;
-  for (int c = 0; c < nrhs; c++) {
-    for (int i = 0; i < n2; i++) out[i + (size_t)c * nd] = r2[(size_t)(pos2[i] - 1) * nrhs + c];
-    for (int a = 0; a < ngen; a++) out[(n2 + a) + (size_t)c * nd] = r1[(size_t)a * nrhs + c];
-  }
+  if (out.empty()) return 0;
+  // the same launches as reduce_loads_noalloc, on buffers of the handle: the
+  // load vectors cross the bus in the caller's order, the result once
+  const size_t nF = (size_t)neq * nrhs, maxa = (size_t)std::max(n2, ngen);
+  HIPCHK(d.rl_f.alloc(nF));
+  HIPCHK(d.sk_t.alloc(nF));
+  HIPCHK(d.part.alloc((size_t)xty_chunks(neq) * maxa * nrhs));
+  HIPCHK(d.acc.alloc((size_t)(n2 + ngen + nd) * nrhs));
+  double *const f = d.rl_f.p, *const r2 = d.acc.p, *const r1 = r2 + (size_t)n2 * nrhs;
+  double* const red = r1 + (size_t)ngen * nrhs;
+  HIPCHK(hipMemcpyAsync(d.sk_t.p, F_eq, sizeof(double) * nF, hipMemcpyHostToDevice, st_));
+  launch_perm_rows(st_, neq, nrhs, d.p2e.p, d.sk_t.p, f);
+  // rhs2 = f_e + B^T f_i = [B; I]^T f, rhs1 = Phi^T f_i
+  if (n2 > 0) launch_xty(st_, neq, n2, nrhs, d.X.p, n2, f, nrhs, d.part.p, r2);
+  if (ngen > 0) launch_xty(st_, neq, ngen, nrhs, d.Phi.p, nev, f, nrhs, d.part.p, r1);
+  launch_scatter_reduced(st_, nd, n2, ngen, nrhs, d.pos2.p, r2, r1, red);
+  HIPCHK(d2h(out.data(), red, sizeof(double) * out.size()));
   (void)err;
   return 0;
 }
@@ -2086,37 +2074,37 @@ int DeviceReducer::recover(int nrhs, const double* Ub, const double* Fi, double*
   const Symbolic& y = sym_;
   const int neq = y.neq, n1 = y.ndof1, n2 = y.ndof2;
   if (nrhs <= 0) return 0;
-  std::vector<double> acc((size_t)n1 * nrhs, 0.0);
-  if (n2 > 0 && Ub) {
-    // Y = [B; I] U_b in permuted rows, the boundary block of U_b in LDS-sized
-    // column chunks
-    const int cj = std::max(1, std::min(nrhs, 8192 / std::max(n2, 1)));
-    DBuf<double>& S = d.rc_s;
-    DBuf<double>& Yd = d.rc_y;
-    HIPCHK(Yd.alloc((size_t)neq * cj));
-    std::vector<double> hs((size_t)n2 * cj), hy((size_t)neq * cj);
-    for (int j0 = 0; j0 < nrhs; j0 += cj) {
-      const int nj = std::min(cj, nrhs - j0);
-      for (int a = 0; a < n2; a++)
-        for (int j = 0; j < nj; j++) hs[(size_t)a * nj + j] = Ub[a + (size_t)(j0 + j) * n2];
-      std::vector<double> hsn(hs.begin(), hs.begin() + (size_t)n2 * nj);
-      HIPCHK(S.upload(hsn));
-      launch_gemm_small(st_, neq, n2, nj, d.X.p, n2, S.p, Yd.p, nj, 0.0, 1.0);
-      HIPCHK(hipMemcpyAsync(hy.data(), Yd.p, sizeof(double) * (size_t)neq * nj, hipMemcpyDeviceToHost, st_));
-      HIPCHK(hipStreamSynchronize(st_));
-      for (int q = 0; q < n1; q++) {
-        const int r = y.eq_to_perm[sam_.meqn1[q] - 1];
-        for (int j = 0; j < nj; j++) acc[q + (size_t)(j0 + j) * n1] = hy[(size_t)r * nj + j];
-      }
+  const bool bound = n2 > 0 && Ub;
+  if (n1 == 0) return 0;
+  if (!bound && !Fi) {
+    std::fill(Ui, Ui + (size_t)n1 * nrhs, 0.0);
+    return 0;
+  }
+  // x = K_ii^-1 F_i first, then per column chunk Y = [B; I] U_b and the sum of
+  // both in the caller's order
+  int rc = 0;
+  if (Fi && (rc = solve_rows(nrhs, Fi, err))) {
+    (void)hipStreamSynchronize(st_);
+    return rc;
+  }
+  const int cj = bound ? std::min(nrhs, 64) : nrhs;
+  HIPCHK(d.sk_t.alloc((size_t)n1 * nrhs));  // free again once x is there
+  if (bound) {
+    HIPCHK(d.rc_s.alloc(2 * (size_t)n2 * nrhs));
+    HIPCHK(d.rc_y.alloc((size_t)neq * cj));
+    HIPCHK(hipMemcpyAsync(d.rc_s.p, Ub, sizeof(double) * (size_t)n2 * nrhs, hipMemcpyHostToDevice, st_));
+  }
+  for (int j0 = 0; j0 < nrhs; j0 += cj) {
+    const int nj = std::min(cj, nrhs - j0);
+    if (bound) {
+      double* const S = d.rc_s.p + (size_t)n2 * nrhs;  // this chunk of U_b, row-major
+      launch_rows_in(st_, n2, nj, nullptr, d.rc_s.p + (size_t)j0 * n2, n2, S, nj);
+      launch_gemm_small(st_, neq, n2, nj, d.X.p, n2, S, d.rc_y.p, nj, 0.0, 1.0);
     }
+    launch_rows_out(st_, n1, nj, d.p1.p, bound ? d.rc_y.p : nullptr, nj, Fi ? d.sk_x.p + j0 : nullptr, nrhs,
+                    d.sk_t.p + (size_t)j0 * n1, n1);
   }
-  if (Fi) {
-    std::vector<double> x((size_t)n1 * nrhs);
-    int rc = solve_kii(nrhs, Fi, x.data(), err);
-    if (rc) return rc;
-    for (size_t k = 0; k < x.size(); k++) acc[k] += x[k];
-  }
-  std::copy(acc.begin(), acc.end(), Ui);
+  HIPCHK(d2h(Ui, d.sk_t.p, sizeof(double) * (size_t)n1 * nrhs));
   return 0;
 }
 

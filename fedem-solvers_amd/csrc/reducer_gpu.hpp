@@ -140,6 +140,8 @@ class DeviceReducer {
   hipStream_t st_ = nullptr;
   // device-to-host copy ordered after the handle's stream work
   hipError_t d2h(void* dst, const void* src, size_t bytes) const;
+  int internal_to_host(const double* A, int nc, double* out) const;
+  int solve_rows(int nrhs, const double* R_eq, std::string& err);
   bool uploaded_ = false;
   double upd_flops_ = 0;
   int64_t upd_launches_ = 0;
