@@ -219,11 +219,23 @@ __global__ __launch_bounds__(256) void k_diag_extract(int n, const int* __restri
     atomicMax(amax, (unsigned long long)__double_as_longlong(fmax(fmax(top[0], top[1]), fmax(top[2], top[3]))));
 }
 
+// Start values of a reduction, in one launch: no element and no pivot flagged,
+// the pivot statistics below, *amax = 0.
+__global__ __launch_bounds__(256) void k_begin(int nel, int* __restrict__ ebad, int n, int* __restrict__ sing,
+                                               int* __restrict__ stats, double* __restrict__ amax) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < nel) ebad[i] = 0;
+  if (i < n) sing[i] = 0;
+  if (i < PIVOT_STATS) stats[i] = i < 3 ? 0 : INT_MAX;
+  if (i == 0) *amax = 0.0;
+}
+
 // pivot statistics of the factor: out[0] negative pivots, out[1] true-zero
 // and out[2] reduced-to-zero pivots replaced, out[3..5] the first such
-// pivot columns (INT_MAX: none); out starts at {0, 0, 0, INT_MAX x 3}
-__global__ void k_pivot_stats(int n, const double* __restrict__ dpiv, const int* __restrict__ sing,
-                              int* __restrict__ out) {
+// pivot columns, out[6] the first flagged element (INT_MAX: none); k_begin's
+// start values
+__global__ void k_pivot_stats(int n, const double* __restrict__ dpiv, const int* __restrict__ sing, int nel,
+                              const int* __restrict__ ebad, int* __restrict__ out) {
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
     if (sing[c]) {
       atomicAdd(&out[sing[c]], 1);
@@ -233,6 +245,44 @@ __global__ void k_pivot_stats(int n, const double* __restrict__ dpiv, const int*
       atomicMin(&out[3], c);
     }
   }
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < nel; e += gridDim.x * blockDim.x)
+    if (ebad[e]) atomicMin(&out[6], e);
+}
+
+// The reduced matrices in the reference's layout (CMSTRS, GRAV), nd x nd and
+// column-major: first the n2 boundary rows in DOF order (pos2, 1-based), then
+// the ngen component modes, zeros up to nd.  SK from the Schur complement
+// (lower triangle of the root front, ld n2; null: left zero) and K11, SM from
+// M22, M12 (ngen x n2) and M11, G (nd x 3) from Ge (n2 x 3) and Gg (ngen x 3),
+// the products row-major, squares symmetrised; the element mass total follows.
+// One launch and one copy instead of up to eight copies, each waited for.
+__global__ __launch_bounds__(256) void k_reduced(int nd, int n2, int ngen, const int* __restrict__ pos2,
+                                                 const double* __restrict__ S22, ReducedParts q,
+                                                 const double* __restrict__ mass, double* __restrict__ out) {
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x, nn = (int64_t)nd * nd;
+  const bool has_mass = mass != nullptr;
+  if (g < nn) {
+    const int i = (int)(g % nd), j = (int)(g / nd);
+    double k = 0.0, m = 0.0;
+    if (i < n2 && j < n2) {
+      const int a = pos2[i] - 1, b = pos2[j] - 1, lo = min(a, b), hi = max(a, b);
+      if (S22) k = S22[hi + (int64_t)lo * n2];
+      if (has_mass) m = 0.5 * (q.M22[(int64_t)a * n2 + b] + q.M22[(int64_t)b * n2 + a]);
+    } else if (min(i, j) >= n2 && max(i, j) < n2 + ngen) {
+      const int a = i - n2, b = j - n2;
+      k = 0.5 * (q.K11[a * ngen + b] + q.K11[b * ngen + a]);
+      if (has_mass) m = 0.5 * (q.M11[a * ngen + b] + q.M11[b * ngen + a]);
+    } else if (max(i, j) < n2 + ngen && has_mass) {
+      m = q.M12[(int64_t)(max(i, j) - n2) * n2 + pos2[min(i, j)] - 1];
+    }
+    out[g] = k;
+    if (has_mass) out[nn + g] = m;
+  }
+  if (has_mass && g < 3 * nd) {
+    const int i = (int)(g % nd), c = (int)(g / nd);
+    out[2 * nn + g] = i < n2 ? q.Ge[(pos2[i] - 1) * 3 + c] : i < n2 + ngen ? q.Gg[(i - n2) * 3 + c] : 0.0;
+  }
+  if (has_mass && g == 0) out[2 * nn + 3 * nd] = *mass;
 }
 
 __global__ void k_fill(double* __restrict__ p, int64_t n, double v) {
@@ -1570,8 +1620,18 @@ void launch_diag_extract(hipStream_t st, int n, const int* dpos, const double* v
     k_diag_extract<<<std::min(256u, nblk(n, 256)), 256, 0, st>>>(n, dpos, val, rs, adiag,
                                                                  reinterpret_cast<unsigned long long*>(amax));
 }
-void launch_pivot_stats(hipStream_t st, int n, const double* dpiv, const int* sing, int* out) {
-  if (n > 0) k_pivot_stats<<<std::min(1024u, nblk(n, 256)), 256, 0, st>>>(n, dpiv, sing, out);
+void launch_begin(hipStream_t st, int nel, int* ebad, int n, int* sing, int* stats, double* amax) {
+  k_begin<<<nblk(std::max({nel, n, PIVOT_STATS}), 256), 256, 0, st>>>(nel, ebad, n, sing, stats, amax);
+}
+void launch_pivot_stats(hipStream_t st, int n, const double* dpiv, const int* sing, int nel, const int* ebad,
+                        int* out) {
+  const int most = std::max(n, nel);
+  if (most > 0) k_pivot_stats<<<std::min(1024u, nblk(most, 256)), 256, 0, st>>>(n, dpiv, sing, nel, ebad, out);
+}
+void launch_reduced(hipStream_t st, int nd, int n2, int ngen, const int* pos2, const double* S22,
+                    const ReducedParts& q, const double* mass, double* out) {
+  const int64_t n = std::max((int64_t)nd * nd, (int64_t)3 * nd + 1);
+  k_reduced<<<nblk(n, 256), 256, 0, st>>>(nd, n2, ngen, pos2, S22, q, mass, out);
 }
 void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
   if (n > 0) k_fill<<<(unsigned)std::min<int64_t>(nblk(n, 256), 16384), 256, 0, st>>>(p, n, v);

@@ -56,12 +56,24 @@ void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, 
                             const double* r1, double* Fred);
 // singular-pivot support of the factorisation: the original (or, with rs,
 // equilibrated) diagonal of the first n permuted equations and its largest
-// magnitude (amax must start at 0); the pivot statistics
-// out[0..5] = negative, true-zero, reduced-to-zero pivots, first column of
-// each (out must start at {0, 0, 0, INT_MAX, INT_MAX, INT_MAX})
+// magnitude (amax must start at 0)
 void launch_diag_extract(hipStream_t st, int n, const int* dpos, const double* val, const double* rs, double* adiag,
                          double* amax);
-void launch_pivot_stats(hipStream_t st, int n, const double* dpiv, const int* sing, int* out);
+// start values of the element flags, pivot flags, statistics and amax; the
+// statistics out[0..6] = negative, true-zero, reduced-to-zero pivots, first
+// column of each, first flagged element
+constexpr int PIVOT_STATS = 7;
+void launch_begin(hipStream_t st, int nel, int* ebad, int n, int* sing, int* stats, double* amax);
+void launch_pivot_stats(hipStream_t st, int n, const double* dpiv, const int* sing, int nel, const int* ebad,
+                        int* out);
+// the products the reduced matrices are made of (row-major; null if absent),
+// and the matrices SK, SM, G and the element mass in one record (mass null:
+// SK only)
+struct ReducedParts {
+  double *M22, *K11, *M11, *M12, *Ge, *Gg;
+};
+void launch_reduced(hipStream_t st, int nd, int n2, int ngen, const int* pos2, const double* S22,
+                    const ReducedParts& q, const double* mass, double* out);
 // Pivot-block inverse tiles whose sum X_ij = -X_ii sum_k L_ik X_kj has more
 // than INV_CHUNK terms are summed in INV_CHUNK-tile chunks in parallel.
 constexpr int INV_CHUNK = 4;

@@ -238,6 +238,8 @@ struct DeviceReducer::Impl {
   // coefficients; two pinned copies (step parity)
   DBuf<double> lzrec;
   HBuf<double> hrec;
+  HBuf<int> hpiv;     // the pivot statistics and
+  HBuf<double> hred;  // the reduced matrices on their way to the host
   hipEvent_t lz_ev[2]{};
   hipStream_t side = nullptr;  // lookahead stream of the factorisation
   hipEvent_t fj[2]{};          // its fork and join events
@@ -909,7 +911,7 @@ int DeviceReducer::upload(std::string& err) {
   }
   HIPCHK(d.ebad.alloc(part_.nel));
   HIPCHK(d.emass.alloc(part_.nel + 1));
-  HIPCHK(d.piv.alloc(6));
+  HIPCHK(d.piv.alloc(PIVOT_STATS));
   mark("value buffers");
   // gravity directions: unit accelerations on translational equation DOFs
   std::vector<double> a((size_t)y.neq * 3, 0.0);
@@ -1283,7 +1285,7 @@ int DeviceReducer::reduce(std::string& err) {
   HIPCHK(hipEventRecord(d.ev[0], st));
   mark("start issued");
   // ---- element matrices
-  HIPCHK(hipMemsetAsync(d.ebad.p, 0, sizeof(int) * part_.nel, st));
+  launch_begin(st, part_.nel, d.ebad.p, std::max(1, n1), d.sing.p, d.piv.p, d.amax.p);
   launch_hex8(st, (int)d.hexl.size(), d.hexlist.p, d.eptr.p, d.enodes.p, d.xyz.p, d.eprop.p, d.eoff.p, d.Kp.p,
               d.Mp.p, d.ebad.p);
   launch_andes4(st, (int)d.shl.size(), d.shlist.p, d.eptr.p, d.enodes.p, d.xyz.p, d.eprop.p, d.eoff.p, d.Kp.p,
@@ -1310,17 +1312,11 @@ int DeviceReducer::reduce(std::string& err) {
   }
   // original diagonal of K_ii for the singular-pivot test (equilibrated for
   // the mixed-precision factor), no pivot flagged yet
-  HIPCHK(hipMemsetAsync(d.amax.p, 0, sizeof(double), st));
-  HIPCHK(hipMemsetAsync(d.sing.p, 0, sizeof(int) * (size_t)std::max(1, n1), st));
   launch_diag_extract(st, n1, d.dpos.p, d.Kv.p, d.mixed ? d.dscale.p : nullptr, d.adiag.p, d.amax.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(d.ev[2], st));
   mark("elements and assembly issued");
   // ---- multifrontal LDL^T; the Schur front ends up holding K_bb - K_bi K_ii^-1 K_ib
-  {
-    int init[6] = {0, 0, 0, INT_MAX, INT_MAX, INT_MAX};
-    HIPCHK(hipMemcpyAsync(d.piv.p, init, sizeof init, hipMemcpyHostToDevice, st));
-  }
   if (opt_.time_updates && d.upd_ev.size() < 2 * (size_t)upd_launches_) {  // another schedule may launch more
     const size_t have = d.upd_ev.size();
     d.upd_ev.resize(2 * (size_t)upd_launches_);
@@ -1389,7 +1385,7 @@ int DeviceReducer::reduce(std::string& err) {
                      factor_ops));
   }
   HIPCHK(fork_err);
-  launch_pivot_stats(st, n1, d.dpiv.p, d.sing.p, d.piv.p);
+  launch_pivot_stats(st, n1, d.dpiv.p, d.sing.p, part_.nel, d.ebad.p, d.piv.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(d.ev[3], st));
   mark("factor issued");
@@ -1451,18 +1447,19 @@ int DeviceReducer::reduce(std::string& err) {
   HIPCHK(hipEventRecord(d.ev[4], st));
   mark("B issued");
   // error checks of the numeric phase
-  int hbad[6] = {0, 0, 0, 0, 0, 0};
-  HIPCHK(hipMemcpyAsync(hbad, d.piv.p, sizeof hbad, hipMemcpyDeviceToHost, st));
-  std::vector<int> eb(part_.nel);
-  HIPCHK(hipMemcpyAsync(eb.data(), d.ebad.p, sizeof(int) * part_.nel, hipMemcpyDeviceToHost, st));
+  HIPCHK(d.hpiv.alloc(PIVOT_STATS));
+  HIPCHK(hipMemcpyAsync(d.hpiv.p, d.piv.p, sizeof(int) * PIVOT_STATS, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  for (int e = 0; e < part_.nel; e++)
-    if (eb[e]) {
-      err = "element " + std::to_string(e + 1) +
-            (eb[e] == -3 ? " has a degenerate shell geometry (zero area or length)"
-                         : " has a non-positive Jacobian determinant");
-      return -4;
-    }
+  int hbad[PIVOT_STATS];
+  std::copy(d.hpiv.p, d.hpiv.p + PIVOT_STATS, hbad);
+  if (const int e = hbad[6]; e != INT_MAX) {
+    int code = 0;
+    HIPCHK(d2h(&code, d.ebad.p + e, sizeof code));
+    err = "element " + std::to_string(e + 1) +
+          (code == -3 ? " has a degenerate shell geometry (zero area or length)"
+                      : " has a non-positive Jacobian determinant");
+    return -4;
+  }
   res_.n_negative = hbad[0];
   res_.n_true_zero = hbad[1];
   res_.n_reduced_zero = hbad[2];
@@ -1777,66 +1774,79 @@ int DeviceReducer::reduce(std::string& err) {
   HIPCHK(hipEventRecord(d.ev[5], st));
   mark("modes done on host");
   // ---- reduced mass: Z = M [B; I], M22 = [B; I]^T Z ; modes: K11, M11, M12
-  std::vector<double> M22, K11, M11, M12, Ge, Gg, S22((size_t)n2 * n2);
+  const int nd = res_.ndim;
   const int maxab = std::max(std::max(n2, 3), std::max(nev, 1));
+  const size_t nrec = 2 * (size_t)nd * nd + 3 * (size_t)nd + 1;  // SK, SM, G, element mass
   HIPCHK(d.part.alloc((size_t)xty_chunks(neq) * maxab * maxab));
-  HIPCHK(d.acc.alloc((size_t)maxab * maxab));
-  auto xty_host = [&](int na, int nb, const double* X, int ldx, const double* Yv, int ldy,
-                      std::vector<double>& out) -> int {
-    out.assign((size_t)na * nb, 0.0);
-    if (na == 0 || nb == 0) return 0;
-    launch_xty(st, neq, na, nb, X, ldx, Yv, ldy, d.part.p, d.acc.p);
-    HIPCHK(hipMemcpyAsync(out.data(), d.acc.p, sizeof(double) * na * nb, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    return 0;
+  HIPCHK(d.acc.alloc(nrec + (size_t)n2 * n2 + 2 * (size_t)ngen * ngen + (size_t)ngen * n2 + 3 * (size_t)(n2 + ngen)));
+  HIPCHK(d.hred.alloc(nrec));
+  ReducedParts rp{};
+  {
+    double* at = d.acc.p + nrec;
+    auto take = [&](size_t n) {
+      double* r = at;
+      at += n;
+      return r;
+    };
+    rp.M22 = take((size_t)n2 * n2);
+    rp.K11 = take((size_t)ngen * ngen);
+    rp.M11 = take((size_t)ngen * ngen);
+    rp.M12 = take((size_t)ngen * n2);
+    rp.Ge = take(3 * (size_t)n2);
+    rp.Gg = take(3 * (size_t)ngen);
+  }
+  auto xty = [&](int na, int nb, const double* X, int ldx, const double* Yv, int ldy, double* out) {
+    if (na > 0 && nb > 0) launch_xty(st, neq, na, nb, X, ldx, Yv, ldy, d.part.p, out);
   };
   if (!opt_.no_mass && n2 > 0) {
     if (!defer_z) mass_mm(st, neq, d, n2, d.X.p, n2, d.Z.p, n2);
-    if (xty_host(n2, n2, d.X.p, n2, d.Z.p, n2, M22)) return -3;
+    xty(n2, n2, d.X.p, n2, d.Z.p, n2, rp.M22);
   }
   if (ngen > 0) {
     HIPCHK(d.Yl.alloc((size_t)neq * std::max(ngen, opt_.lanczos_block)));
     launch_spmm(st, d.node_rows(neq), ngen, d.rowptr.p, d.colind.p, d.Kv.p, d.Phi.p, nev, d.Yl.p, ngen);
-    if (xty_host(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, K11)) return -3;
+    xty(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, rp.K11);
     if (!opt_.no_mass) {
       mass_mm(st, neq, d, ngen, d.Phi.p, nev, d.Yl.p, ngen);
-      if (xty_host(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, M11)) return -3;
-      if (n2 > 0 && xty_host(ngen, n2, d.Phi.p, nev, d.Z.p, n2, M12)) return -3;
+      xty(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, rp.M11);
+      xty(ngen, n2, d.Phi.p, nev, d.Z.p, n2, rp.M12);
     }
   }
   HIPCHK(hipEventRecord(d.ev[6], st));
   // ---- gravity: g = M a ; G_e = [B; I]^T g ; G_g = Phi^T g
+  const bool vgi = !opt_.no_mass && opt_.want_vgi && n1 > 0;
   if (!opt_.no_mass) {
     HIPCHK(d.Tmp.alloc((size_t)neq * std::max(3, std::max(opt_.lanczos_block, nev))));
     mass_mm(st, neq, d, 3, d.grav.p, 3, d.Tmp.p, 3);
-    if (n2 > 0 && xty_host(n2, 3, d.X.p, n2, d.Tmp.p, 3, Ge)) return -3;
-    if (ngen > 0 && xty_host(ngen, 3, d.Phi.p, nev, d.Tmp.p, 3, Gg)) return -3;
-    if (opt_.want_vgi && n1 > 0) {
+    xty(n2, 3, d.X.p, n2, d.Tmp.p, 3, rp.Ge);
+    xty(ngen, 3, d.Phi.p, nev, d.Tmp.p, 3, rp.Gg);
+    if (vgi) {
       SolvePlan* p3 = nullptr;
       if (get_plan(y, d, 3, p3, err)) return -3;
       if (ensure_work(d, std::max(std::max(n2, 3), opt_.lanczos_block), err)) return -3;
       HIPCHK(d.Zl.alloc((size_t)neq * std::max(3, opt_.lanczos_block)));
       HIPCHK(d.Wl.alloc((size_t)neq * std::max(3, opt_.lanczos_block)));
       if (int rc2 = solve_int(st, d, y, opt_, *p3, d.Tmp.p, d.Zl.p, d.Wl.p, nullptr, err)) return rc2;
-      std::vector<double> v((size_t)neq * 3);
-      HIPCHK(hipMemcpyAsync(v.data(), d.Wl.p, sizeof(double) * v.size(), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      res_.vgi.assign((size_t)n1 * 3, 0.0);
-      for (int q = 0; q < n1; q++) {  // MEQN1 order: equation q+1
-        int r = y.eq_to_perm[sam_.meqn1[q] - 1];
-        for (int c = 0; c < 3; c++) res_.vgi[(size_t)c * n1 + q] = v[(size_t)r * 3 + c];
-      }
+      launch_rows_out(st, n1, 3, d.p1.p, d.Wl.p, 3, nullptr, 0, d.Zl.p, n1);  // MEQN1 order
     }
+  }
+  if (nd > 0) {
+    const bool s22 = n2 > 0 && !d.mixed;  // the Schur complement in the root front
+    launch_reduced(st, nd, n2, ngen, d.pos2.p, s22 ? d.pool.p + y.foff[schur] : nullptr, rp,
+                   opt_.no_mass ? nullptr : d.emass.p + part_.nel, d.acc.p);
+    HIPCHK(hipGetLastError());
   }
   HIPCHK(hipEventRecord(d.ev[7], st));
   mark("mass and gravity issued");
-  // ---- Schur complement out of the root front
-  if (n2 > 0 && d.mixed) S22 = d.s22;
-  else if (n2 > 0) {
-    HIPCHK(hipMemcpyAsync(S22.data(), d.pool.p + y.foff[schur], sizeof(double) * n2 * n2, hipMemcpyDeviceToHost, st));
+  if (nd > 0)
+    HIPCHK(hipMemcpyAsync(d.hred.p, d.acc.p, sizeof(double) * (opt_.no_mass ? (size_t)nd * nd : nrec),
+                          hipMemcpyDeviceToHost, st));
+  else if (!opt_.no_mass)
+    HIPCHK(hipMemcpyAsync(d.hred.p + nrec - 1, d.emass.p + part_.nel, sizeof(double), hipMemcpyDeviceToHost, st));
+  if (vgi) {
+    res_.vgi.resize((size_t)n1 * 3);
+    HIPCHK(hipMemcpyAsync(res_.vgi.data(), d.Zl.p, sizeof(double) * res_.vgi.size(), hipMemcpyDeviceToHost, st));
   }
-  if (!opt_.no_mass)
-    HIPCHK(hipMemcpyAsync(&res_.mass_fe, d.emass.p + part_.nel, sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
   mark("device done");
   times_.elements = ev_ms(d.ev[0], d.ev[1]);
@@ -1854,37 +1864,21 @@ int DeviceReducer::reduce(std::string& err) {
     for (int64_t q = 0; q < ui; q++) times_.update_kernel_ms += ev_ms(d.upd_ev[2 * q], d.upd_ev[2 * q + 1]);
     times_.update_launches = ui;
   }
-  // ---- reduced matrices in the reference layout (CMSTRS, GRAV): first ndof2
-  // rows in DOF order through dofPosIn2, then the ngen component modes, then
-  // zero padding up to ndim
-  const int nd = res_.ndim;
-  const std::vector<int>& pos2 = sam_.dofPosIn2;
-  res_.SK.assign((size_t)nd * nd, 0.0);
-  res_.SM.assign(opt_.no_mass ? 0 : (size_t)nd * nd, 0.0);
-  res_.G.assign(opt_.no_mass ? 0 : (size_t)nd * 3, 0.0);
-  for (int j = 0; j < n2; j++)
-    for (int i = 0; i < n2; i++) {
-      int a = pos2[i] - 1, b = pos2[j] - 1;
-      double v = a >= b ? S22[a + (size_t)b * n2] : S22[b + (size_t)a * n2];
-      res_.SK[i + (size_t)j * nd] = v;
-      if (!opt_.no_mass) res_.SM[i + (size_t)j * nd] = 0.5 * (M22[(size_t)a * n2 + b] + M22[(size_t)b * n2 + a]);
-    }
-  for (int a = 0; a < ngen; a++)
-    for (int b = 0; b < ngen; b++) {
-      res_.SK[(n2 + a) + (size_t)(n2 + b) * nd] = 0.5 * (K11[(size_t)a * ngen + b] + K11[(size_t)b * ngen + a]);
-      if (!opt_.no_mass) res_.SM[(n2 + a) + (size_t)(n2 + b) * nd] = 0.5 * (M11[(size_t)a * ngen + b] + M11[(size_t)b * ngen + a]);
-    }
+  const size_t nn = (size_t)nd * nd;
+  const double* h = d.hred.p;
+  res_.SK.assign(h, h + nn);
   if (!opt_.no_mass) {
-    for (int a = 0; a < ngen; a++)
+    res_.SM.assign(h + nn, h + 2 * nn);
+    res_.G.assign(h + 2 * nn, h + 2 * nn + 3 * (size_t)nd);
+    res_.mass_fe = h[nrec - 1];
+  }
+  if (d.mixed) {  // the Schur complement from the refined B
+    const std::vector<int>& pos2 = sam_.dofPosIn2;
+    for (int j = 0; j < n2; j++)
       for (int i = 0; i < n2; i++) {
-        double v = M12[(size_t)a * n2 + (pos2[i] - 1)];
-        res_.SM[(n2 + a) + (size_t)i * nd] = v;
-        res_.SM[i + (size_t)(n2 + a) * nd] = v;
+        const int a = pos2[i] - 1, b = pos2[j] - 1;
+        res_.SK[i + (size_t)j * nd] = d.s22[std::max(a, b) + (size_t)std::min(a, b) * n2];
       }
-    for (int c = 0; c < 3; c++) {
-      for (int i = 0; i < n2; i++) res_.G[i + (size_t)c * nd] = Ge[(size_t)(pos2[i] - 1) * 3 + c];
-      for (int a = 0; a < ngen; a++) res_.G[(n2 + a) + (size_t)c * nd] = Gg[(size_t)a * 3 + c];
-    }
   }
   return 0;
 }
