@@ -46,6 +46,14 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v);
 // (address and size), the permuted-row gather of column-major load vectors
 // and the scatter of the reduced rows into Fred
 int noalloc_scratch(double** ptr, size_t* bytes, std::string& err);
+// one block of a gathered upload: `bytes` (a multiple of 4, at most COPY_BLOCK)
+// from offset `from` of the pinned memory to dst
+struct CopyBlock {
+  void* dst;
+  unsigned from, bytes;
+};
+constexpr size_t COPY_BLOCK = 8192;
+void launch_copy_blocks(hipStream_t st, int n, const CopyBlock* table, const char* stage);
 // order changes (order.hip): rows of a column-major array into row-major rows
 // map[q], and the sum of up to two row-major arrays' rows map[q] back
 void launch_rows_in(hipStream_t st, int n, int nc, const int* map, const double* in, int64_t ldi, double* out, int ldo);

@@ -1,7 +1,7 @@
 // Change of order between the callers' vectors (column-major, equations in
 // SAM order) and the reducer's (row-major, rows in elimination order), on the
 // device, so that a vector crosses the bus once and the host does not touch
-// it.
+// it; and the gathered upload of small arrays.
 #include "kernels.hpp"
 
 namespace fgpu {
@@ -79,6 +79,20 @@ void launch_rows_out(hipStream_t st, int n, int nc, const int* map, const double
   by_columns(n, nc, [&](dim3 g, int c0, int k) {
     k_rows_out<<<g, 256, 0, st>>>(n, k, map, A ? A + c0 : nullptr, lda, B ? B + c0 : nullptr, ldb, out + c0 * ldo, ldo);
   });
+}
+
+// One workgroup per block of a gathered upload, table and data read straight
+// from pinned host memory (four words in flight per thread).
+__global__ __launch_bounds__(256) void k_copy_blocks(const CopyBlock* __restrict__ table, const char* __restrict__ stage) {
+  const CopyBlock b = table[blockIdx.x];
+  const unsigned* in = reinterpret_cast<const unsigned*>(stage + b.from);
+  unsigned* out = static_cast<unsigned*>(b.dst);
+#pragma unroll 4
+  for (unsigned i = threadIdx.x; i < b.bytes / 4; i += 256) out[i] = in[i];
+}
+
+void launch_copy_blocks(hipStream_t st, int n, const CopyBlock* table, const char* stage) {
+  if (n > 0) k_copy_blocks<<<n, 256, 0, st>>>(table, stage);
 }
 
 }  // namespace fgpu
