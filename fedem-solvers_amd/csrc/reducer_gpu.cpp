@@ -375,6 +375,7 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
                                   std::vector<Op>& ops, std::vector<int>& xrange, double& flops, int panel,
                                   int& inv_slots, bool lookahead) {
   xrange.clear();
+  std::vector<int> at;
   inv_slots = 0;
   flops = 0;
   // columns of a front cleared before the original entries go in (k_front_zero),
@@ -394,13 +395,16 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
       // extend-add task (front s, 16-column block j0): the (child, first,
       // end) ranges of child update columns landing in the block, in child
       // order, at xrange[3 b ..], kb of them
+      at.assign(y.chptr[s + 1] - y.chptr[s], 0);  // every child's first column not yet placed
       for (int j0 = 0; j0 < y.nrow[s]; j0 += 16) {
         FTask t{s, j0, (int)xrange.size() / 3, own(s), 0, 0};
         for (int q = y.chptr[s]; q < y.chptr[s + 1]; q++) {
           const int c = y.chlist[q], nu = y.nrow[c] - y.ncol[c];
           const int* rel = y.rel.data() + y.relptr[c];
-          const int ka = (int)(std::lower_bound(rel, rel + nu, j0) - rel);
-          const int kb = (int)(std::lower_bound(rel, rel + nu, j0 + 16) - rel);
+          const int ka = at[q - y.chptr[s]];
+          int kb = ka;
+          while (kb < nu && rel[kb] < j0 + 16) kb++;
+          at[q - y.chptr[s]] = kb;
           if (kb > ka) {
             xrange.push_back(c);
             xrange.push_back(ka);
