@@ -1501,16 +1501,17 @@ __global__ void k_front_scatter32(int n, const int* __restrict__ rowptr, const i
   }
 }
 
-// X[r][j] *= rs[r] (rows 0..nrows-1) and, with cs, *= cs[j] (row-major, nrhs columns)
+// Y[r][j] = X[r][j] rs[r] (rows 0..nrows-1) and, with cs, times cs[j]
+// (row-major, nrhs columns; Y may be X)
 __global__ void k_scale_rc(int64_t nrows, int nrhs, const double* __restrict__ rs, const double* __restrict__ cs,
-                           double* __restrict__ X) {
+                           const double* X, double* Y) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nrows * nrhs) return;
   const int64_t r = g / nrhs;
   const int j = (int)(g % nrhs);
   double v = X[g] * rs[r];
   if (cs) v *= cs[j];
-  X[g] = v;
+  Y[g] = v;
 }
 
 // y[i] = 1 / x[i]
@@ -1555,35 +1556,78 @@ __global__ __launch_bounds__(256) void k_sumsq2(int64_t n, const double* __restr
 }
 
 // Column dot products of up to three pairs (A_k, B_k) of row-major n x nr
-// arrays: block b sums rows [b COLDOT_ROWS, (b+1) COLDOT_ROWS) of each
-// column in row order into part[(b * npair + k) * nr + c]; k_coldot_sum
-// then adds the blocks in block order (a fixed order: same bits every run).
+// arrays: block b sums rows [b COLDOT_ROWS, (b+1) COLDOT_ROWS) of each column
+// into part[(b * npair + k) * nr + c].  Its threads stand W = min(nr, 256)
+// columns wide and as many rows high as fit, take every so many-th row and
+// add their sums in row order through LDS; k_coldot_sum then adds the blocks
+// in a fixed order (16 groups of them per column).  Bound by HBM: 45,000 rows
+// by 66 columns, one to three pairs, 158 + 44 -> 16 + 9 us on average (one
+// thread per column and 256 rows, one thread per column over all blocks).
 __global__ __launch_bounds__(256) void k_coldot_part(int64_t n, int nr, int npair, const double* __restrict__ A0,
                                                      const double* __restrict__ B0, const double* __restrict__ A1,
                                                      const double* __restrict__ B1, const double* __restrict__ A2,
                                                      const double* __restrict__ B2, double* __restrict__ part) {
+  __shared__ double red[3][256];
+  const int W = min(nr, 256), H = 256 / W, tid = threadIdx.x, g = tid / W;
   const int64_t r0 = (int64_t)blockIdx.x * COLDOT_ROWS, r1 = min(n, r0 + COLDOT_ROWS);
-  for (int c = threadIdx.x; c < nr; c += 256) {
+  for (int c0 = 0; c0 < nr; c0 += W) {
+    const int c = c0 + tid % W;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int64_t r = r0; r < r1; r++) {
-      const int64_t o = r * nr + c;
-      s0 += A0[o] * B0[o];
-      if (npair > 1) s1 += A1[o] * B1[o];
-      if (npair > 2) s2 += A2[o] * B2[o];
+    if (g < H && c < nr) {
+      if (npair == 3) {
+#pragma unroll 4
+        for (int64_t r = r0 + g; r < r1; r += H) {
+          const int64_t o = r * nr + c;
+          s0 += A0[o] * B0[o];
+          s1 += A1[o] * B1[o];
+          s2 += A2[o] * B2[o];
+        }
+      } else if (npair == 2) {
+#pragma unroll 4
+        for (int64_t r = r0 + g; r < r1; r += H) {
+          const int64_t o = r * nr + c;
+          s0 += A0[o] * B0[o];
+          s1 += A1[o] * B1[o];
+        }
+      } else {
+#pragma unroll 4
+        for (int64_t r = r0 + g; r < r1; r += H) s0 += A0[r * nr + c] * B0[r * nr + c];
+      }
     }
-    double* P = part + (int64_t)blockIdx.x * npair * nr + c;
-    P[0] = s0;
-    if (npair > 1) P[nr] = s1;
-    if (npair > 2) P[2 * nr] = s2;
+    red[0][tid] = s0;
+    red[1][tid] = s1;
+    red[2][tid] = s2;
+    __syncthreads();
+    if (tid < W && c < nr)
+      for (int k = 0; k < npair; k++) {
+        double s = red[k][tid];
+        for (int h = 1; h < H; h++) s += red[k][h * W + tid];
+        part[((int64_t)blockIdx.x * npair + k) * nr + c] = s;
+      }
+    __syncthreads();
   }
 }
 
-__global__ __launch_bounds__(256) void k_coldot_sum(int nb, int nr, int npair, const double* __restrict__ part,
-                                                    double* __restrict__ out) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx >= npair * nr) return;
+__global__ __launch_bounds__(1024) void k_coldot_sum(int nb, int n, const double* __restrict__ part,
+                                                     double* __restrict__ out) {
+  __shared__ double red[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, idx = blockIdx.x * 64 + lane;
+  const double* p = part + min(idx, n - 1);
   double s = 0.0;
-  for (int b = 0; b < nb; b++) s += part[(int64_t)b * npair * nr + idx];
+  int b = w;
+  for (; b + 7 * 16 < nb; b += 8 * 16) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = p[(int64_t)(b + 16 * u) * n];
+#pragma unroll
+    for (int u = 0; u < 8; u++) s += v[u];
+  }
+  for (; b < nb; b += 16) s += p[(int64_t)b * n];
+  red[w][lane] = s;
+  __syncthreads();
+  if (w > 0 || idx >= n) return;
+#pragma unroll
+  for (int k = 1; k < 16; k++) s += red[k][lane];
   out[idx] = s;
 }
 
@@ -1741,8 +1785,9 @@ void launch_front_scatter32(hipStream_t st, int n, const int* rowptr, const int*
                             const double* s, const int64_t* fmap, float* pool) {
   if (n > 0) k_front_scatter32<<<nblk(n, 256), 256, 0, st>>>(n, rowptr, colind, val, s, fmap, pool);
 }
-void launch_scale_rc(hipStream_t st, int64_t nrows, int nrhs, const double* rs, const double* cs, double* X) {
-  if (nrows * nrhs > 0) k_scale_rc<<<nblk(nrows * nrhs, 256), 256, 0, st>>>(nrows, nrhs, rs, cs, X);
+void launch_scale_rc(hipStream_t st, int64_t nrows, int nrhs, const double* rs, const double* cs, const double* X,
+                     double* Y) {
+  if (nrows * nrhs > 0) k_scale_rc<<<nblk(nrows * nrhs, 256), 256, 0, st>>>(nrows, nrhs, rs, cs, X, Y);
 }
 void launch_recip(hipStream_t st, int n, const double* x, double* y) {
   if (n > 0) k_recip<<<nblk(n, 256), 256, 0, st>>>(n, x, y);
@@ -1756,7 +1801,7 @@ void launch_coldots(hipStream_t st, int64_t n, int nr, int npair, const double* 
                     double* out) {
   const int nb = coldot_blocks(n);
   if (nb > 0) k_coldot_part<<<nb, 256, 0, st>>>(n, nr, npair, A0, B0, A1, B1, A2, B2, part);
-  k_coldot_sum<<<nblk((int64_t)npair * nr, 256), 256, 0, st>>>(nb, nr, npair, part, out);
+  k_coldot_sum<<<nblk((int64_t)npair * nr, 64), 1024, 0, st>>>(nb, npair * nr, part, out);
 }
 void launch_col_axpby(hipStream_t st, int64_t n, int nr, const double* a, const double* X, const double* b,
                       double* Y) {

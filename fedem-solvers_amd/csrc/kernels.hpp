@@ -165,14 +165,15 @@ constexpr int SUMSQ_BLOCKS = 512;
 void launch_diag_scale(hipStream_t st, int n, const int* dpos, const double* val, double* s);
 void launch_front_scatter32(hipStream_t st, int n, const int* rowptr, const int* colind, const double* val,
                             const double* s, const int64_t* fmap, float* pool);
-void launch_scale_rc(hipStream_t st, int64_t nrows, int nrhs, const double* rs, const double* cs, double* X);
+void launch_scale_rc(hipStream_t st, int64_t nrows, int nrhs, const double* rs, const double* cs, const double* X,
+                     double* Y);
 void launch_recip(hipStream_t st, int n, const double* x, double* y);
 void launch_axpby(hipStream_t st, int64_t n, double a, const double* X, double b, double* Y);
 void launch_sumsq2(hipStream_t st, int64_t n, const double* x, const double* y, double* part);
 // Column dot products out[k * nr + c] = sum_r A_k[r][c] B_k[r][c] of npair
 // (<= 3) pairs of row-major n x nr arrays, summed in a fixed order; part
 // holds coldot_blocks(n) * npair * nr doubles.
-constexpr int COLDOT_ROWS = 256;
+constexpr int COLDOT_ROWS = 64;
 int coldot_blocks(int64_t n);
 void launch_coldots(hipStream_t st, int64_t n, int nr, int npair, const double* A0, const double* B0,
                     const double* A1, const double* B1, const double* A2, const double* B2, double* part,

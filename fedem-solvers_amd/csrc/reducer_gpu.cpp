@@ -1186,17 +1186,17 @@ static int refine_state(double rel, double prev, int steps, const ReduceOptions&
   return 0;
 }
 
-// One approximate solve D = K_ii^{-1} Rin on the mixed-precision factor:
-// D = S (K~_ii)^{-1} S Rin with K~ = S K S the equilibrated matrix whose FP32
-// LDL^T the fronts hold.  Rin (neq x nrhs, internal rows read) is scaled in
-// place; D's boundary rows are zero.
+// One approximate solve D = K_ii^{-1} R on the mixed-precision factor:
+// D = S (K~_ii)^{-1} S R with K~ = S K S the equilibrated matrix whose FP32
+// LDL^T the fronts hold.  R's internal rows are read, `scaled` takes S R (neq x
+// nrhs); D's boundary rows are zero.
 static void approx_solve(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, int neq, int ndof1,
-                         double* Rin, double* Yw, double* D) {
-  launch_scale_rc(st, ndof1, sp.nrhs, d.dscale.p, nullptr, Rin);
-  run_forward(st, d, sp, Rin, Yw);
+                         const double* R, double* scaled, double* Yw, double* D) {
+  launch_scale_rc(st, ndof1, sp.nrhs, d.dscale.p, nullptr, R, scaled);
+  run_forward(st, d, sp, scaled, Yw);
   launch_fill(st, D + (size_t)ndof1 * sp.nrhs, (int64_t)(neq - ndof1) * sp.nrhs, 0.0);  // boundary rows
   run_backward(st, d, sp, Yw, D);
-  launch_scale_rc(st, ndof1, sp.nrhs, d.dscale.p, nullptr, D);
+  launch_scale_rc(st, ndof1, sp.nrhs, d.dscale.p, nullptr, D, D);
 }
 
 // Mixed precision: conjugate gradients on K_ii X = b, one independent CG
@@ -1231,15 +1231,11 @@ static int pcg_int(hipStream_t st, DeviceReducer::Impl& d, const Symbolic& y, co
     HIPCHK(hipStreamSynchronize(st));
     return 0;
   };
-  // z = K~^-1 r (approx_solve scales its input in place: it gets a copy)
-  auto precond = [&]() -> int {
-    HIPCHK(hipMemcpyAsync(d.cg_t.p, R, sizeof(double) * nint, hipMemcpyDeviceToDevice, st));
-    approx_solve(st, d, sp, neq, n1, d.cg_t.p, Yw, d.cg_z.p);
-    return 0;
-  };
+  // z = K~^-1 r
+  auto precond = [&]() { approx_solve(st, d, sp, neq, n1, R, d.cg_t.p, Yw, d.cg_z.p); };
   bool stationary = false;
   double prev = INFINITY;
-  if (int rc = precond()) return rc;
+  precond();
   if (int rc = dots(2, R, d.cg_z.p, X, X, nullptr, nullptr)) return rc;
   for (int c = 0; c < nr; c++) {
     rz[c] = h[c];
@@ -1290,7 +1286,7 @@ static int pcg_int(hipStream_t st, DeviceReducer::Impl& d, const Symbolic& y, co
     if (state > 0) return 0;
     if (state < 0) return -6;
     prev = rel;
-    if (int rc = precond()) return rc;
+    precond();
     if (stationary) continue;
     if (int rc = dots(1, R, d.cg_z.p, nullptr, nullptr, nullptr, nullptr)) return rc;
     for (int c = 0; c < nr; c++) {
@@ -1501,7 +1497,7 @@ int DeviceReducer::reduce(std::string& err) {
     if (d.mixed) {
       // the backward pass of the equilibrated factor gives S_i^-1 B S_b
       launch_recip(st, n2, d.dscale.p + n1, d.dcs.p);
-      launch_scale_rc(st, n1, n2, d.dscale.p, d.dcs.p, d.X.p);
+      launch_scale_rc(st, n1, n2, d.dscale.p, d.dcs.p, d.X.p, d.X.p);
       // refinement against the FP64 matrix: Z = K [B; I] has the residual
       // -(K_ii B + K_ib) in its internal rows and K_bb + K_bi B in its
       // boundary rows (the Schur complement once B has converged)
