@@ -254,7 +254,8 @@ __global__ void k_pivot_stats(int n, const double* __restrict__ dpiv, const int*
 // the ngen component modes, zeros up to nd.  SK from the Schur complement
 // (lower triangle of the root front, ld n2; null: left zero) and K11, SM from
 // M22, M12 (ngen x n2) and M11, G (nd x 3) from Ge (n2 x 3) and Gg (ngen x 3),
-// the products row-major, squares symmetrised; the element mass total follows.
+// the products row-major, of squares the lower triangle; the element mass
+// total follows.
 // One launch and one copy instead of up to eight copies, each waited for.
 __global__ __launch_bounds__(256) void k_reduced(int nd, int n2, int ngen, const int* __restrict__ pos2,
                                                  const double* __restrict__ S22, ReducedParts q,
@@ -267,11 +268,11 @@ __global__ __launch_bounds__(256) void k_reduced(int nd, int n2, int ngen, const
     if (i < n2 && j < n2) {
       const int a = pos2[i] - 1, b = pos2[j] - 1, lo = min(a, b), hi = max(a, b);
       if (S22) k = S22[hi + (int64_t)lo * n2];
-      if (has_mass) m = 0.5 * (q.M22[(int64_t)a * n2 + b] + q.M22[(int64_t)b * n2 + a]);
+      if (has_mass) m = q.M22[(int64_t)hi * n2 + lo];
     } else if (min(i, j) >= n2 && max(i, j) < n2 + ngen) {
-      const int a = i - n2, b = j - n2;
-      k = 0.5 * (q.K11[a * ngen + b] + q.K11[b * ngen + a]);
-      if (has_mass) m = 0.5 * (q.M11[a * ngen + b] + q.M11[b * ngen + a]);
+      const int at = (max(i, j) - n2) * ngen + min(i, j) - n2;
+      k = q.K11[at];
+      if (has_mass) m = q.M11[at];
     } else if (max(i, j) < n2 + ngen && has_mass) {
       m = q.M12[(int64_t)(max(i, j) - n2) * n2 + pos2[min(i, j)] - 1];
     }

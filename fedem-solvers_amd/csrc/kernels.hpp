@@ -132,8 +132,9 @@ void launch_diag_mm(hipStream_t st, int n, int nrhs, const int* dpos, const doub
 int xty_chunks(int n);
 // C = X^T Y (X n x na, Y n x nb, row-major; C na x nb row-major); acc
 // (optional) = C, or acc + C with acc_add
+// sym: C is symmetric, its strict upper triangle is not needed
 void launch_xty(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Y, int ldy,
-                double* part, double* C, double* acc = nullptr, bool acc_add = false);
+                double* part, double* C, double* acc = nullptr, bool acc_add = false, bool sym = false);
 // Y = alpha Y + beta X S (X n x na, S na x nb, row-major); up to 64 columns
 // on FP64 MFMA, where Y may be X itself (same leading dimension).
 void launch_gemm_small(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Sm,

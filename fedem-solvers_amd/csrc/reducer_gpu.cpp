@@ -1871,20 +1871,20 @@ int DeviceReducer::reduce(std::string& err) {
     rp.Ge = take(3 * (size_t)n2);
     rp.Gg = take(3 * (size_t)ngen);
   }
-  auto xty = [&](int na, int nb, const double* X, int ldx, const double* Yv, int ldy, double* out) {
-    if (na > 0 && nb > 0) launch_xty(st, neq, na, nb, X, ldx, Yv, ldy, d.part.p, out);
+  auto xty = [&](int na, int nb, const double* X, int ldx, const double* Yv, int ldy, double* out, bool sym = false) {
+    if (na > 0 && nb > 0) launch_xty(st, neq, na, nb, X, ldx, Yv, ldy, d.part.p, out, nullptr, false, sym);
   };
   if (!opt_.no_mass && n2 > 0) {
     if (!defer_z) mass_mm(st, neq, d, n2, d.X.p, n2, d.Z.p, n2);
-    xty(n2, n2, d.X.p, n2, d.Z.p, n2, rp.M22);
+    xty(n2, n2, d.X.p, n2, d.Z.p, n2, rp.M22, true);
   }
   if (ngen > 0) {
     HIPCHK(d.Yl.alloc((size_t)neq * std::max(ngen, opt_.lanczos_block)));
     launch_spmm(st, d.node_rows(neq), ngen, d.rowptr.p, d.colind.p, d.Kv.p, d.Phi.p, nev, d.Yl.p, ngen);
-    xty(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, rp.K11);
+    xty(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, rp.K11, true);
     if (!opt_.no_mass) {
       mass_mm(st, neq, d, ngen, d.Phi.p, nev, d.Yl.p, ngen);
-      xty(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, rp.M11);
+      xty(ngen, ngen, d.Phi.p, nev, d.Yl.p, ngen, rp.M11, true);
       xty(ngen, n2, d.Phi.p, nev, d.Z.p, n2, rp.M12);
     }
   }
