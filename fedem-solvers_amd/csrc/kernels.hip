@@ -842,7 +842,8 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
 
 // ---------------------------------------------------------------- update
 // Task: sn, a = ti, b = tj (64x64 tiles of the trailing lower triangle),
-// k0 = panel, kb = panel width (<= 256), je = column limit.  F[I,J] -= (L_I
+// k0 = panel, kb = panel width (<= 256), je = column limit; blockIdx.y the
+// quadrant of the tile where a launch has four.  F[I,J] -= (L_I
 // D) L_J^T over the panel.  A wave holds 16 XA x 32 of the tile in its MFMA accumulators and
 // reads both operands straight from the panel (128 contiguous bytes per
 // column and 16 rows), eight columns ahead of their products: a 16x16x4 FP64
@@ -858,18 +859,24 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
 // and write (16 flop per byte of it).  Measured at 128 columns: one front of
 // 6000 rows 45 TFLOP/s (four waves of 32x32: 42; staged through LDS: 37),
 // 16 fronts of 1500 rows 44 (41; 36), one of 1900 rows 17 (24; 21): the wide
-// waves where a launch has UPD_WIDE or more tiles, else the four.
-constexpr int UPD_WIDE = 2048;
+// waves where a launch has UPD_WIDE or more tiles, else the four.  A tile of
+// 256 columns keeps the matrix cores of its CU for 7 us, so up to UPD_NARROW
+// tiles, half as many as CUs, go as four workgroups of 32 x 32 each: 7 us a
+// launch; 17x13x11 block 291 -> 230 us in all, 117x109 plate 671 -> 613 (limit
+// 256: 237, 630; 512: 242, 659).
+constexpr int UPD_WIDE = 2048, UPD_NARROW = 128;
 
-template <int XA, class T>
-__global__ __launch_bounds__(XA == 2 ? 256 : 128, XA == 2 ? 4 : 3) void k_update(const FTask* __restrict__ tasks, DevSym S,
+template <int XA, int YB, class T>
+__global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update(const FTask* __restrict__ tasks, DevSym S,
                                                                 T* __restrict__ pool) {
-  constexpr int YB = 2, CH = 8, ST = CH / 4;
+  constexpr int CH = 8, ST = CH / 4;
   const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
   const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn], kb = t.kb;
   T* F = pool + S.foff[sn];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
-  const int I0 = k0 + kb + 64 * t.a + 16 * XA * (wv >> 1), J0 = k0 + kb + 64 * t.b + 32 * (wv & 1);
+  const int quad = blockIdx.y;  // 0 of 1, or the quadrant of the tile
+  const int I0 = k0 + kb + 64 * t.a + 32 * (quad >> 1) + 16 * XA * (wv >> 1);
+  const int J0 = k0 + kb + 64 * t.b + 32 * (quad & 1) + 16 * YB * (wv & 1);
   const int je = t.je > 0 ? t.je : ld;
   if (I0 >= ld || J0 >= je || J0 >= I0 + 16 * XA) return;  // nothing of this part is stored
   // rows past the front repeat its last one and are not stored
@@ -902,8 +909,8 @@ __global__ __launch_bounds__(XA == 2 ? 256 : 128, XA == 2 ? 4 : 3) void k_update
     for (int y = 0; y < YB; y++) Jp[y] += ST * step;
     Dq += CH;
   };
-  const int kf = kb & ~(2 * CH - 1);
-  // a chunk from column c on, after the whole pairs of chunks; the columns
+  const int kf = kb & ~(CH - 1);
+  // a chunk from column c on, after the whole chunks; the columns
   // past the panel repeat the last one with a zero pivot
   auto load_tail = [&](int c, Stage& g) {
 #pragma unroll
@@ -942,13 +949,13 @@ __global__ __launch_bounds__(XA == 2 ? 256 : 128, XA == 2 ? 4 : 3) void k_update
         acc[x][y][r] = seed ? F[(int64_t)i + (int64_t)j * ld] : (T)0;
       }
   for (int c = 0; c < kf; c += 2 * CH) {
-    load(g1);
+    if (c + CH < kf) load(g1);
     multiply(g0);
     if (c + 2 * CH < kf) load(g0);
-    multiply(g1);
+    if (c + CH < kf) multiply(g1);
   }
-  for (int c = kf; c < kb; c += CH) {
-    load_tail(c, g0);
+  if (kf < kb) {
+    load_tail(kf, g0);
     multiply(g0);
   }
 #pragma unroll
@@ -1702,8 +1709,9 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
     if (n > 0) k_trsm<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                        \
   }                                                                                                        \
   void launch_update(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {                    \
-    if (n >= UPD_WIDE) k_update<4, T><<<n, 128, 0, st>>>(t, S, pool);                                       \
-    else if (n > 0) k_update<2, T><<<n, 256, 0, st>>>(t, S, pool);                                          \
+    if (n >= UPD_WIDE) k_update<4, 2, T><<<n, 128, 0, st>>>(t, S, pool);                                     \
+    else if (n > UPD_NARROW) k_update<2, 2, T><<<n, 256, 0, st>>>(t, S, pool);                               \
+    else if (n > 0) k_update<1, 1, T><<<dim3(n, 4), 256, 0, st>>>(t, S, pool);                               \
   }                                                                                                        \
   void launch_inv_off(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,               \
                       const int64_t* ioff, T* ipool) {                                                     \
