@@ -1,13 +1,16 @@
 // gfx950 kernel of the 4-noded ANDES shell element: one 64-lane workgroup
 // per element runs the phases of shell_andes4.hpp (each phase on all lanes,
 // a barrier between phases) and writes the packed lower node-pair 6x6
-// blocks of the projected stiffness and of the lumped mass.
+// blocks of the projected stiffness and of the lumped mass.  Bound by the
+// phases' LDS reads and their latency: two waves per SIMD (256 registers, 21
+// KB of LDS) and 3x3 blocks of the 24x24 products per lane take 334 us for
+// 12,753 elements, one wave per SIMD with 28 KB and a lane per entry 505.
 #include "kernels.hpp"
 #include "shell_andes4.hpp"
 
 namespace fgpu {
 
-__global__ __launch_bounds__(64) void k_andes4(int nel, const int* __restrict__ elist, const int* __restrict__ eptr,
+__global__ __launch_bounds__(64, 2) void k_andes4(int nel, const int* __restrict__ elist, const int* __restrict__ eptr,
                                                const int* __restrict__ enodes, const double* __restrict__ xyz,
                                                const double* __restrict__ eprop, const int64_t* __restrict__ eoff,
                                                double* __restrict__ Kp, double* __restrict__ Mp,

@@ -65,17 +65,28 @@ struct Work {
   // bending directions of each corner: to the previous, next and opposite corner
   double bdir[4][3][3];  // (s_x, s_y, l)
   double binv[4][9], minv[4][9];     // inverses of the direction matrices (row-major)
-  double bnat[4][3][12];             // directional second derivatives (cols w0..3, tx0..3, ty0..3)
-  double mnat[4][3][7];              // natural membrane strains over the higher-order coordinates
-  double Kn[4][3][12], Qn[4][3][7];  // Cartesian nodal tables
-  double Kbar[3][12], Qbar[3][7];
-  double H[7][12];                   // membrane DOFs (u0..3, v0..3, rz0..3) -> higher-order coordinates
-  double Lm[3][12], Lb[3][12];       // lumping tables (membrane: u, v, rz; bending: w, tx, ty)
-  double B[4][6][24], CB[4][6][24];  // strain-displacement at the Gauss points; C |J| B (later K P)
-  double K[24][25];                  // global-frame stiffness before projection
-  double R[24][6], Rs[24][6];        // rigid-body basis (unit columns) and R (R^T R)^-1
-  double cr[4][3];                   // corners relative to the centroid
+  // the tables' last reader is step 7, K's first writer step 9
+  union {
+    struct {
+      double bnat[4][3][12];             // directional second derivatives (cols w0..3, tx0..3, ty0..3)
+      double mnat[4][3][7];              // natural membrane strains over the higher-order coordinates
+      double Kn[4][3][12], Qn[4][3][7];  // Cartesian nodal tables
+      double Kbar[3][12], Qbar[3][7];
+      double H[7][12];                   // membrane DOFs (u0..3, v0..3, rz0..3) -> higher-order coordinates
+      double Lm[3][12], Lb[3][12];       // lumping tables (membrane: u, v, rz; bending: w, tx, ty)
+    };
+    double K[24][25];  // global-frame stiffness before projection
+  };
+  double cr[4][3];  // corners relative to the centroid
   double Si[9];
+  // the basis' last reader runs beside step 6, B's writer is step 7
+  union {
+    struct {
+      double R[24][6], Rs[24][6];  // rigid-body basis (unit columns) and R (R^T R)^-1
+    };
+    double B[4][6][24];  // strain-displacement at the Gauss points
+  };
+  double CB[4][6][24];  // C |J| B (later K P)
   double P[24][25];
   double em[24];                     // lumped mass diagonal
 };
@@ -445,14 +456,13 @@ SHELL_HD inline void step_cb(int lane, Work& w) {
 // to the global axes (lane = 8 a + b)
 SHELL_HD inline void step_stiffness(int lane, Work& w) {
   const int a = lane / 8, b = lane % 8;
-  double k[3][3];
-  for (int i = 0; i < 3; i++)
-    for (int j = 0; j < 3; j++) {
-      double s = 0.0;
-      for (int g = 0; g < 4; g++)
-        for (int r = 0; r < 6; r++) s += w.B[g][r][3 * a + i] * w.CB[g][r][3 * b + j];
-      k[i][j] = s;
-    }
+  double k[3][3] = {};
+  const double(*B)[24] = w.B[0];
+  const double(*CB)[24] = w.CB[0];
+#pragma unroll 4
+  for (int gr = 0; gr < 24; gr++)
+    for (int i = 0; i < 3; i++)
+      for (int j = 0; j < 3; j++) k[i][j] += B[gr][3 * a + i] * CB[gr][3 * b + j];
   for (int i = 0; i < 3; i++)
     for (int j = 0; j < 3; j++) {
       double s = 0.0;
@@ -468,25 +478,17 @@ SHELL_HD inline void step_stiffness(int lane, Work& w) {
 SHELL_HD inline void step_rigid(int lane, Work& w) {
   if (lane >= 6) return;
   const int k = lane;
-  double col[24];
-  for (int i = 0; i < 24; i++) col[i] = 0.0;
-  for (int n = 0; n < 4; n++) {
-    const double* x = w.cr[n];
-    double* u = col + 6 * n;
-    if (k < 3) {
-      u[k] = 1.0;
-    } else {
-      const int a = k - 3;  // rotation about axis a: displacement e_a x x
-      const int b = (a + 1) % 3, c = (a + 2) % 3;
-      u[b] = -x[c];
-      u[c] = x[b];
-      u[3 + a] = 1.0;
-    }
-  }
+  // entry (corner n, component q) of column k: translation along k, or the
+  // displacement e_a x x of a rotation about axis a = k - 3
+  const int a = k - 3, b = (a + 4) % 3, c = (a + 5) % 3;
+  auto entry = [&](int n, int q) {
+    if (k < 3) return q == k ? 1.0 : 0.0;
+    return q == b ? -w.cr[n][c] : q == c ? w.cr[n][b] : q == 3 + a ? 1.0 : 0.0;
+  };
   double s = 0.0;
-  for (int i = 0; i < 24; i++) s += col[i] * col[i];
+  for (int i = 0; i < 24; i++) s += entry(i / 6, i % 6) * entry(i / 6, i % 6);
   s = sqrt(s);
-  for (int i = 0; i < 24; i++) w.R[i][k] = col[i] / s;
+  for (int i = 0; i < 24; i++) w.R[i][k] = entry(i / 6, i % 6) / s;
 }
 
 // ---- step 11 (lane 0): inverse Gram matrix of the rotation columns
@@ -512,24 +514,28 @@ SHELL_HD inline void step_projector(int lane, Work& w) {
     }
   }
 }
+// 3x3 blocks (lane = 8 a + b) here and in step 13: six loads for nine products
 SHELL_HD inline void step_projector2(int lane, Work& w) {
-  for (int idx = lane; idx < 576; idx += 64) {
-    const int i = idx / 24, j = idx % 24;
-    double s = 0.0;
-    for (int k = 0; k < 6; k++) s += w.Rs[i][k] * w.R[j][k];
-    w.P[i][j] = (i == j ? 1.0 : 0.0) - s;
-  }
+  const int a = 3 * (lane / 8), b = 3 * (lane % 8);
+  double s[3][3] = {};
+  for (int k = 0; k < 6; k++)
+    for (int i = 0; i < 3; i++)
+      for (int j = 0; j < 3; j++) s[i][j] += w.Rs[a + i][k] * w.R[b + j][k];
+  for (int i = 0; i < 3; i++)
+    for (int j = 0; j < 3; j++) w.P[a + i][b + j] = (a + i == b + j ? 1.0 : 0.0) - s[i][j];
 }
 
 // ---- step 13: K P into CB (as a 24 x 24 array)
 SHELL_HD inline void step_kp(int lane, Work& w) {
   double* KP = &w.CB[0][0][0];
-  for (int idx = lane; idx < 576; idx += 64) {
-    const int i = idx / 24, j = idx % 24;
-    double s = 0.0;
-    for (int k = 0; k < 24; k++) s += w.K[i][k] * w.P[k][j];
-    KP[i * 24 + j] = s;
-  }
+  const int a = 3 * (lane / 8), b = 3 * (lane % 8);
+  double s[3][3] = {};
+#pragma unroll 4
+  for (int k = 0; k < 24; k++)
+    for (int i = 0; i < 3; i++)
+      for (int j = 0; j < 3; j++) s[i][j] += w.K[a + i][k] * w.P[k][b + j];
+  for (int i = 0; i < 3; i++)
+    for (int j = 0; j < 3; j++) KP[(a + i) * 24 + b + j] = s[i][j];
 }
 
 // entry idx (< 360) of the packed lower node-pair blocks of P^T (K P):
@@ -543,6 +549,7 @@ SHELL_HD inline double projected_entry(int idx, const Work& w, int& r, int& c) {
   c = 6 * b + q % 6;
   const double* KP = &w.CB[0][0][0];
   double s = 0.0;
+#pragma unroll 8
   for (int k = 0; k < 24; k++) s += w.P[k][r] * KP[k * 24 + c];
   return s;
 }
