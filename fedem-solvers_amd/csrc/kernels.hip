@@ -843,24 +843,26 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
 // ---------------------------------------------------------------- update
 // Task: sn, a = ti, b = tj (64x64 tiles of the trailing lower triangle),
 // k0 = panel, kb = panel width (<= 256), je = column limit; blockIdx.y the
-// quadrant of the tile where a launch has four.  F[I,J] -= (L_I
-// D) L_J^T over the panel.  A wave holds 16 XA x 32 of the tile in its MFMA accumulators and
-// reads both operands straight from the panel (128 contiguous bytes per
-// column and 16 rows), eight columns ahead of their products: a 16x16x4 FP64
-// step keeps the matrix core for 64 cycles, so the first-level cache feeds
-// it without staging, barriers or staging arithmetic.  FP64: the
-// accumulators start from the tile's current values and the A operand is
-// negated, so the chain forms F - sum (L_I D) L_J^T and the tile is only
-// stored at the end.  FP32 (mixed precision) sums the products from zero and
-// subtracts them from the tile at the end: accumulating onto the tile
-// through the FP32 MFMA left the factor too inexact for the FP64 refinement
-// of a thin 200x200 plate to converge.
-// Bound by the matrix cores and, at 128 columns a panel, by the tile's read
-// and write (16 flop per byte of it).  Measured at 128 columns: one front of
-// 6000 rows 45 TFLOP/s (four waves of 32x32: 42; staged through LDS: 37),
-// 16 fronts of 1500 rows 44 (41; 36), one of 1900 rows 17 (24; 21): the wide
-// waves where a launch has UPD_WIDE or more tiles, else the four.  A tile of
-// 256 columns keeps the matrix cores of its CU for 7 us, so up to UPD_NARROW
+// quadrant of the tile where a launch has four.  F[I,J] -= (L_I D) L_J^T over
+// the panel.  A wave holds 16 XA x 16 YB of the tile in its MFMA accumulators
+// and reads both operands straight from the panel, eight columns ahead of
+// their products: a 16x16x4 FP64 step keeps the matrix core for 64 cycles, so
+// the first-level cache feeds it without staging, barriers or staging
+// arithmetic.  FP64: the accumulators start from the tile's current values and
+// the J operand is scaled by -D, so the chain forms F - sum (L_I D) L_J^T and
+// the tile is only stored at the end.  FP32 (mixed precision) sums the products
+// from zero and subtracts them from the tile at the end: accumulating onto the
+// tile through the FP32 MFMA left the factor too inexact for the FP64
+// refinement of a thin 200x200 plate to converge.
+// Bound by the matrix cores and by the rate of the first-level cache, which
+// takes a quarter of a line a lane group: 16-byte loads of row pairs need half
+// its cycles.  At 256 columns a panel two fronts of 6000 rows take 50 TFLOP/s
+// and 16 of 1500 rows 51 (8-byte loads 43 and 44; waves of 64x64 46 and 40; at
+// 128 columns, staged through LDS, 37 and 36); three or four chunks in flight
+// and scalar address bases make no difference.  One front of 1900 rows has
+// too few 64x32 waves (17 TFLOP/s, four waves of 32x32 24): the wide waves
+// where a launch has UPD_WIDE or more tiles, else the four.  A tile of 256
+// columns keeps the matrix cores of its CU for 7 us, so up to UPD_NARROW
 // tiles, half as many as CUs, go as four workgroups of 32 x 32 each: 7 us a
 // launch; 17x13x11 block 291 -> 230 us in all, 117x109 plate 671 -> 613 (limit
 // 256: 237, 630; 512: 242, 659).
@@ -879,16 +881,25 @@ __global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update
   const int J0 = k0 + kb + 64 * t.b + 32 * (quad & 1) + 16 * YB * (wv & 1);
   const int je = t.je > 0 ? t.je : ld;
   if (I0 >= ld || J0 >= je || J0 >= I0 + 16 * XA) return;  // nothing of this part is stored
-  // rows past the front repeat its last one and are not stored
+  // Rows go to the lanes in pairs where a wave has 32 of them: lane lr takes
+  // rows 2 lr and 2 lr + 1, which are row lr of two MFMA tiles, by one 16-byte
+  // load.  Rows past the front repeat its last one (and the entry behind it)
+  // and are not stored.
+  constexpr int VI = XA > 1 ? 2 : 1, VJ = YB > 1 ? 2 : 1;
+  typedef T veci __attribute__((ext_vector_type(VI), aligned(sizeof(T))));
+  typedef T vecj __attribute__((ext_vector_type(VJ), aligned(sizeof(T))));
+  auto row_i = [&](int x) { return I0 + 16 * VI * x + VI * lr; };  // first row of lane's group x
   const T* base = F + (int64_t)(k0 + lk) * ld;
-  const T *Ip[XA], *Jp[YB];
+  const T *Ip[XA / VI], *Jp[YB / VJ];
 #pragma unroll
-  for (int x = 0; x < XA; x++) Ip[x] = base + min(I0 + 16 * x + lr, ld - 1);
+  for (int x = 0; x < XA / VI; x++) Ip[x] = base + min(row_i(x), ld - 1);
 #pragma unroll
-  for (int y = 0; y < YB; y++) Jp[y] = base + min(J0 + 16 * y + lr, ld - 1);
+  for (int y = 0; y < YB / VJ; y++) Jp[y] = base + min(J0 + 16 * VJ * y + VJ * lr, ld - 1);
   const double* Dp = S.dpiv + S.col0[sn] + k0;
   struct Stage {
-    T a[ST][XA], b[ST][YB], d[ST];
+    veci a[ST][XA / VI];
+    vecj b[ST][YB / VJ];
+    T d[ST];
   };
   // the next whole chunk, the pointers moving on (an address product per
   // load costs as much as the matrix step: 23 TFLOP/s)
@@ -898,19 +909,19 @@ __global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update
 #pragma unroll
     for (int s = 0; s < ST; s++) {
 #pragma unroll
-      for (int x = 0; x < XA; x++) g.a[s][x] = Ip[x][s * step];
+      for (int x = 0; x < XA / VI; x++) g.a[s][x] = *(const veci*)(Ip[x] + s * step);
 #pragma unroll
-      for (int y = 0; y < YB; y++) g.b[s][y] = Jp[y][s * step];
+      for (int y = 0; y < YB / VJ; y++) g.b[s][y] = *(const vecj*)(Jp[y] + s * step);
       g.d[s] = (T)Dq[4 * s];
     }
 #pragma unroll
-    for (int x = 0; x < XA; x++) Ip[x] += ST * step;
+    for (int x = 0; x < XA / VI; x++) Ip[x] += ST * step;
 #pragma unroll
-    for (int y = 0; y < YB; y++) Jp[y] += ST * step;
+    for (int y = 0; y < YB / VJ; y++) Jp[y] += ST * step;
     Dq += CH;
   };
-  const int kf = kb & ~(CH - 1);
-  // a chunk from column c on, after the whole chunks; the columns
+  const int kf = kb & ~(2 * CH - 1);
+  // a chunk from column c on, after the whole pairs of chunks; the columns
   // past the panel repeat the last one with a zero pivot
   auto load_tail = [&](int c, Stage& g) {
 #pragma unroll
@@ -918,9 +929,9 @@ __global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update
       const int k = c + 4 * s + lk, kc = min(k, kb - 1);
       const int64_t o = (int64_t)(kc - kf - lk) * ld;
 #pragma unroll
-      for (int x = 0; x < XA; x++) g.a[s][x] = Ip[x][o];
+      for (int x = 0; x < XA / VI; x++) g.a[s][x] = *(const veci*)(Ip[x] + o);
 #pragma unroll
-      for (int y = 0; y < YB; y++) g.b[s][y] = Jp[y][o];
+      for (int y = 0; y < YB / VJ; y++) g.b[s][y] = *(const vecj*)(Jp[y] + o);
       const T d = (T)Dp[kc];
       g.d[s] = k < kb ? d : (T)0;
     }
@@ -929,45 +940,69 @@ __global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update
   typename MF<T>::acc acc[XA][YB];
   auto multiply = [&](const Stage& g) {
 #pragma unroll
-    for (int s = 0; s < ST; s++)
+    for (int s = 0; s < ST; s++) {
+      T b[YB];
 #pragma unroll
-      for (int x = 0; x < XA; x++) {
-        const T a = seed ? -(g.a[s][x] * g.d[s]) : g.a[s][x] * g.d[s];
-#pragma unroll
-        for (int y = 0; y < YB; y++) acc[x][y] = MF<T>::op(g.b[s][y], a, acc[x][y]);
+      for (int y = 0; y < YB; y++) {
+        const T v = g.b[s][y / VJ][y % VJ] * g.d[s];
+        b[y] = seed ? -v : v;
       }
+#pragma unroll
+      for (int x = 0; x < XA; x++)
+#pragma unroll
+        for (int y = 0; y < YB; y++) acc[x][y] = MF<T>::op(b[y], g.a[s][x / VI][x % VI], acc[x][y]);
+    }
   };
+  // column of the accumulators' entry r
+  auto col_j = [&](int y, int r) { return J0 + 16 * VJ * (y / VJ) + VJ * MF<T>::col(lk, r) + y % VJ; };
   Stage g0, g1;
   if (kf > 0) load(g0);
 #pragma unroll
-  for (int x = 0; x < XA; x++)
+  for (int x = 0; x < XA / VI; x++)
 #pragma unroll
     for (int y = 0; y < YB; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = min(I0 + 16 * x + lr, ld - 1), j = min(J0 + 16 * y + MF<T>::col(lk, r), ld - 1);
-        acc[x][y][r] = seed ? F[(int64_t)i + (int64_t)j * ld] : (T)0;
+        veci v{};
+        if (seed) v = *(const veci*)(F + min(row_i(x), ld - 1) + (int64_t)min(col_j(y, r), ld - 1) * ld);
+#pragma unroll
+        for (int m = 0; m < VI; m++) acc[VI * x + m][y][r] = v[m];
       }
-  for (int c = 0; c < kf; c += 2 * CH) {
-    if (c + CH < kf) load(g1);
+  // (no load under a condition in here: where the paths join, the compiler
+  // waits for all that either may have in flight)
+  for (int c = 2 * CH; c < kf; c += 2 * CH) {
+    load(g1);
     multiply(g0);
-    if (c + 2 * CH < kf) load(g0);
-    if (c + CH < kf) multiply(g1);
+    load(g0);
+    multiply(g1);
   }
-  if (kf < kb) {
-    load_tail(kf, g0);
+  if (kf > 0) {
+    load(g1);
+    multiply(g0);
+    multiply(g1);
+  }
+  for (int c = kf; c < kb; c += CH) {
+    load_tail(c, g0);
     multiply(g0);
   }
 #pragma unroll
-  for (int x = 0; x < XA; x++)
+  for (int x = 0; x < XA / VI; x++)
 #pragma unroll
     for (int y = 0; y < YB; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = I0 + 16 * x + lr, j = J0 + 16 * y + MF<T>::col(lk, r);
-        if (i < ld && j < je && i >= j) {
-          if (seed) F[(int64_t)i + (int64_t)j * ld] = acc[x][y][r];
-          else F[(int64_t)i + (int64_t)j * ld] -= acc[x][y][r];
+        const int i = row_i(x), j = col_j(y, r);
+        if (i + VI - 1 < j || i >= ld || j >= je) continue;
+        T* out = F + (int64_t)i + (int64_t)j * ld;
+        veci v;
+#pragma unroll
+        for (int m = 0; m < VI; m++) v[m] = acc[VI * x + m][y][r];
+        if (i >= j && i + VI <= ld) {
+          *(veci*)out = seed ? v : *(veci*)out - v;
+        } else {
+#pragma unroll
+          for (int m = 0; m < VI; m++)
+            if (i + m >= j && i + m < ld) out[m] = seed ? v[m] : out[m] - v[m];
         }
       }
 }

@@ -980,13 +980,13 @@ int DeviceReducer::upload(std::string& err) {
   HIPCHK(d.Mv.alloc(nnz));
   if (d.mixed) {
     d.pool.release();
-    HIPCHK(d.pool32.alloc(y.fpool));
+    HIPCHK(d.pool32.alloc(y.fpool + PANEL_PAD));
     HIPCHK(d.dscale.alloc(y.neq));
     HIPCHK(d.dcs.alloc(std::max(1, y.ndof2)));
     HIPCHK(d.irpart.alloc(2 * SUMSQ_BLOCKS));
   } else {
     d.pool32.release();
-    HIPCHK(d.pool.alloc(y.fpool));
+    HIPCHK(d.pool.alloc(y.fpool + PANEL_PAD));
   }
   HIPCHK(d.ebad.alloc(part_.nel));
   HIPCHK(d.emass.alloc(part_.nel + 1));
