@@ -509,12 +509,17 @@ __device__ __forceinline__ float div_pivot(float a, double d) { return a / (floa
 // are carried as identity rows.
 // Bound by the dependent chain over the pivots (a reciprocal, a quotient and
 // a broadcast each): it sets the pace of every panel of the top separators.
-// A k_diag_trsm launch takes 18-19 us (117 x 109 plate, 48 x 24 x 24 block)
-// where 16-row sweeps with a division per pivot, L21 through X11 and loads
-// under conditions (each waiting for the one before) took 37-39 us.
+// 64 pivots take 25,400 cycles in one workgroup: 2500 of loads, four sweeps of
+// 2800 (issue bound: 15 broadcasts by two readlanes and a product per pivot),
+// 2000 around each (panel to and from LDS, its tiles), 1700 of stores.  A
+// k_diag_trsm launch of the 117 x 109 plate takes 14.7 us (18.2 with LDS reads
+// and stores under conditions, one wait each, and selects in the sweep that
+// kept the unread upper entries; 37-39 with 16-row sweeps, a division per pivot
+// and L21 through X11).
 //
-// diag_block: that factorisation in LDS; sA holds L (unit lower) below D,
-// sD = D, sX = L^-1 with zeros above it, all in FP64.
+// diag_block: that factorisation in LDS; sA holds L below its unit diagonal,
+// sD = D, sX = L^-1 with zeros above it, all in FP64 (sA on and above the
+// diagonal holds left-overs).
 template <class T>
 __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int k0, int kb, double (&sA)[64][65],
                                            double (&sX)[64][65], double (&sD)[64], double (&sT)[4][16][17],
@@ -549,17 +554,22 @@ __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int 
   };
   // A(ti, tj) -= (L(ti, p) D_p) L(tj, p)^T, 16 x 16 tiles, lower entries
   auto update_tile = [&](int ti, int tj, int p) {
+    // (all reads at once, and of whole tiles: nobody reads the entries above
+    // the diagonal)
+    double a[4], b[4], c[4];
+    double* out = &sA[16 * ti + lr][16 * tj + lk];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int m = 16 * p + 4 * q + lk;
+      a[q] = sA[16 * tj + lr][m];
+      b[q] = sA[16 * ti + lr][m] * sD[m];
+      c[q] = out[4 * q];
+    }
     f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int m0 = 0; m0 < 16; m0 += 4) {
-      const int m = 16 * p + m0 + lk;
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[16 * tj + lr][m], sA[16 * ti + lr][m] * sD[m], acc, 0, 0, 0);
-    }
+    for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[q], acc, 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int i = 16 * ti + lr, j = 16 * tj + lk + 4 * r;
-      if (i >= j) sA[i][j] -= acc[r];
-    }
+    for (int r = 0; r < 4; r++) out[4 * r] = c[r] - acc[r];
   };
   // X_00 = L_00^-1 where the sweep had no free lanes: lane c < 16 solves
   // column c against the uniformly read L
@@ -612,7 +622,9 @@ __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int 
       auto sweep = [&](auto test) {
         constexpr bool TEST = decltype(test)::value;
 #pragma unroll
-        for (int m = 0; m < 16; m++) a[m] = unit < 0 ? sA[row][c0 + m] : (unit == m ? 1.0 : 0.0);
+        for (int m = 0; m < 16; m++) u[m] = sA[row][c0 + m];
+#pragma unroll
+        for (int m = 0; m < 16; m++) a[m] = unit < 0 ? u[m] : (unit == m ? 1.0 : 0.0);
         auto pivot = [&](double v, int j) { return lane_bcast(TEST ? (fabs(v) > thr ? v : rep) : v, j); };
         d0 = a[0];
         double dj = pivot(a[0], 0), rj = recip64(dj);
@@ -625,7 +637,7 @@ __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int 
 #pragma unroll
           for (int m = j + 1; m < 16; m++) ub[m] = lane_bcast(u[j], m);
           const double l = quot64(u[j], dj, rj);
-          a[j] = lane > j ? l : (lane == j ? dj : a[j]);
+          a[j] = l;  // (on and above the diagonal as well, where nobody reads it)
           if (j == 15) break;
           __builtin_amdgcn_sched_barrier(0);
           a[j + 1] = __builtin_fma(-l, ub[j + 1], a[j + 1]);
@@ -646,11 +658,7 @@ __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int 
           S.sing[colbase + c0 + lane] = ac == 0.0 || fabs(d0) <= 1.0e3 * 2.220446049250313e-16 * ac ? 1 : 2;
       }
       if (unit < 0) {
-        // (the entries above the diagonal are not read again)
-        double dd = a[0];
-#pragma unroll
-        for (int m = 1; m < 16; m++) dd = m == lane ? a[m] : dd;
-        if (lane < 16) sD[c0 + lane] = dd;
+        if (lane < 16) sD[c0 + lane] = fabs(d0) > thr ? d0 : rep;
 #pragma unroll
         for (int m = 0; m < 16; m++) sA[row][c0 + m] = a[m];
       } else if (unit < 16) {
@@ -686,13 +694,19 @@ __device__ __forceinline__ void diag_block(const T* __restrict__ F, int ld, int 
 }
 
 // L_r = F_r L_kk^-T D^-1 for a 64-row tile at row R0: sF the rows, sL =
-// L_kk^-1 (lower, zeros above), C the panel's first column, d(j) its pivots.
-// Wave w takes rows 16 w .. 16 w + 15; column tile y only sums over the
-// column tiles m <= y, 40 MFMA steps a wave instead of 64.
+// L_kk^-1 (lower, zeros above), C the panel's first column, d(j) its pivots
+// (j < kb), read ahead of the products.  Wave w takes rows 16 w .. 16 w + 15;
+// column tile y only sums over the column tiles m <= y, 40 MFMA steps a wave
+// instead of 64.
 template <class T, class D>
 __device__ __forceinline__ void trsm_product(const T (*sF)[65], const T (*sL)[65], T* __restrict__ C, int ld, int R0,
                                              int kb, D d) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4, nsb = (kb + 15) >> 4;
+  double dv[4][4];
+#pragma unroll
+  for (int y = 0; y < 4; y++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) dv[y][r] = d(min(16 * y + MF<T>::col(lk, r), kb - 1));
   typename MF<T>::acc acc[4];
 #pragma unroll
   for (int y = 0; y < 4; y++) acc[y] = typename MF<T>::acc{};
@@ -714,7 +728,7 @@ __device__ __forceinline__ void trsm_product(const T (*sF)[65], const T (*sL)[65
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int j = 16 * y + MF<T>::col(lk, r);
-      if (j < kb) C[(int64_t)j * ld + i] = div_pivot(acc[y][r], d(j));
+      if (j < kb) C[(int64_t)j * ld + i] = div_pivot(acc[y][r], dv[y][r]);
     }
 }
 
@@ -727,12 +741,15 @@ template <class T>
 __device__ __forceinline__ void diag_store(T* __restrict__ Xg, double* __restrict__ dpiv, int xld, int k0, int kb,
                                            int col0, const double (&sD)[64], const double (&sX)[64][65],
                                            int* __restrict__ piv) {
-  const int tid = threadIdx.x;
-  for (int idx = tid; idx < 64 * 64; idx += 256) {
-    const int i = idx & 63, m = idx >> 6;
-    if (i < kb && m < kb) Xg[(int64_t)(k0 + i) + (int64_t)(k0 + m) * xld] = (T)sX[i][m];
-  }
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (tid < kb) dpiv[col0 + k0 + tid] = sD[tid];
+  double x[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) x[q] = sX[lane][wv + 4 * q];
+  T* out = Xg + (int64_t)k0 * (xld + 1) + lane;
+#pragma unroll
+  for (int q = 0; q < 16; q++)
+    if (lane < kb && wv + 4 * q < kb) out[(int64_t)(wv + 4 * q) * xld] = (T)x[q];
   (void)piv;
 }
 
