@@ -34,12 +34,20 @@ struct MvTask {
   int dst2;    // MV_Y: first row of V to keep the result in (-1: none); MV_YSUB: first row of Y
   int flags;
   int j0;
-  int pad;
+  int rsrc;    // MV_FORWARD_ALL: first right-hand side row of the source rows
 };
+// A level whose products read up to GM_BYTES of source rows gathers them itself
+// (up to three times the reads against a launch less), with up to GM_TILES
+// 16-column groups (registers).  Limits of 32 and 200 MiB came out the same to
+// 0.5 % from the 17x13x11 to the 45x41x43 block; the one that reads least stands.
+constexpr int64_t GM_BYTES = 8 << 20;
+constexpr int GM_TILES = 2;
 enum MvKind : int {
-  MV_FORWARD,    // operand rows contiguous
-  MV_BACK_ROWS,  // operand k contiguous, source rows through the fronts' row list
-  MV_BACK        // operand k contiguous, source rows contiguous in W
+  MV_FORWARD,      // operand rows contiguous
+  MV_FORWARD_ADD,  // the same, MV_ADD and MV_SUB targets gathered from the children
+  MV_FORWARD_ALL,  // source rows gathered from right-hand sides and children as well (up to GM_TILES column groups)
+  MV_BACK_ROWS,    // operand k contiguous, source rows through the fronts' row list
+  MV_BACK          // operand k contiguous, source rows contiguous in W
 };
 enum MvFlags : int {
   MV_FRONT = 1,                  // operand in the fronts (L21), not the solve panels

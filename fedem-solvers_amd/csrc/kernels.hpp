@@ -111,8 +111,8 @@ constexpr int INV_CHUNK = 4;
                     const int64_t* ioff, T* ipool);                                                       \
   /* solve products (solve.hip): nt 16-column groups of right-hand sides per task, kw K parts */         \
   void launch_mv(hipStream_t st, const MvTask* t, int n, int kind, int nt, int kw, const T* pool,         \
-                 const T* panel, const int* rows, const double* dpiv, double* W, double* V,               \
-                 const double* R, double* Y, double* X, int nrhs);
+                 const T* panel, const int* rows, const double* dpiv, const int2* kids, double* W,        \
+                 double* V, const double* R, double* Y, double* X, int nrhs);
 FGPU_FACTOR_DECLS(double)
 FGPU_FACTOR_DECLS(float)
 #undef FGPU_FACTOR_DECLS

@@ -183,7 +183,7 @@ enum OpKind {
   FRONT_ZERO,  // the first of the factor schedule, issued before the assembly
   EXTADD, DIAG, TRSM, DIAG_TRSM, UPDATE, INV_OFF, INV_PART, INV_FIN, PANEL,
   UPDATE_SIDE, FORK, JOIN,  // lookahead: trailing tiles on the side stream, fork/join with the main one
-  FW_INIT, FW_MV, BW_ROWS, BW_MV  // solve plans
+  FW_INIT, FW_MV, FW_MV_ADD, FW_MV_ALL, BW_ROWS, BW_MV  // solve plans
 };
 struct Op {
   int kind, off, n;
@@ -265,6 +265,7 @@ struct DeviceReducer::Impl {
   DBuf<int> ild;
   SolveLayout lay;
   DBuf<int> gptr, gsrc;  // forward init: the child update rows added to each work row, in child order
+  DBuf<int2> kids;       // the first two of them (-1: none)
   // inputs of the device structure build: SAM arrays, element types, per
   // node first equation / equation count / neighbour lists (+ DOF offsets),
   // per row its node, per column its front
@@ -593,7 +594,7 @@ static std::vector<int> work_rows(const Symbolic& y) {
   for (int s = 0; s < y.nsup; s++) woff[s + 1] = woff[s] + y.nrow[s];
   return woff;
 }
-static void build_gather(const Symbolic& y, std::vector<int>& gptr, std::vector<int>& gsrc) {
+static void build_gather(const Symbolic& y, std::vector<int>& gptr, std::vector<int>& gsrc, std::vector<int2>& kids) {
   const std::vector<int> woff = work_rows(y);
   gptr.assign(woff[y.nsup] + 1, 0);
   for (int s = 0; s < y.nsup; s++)
@@ -611,11 +612,22 @@ static void build_gather(const Symbolic& y, std::vector<int>& gptr, std::vector<
       const int* rel = y.rel.data() + y.relptr[c];
       for (int k = 0; k < nu; k++) gsrc[fill[woff[s] + rel[k]]++] = woff[c] + y.ncol[c] + k;
     }
+  kids.resize(std::max(1, woff[y.nsup]));
+  for (int w = 0; w < woff[y.nsup]; w++) {
+    const int n = gptr[w + 1] - gptr[w];
+    kids[w] = int2{n > 0 ? gsrc[gptr[w]] : -1, n > 1 ? gsrc[gptr[w] + 1] : -1};
+  }
 }
 
 // Solve plan for sp.nrhs right-hand sides: per level a forward init (fronts
 // with children), one product in a fused level and two in another, then the
-// levels top-down.  zero_start: also the backward pass from Y = 0.
+// levels top-down.  zero_start: also the backward pass from Y = 0.  Where no
+// front of a level has more than two children (a separator that is empty or
+// falls apart gives more), the products gather the update rows, and the pivot
+// rows too in a level of few source bytes (GM_BYTES): the init is left with the
+// pivot rows or with nothing.  A step of the 17x13x11 block's Lanczos loop is 8
+// launches shorter (reduction 4.83 -> 4.65 ms), the inits of a forward pass of
+// the 45x41x43 block take 70 us instead of 170.
 //
 // Right-hand sides go in groups of up to 96 columns, as even as 16-column
 // tiles allow.  A task's K range is split over the 4 waves of a workgroup
@@ -644,11 +656,12 @@ static void build_solve_plan(const Symbolic& y, const SolveLayout& lay, SolvePla
       t16 += (p.t.rn + 15) / 16 * ngrp;
       kmax = std::max(kmax, p.t.kn);
     }
-    const bool wide = kind == FW_MV && t16 >= 4096 && kmax <= ksplit;
+    const bool fw = kind == FW_MV || kind == FW_MV_ADD || kind == FW_MV_ALL;
+    const bool wide = fw && t16 >= 4096 && kmax <= ksplit;
     Op op{kind, (int)h.tasks.size(), 0, 4};
     if (wide || kmax <= 32) op.kw = 1;
     else if (t16 <= 256 && kmax > 4 * ksplit) op.kw = 16;
-    const int rt = op.kw == 1 && kind == FW_MV ? 64 : 16;
+    const int rt = op.kw == 1 && fw ? 64 : 16;
     for (const Piece& p : ps)
       for (int r0 = 0; r0 < p.t.rn; r0 += rt) {
         MvTask t = p.t;
@@ -675,17 +688,26 @@ static void build_solve_plan(const Symbolic& y, const SolveLayout& lay, SolvePla
   for (int l = 0; l < y.nlevels; l++) {
     const int i0 = (int)h.inits.size();
     std::vector<Piece> first, second;
+    bool pairs = l > 0;  // (the fronts of level 0 have no children)
+    int64_t bytes = 0;
+    for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++) {
+      const int s = y.lvsup[q];
+      pairs = pairs && (s == schur || y.chptr[s + 1] - y.chptr[s] <= 2);
+      bytes += (int64_t)((y.nrow[s] + 15) / 16) * y.ncol[s] * 128 * sp.nt * ngrp;
+    }
+    const bool all = pairs && sp.nt <= GM_TILES && bytes <= GM_BYTES;
     for (int q = y.lvptr[l]; q < y.lvptr[l + 1]; q++) {
       const int s = y.lvsup[q];
       if (s == schur) continue;
       const int nc = y.ncol[s], nu = y.nrow[s] - nc, ld = lay.ild[s];
       const bool leaf = y.chptr[s + 1] == y.chptr[s], up = y.parent[s] != schur && y.parent[s] >= 0;
       // rows that only the boundary would take are not formed
-      const int rows = up ? y.nrow[s] : nc;
-      if (!leaf)
+      const int rows = up && !pairs ? y.nrow[s] : nc;
+      if (!leaf && !all)
         for (int r0 = 0; r0 < rows; r0 += 64)
           h.inits.push_back({woff[s] + r0, std::min(64, rows - r0), std::max(0, std::min(64, nc - r0)), y.col0[s] + r0});
       const int from = leaf ? y.col0[s] : woff[s], ff = leaf ? MV_SRC_R : 0;
+      const size_t pieces = first.size();
       if (lay.fused[l]) {
         if (up)
           first.push_back({{lay.ioff[s] + nc, ld, nu, nc, from, 0, woff[s] + nc, -1, ff | (leaf ? MV_SET : MV_ADD), 0, 0}, 1, 0});
@@ -696,10 +718,11 @@ static void build_solve_plan(const Symbolic& y, const SolveLayout& lay, SolvePla
           second.push_back({{y.foff[s] + nc, y.nrow[s], nu, nc, woff[s], 0, woff[s] + nc, -1,
                              MV_FRONT | MV_SRC_V | (leaf ? MV_NEG : MV_SUB), 0, 0}, 1, 0});
       }
+      for (size_t p = pieces; p < first.size(); p++) first[p].t.rsrc = y.col0[s];
     }
     if ((int)h.inits.size() > i0) sp.fw.push_back({FW_INIT, i0, (int)h.inits.size() - i0});
-    cut(sp.fw, FW_MV, first);
-    cut(sp.fw, FW_MV, second);
+    cut(sp.fw, all ? FW_MV_ALL : pairs ? FW_MV_ADD : FW_MV, first);
+    cut(sp.fw, pairs ? FW_MV_ADD : FW_MV, second);
   }
   for (int z = 0; z < (zero_start ? 2 : 1); z++) {
     std::vector<Op>& ops = z ? sp.bw0 : sp.bw;
@@ -950,7 +973,8 @@ int DeviceReducer::upload(std::string& err) {
     build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_slots, opt_.factor_lookahead);
   }));
   std::vector<int> gptr, gsrc;
-  host_jobs.push_back(std::async(std::launch::async, [&]() { build_gather(y, gptr, gsrc); }));
+  std::vector<int2> kids;
+  host_jobs.push_back(std::async(std::launch::async, [&]() { build_gather(y, gptr, gsrc, kids); }));
   for (size_t i = 0; i < sps.size(); i++)
     host_jobs.push_back(std::async(std::launch::async, [&, i]() { plan_host(y, d, *sps[i], phs[i]); }));
   const int src = build_structure(err);
@@ -959,6 +983,7 @@ int DeviceReducer::upload(std::string& err) {
   mark("structure built");
   HIPCHK(d.gptr.upload(gptr));
   HIPCHK(d.gsrc.upload(gsrc));
+  HIPCHK(d.kids.upload(kids));
   for (size_t i = 0; i < sps.size(); i++)
     if (int rc = plan_upload(*sps[i], phs[i], err)) return rc;
   HIPCHK(ensure_side(d));
@@ -1117,12 +1142,14 @@ int DeviceReducer::prepare_solves(std::string& err) {
 static void run_mv(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const Op& op, const double* R,
                    double* Y, double* X) {
   const MvTask* t = sp.tasks.p + op.off;
-  const int kind = op.kind == FW_MV ? MV_FORWARD : op.kind == BW_ROWS ? MV_BACK_ROWS : MV_BACK;
+  const int kind = op.kind == FW_MV ? MV_FORWARD : op.kind == FW_MV_ADD ? MV_FORWARD_ADD :
+                   op.kind == FW_MV_ALL ? MV_FORWARD_ALL : op.kind == BW_ROWS ? MV_BACK_ROWS : MV_BACK;
   if (d.mixed)
-    launch_mv(st, t, op.n, kind, sp.nt, op.kw, d.pool32.p, d.ipool32.p, d.S.rows, d.S.dpiv, d.W.p, d.V.p, R, Y, X,
-              sp.nrhs);
+    launch_mv(st, t, op.n, kind, sp.nt, op.kw, d.pool32.p, d.ipool32.p, d.S.rows, d.S.dpiv, d.kids.p, d.W.p, d.V.p, R, Y,
+              X, sp.nrhs);
   else
-    launch_mv(st, t, op.n, kind, sp.nt, op.kw, d.pool.p, d.ipool.p, d.S.rows, d.S.dpiv, d.W.p, d.V.p, R, Y, X, sp.nrhs);
+    launch_mv(st, t, op.n, kind, sp.nt, op.kw, d.pool.p, d.ipool.p, d.S.rows, d.S.dpiv, d.kids.p, d.W.p, d.V.p, R, Y, X,
+              sp.nrhs);
 }
 
 // Y = D^{-1} L^{-1} R on the internal rows

@@ -23,31 +23,35 @@ __device__ __forceinline__ int xcd_task(int b, int n) {
   return c < r ? c * (q + 1) + m : r * (q + 1) + (c - r) * q + m;
 }
 
-// Result v of target row r, right-hand side j of task t.
-template <class T>
-__device__ __forceinline__ void mv_apply(const MvTask& t, int r, int j, double v, const double* __restrict__ dpiv,
-                                         double* W, double* V, double* Y, double* X, int nrhs) {
+// Result v of target row r, right-hand side j of task t.  GM > 0: base is what
+// the children add to a row of W, which the row itself does not hold.
+template <int GM, class T>
+__device__ __forceinline__ void mv_apply(const MvTask& t, int r, int j, double v, double base,
+                                         const double* __restrict__ dpiv, double* W, double* V, double* Y, double* X,
+                                         int nrhs) {
+  double* w = W + (int64_t)(t.dst + r) * nrhs + j;
   switch (t.flags & MV_APPLY) {
     case MV_Y:
       if (t.dst2 >= 0) V[(int64_t)(t.dst2 + r) * nrhs + j] = v;
       Y[(int64_t)(t.dst + r) * nrhs + j] = v / (double)(T)dpiv[t.dst + r];
       break;
-    case MV_SET: W[(int64_t)(t.dst + r) * nrhs + j] = v; break;
-    case MV_NEG: W[(int64_t)(t.dst + r) * nrhs + j] = -v; break;
-    case MV_ADD: W[(int64_t)(t.dst + r) * nrhs + j] += v; break;
-    case MV_SUB: W[(int64_t)(t.dst + r) * nrhs + j] -= v; break;
+    case MV_SET: *w = v; break;
+    case MV_NEG: *w = -v; break;
+    case MV_ADD: *w = (GM ? base : *w) + v; break;
+    case MV_SUB: *w = (GM ? base : *w) - v; break;
     case MV_X: X[(int64_t)(t.dst + r) * nrhs + j] = v; break;
     default:  // MV_YSUB
-      W[(int64_t)(t.dst + r) * nrhs + j] = (Y ? Y[(int64_t)(t.dst2 + r) * nrhs + j] : 0.0) - v;
+      *w = (Y ? Y[(int64_t)(t.dst2 + r) * nrhs + j] : 0.0) - v;
   }
 }
 
 // Sum of the K parts' 16 x 16 NT results in part order through LDS (red: KW
 // x 16 x 17 values) and their application; acc[y][q] holds target row lr,
-// right-hand side 16 y + lk + 4 q.
-template <int NT, int KW, class T>
-__device__ __forceinline__ void mv_combine(const MvTask& t, const f64x4 (&acc)[NT], double* red,
-                                           const double* __restrict__ dpiv, double* W, double* V, double* Y,
+// right-hand side 16 y + lk + 4 q; base[y] belongs to row (thread / 16) mod 16,
+// right-hand side 16 y + thread mod 16.
+template <int NT, int KW, int GM, class T>
+__device__ __forceinline__ void mv_combine(const MvTask& t, const f64x4 (&acc)[NT], const double (&base)[NT],
+                                           double* red, const double* __restrict__ dpiv, double* W, double* V, double* Y,
                                            double* X, int nrhs) {
   const int lane = threadIdx.x & 63, kw = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
 #pragma unroll
@@ -61,7 +65,7 @@ __device__ __forceinline__ void mv_combine(const MvTask& t, const f64x4 (&acc)[N
       double v = red[c * 17 + r];
 #pragma unroll
       for (int w = 1; w < KW; w++) v += red[w * 272 + c * 17 + r];
-      if (r < t.rn && j < nrhs) mv_apply<T>(t, r, j, v, dpiv, W, V, Y, X, nrhs);
+      if (r < t.rn && j < nrhs) mv_apply<GM, T>(t, r, j, v, base[y], dpiv, W, V, Y, X, nrhs);
     }
   }
 }
@@ -80,12 +84,20 @@ __device__ __forceinline__ void mv_combine(const MvTask& t, const f64x4 (&acc)[N
 // cores could take 19 TB/s.  KW = 4 reads 4.2-5.6 TB/s on fronts of 260 to
 // 5544 pivot columns (a plain copy moves 5.05 here); 64-row tasks 2.1-5.0,
 // 16 K parts 1.2-4.5 and only ahead when a level has few rows.
-template <int NT, int RT, int KW, class T>
+//
+// GM = 1: the rows of W that a task adds to hold nothing yet; it takes what
+// the front's (at most two) children add there, kids[row] being their rows of
+// W (-1: none), instead of a launch before it.  GM = 2: it takes its source
+// rows that way too, right-hand side row rsrc + k plus the children's, so that
+// the level is one launch (GM_BYTES).
+template <int NT, int RT, int KW, int GM, class T>
 __global__ __launch_bounds__(64 * RT * KW) void k_fw(const MvTask* __restrict__ tasks, const T* __restrict__ pool,
                                                      const T* __restrict__ panel, const double* __restrict__ dpiv,
-                                                     double* W, double* V, const double* R, double* Y, int nrhs) {
+                                                     const int2* __restrict__ kids, double* W, double* V,
+                                                     const double* R, double* Y, int nrhs) {
   static_assert(KW == 1 || RT == 1, "the K split works on 16-row tasks");
-  constexpr int CH = NT == 1 ? 32 : 16, ST = CH / 4;
+  constexpr int CH = NT == 1 && GM < 2 ? 32 : 16, ST = CH / 4;
+  constexpr int NB = KW == 1 ? 4 * NT : NT;  // results of a thread
   const MvTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
   const int r0 = 16 * (wv % RT), kw = wv / RT;
@@ -101,18 +113,55 @@ __global__ __launch_bounds__(64 * RT * KW) void k_fw(const MvTask* __restrict__ 
   f64x4 acc[NT];
 #pragma unroll
   for (int y = 0; y < NT; y++) acc[y] = f64x4{0.0, 0.0, 0.0, 0.0};
+  // row of W: the value at column c of the child's row q, 0.0 for none
+  auto kid = [&](int q, int c) { return W[(int64_t)max(q, 0) * nrhs + c]; };
+  // the children's part of this thread's results: rows first, values behind
+  // the first operand loads
+  double base[NB] = {}, add[2][NB];
+  int2 own{-1, -1};
+  const int erow = KW == 1 ? r0 + lr : (threadIdx.x >> 4) & 15;
+  auto ecol = [&](int e) { return KW == 1 ? 16 * (e / 4) + lk + 4 * (e % 4) : 16 * e + ((int)threadIdx.x & 15); };
+  if constexpr (GM > 0) own = kids[t.dst + min(erow, t.rn - 1)];
+  auto load_base = [&]() {
+    if constexpr (GM > 0)
+#pragma unroll
+      for (int e = 0; e < NB; e++) {
+        const int c = min(t.j0 + ecol(e), nrhs - 1);
+        add[0][e] = kid(own.x, c);
+        add[1][e] = kid(own.y, c);
+      }
+  };
   struct Stage {
     T a[ST];
-    double b[ST][NT];
+    double b[ST][NT], k0[GM == 2 ? ST : 1][NT], k1[GM == 2 ? ST : 1][NT];
+    int2 q[GM == 2 ? ST : 1];
+  };
+  int2 next[GM == 2 ? ST : 1];  // the children's rows of the chunk that is loaded next
+  auto load_kids = [&](int kc) {
+    if constexpr (GM == 2)
+#pragma unroll
+      for (int s = 0; s < ST; s++) next[s] = kids[t.src + min(kc + 4 * s + lk, ke - 1)];
   };
   auto load = [&](int kc, Stage& g) {
 #pragma unroll
     for (int s = 0; s < ST; s++) {
       const int k = min(kc + 4 * s + lk, ke - 1);
       g.a[s] = A[(int64_t)k * t.ld];
-      const double* b = src + (int64_t)k * nrhs;
+      const double* b = GM == 2 ? R + (int64_t)(t.rsrc + k) * nrhs : src + (int64_t)k * nrhs;
 #pragma unroll
       for (int y = 0; y < NT; y++) g.b[s][y] = b[col[y]];
+    }
+    if constexpr (GM == 2) {
+#pragma unroll
+      for (int s = 0; s < ST; s++) {
+        g.q[s] = next[s];
+#pragma unroll
+        for (int y = 0; y < NT; y++) {
+          g.k0[s][y] = kid(next[s].x, col[y]);
+          g.k1[s][y] = kid(next[s].y, col[y]);
+        }
+      }
+      load_kids(kc + CH);
     }
   };
   auto multiply = [&](int kc, const Stage& g) {
@@ -120,12 +169,21 @@ __global__ __launch_bounds__(64 * RT * KW) void k_fw(const MvTask* __restrict__ 
     for (int s = 0; s < ST; s++) {
       const double a = kc + 4 * s + lk < ke ? (double)g.a[s] : 0.0;
 #pragma unroll
-      for (int y = 0; y < NT; y++) acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(g.b[s][y], a, acc[y], 0, 0, 0);
+      for (int y = 0; y < NT; y++) {
+        double b = g.b[s][y];
+        if constexpr (GM == 2) {
+          b += g.q[s].x >= 0 ? g.k0[s][y] : 0.0;
+          b += g.q[s].y >= 0 ? g.k1[s][y] : 0.0;
+        }
+        acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc[y], 0, 0, 0);
+      }
     }
   };
   if (kb < ke) {
     Stage g0, g1;
+    load_kids(kb);
     load(kb, g0);
+    load_base();
     for (int kc = kb; kc < ke; kc += 2 * CH) {
       if (kc + CH < ke) load(kc + CH, g1);
       multiply(kc, g0);
@@ -133,6 +191,11 @@ __global__ __launch_bounds__(64 * RT * KW) void k_fw(const MvTask* __restrict__ 
       if (kc + 2 * CH < ke) load(kc + 2 * CH, g0);
       multiply(kc + CH, g1);
     }
+  }
+  if constexpr (GM > 0) {
+    if (kb >= ke) load_base();
+#pragma unroll
+    for (int e = 0; e < NB; e++) base[e] = (own.x >= 0 ? add[0][e] : 0.0) + (own.y >= 0 ? add[1][e] : 0.0);
   }
   if constexpr (KW == 1) {
     // acc[y][q]: target row r0 + lr, right-hand side 16 y + lk + 4 q
@@ -142,11 +205,11 @@ __global__ __launch_bounds__(64 * RT * KW) void k_fw(const MvTask* __restrict__ 
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           const int j = t.j0 + 16 * y + lk + 4 * q;
-          if (j < nrhs) mv_apply<T>(t, r0 + lr, j, acc[y][q], dpiv, W, V, Y, nullptr, nrhs);
+          if (j < nrhs) mv_apply<GM, T>(t, r0 + lr, j, acc[y][q], base[4 * y + q], dpiv, W, V, Y, nullptr, nrhs);
         }
   } else {
     __shared__ double red[KW * 272];
-    mv_combine<NT, KW, T>(t, acc, red, dpiv, W, V, Y, nullptr, nrhs);
+    mv_combine<NT, KW, GM, T>(t, acc, base, red, dpiv, W, V, Y, nullptr, nrhs);
   }
 }
 
@@ -237,12 +300,13 @@ __global__ __launch_bounds__(64 * KW) void k_bw(const MvTask* __restrict__ tasks
     }
   }
   if constexpr (KW > 1) __syncthreads();  // the tiles' space takes the partial sums
-  mv_combine<NT, KW, T>(t, acc, lds, nullptr, W, nullptr, Y, X, nrhs);
+  const double base[NT] = {};
+  mv_combine<NT, KW, 0, T>(t, acc, base, lds, nullptr, W, nullptr, Y, X, nrhs);
 }
 
-// Forward-solve initialisation of the work rows of fronts with children:
-// row w takes the right-hand side row (pivot rows) plus the children's
-// update rows that land in it, in child order.  Task: up to 64 work rows
+// Forward-solve initialisation of the work rows of fronts with children, as
+// far as the products do not gather them: row w takes the right-hand side row
+// (pivot rows) plus the children's update rows that land in it, in child order.  Task: up to 64 work rows
 // from w0, the first np of them pivot rows with right-hand side rows r0 ..
 __global__ __launch_bounds__(1024) void k_fw_init(const InitTask* __restrict__ tasks, const int* __restrict__ gptr,
                                                   const int* __restrict__ gsrc, const double* __restrict__ R,
@@ -259,8 +323,8 @@ __global__ __launch_bounds__(1024) void k_fw_init(const InitTask* __restrict__ t
 
 template <int NT, class T>
 static void mv_launch(hipStream_t st, const MvTask* t, int n, int kind, int kw, const T* pool, const T* panel,
-                      const int* rows, const double* dpiv, double* W, double* V, const double* R, double* Y, double* X,
-                      int nrhs) {
+                      const int* rows, const double* dpiv, const int2* kids, double* W, double* V, const double* R,
+                      double* Y, double* X, int nrhs) {
   constexpr int KMAX = NT == 1 ? 16 : 8;  // registers: a 1024-thread workgroup has 128 a lane
   auto bw = [&](auto g) {
     constexpr bool G = decltype(g)::value;
@@ -268,10 +332,18 @@ static void mv_launch(hipStream_t st, const MvTask* t, int n, int kind, int kw, 
     else if (kw == 4) k_bw<G, NT, 4, T><<<n, 256, 0, st>>>(t, pool, panel, rows, W, Y, X, nrhs);
     else k_bw<G, NT, KMAX, T><<<n, 64 * KMAX, 0, st>>>(t, pool, panel, rows, W, Y, X, nrhs);
   };
+  auto fw = [&](auto g) {
+    constexpr int GM = decltype(g)::value;
+    if (kw == 1) k_fw<NT, 4, 1, GM, T><<<n, 256, 0, st>>>(t, pool, panel, dpiv, kids, W, V, R, Y, nrhs);
+    else if (kw == 4) k_fw<NT, 1, 4, GM, T><<<n, 256, 0, st>>>(t, pool, panel, dpiv, kids, W, V, R, Y, nrhs);
+    else k_fw<NT, 1, KMAX, GM, T><<<n, 64 * KMAX, 0, st>>>(t, pool, panel, dpiv, kids, W, V, R, Y, nrhs);
+  };
   if (kind == MV_FORWARD) {
-    if (kw == 1) k_fw<NT, 4, 1, T><<<n, 256, 0, st>>>(t, pool, panel, dpiv, W, V, R, Y, nrhs);
-    else if (kw == 4) k_fw<NT, 1, 4, T><<<n, 256, 0, st>>>(t, pool, panel, dpiv, W, V, R, Y, nrhs);
-    else k_fw<NT, 1, KMAX, T><<<n, 64 * KMAX, 0, st>>>(t, pool, panel, dpiv, W, V, R, Y, nrhs);
+    fw(std::integral_constant<int, 0>{});
+  } else if (kind == MV_FORWARD_ADD) {
+    fw(std::integral_constant<int, 1>{});
+  } else if (kind == MV_FORWARD_ALL) {
+    if constexpr (NT <= GM_TILES) fw(std::integral_constant<int, 2>{});
   } else if (kind == MV_BACK_ROWS) {
     bw(std::true_type{});
   } else {
@@ -281,16 +353,16 @@ static void mv_launch(hipStream_t st, const MvTask* t, int n, int kind, int kw, 
 
 #define FGPU_MV(T)                                                                                                  \
   void launch_mv(hipStream_t st, const MvTask* t, int n, int kind, int nt, int kw, const T* pool, const T* panel,   \
-                 const int* rows, const double* dpiv, double* W, double* V, const double* R, double* Y, double* X,  \
-                 int nrhs) {                                                                                        \
+                 const int* rows, const double* dpiv, const int2* kids, double* W, double* V, const double* R,      \
+                 double* Y, double* X, int nrhs) {                                                                                        \
     if (n <= 0) return;                                                                                             \
     switch (nt) {                                                                                                   \
-      case 1: mv_launch<1, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, W, V, R, Y, X, nrhs); break;              \
-      case 2: mv_launch<2, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, W, V, R, Y, X, nrhs); break;              \
-      case 3: mv_launch<3, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, W, V, R, Y, X, nrhs); break;              \
-      case 4: mv_launch<4, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, W, V, R, Y, X, nrhs); break;              \
-      case 5: mv_launch<5, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, W, V, R, Y, X, nrhs); break;              \
-      default: mv_launch<6, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, W, V, R, Y, X, nrhs); break;             \
+      case 1: mv_launch<1, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
+      case 2: mv_launch<2, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
+      case 3: mv_launch<3, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
+      case 4: mv_launch<4, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
+      case 5: mv_launch<5, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
+      default: mv_launch<6, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;             \
     }                                                                                                               \
   }
 FGPU_MV(double)
