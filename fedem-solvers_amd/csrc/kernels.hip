@@ -410,16 +410,14 @@ __global__ __launch_bounds__(256) void k_extend_add(const FTask* __restrict__ ta
 }
 
 // ---------------------------------------------------------------- MFMA tile
-// acc[x][y] += sum_m sA[wr+16x+(lane&15)][m] * sB[wc+16y+...][m] on the
-// 16x16x4 MFMA of the storage type (v_mfma_f64_16x16x4f64 for the FP64
-// factor, v_mfma_f32_16x16x4f32 for the mixed-precision one) for a 64x64
-// tile split in four 32x32 wave quarters.  The A operand of the instruction
-// takes the sB rows and its B operand the sA rows, so for fixed register
-// consecutive lanes hold consecutive rows of sA (coalesced stores into
+// The 16x16x4 MFMA of the storage type (v_mfma_f64_16x16x4f64 for the FP64
+// factor, v_mfma_f32_16x16x4f32 for the mixed-precision one).  The first
+// operand takes the columns of a result tile and the second its rows, so for a
+// fixed register consecutive lanes hold consecutive rows (coalesced stores into
 // column-major fronts).  The two instructions place the 16x16 result
 // differently: D[p][q] sits in lane q + 16*(p % 4), register p / 4 for FP64
-// and in lane q + 16*(p / 4), register p % 4 for FP32.  Result element of
-// acc[x][y][r]: row wr + 16x + (lane & 15), column wc + 16y + MF<T>::col(lane >> 4, r).
+// and in lane q + 16*(p / 4), register p % 4 for FP32.  Result register r: row
+// lane & 15, column MF<T>::col(lane >> 4, r).
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 
 template <class T> struct MF;
@@ -437,24 +435,6 @@ template <> struct MF<float> {
   }
   static __device__ __forceinline__ int col(int lk, int r) { return 4 * lk + r; }
 };
-
-template <class T, int LD>
-__device__ __forceinline__ void mfma_tile(const T (*sA)[LD], const T (*sB)[LD], int kbr,
-                                          typename MF<T>::acc (&acc)[2][2], int lane, int wr, int wc) {
-  const int lr = lane & 15, lk = lane >> 4;
-  for (int m0 = 0; m0 < kbr; m0 += 4) {
-    T ab[2], aa[2];
-#pragma unroll
-    for (int x = 0; x < 2; x++) {
-      ab[x] = sB[wc + 16 * x + lr][m0 + lk];
-      aa[x] = sA[wr + 16 * x + lr][m0 + lk];
-    }
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-      for (int y = 0; y < 2; y++) acc[x][y] = MF<T>::op(ab[y], aa[x], acc[x][y]);
-  }
-}
 
 template <class A>
 __device__ __forceinline__ void zero_acc(A (&acc)[2][2]) {
@@ -1032,197 +1012,100 @@ __global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update
 // into a few wide launches per tree level instead of a sequence of dependent
 // 64-column substitutions.
 //
-// k_inv_off task: sn, a = tile column j, b = tile row i > j:
-//   X_ij = - X_ii * sum_{k=j}^{i-1} L_ik X_kj
-// (all tiles at smaller distance i-j are complete).
+// The diagonal 64-column tiles come from the diagonal blocks.  From blocks of
+// 64 h columns pairs are joined, h = 1, 2, 4, ...:
+//   [X11     ]
+//   [X21  X22]   X21 = -X22 T,  T = L21 X11
+// by two launches over all fronts at once, so a front of n tiles takes 2 log2 n
+// dependent launches of whole tiles instead of up to 2 n.
+// k_inv_mul task: sn, a = tile column j, b = tile row i, k0 = the pair's first
+// column of X22, kb = 0: T_ij = sum_{j<=k<k0} L_ik X_kj, 1: X_ij = -sum_{k0<=k<=i}
+// X_ik T_kj, je = the place of the pair's T in tmp (16-element units; column-
+// major, its rows those of X22).  Operands as in k_panel, three chunks ahead of
+// their products (a small launch is bound by the latency of its loads); chunks
+// past the sum repeat its last column and meet zeros.
+// Fronts of 5544 and 3000 columns (45x41x43 block): 14 launches of 170 us
+// (tile by tile at growing distance from the diagonal, staged through LDS: 164
+// launches, 4.65 ms); 117x109 plate 8 of 19 us (16 launches, 223 us).
 template <class T>
-__global__ __launch_bounds__(256) void k_inv_off(const FTask* __restrict__ tasks, DevSym S,
-                                                 const T* __restrict__ pool, const int64_t* __restrict__ ioff,
-                                                 T* __restrict__ ipool) {
-  __shared__ T sA[64][65];
-  __shared__ T sB[64][65];
+__global__ __launch_bounds__(256) void k_inv_mul(const FTask* __restrict__ tasks, DevSym S, const T* __restrict__ pool,
+                                                 const int64_t* __restrict__ ioff, T* ipool, T* tmp) {
   const FTask t = tasks[blockIdx.x];
-  const int sn = t.sn, ld = S.nrow[sn], nc = S.ncol[sn];
-  const int rj = 64 * t.a, nj = min(64, nc - rj);
-  const int ri = 64 * t.b, ni = min(64, nc - ri);
+  const int sn = t.sn, ld = S.nrow[sn], nc = S.ncol[sn], xld = S.ild[sn], m = t.k0;
+  const int h = (m / 64) & -(m / 64), first = m - 64 * h, end = min(m + 64 * h, nc), lt = end - m;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int i0 = 64 * t.b + (wv >> 1) * 32, j0 = 64 * t.a + (wv & 1) * 32;
+  if (i0 >= end) return;
   const T* F = pool + S.foff[sn];
   T* X = ipool + ioff[sn];
-  const int xld = S.ild[sn];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
-  typename MF<T>::acc acc[2][2];
-  zero_acc(acc);
-  T ra[16], rb[16];
-  // global loads of tile k (sA rows of tile i, sB the transposed column tile of X)
-  auto load = [&](int kt) {
-    const int rk = 64 * kt, nk = min(64, nc - rk);
+  T* P = tmp + (int64_t)16 * t.je;  // element (i, j) of T at i - m + (j - first) lt
+  const bool fin = t.kb != 0;
+  // the sum from column kb on, kn of it (X is zero above its diagonal)
+  const int kb = fin ? m : j0, kn = fin ? min(i0 + 32, end) - m : m - j0, lda = fin ? xld : ld;
+  const T* A = (fin ? X : F) + (int64_t)kb * lda;
+  const T* B = fin ? P + (int64_t)(j0 - first) * lt : X + (int64_t)j0 * xld + kb;
+  const int ldb = fin ? lt : xld;
+  const T *Ar[2], *Bc[2];
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q, r = idx & 63, m = idx >> 6;
-      // sA[r][m] = L[ri+r][rk+m]  (rows of tile i, columns of tile k)
-      ra[q] = (r < ni && m < nk) ? F[(int64_t)(ri + r) + (int64_t)(rk + m) * ld] : (T)0;
-      // sB[c][m] = X[rk+m][rj+c]  (transposed, lower part only on the diagonal tile)
-      const int c = idx >> 6, mm = idx & 63;
-      const bool ok = c < nj && mm < nk && (kt > t.a || mm >= c);
-      rb[q] = ok ? X[(int64_t)(rk + mm) + (int64_t)(rj + c) * xld] : (T)0;
+  for (int x = 0; x < 2; x++) {
+    Ar[x] = A + min(i0 + 16 * x + lr, end - 1);
+    Bc[x] = B + (int64_t)(16 * x + lr) * ldb;
+  }
+  constexpr int VK = 16 / sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(VK), aligned(sizeof(T))));
+  struct Stage {
+    T a[4][2], b[4][2];
+  };
+  auto kof = [&](int kc, int s) { return kc + 4 * VK * (s / VK) + VK * lk + s % VK; };
+  auto load = [&](int kc, Stage& g) {
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+#pragma unroll
+      for (int s = 0; s < 4; s += VK) {
+        const vec v = *(const vec*)(Bc[x] + min(kof(kc, s), kn - 1));
+#pragma unroll
+        for (int q = 0; q < VK; q++) g.b[s + q][x] = v[q];
+      }
+#pragma unroll
+      for (int s = 0; s < 4; s++) g.a[s][x] = Ar[x][(int64_t)min(kof(kc, s), kn - 1) * lda];
     }
   };
-  load(t.a);
-  for (int kt = t.a; kt < t.b; kt++) {
-    __syncthreads();  // the previous tile's products are done with the LDS tiles
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q;
-      sA[idx & 63][idx >> 6] = ra[q];
-      sB[idx >> 6][idx & 63] = rb[q];
-    }
-    __syncthreads();
-    if (kt + 1 < t.b) load(kt + 1);  // the next tile's loads are in flight during the products
-    mfma_tile<T>(sA, sB, 64, acc, lane, wr, wc);
-  }
-  // T = acc (rows i, cols j) -> LDS as sB[c][m] = T[m][c] for the second product
-  __syncthreads();
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) sB[wc + 16 * y + MF<T>::col(lk, r)][wr + 16 * x + lr] = acc[x][y][r];
-  for (int idx = tid; idx < 64 * 64; idx += 256) {
-    int r = idx & 63, m = idx >> 6;
-    sA[r][m] = (r < ni && m < ni && r >= m) ? X[(int64_t)(ri + r) + (int64_t)(ri + m) * xld] : (T)0;
-  }
-  __syncthreads();
+  typename MF<T>::acc acc[2][2];
   zero_acc(acc);
-  mfma_tile<T>(sA, sB, 64, acc, lane, wr, wc);
+  auto multiply = [&](int kc, const Stage& g) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const bool in = kof(kc, s) < kn;
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int y = 0; y < 2; y++) acc[x][y] = MF<T>::op(in ? g.b[s][y] : (T)0, in ? g.a[s][x] : (T)0, acc[x][y]);
+    }
+  };
+  Stage g0, g1, g2, g3;
+  load(0, g0);
+  load(16, g1);
+  load(32, g2);
+  for (int kc = 0; kc < kn; kc += 64) {
+    load(kc + 48, g3);
+    multiply(kc, g0);
+    load(kc + 64, g0);
+    multiply(kc + 16, g1);
+    load(kc + 80, g1);
+    multiply(kc + 32, g2);
+    load(kc + 96, g2);
+    multiply(kc + 48, g3);
+  }
 #pragma unroll
   for (int x = 0; x < 2; x++)
 #pragma unroll
     for (int y = 0; y < 2; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = wr + 16 * x + lr, c = wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ni && c < nj) X[(int64_t)(ri + i) + (int64_t)(rj + c) * xld] = -acc[x][y][r];
-      }
-}
-
-// Split inverse tiles.  k_inv_part task: sn, a = tile column j, b = tile
-// row i, k0 = first k tile of the chunk, kb = partial slot:
-//   part[slot] = sum_{k=k0}^{min(k0+INV_CHUNK,i)-1} L_ik X_kj   (64 x 64, row-major)
-// k_inv_fin task: sn, a = j, b = i, k0 = first slot, kb = number of slots:
-//   X_ij = - X_ii * (sum of the partials in slot order).
-template <class T>
-__global__ __launch_bounds__(256) void k_inv_part(const FTask* __restrict__ tasks, DevSym S,
-                                                  const T* __restrict__ pool, const int64_t* __restrict__ ioff,
-                                                  const T* __restrict__ ipool, T* __restrict__ part) {
-  __shared__ T sA[64][65];
-  __shared__ T sB[64][65];
-  const FTask t = tasks[blockIdx.x];
-  const int sn = t.sn, ld = S.nrow[sn], nc = S.ncol[sn];
-  const int rj = 64 * t.a, nj = min(64, nc - rj);
-  const int ri = 64 * t.b, ni = min(64, nc - ri);
-  const T* F = pool + S.foff[sn];
-  const T* X = ipool + ioff[sn];
-  const int xld = S.ild[sn];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
-  const int kend = min(t.k0 + INV_CHUNK, t.b);
-  typename MF<T>::acc acc[2][2];
-  zero_acc(acc);
-  T ra[16], rb[16];
-  auto load = [&](int kt) {
-    const int rk = 64 * kt, nk = min(64, nc - rk);
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q, r = idx & 63, m = idx >> 6;
-      ra[q] = (r < ni && m < nk) ? F[(int64_t)(ri + r) + (int64_t)(rk + m) * ld] : (T)0;
-      const int c = idx >> 6, mm = idx & 63;
-      const bool ok = c < nj && mm < nk && (kt > t.a || mm >= c);
-      rb[q] = ok ? X[(int64_t)(rk + mm) + (int64_t)(rj + c) * xld] : (T)0;
-    }
-  };
-  load(t.k0);
-  for (int kt = t.k0; kt < kend; kt++) {
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int idx = tid + 256 * q;
-      sA[idx & 63][idx >> 6] = ra[q];
-      sB[idx >> 6][idx & 63] = rb[q];
-    }
-    __syncthreads();
-    if (kt + 1 < kend) load(kt + 1);
-    mfma_tile<T>(sA, sB, 64, acc, lane, wr, wc);
-  }
-  T* P = part + (int64_t)t.kb * 4096;
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) P[(wr + 16 * x + lr) * 64 + wc + 16 * y + MF<T>::col(lk, r)] = acc[x][y][r];
-}
-
-template <class T>
-__global__ __launch_bounds__(1024) void k_inv_fin(const FTask* __restrict__ tasks, DevSym S,
-                                                  const int64_t* __restrict__ ioff, T* __restrict__ ipool,
-                                                  const T* __restrict__ part) {
-  __shared__ T sA[64][65];
-  __shared__ T sB[64][65];
-  const FTask t = tasks[blockIdx.x];
-  const int sn = t.sn, nc = S.ncol[sn];
-  const int rj = 64 * t.a, nj = min(64, nc - rj);
-  const int ri = 64 * t.b, ni = min(64, nc - ri);
-  T* X = ipool + ioff[sn];
-  const int xld = S.ild[sn];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  // sum of the partials (slot order) for four entries per thread, every
-  // slot's loads issued before the additions; X_ii lower -> sA
-  {
-    T v[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = (T)0;
-    const T* p = part + (int64_t)t.k0 * 4096 + tid;
-    int q = 0;
-    for (; q + 1 < t.kb; q += 2) {
-      T a0[4], a1[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        a0[e] = p[(int64_t)q * 4096 + 1024 * e];
-        a1[e] = p[(int64_t)(q + 1) * 4096 + 1024 * e];
-      }
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[e] += a0[e];
-        v[e] += a1[e];
-      }
-    }
-    if (q < t.kb) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) v[e] += p[(int64_t)q * 4096 + 1024 * e];
-    }
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int idx = tid + 1024 * e, m = idx >> 6, c = idx & 63;  // T[m][c] -> sB[c][m]
-      sB[c][m] = v[e];
-      const int r = idx & 63, mm = idx >> 6;  // X_ii lower -> sA[r][mm]
-      sA[r][mm] = (r < ni && mm < ni && r >= mm) ? X[(int64_t)(ri + r) + (int64_t)(ri + mm) * xld] : (T)0;
-    }
-  }
-  __syncthreads();
-  if (wv >= 4) return;
-  const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
-  typename MF<T>::acc acc[2][2];
-  zero_acc(acc);
-  mfma_tile<T>(sA, sB, 64, acc, lane, wr, wc);
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = wr + 16 * x + lr, c = wc + 16 * y + MF<T>::col(lk, r);
-        if (i < ni && c < nj) X[(int64_t)(ri + i) + (int64_t)(rj + c) * xld] = -acc[x][y][r];
+        const int i = i0 + 16 * x + lr, j = j0 + 16 * y + MF<T>::col(lk, r);
+        if (i >= end) continue;
+        if (fin) X[i + (int64_t)j * xld] = -acc[x][y][r];
+        else P[i - m + (int64_t)(j - first) * lt] = acc[x][y][r];
       }
 }
 
@@ -1765,17 +1648,9 @@ void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
     else if (n > UPD_NARROW) k_update<2, 2, T><<<n, 256, 0, st>>>(t, S, pool);                               \
     else if (n > 0) k_update<1, 1, T><<<dim3(n, 4), 256, 0, st>>>(t, S, pool);                               \
   }                                                                                                        \
-  void launch_inv_off(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,               \
-                      const int64_t* ioff, T* ipool) {                                                     \
-    if (n > 0) k_inv_off<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                     \
-  }                                                                                                        \
-  void launch_inv_part(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,              \
-                       const int64_t* ioff, const T* ipool, T* ipart) {                                    \
-    if (n > 0) k_inv_part<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, ipart);                             \
-  }                                                                                                        \
-  void launch_inv_fin(hipStream_t st, const FTask* t, int n, const DevSym& S, const int64_t* ioff,         \
-                      T* ipool, const T* ipart) {                                                          \
-    if (n > 0) k_inv_fin<T><<<n, 1024, 0, st>>>(t, S, ioff, ipool, ipart);                                    \
+  void launch_inv_mul(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,               \
+                      const int64_t* ioff, T* ipool, T* tmp) {                                             \
+    if (n > 0) k_inv_mul<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, tmp);                                \
   }                                                                                                        \
   void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                 \
                     const int64_t* ioff, T* ipool) {                                                       \

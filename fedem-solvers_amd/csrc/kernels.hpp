@@ -82,9 +82,6 @@ struct ReducedParts {
 };
 void launch_reduced(hipStream_t st, int nd, int n2, int ngen, const int* pos2, const double* S22,
                     const ReducedParts& q, const double* mass, double* out);
-// Pivot-block inverse tiles whose sum X_ij = -X_ii sum_k L_ik X_kj has more
-// than INV_CHUNK terms are summed in INV_CHUNK-tile chunks in parallel.
-constexpr int INV_CHUNK = 4;
 
 // Factorisation and solve launchers for both factor storage types: double
 // (FP64 path) and float (mixed precision: FP32 fronts and FP32 MFMA updates,
@@ -100,12 +97,9 @@ constexpr int INV_CHUNK = 4;
   void launch_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,  \
                    const T* ipool);                                                                       \
   void launch_update(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool);                    \
-  void launch_inv_off(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,              \
-                      const int64_t* ioff, T* ipool);                                                     \
-  void launch_inv_part(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,             \
-                       const int64_t* ioff, const T* ipool, T* ipart);                                    \
-  void launch_inv_fin(hipStream_t st, const FTask* t, int n, const DevSym& S, const int64_t* ioff,        \
-                      T* ipool, const T* ipart);                                                          \
+  /* pivot-block inverses (tmp: the products that the pairs of blocks are joined by) */                   \
+  void launch_inv_mul(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,              \
+                      const int64_t* ioff, T* ipool, T* tmp);                                             \
   /* Y21 = -L21 L11^-1 of the fused levels below L11^-1 (solve panels) */                               \
   void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                \
                     const int64_t* ioff, T* ipool);                                                       \

@@ -181,7 +181,7 @@ struct DBuf {
 
 enum OpKind {
   FRONT_ZERO,  // the first of the factor schedule, issued before the assembly
-  EXTADD, DIAG, TRSM, DIAG_TRSM, UPDATE, INV_OFF, INV_PART, INV_FIN, PANEL,
+  EXTADD, DIAG, TRSM, DIAG_TRSM, UPDATE, INV_MUL, PANEL,
   UPDATE_SIDE, FORK, JOIN,  // lookahead: trailing tiles on the side stream, fork/join with the main one
   FW_INIT, FW_MV, FW_MV_ADD, FW_MV_ALL, BW_ROWS, BW_MV  // solve plans
 };
@@ -283,7 +283,7 @@ struct DeviceReducer::Impl {
   DBuf<double> dpiv;   // pivots D of the factor by pivot column (FP64 for both factor types)
   DBuf<double> adiag, amax;  // original (mixed: equilibrated) diagonal of K_ii and its largest magnitude
   DBuf<int> sing;            // per pivot column: 0, 1 true zero replaced, 2 reduced-to-zero replaced
-  DBuf<double> ipart;  // partial sums of split pivot-block inverse tiles (64 x 64 each; FP32 ones use half)
+  DBuf<double> itmp;  // products of the pairs that the pivot-block inverses are joined from (FP32 ones use half)
   std::vector<Op> fops;
   std::map<int, std::unique_ptr<SolvePlan>> plans;
   // values
@@ -374,10 +374,9 @@ static SolveLayout solve_layout(const Symbolic& y, const ReduceOptions& o) {
 
 static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std::vector<FTask>& tasks,
                                   std::vector<Op>& ops, std::vector<int>& xrange, double& flops, int panel,
-                                  int& inv_slots, bool lookahead) {
+                                  int64_t& inv_tmp, bool lookahead) {
   xrange.clear();
   std::vector<int> at;
-  inv_slots = 0;
   flops = 0;
   // columns of a front cleared before the original entries go in (k_front_zero),
   // the largest fronts first
@@ -532,41 +531,32 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
     }
     if (side_pending) ops.push_back({JOIN, 0, 0});
   }
-  // Explicit inverse of every pivot block: the diagonal tiles come from
-  // k_diag, the tiles at growing distance from the diagonal follow.  Only the
-  // solves read the inverses, so they are formed after the whole
-  // factorisation, distance by distance over all fronts at once.
+  // Explicit inverse of every pivot block, joined pairwise from its diagonal
+  // tiles (k_inv_mul).  Only the solves read the inverses, so they are formed
+  // after the whole factorisation, over all fronts at once, long sums first.
   int maxT = 0;
   for (int s = 0; s < y.nsup; s++) maxT = std::max(maxT, (y.ncol[s] + 63) / 64);
-  // A tile whose sum has more than INV_CHUNK terms is split: partial sums
-  // over INV_CHUNK-tile chunks in parallel (k_inv_part), then their sum in
-  // chunk order and the product with X_ii (k_inv_fin).
-  for (int dist = 1; dist < maxT; dist++) {
-    int off = (int)tasks.size();
-    std::vector<FTask> part, fin;
-    int slot = 0;
+  inv_tmp = 0;
+  for (int h = 1; h < maxT; h *= 2) {
+    std::vector<FTask> join[2];
+    int at = 0;  // in 16-element units
     for (int s = 0; s < y.nsup; s++) {
       const int T = (y.ncol[s] + 63) / 64;
-      for (int j = 0; j + dist < T; j++) {
-        if (dist <= INV_CHUNK) {
-          tasks.push_back({s, j, j + dist, 0, 0, 0});
-          continue;
-        }
-        const int first = slot;
-        for (int k = j; k < j + dist; k += INV_CHUNK) part.push_back({s, j, j + dist, k, slot++, 0});
-        fin.push_back({s, j, j + dist, first, slot - first, 0});
+      for (int m = h; m < T; m += 2 * h) {
+        const int end = std::min(m + h, T);
+        for (int i = m; i < end; i++)
+          for (int j = m - h; j < m; j++)
+            for (int f = 0; f < 2; f++) join[f].push_back({s, j, i, 64 * m, f, at});
+        at += 4 * h * (std::min(64 * (m + h), y.ncol[s]) - 64 * m);
       }
     }
-    if ((int)tasks.size() > off) ops.push_back({INV_OFF, off, (int)tasks.size() - off});
-    if (!part.empty()) {
-      off = (int)tasks.size();
-      tasks.insert(tasks.end(), part.begin(), part.end());
-      ops.push_back({INV_PART, off, (int)part.size()});
-      off = (int)tasks.size();
-      tasks.insert(tasks.end(), fin.begin(), fin.end());
-      ops.push_back({INV_FIN, off, (int)fin.size()});
+    inv_tmp = std::max(inv_tmp, (int64_t)16 * at);
+    auto terms = [](const FTask& t) { return t.kb ? t.b - t.k0 / 64 + 1 : t.k0 / 64 - t.a; };
+    for (auto& q : join) {
+      std::stable_sort(q.begin(), q.end(), [&](const FTask& a, const FTask& b) { return terms(a) > terms(b); });
+      ops.push_back({INV_MUL, (int)tasks.size(), (int)q.size()});
+      tasks.insert(tasks.end(), q.begin(), q.end());
     }
-    inv_slots = std::max(inv_slots, slot);
   }
   // Y21 of the fused levels, long sums first
   std::vector<FTask> pan;
@@ -966,11 +956,11 @@ int DeviceReducer::upload(std::string& err) {
   std::vector<FTask> ft;
   d.fops.clear();
   std::vector<int> xr;
-  int inv_slots = 0;
+  int64_t inv_tmp = 0;
   const int panel = std::min(256, std::max(64, (opt_.factor_panel / 64) * 64));
   std::vector<std::future<void>> host_jobs;
   host_jobs.push_back(std::async(std::launch::async, [&]() {
-    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_slots, opt_.factor_lookahead);
+    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_tmp, opt_.factor_lookahead);
   }));
   std::vector<int> gptr, gsrc;
   std::vector<int2> kids;
@@ -990,7 +980,7 @@ int DeviceReducer::upload(std::string& err) {
   HIPCHK(d.ftasks.upload(ft));
   mark("factor schedule built");
   HIPCHK(d.xrange.upload(xr));
-  HIPCHK(d.ipart.alloc((size_t)std::max(1, inv_slots) * 4096));
+  HIPCHK(d.itmp.alloc((size_t)inv_tmp + PANEL_PAD));
   upd_launches_ = 0;
   for (auto& op : d.fops)
     if (op.kind == UPDATE || op.kind == UPDATE_SIDE) upd_launches_++;
@@ -1459,16 +1449,11 @@ int DeviceReducer::reduce(std::string& err) {
             note(hipStreamWaitEvent(st, d.fj[1], 0));
           }
           break;
-        case INV_OFF: launch_inv_off(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
-        case INV_PART:
-          launch_inv_part(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool,
-                          reinterpret_cast<decltype(pool)>(d.ipart.p));
+        case INV_MUL:
+          launch_inv_mul(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool,
+                         reinterpret_cast<decltype(pool)>(d.itmp.p));
           break;
         case PANEL: launch_panel(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
-        case INV_FIN:
-          launch_inv_fin(st, d.ftasks.p + op.off, op.n, d.S, d.ioff.p, ipool,
-                         reinterpret_cast<decltype(pool)>(d.ipart.p));
-          break;
       }
     }
   };
@@ -1483,7 +1468,7 @@ int DeviceReducer::reduce(std::string& err) {
   } else {
     // the factor schedule is fixed per symbolic structure: one graph
     HIPCHK(run_graph(st, d.g_factor,
-                     {d.ftasks.p, d.xrange.p, d.ipart.p, d.pool.p, d.ipool.p, d.pool32.p, d.ipool32.p, d.ioff.p,
+                     {d.ftasks.p, d.xrange.p, d.itmp.p, d.pool.p, d.ipool.p, d.pool32.p, d.ipool32.p, d.ioff.p,
                       d.piv.p, d.S.foff, d.S.rows, d.S.dpiv},
                      factor_ops));
   }
@@ -2212,10 +2197,10 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
     std::vector<FTask> ft;
     std::vector<int> xr;
     d.fops.clear();
-    int inv_slots = 0;
-    build_factor_schedule(sym_, d.lay, ft, d.fops, xr, upd_flops_, P, inv_slots, opt_.factor_lookahead);
+    int64_t inv_tmp = 0;
+    build_factor_schedule(sym_, d.lay, ft, d.fops, xr, upd_flops_, P, inv_tmp, opt_.factor_lookahead);
     HIPCHK(ensure_side(d));
-    HIPCHK(d.ipart.alloc((size_t)std::max(1, inv_slots) * 4096));
+    HIPCHK(d.itmp.alloc((size_t)inv_tmp + PANEL_PAD));
     HIPCHK(d.ftasks.upload(ft));
     HIPCHK(d.xrange.upload(xr));
     upd_launches_ = 0;
