@@ -1115,11 +1115,13 @@ __global__ __launch_bounds__(256) void k_inv_mul(const FTask* __restrict__ tasks
 // 32 quarter with both operands straight from memory (rows of L contiguous;
 // X along k: each lane takes the VK neighbouring k of 16 bytes, step m of a
 // 4 VK-chunk multiplies k = VK (lane / 16) + m), one chunk ahead of its
-// products.
+// products.  The tasks come with the longest sums first and are dealt out one by
+// one: in contiguous ranges per XCD the first XCD got all long ones (45x41x43
+// block 2236 -> 890 us, 117x109 plate 265 -> 131, 17x13x11 block 52 -> 38).
 template <class T>
 __global__ __launch_bounds__(256) void k_panel(const FTask* __restrict__ tasks, DevSym S, const T* __restrict__ pool,
                                                const int64_t* __restrict__ ioff, T* __restrict__ ipool) {
-  const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const FTask t = tasks[blockIdx.x];
   const int sn = t.sn, ld = S.nrow[sn], nc = S.ncol[sn], nu = ld - nc;
   const T* F = pool + S.foff[sn] + nc;
   T* Z = ipool + ioff[sn];
