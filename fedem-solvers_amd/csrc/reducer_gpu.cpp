@@ -633,6 +633,9 @@ static void build_solve_plan(const Symbolic& y, const SolveLayout& lay, SolvePla
   const int ngrp = (nrhs + 95) / 96;
   sp.nt = ((nrhs + ngrp - 1) / ngrp + 15) / 16;
   const std::vector<int> woff = work_rows(y);
+  // rows of an init task: one value a thread, as each is a chain of three loads
+  // (64 rows by 66 columns took four in turn: a launch 9.6 us, now 4.7)
+  const int ir = std::max(4, std::min(64, 1024 / nrhs));
   // one launch: (task with its whole row range, rows) pieces, cut into row tiles
   struct Piece {
     MvTask t;      // rn = all rows
@@ -694,8 +697,8 @@ static void build_solve_plan(const Symbolic& y, const SolveLayout& lay, SolvePla
       // rows that only the boundary would take are not formed
       const int rows = up && !pairs ? y.nrow[s] : nc;
       if (!leaf && !all)
-        for (int r0 = 0; r0 < rows; r0 += 64)
-          h.inits.push_back({woff[s] + r0, std::min(64, rows - r0), std::max(0, std::min(64, nc - r0)), y.col0[s] + r0});
+        for (int r0 = 0; r0 < rows; r0 += ir)
+          h.inits.push_back({woff[s] + r0, std::min(ir, rows - r0), std::max(0, std::min(ir, nc - r0)), y.col0[s] + r0});
       const int from = leaf ? y.col0[s] : woff[s], ff = leaf ? MV_SRC_R : 0;
       const size_t pieces = first.size();
       if (lay.fused[l]) {
