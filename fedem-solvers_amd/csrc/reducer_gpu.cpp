@@ -1701,8 +1701,8 @@ int DeviceReducer::reduce(std::string& err) {
     // device computes the next blocks: one for every second block from the
     // first that can hold the modes, at most CHECKS at a time.  The first in
     // their order that passes decides the basis whatever the timing, so every
-    // result bit depends on the data only; blocks computed meanwhile are
-    // dropped.  (A test takes 0.9 ms at 176 vectors, six steps of a small part,
+    // result bit, and whether there is a result, depends on the data only;
+    // blocks computed meanwhile are dropped.  (A test takes 0.9 ms at 176 vectors, six steps of a small part,
     // which waited for it two steps later.)
     constexpr size_t CHECKS = 3;
     struct Pending {
@@ -1779,11 +1779,12 @@ int DeviceReducer::reduce(std::string& err) {
       const int mj = (j + 1) * bs, par = j & 1;
       const bool last = mj + bs > mcap;
       if (collect(-1) || collect(expected())) break;
-      // an error in a block that only the tests' duration let be computed
-      // does not count: the loop ended before it whenever a test up to j - 3
-      // had passed
+      // a block that cannot be made (breakdown, refinement that does not
+      // converge) is an error only if no test of the blocks before it passes:
+      // which of them have been started depends on j alone, and all of them
+      // are waited for
       auto ended = [&]() {
-        if (collect(j - 3)) err.clear();
+        if (rc == -6 && collect(INT_MAX)) err.clear();
         return conv;
       };
       if (!last && (rc = issue_step(j + 1))) {
