@@ -21,6 +21,7 @@
 #include <deque>
 #include <future>
 #include "dense_small.hpp"
+#include "host_jobs.hpp"
 #include "kernels.hpp"
 
 namespace fgpu {
@@ -961,17 +962,16 @@ int DeviceReducer::upload(std::string& err) {
   std::vector<int> xr;
   int64_t inv_tmp = 0;
   const int panel = std::min(256, std::max(64, (opt_.factor_panel / 64) * 64));
-  std::vector<std::future<void>> host_jobs;
-  host_jobs.push_back(std::async(std::launch::async, [&]() {
-    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_tmp, opt_.factor_lookahead);
-  }));
   std::vector<int> gptr, gsrc;
   std::vector<int2> kids;
-  host_jobs.push_back(std::async(std::launch::async, [&]() { build_gather(y, gptr, gsrc, kids); }));
-  for (size_t i = 0; i < sps.size(); i++)
-    host_jobs.push_back(std::async(std::launch::async, [&, i]() { plan_host(y, d, *sps[i], phs[i]); }));
+  HostJobs host_jobs;  // (after all that the jobs write)
+  host_jobs.start([&]() {
+    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_tmp, opt_.factor_lookahead);
+  });
+  host_jobs.start([&]() { build_gather(y, gptr, gsrc, kids); });
+  for (size_t i = 0; i < sps.size(); i++) host_jobs.start([&, i]() { plan_host(y, d, *sps[i], phs[i]); });
   const int src = build_structure(err);
-  for (auto& f : host_jobs) f.get();
+  host_jobs.wait();
   if (src) return src;
   mark("structure built");
   HIPCHK(d.gptr.upload(gptr));
