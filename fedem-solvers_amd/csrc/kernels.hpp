@@ -42,9 +42,7 @@ void launch_fmap(hipStream_t st, int neq, const int* rowptr, const int* colind, 
 int scan_tiles(int n);
 void launch_exclusive_scan(hipStream_t st, int n, const int* in, int* out, int* tsum);
 void launch_fill(hipStream_t st, double* p, int64_t n, double v);
-// no-allocation reduced loads (noalloc.hip): this GPU's scratch array
-// (address and size), the permuted-row gather of column-major load vectors
-// and the scatter of the reduced rows into Fred
+// no-allocation reduced loads (noalloc.hip): this GPU's scratch array (address and size)
 int noalloc_scratch(double** ptr, size_t* bytes, std::string& err);
 // one block of a gathered upload: `bytes` (a multiple of 4, at most COPY_BLOCK)
 // from offset `from` of the pinned memory to dst
@@ -59,6 +57,8 @@ void launch_copy_blocks(hipStream_t st, int n, const CopyBlock* table, const cha
 void launch_rows_in(hipStream_t st, int n, int nc, const int* map, const double* in, int64_t ldi, double* out, int ldo);
 void launch_rows_out(hipStream_t st, int n, int nc, const int* map, const double* A, int lda, const double* B, int ldb,
                      double* out, int64_t ldo);
+// reduced loads: permuted rows of column-major load vectors, and the scatter of
+// the reduced rows into Fred (order.hip)
 void launch_perm_rows(hipStream_t st, int neq, int nrhs, const int* p2e, const double* F, double* Fp);
 void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, const int* pos2, const double* r2,
                             const double* r1, double* Fred);
