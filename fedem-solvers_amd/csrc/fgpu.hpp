@@ -134,6 +134,7 @@ struct Symbolic {
 
 struct SymbolicOptions {
   int leaf_nodes = 24;  // stop nested dissection below this many nodes
+  int threads = 0;      // host threads of the ordering and the front lists (0: by the part's size)
 };
 
 int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,

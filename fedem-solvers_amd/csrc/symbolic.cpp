@@ -212,11 +212,17 @@ int build_symbolic(const Part& p, const Sam& s, const SymbolicOptions& o,
       for (int k = ecptr[e]; k < ecptr[e + 1]; k++) elist[fill[ecn[k]]++] = e;
   }
   // The lists that follow are made by several threads where the part is large
-  // enough to pay for them (a thread starts in 20 us, 1000 nodes take 0.6 ms
-  // in all); they do not depend on the number.  48x24x24 block: 25 ms with one
-  // thread, indirect sort keys, a search per update row and a second graph
-  // without boundary nodes, 13 now (61x47 plate, one thread: 1.07 and 0.91).
-  const int threads = nnod < 4000 ? 1 : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
+  // enough to pay for them; they do not depend on the number.  What grows with
+  // the work are the node pairs of the elements, of which a solid node has four
+  // times a shell node's: 8 threads against one take 1.6 and 1.1 ms for 61,000
+  // pairs (63x61 plate), 2.0 and 1.9 for 170,000 (17x13x12 block), 3.7 both for
+  // 208,000 (115x113 plate), 2.75 and 3.0 for 269,000 (20x15x14 block), 4.0 and
+  // 4.9 for 418,000 (24x17x16), 6.5 and 9.0 for 730,000 (30x20x19).
+  int64_t pairs = 0;
+  for (int e = 0; e < p.nel; e++) pairs += (int64_t)(ecptr[e + 1] - ecptr[e]) * (ecptr[e + 1] - ecptr[e]);
+  const int threads = o.threads > 0     ? std::min(o.threads, 64)
+                      : pairs < 250'000 ? 1
+                                        : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
   std::vector<int> adjptr(nnod + 1, 0), adj;
   {
     constexpr int BLOCK = 1024;  // nodes of one list
