@@ -120,13 +120,17 @@ void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, 
 }
 
 // One workgroup per block of a gathered upload, table and data read straight
-// from pinned host memory (four words in flight per thread).
+// from pinned host memory: 16 bytes a load, two in flight per thread, the last
+// words of an array one by one (blocks start at multiples of 16 on both sides).
 __global__ __launch_bounds__(256) void k_copy_blocks(const CopyBlock* __restrict__ table, const char* __restrict__ stage) {
   const CopyBlock b = table[blockIdx.x];
-  const unsigned* in = reinterpret_cast<const unsigned*>(stage + b.from);
-  unsigned* out = static_cast<unsigned*>(b.dst);
-#pragma unroll 4
-  for (unsigned i = threadIdx.x; i < b.bytes / 4; i += 256) out[i] = in[i];
+  const uint4* in = reinterpret_cast<const uint4*>(stage + b.from);
+  uint4* out = static_cast<uint4*>(b.dst);
+  const unsigned n = b.bytes / 16;
+#pragma unroll 2
+  for (unsigned i = threadIdx.x; i < n; i += 256) out[i] = in[i];
+  const unsigned w = 4 * n + threadIdx.x;
+  if (w < b.bytes / 4) reinterpret_cast<unsigned*>(out)[w] = reinterpret_cast<const unsigned*>(in)[w];
 }
 
 void launch_copy_blocks(hipStream_t st, int n, const CopyBlock* table, const char* stage) {

@@ -20,6 +20,7 @@
 #include <cstring>
 #include <deque>
 #include <future>
+#include <mutex>
 #include "dense_small.hpp"
 #include "host_jobs.hpp"
 #include "kernels.hpp"
@@ -49,7 +50,62 @@ struct StreamScope {
   ~StreamScope() { tl_stream = prev; }
 };
 
-// Pinned host memory (hipHostMalloc) for asynchronous copies.
+// Pinned host memory that no handle of the process uses, for the next one that
+// asks for as much on the same device: a call for it takes 11-15 us, every so
+// often 60-330 (a new mapping, whose pages are then touched for the first
+// time), and as much to give it back.  Blocks are powers of two; at most MOST
+// bytes stay here, the others go back to the system.  One object for the
+// process, never destroyed (at its end the runtime may be gone before it).
+class PinnedPool {
+ public:
+  static PinnedPool& get() {
+    static PinnedPool* pool = new PinnedPool;
+    return *pool;
+  }
+  hipError_t take(size_t bytes, void** p, int* dev) {
+    if (hipError_t e = hipGetDevice(dev)) return e;
+    {
+      std::lock_guard<std::mutex> g(mu_);
+      for (size_t k = 0; k < idle_.size(); k++)
+        if (idle_[k].bytes == bytes && idle_[k].dev == *dev) {
+          *p = idle_[k].p;
+          held_ -= bytes;
+          idle_.erase(idle_.begin() + k);
+          return hipSuccess;
+        }
+    }
+    return hipHostMalloc(p, bytes, hipHostMallocDefault);
+  }
+  // no work of the device on the block may be outstanding
+  void give(void* p, size_t bytes, int dev) {
+    {
+      std::lock_guard<std::mutex> g(mu_);
+      if (held_ + bytes <= MOST) {
+        try {
+          idle_.push_back({p, bytes, dev});
+          held_ += bytes;
+          return;
+        } catch (const std::bad_alloc&) {
+        }
+      }
+    }
+    (void)hipHostFree(p);
+  }
+
+ private:
+  static constexpr size_t MOST = 8 << 20;
+  struct Block {
+    void* p;
+    size_t bytes;
+    int dev;
+  };
+  std::mutex mu_;
+  std::vector<Block> idle_;
+  size_t held_ = 0;
+};
+
+// Pinned host memory for asynchronous copies.  Growing it waits for the
+// thread's stream; an owner that releases it has waited for its own.
 template <class T>
 struct HBuf {
   T* p = nullptr;
@@ -59,81 +115,117 @@ struct HBuf {
   HBuf& operator=(const HBuf&) = delete;
   ~HBuf() { release(); }
   void release() {
-    if (p) (void)hipHostFree(p);
+    if (p) PinnedPool::get().give(p, bytes_, dev_);
     p = nullptr;
     n = 0;
   }
   hipError_t alloc(size_t count) {
     if (count <= n && p) return hipSuccess;
+    if (p && tl_stream)
+      if (hipError_t e = hipStreamSynchronize(tl_stream)) return e;
     release();
-    n = count;
-    return hipHostMalloc((void**)&p, std::max<size_t>(1, count) * sizeof(T), hipHostMallocDefault);
-  }
-};
-
-// Small arrays on their way to the device.  While a batch is open on the
-// thread, uploads of up to MOST bytes are gathered in pinned memory; flush()
-// launches one kernel that reads it and writes all of them.  An array by
-// itself costs a staged copy and a wait, 15 us each: the 45 of an upload made
-// 0.8 of the 1.46 ms in which a 20x10 plate is analysed, uploaded and reduced
-// (now 0.74 in all).  Larger ones go by themselves: their time is the copy's.
-struct UploadBatch {
-  static constexpr size_t BYTES = 1 << 20, MOST = 1 << 18, BLOCKS = 1024;
-  HBuf<char> stage;
-  HBuf<CopyBlock> table;
-  size_t used = 0, blocks = 0;
-  hipStream_t st = nullptr;
-
-  hipError_t open(hipStream_t s) {
-    st = s;
-    used = blocks = 0;
-    hipError_t e = stage.alloc(BYTES);
-    if (e == hipSuccess) e = table.alloc(BLOCKS);
-    // the last batch's kernel has read the memory
-    return e == hipSuccess ? hipStreamSynchronize(st) : e;
-  }
-  bool take(void* dst, const void* src, size_t bytes) {
-    const size_t need = (bytes + COPY_BLOCK - 1) / COPY_BLOCK;
-    if (bytes > MOST || bytes % 4 || used + bytes > BYTES || blocks + need > BLOCKS) return false;
-    if (pending(dst, bytes) && flush() != hipSuccess) return false;  // written twice: in order
-    std::memcpy(stage.p + used, src, bytes);
-    for (size_t o = 0; o < bytes; o += COPY_BLOCK)
-      table.p[blocks++] = {static_cast<char*>(dst) + o, (unsigned)(used + o),
-                           (unsigned)std::min<size_t>(COPY_BLOCK, bytes - o)};
-    used = (used + bytes + 15) & ~(size_t)15;
-    return true;
-  }
-  hipError_t flush() {
-    if (sent == blocks) return hipSuccess;
-    launch_copy_blocks(st, (int)(blocks - sent), table.p + sent, stage.p);
-    sent = blocks;
-    return hipGetLastError();
-  }
-  bool pending(const void* p, size_t bytes) const {
-    const char* lo = static_cast<const char*>(p);
-    for (size_t q = sent; q < blocks; q++)
-      if (static_cast<char*>(table.p[q].dst) >= lo && static_cast<char*>(table.p[q].dst) < lo + bytes) return true;
-    return false;
-  }
-  // memory about to be freed: nothing may be on its way there
-  void settle(const void* p, size_t bytes) {
-    if (!pending(p, bytes)) return;
-    (void)flush();
-    (void)hipStreamSynchronize(st);
+    bytes_ = 4096;
+    while (bytes_ < count * sizeof(T)) bytes_ *= 2;
+    const hipError_t e = PinnedPool::get().take(bytes_, (void**)&p, &dev_);
+    if (e == hipSuccess) n = count;
+    else p = nullptr;
+    return e;
   }
 
  private:
-  size_t sent = 0;
-  friend struct BatchScope;
+  size_t bytes_ = 0;
+  int dev_ = 0;
+};
+
+// Two pieces of pinned memory through which arrays go to and from the device:
+// the host fills or reads one while the device reads or fills the other.
+struct Stage {
+  static constexpr size_t PIECE = 512 << 10;
+  HBuf<char> mem;
+  hipEvent_t passed[2]{};
+  bool in_use[2]{};
+
+  ~Stage() {
+    for (hipEvent_t& e : passed)
+      if (e) (void)hipEventDestroy(e);
+  }
+  hipError_t open() {
+    if (mem.p) return hipSuccess;
+    for (hipEvent_t& ev : passed)
+      if (!ev)
+        if (hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) return e;
+    return mem.alloc(2 * PIECE);
+  }
+  char* piece(int h) { return mem.p + h * PIECE; }
+  // the device's work on piece h is what the stream has been given so far
+  hipError_t mark(int h, hipStream_t st) {
+    in_use[h] = true;
+    return hipEventRecord(passed[h], st);
+  }
+  // piece h is the host's again
+  hipError_t wait(int h) {
+    if (!in_use[h]) return hipSuccess;
+    in_use[h] = false;
+    return hipEventSynchronize(passed[h]);
+  }
+};
+
+// Arrays on their way to the device.  While a batch is open on the thread its
+// uploads are gathered in the stage's pieces, behind a table of blocks of up to
+// 8 KB; a kernel reads a full piece and writes its blocks while the host fills
+// the other, flush() sends what is there.  Each array is uploaded once and
+// kept until the batch ends.  An array by itself costs a staged copy and a
+// wait, 15 us each (0.8 of the 1.46 ms in which a 20x10 plate was analysed,
+// uploaded and reduced; 0.74 in all with its 45 small arrays gathered), and a
+// large one goes through staging memory of the runtime's own, whose pages are
+// new with most handles: 2.4 GB/s, until 16 MB have passed.
+struct UploadBatch {
+  static constexpr size_t TABLE = 16 << 10, MOST = TABLE / sizeof(CopyBlock), DATA = Stage::PIECE - TABLE;
+  Stage& stage;
+  hipStream_t st = nullptr;
+  hipError_t err = hipSuccess;
+  int h = 0;
+  size_t used = 0, blocks = 0;
+
+  explicit UploadBatch(Stage& s) : stage(s) {}
+  hipError_t open(hipStream_t s) {
+    st = s;
+    err = stage.open();
+    used = blocks = 0;
+    return err == hipSuccess ? err = stage.wait(h) : err;
+  }
+  hipError_t put(void* dst, const void* src, size_t bytes) {
+    for (size_t o = 0; o < bytes && err == hipSuccess;) {
+      const size_t n = std::min({bytes - o, DATA - used, (MOST - blocks) * COPY_BLOCK});
+      if (n == 0) {
+        (void)flush();  // (err)
+        continue;
+      }
+      CopyBlock* t = reinterpret_cast<CopyBlock*>(stage.piece(h));
+      std::memcpy(stage.piece(h) + TABLE + used, static_cast<const char*>(src) + o, n);
+      for (size_t q = 0; q < n; q += COPY_BLOCK)
+        t[blocks++] = {static_cast<char*>(dst) + o + q, (unsigned)(TABLE + used + q),
+                       (unsigned)std::min(COPY_BLOCK, n - q)};
+      used = std::min(DATA, (used + n + 15) & ~(size_t)15);
+      o += n;
+    }
+    return err;
+  }
+  hipError_t flush() {
+    if (blocks == 0 || err != hipSuccess) return err;
+    launch_copy_blocks(st, (int)blocks, reinterpret_cast<const CopyBlock*>(stage.piece(h)), stage.piece(h));
+    used = blocks = 0;
+    err = hipGetLastError();
+    if (err == hipSuccess) err = stage.mark(h, st);
+    h ^= 1;
+    return err == hipSuccess ? err = stage.wait(h) : err;
+  }
 };
 static thread_local UploadBatch* tl_batch = nullptr;
 struct BatchScope {
-  explicit BatchScope(UploadBatch& b) {
-    b.sent = 0;
-    tl_batch = &b;
-  }
+  explicit BatchScope(UploadBatch& b) { tl_batch = &b; }
   ~BatchScope() {
-    if (tl_batch) (void)tl_batch->flush();
+    (void)tl_batch->flush();
     tl_batch = nullptr;
   }
 };
@@ -149,7 +241,6 @@ struct DBuf {
   ~DBuf() { release(); }
   void release() {
     if (p) {
-      if (tl_batch) tl_batch->settle(p, n * sizeof(T));
       (void)hipFree(p);
       if (acct) *acct -= (int64_t)(std::max<size_t>(1, n) * sizeof(T));
     }
@@ -173,7 +264,8 @@ struct DBuf {
   hipError_t upload(const std::vector<T>& v) {
     hipError_t e = alloc(v.size());
     if (e != hipSuccess || v.empty()) return e;
-    if (tl_batch && tl_batch->take(p, v.data(), v.size() * sizeof(T))) return hipSuccess;
+    static_assert(sizeof(T) % 4 == 0, "a batch moves whole words");
+    if (tl_batch) return tl_batch->put(p, v.data(), v.size() * sizeof(T));
     if (!tl_stream) return hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice);
     e = hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, tl_stream);
     return e == hipSuccess ? hipStreamSynchronize(tl_stream) : e;  // v may go out of scope after the call
@@ -253,7 +345,8 @@ static hipError_t run_graph(hipStream_t st, GraphCache& gc, const std::vector<co
 
 struct DeviceReducer::Impl {
   GraphCache g_factor;
-  UploadBatch batch;
+  Stage stage;
+  UploadBatch batch{stage};
   DBuf<int> sb_cnt, sb_tsum, sb_bad;  // the structure build's counts
   int factor_runs = 0;  // factorisations since the last upload
   // part
