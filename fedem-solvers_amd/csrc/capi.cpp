@@ -260,9 +260,7 @@ int fgpu_get_eigen(const fgpu_reducer* h, int* nev, double* lambda, double* evl)
 int fgpu_get_B(fgpu_reducer* h, double* B) {
   GUARD(h)
   if (!h->reduced || !B) return -1;
-  std::vector<double> b;
-  if (h->red.get_B(b)) { h->err = "fgpu_get_B: copy failed"; return -3; }
-  std::memcpy(B, b.data(), b.size() * sizeof(double));
+  if (h->red.get_B(B)) { h->err = "fgpu_get_B: copy failed"; return -3; }
   return 0;
   END_GUARD(h)
 }
@@ -270,9 +268,7 @@ int fgpu_get_B(fgpu_reducer* h, double* B) {
 int fgpu_get_phi(fgpu_reducer* h, double* phi) {
   GUARD(h)
   if (!h->reduced || !phi) return -1;
-  std::vector<double> p;
-  if (h->red.get_phi(p)) { h->err = "fgpu_get_phi: copy failed"; return -3; }
-  std::memcpy(phi, p.data(), p.size() * sizeof(double));
+  if (h->red.get_phi(phi)) { h->err = "fgpu_get_phi: copy failed"; return -3; }
   return 0;
   END_GUARD(h)
 }
@@ -333,10 +329,7 @@ int fgpu_solve_internal(fgpu_reducer* h, int nrhs, const double* R, double* X) {
 int fgpu_get_gravity_internal(fgpu_reducer* h, double* gi) {
   GUARD(h)
   if (!h->reduced || !gi) return -1;
-  std::vector<double> g;
-  int rc = h->red.gravity_internal(g, h->err);
-  if (rc == 0) std::copy(g.begin(), g.end(), gi);
-  return rc;
+  return h->red.gravity_internal(gi, h->err);
   END_GUARD(h)
 }
 

@@ -57,9 +57,7 @@ void launch_copy_blocks(hipStream_t st, int n, const CopyBlock* table, const cha
 void launch_rows_in(hipStream_t st, int n, int nc, const int* map, const double* in, int64_t ldi, double* out, int ldo);
 void launch_rows_out(hipStream_t st, int n, int nc, const int* map, const double* A, int lda, const double* B, int ldb,
                      double* out, int64_t ldo);
-// reduced loads: permuted rows of column-major load vectors, and the scatter of
-// the reduced rows into Fred (order.hip)
-void launch_perm_rows(hipStream_t st, int neq, int nrhs, const int* p2e, const double* F, double* Fp);
+// the reduced load vectors' rows into Fred
 void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, const int* pos2, const double* r2,
                             const double* r1, double* Fred);
 // singular-pivot support of the factorisation: the original (or, with rs,

@@ -81,20 +81,9 @@ void launch_rows_out(hipStream_t st, int n, int nc, const int* map, const double
   });
 }
 
-// The two below serve the reduced load vectors with and without allocation.
-// They are here and not beside the scratch array of the latter, whose code
-// object a program would load with its first load case: 13 ms and 32 MiB.
-
-// Fp[r * nrhs + c] = F[p2e[r] + c * neq]: column-major load vectors in
-// equation order to row-major permuted rows
-__global__ void k_perm_rows(int neq, int nrhs, const int* __restrict__ p2e, const double* __restrict__ F,
-                            double* __restrict__ Fp) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= (int64_t)neq * nrhs) return;
-  const int r = (int)(g / nrhs), c = (int)(g % nrhs);
-  Fp[g] = F[p2e[r] + (int64_t)c * neq];
-}
-
+// (Here and not beside the scratch array of the load vectors without
+// allocation, whose code object a program would load with its first load case:
+// 13 ms and 32 MiB.)
 // Fred (nd x nrhs, column-major) = [r2 rows in dofPosIn2 order; r1; 0]
 __global__ void k_scatter_reduced(int nd, int n2, int ngen, int nrhs, const int* __restrict__ pos2,
                                   const double* __restrict__ r2, const double* __restrict__ r1,
@@ -106,11 +95,6 @@ __global__ void k_scatter_reduced(int nd, int n2, int ngen, int nrhs, const int*
   if (i < n2) v = r2[(int64_t)(pos2[i] - 1) * nrhs + c];
   else if (i < n2 + ngen) v = r1[(int64_t)(i - n2) * nrhs + c];
   Fred[g] = v;
-}
-
-void launch_perm_rows(hipStream_t st, int neq, int nrhs, const int* p2e, const double* F, double* Fp) {
-  const int64_t n = (int64_t)neq * nrhs;
-  if (n > 0) k_perm_rows<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(neq, nrhs, p2e, F, Fp);
 }
 
 void launch_scatter_reduced(hipStream_t st, int nd, int n2, int ngen, int nrhs, const int* pos2, const double* r2,

@@ -370,7 +370,7 @@ struct DeviceReducer::Impl {
   DBuf<double> sk_r, sk_t, sk_x, rl_f, rc_s, rc_y, gi_g;
   DBuf<int> ceq_ptr, ceq_node, ceq_dof;  // constraint equations of the dependent DOFs
   DBuf<double> ceq_coef;
-  DBuf<int> p2e, pos2;  // perm row -> 0-based equation; dofPosIn2 (for the device-side reduced loads)
+  DBuf<int> e2p, pos2;  // perm row of every equation; dofPosIn2 (for the device-side reduced loads)
   DevSym S{};
   DBuf<FTask> ftasks;
   DBuf<int> xrange;  // extend-add tasks: (child, first, end) column ranges
@@ -1111,7 +1111,7 @@ int DeviceReducer::upload(std::string& err) {
       if (sam_.meqn[dof] > 0) a[(size_t)y.eq_to_perm[sam_.meqn[dof] - 1] * 3 + j] = 1.0;
     }
   HIPCHK(d.grav.upload(a));
-  HIPCHK(d.p2e.upload(y.perm_to_eq));
+  HIPCHK(d.e2p.upload(y.eq_to_perm));
   HIPCHK(d.pos2.upload(sam_.dofPosIn2.empty() ? std::vector<int>(1, 1) : sam_.dofPosIn2));
   mark("gravity and maps");
   // the solve plans and work buffers the reduction will use, made here (on
@@ -2074,30 +2074,100 @@ hipError_t DeviceReducer::d2h(void* dst, const void* src, size_t bytes) const {
   return e == hipSuccess ? hipStreamSynchronize(st_) : e;
 }
 
-// Internal rows of the row-major neq x nc array A, in equation order and
-// column-major, to the host: ordered on the device, at most 2^23 values (64
-// MiB of device memory) at a time.
-int DeviceReducer::internal_to_host(const double* A, int nc, double* out) const {
-  Impl& d = *d_;
-  std::string err;
-  const int n1 = sym_.ndof1, step = std::max(1, std::min(nc, (1 << 23) / std::max(1, n1)));
-  HIPCHK(d.sk_t.alloc((size_t)n1 * step));
-  for (int c0 = 0; c0 < nc; c0 += step) {
-    const int k = std::min(step, nc - c0);
-    launch_rows_out(st_, n1, k, d.p1.p, A + c0, nc, nullptr, 0, d.sk_t.p, n1);
-    HIPCHK(d2h(out + (size_t)c0 * n1, d.sk_t.p, sizeof(double) * (size_t)n1 * k));
+// The parts of a column-major n x nc array that go through a piece of the stage
+// at a time: whole columns where one fits, else rows of up to 16 columns (the
+// width of an ordering kernel's tile).
+struct Pieces {
+  int n, nc, rows, cols;
+  Pieces(int n_, int nc_) : n(n_), nc(nc_) {
+    const int most = Stage::PIECE / sizeof(double);
+    cols = std::min(nc, std::max(16, most / std::max(1, n)));
+    rows = std::min(n, most / std::max(1, cols));
   }
-  return 0;
+  // go(h, q0, m, c0, k): rows q0 .. q0 + m and columns c0 .. c0 + k, piece h
+  template <class F>
+  int each(F&& go) const {
+    int h = 0;
+    for (int c0 = 0; c0 < nc; c0 += cols)
+      for (int q0 = 0; q0 < n; q0 += rows, h ^= 1)
+        if (int rc = go(h, q0, std::min(rows, n - q0), c0, std::min(cols, nc - c0))) return rc;
+    return 0;
+  }
+};
+
+// copy(piece, array, doubles) for the contiguous runs of a part
+template <class F>
+static void runs(char* piece, double* array, int n, int q0, int m, int c0, int k, F&& copy) {
+  double* p = reinterpret_cast<double*>(piece);
+  array += q0 + (size_t)c0 * n;
+  if (m == n) return copy(p, array, (size_t)m * k);
+  for (int c = 0; c < k; c++) copy(p + (size_t)c * m, array + (size_t)c * n, (size_t)m);
 }
 
-int DeviceReducer::get_B(std::vector<double>& B) {
-  B.resize((size_t)sym_.ndof1 * sym_.ndof2);
-  return B.empty() ? 0 : internal_to_host(d_->X.p, sym_.ndof2, B.data());
+// Rows map[0..n) of A + B (row-major, either may be null) to the host, column-
+// major.  A kernel writes them in their order into a piece of the stage, and
+// the host copies one piece out while the device fills the other: no device
+// buffer, and the data crosses the bus once.  (With copies behind an ordering
+// kernel into a buffer of its own, through the runtime's staging memory, B of a
+// 16x12x10 block took 0.98 ms where the order on the host took 0.53.)
+int DeviceReducer::rows_to_host(int n, int nc, const int* map, const double* A, int lda, const double* B, int ldb,
+                                double* out, std::string& err) const {
+  Stage& s = d_->stage;
+  HIPCHK(s.open());
+  struct {
+    int q0, m = 0, c0, k;
+  } full[2];
+  auto drain = [&](int h) -> int {
+    HIPCHK(s.wait(h));
+    auto& f = full[h];
+    if (f.m > 0)
+      runs(s.piece(h), out, n, f.q0, f.m, f.c0, f.k,
+           [](const double* p, double* a, size_t count) { std::memcpy(a, p, count * sizeof(double)); });
+    f.m = 0;
+    return 0;
+  };
+  int last = 0;
+  const int rc = Pieces(n, nc).each([&](int h, int q0, int m, int c0, int k) -> int {
+    if (int rc = drain(h)) return rc;
+    launch_rows_out(st_, m, k, map + q0, A ? A + c0 : nullptr, lda, B ? B + c0 : nullptr, ldb,
+                    reinterpret_cast<double*>(s.piece(h)), m);
+    HIPCHK(hipGetLastError());
+    HIPCHK(s.mark(h, st_));
+    full[h] = {q0, m, c0, k};
+    last = h;
+    return 0;
+  });
+  if (rc) return rc;
+  if (int rc2 = drain(last ^ 1)) return rc2;
+  return drain(last);
 }
 
-int DeviceReducer::get_phi(std::vector<double>& P) {
-  P.resize((size_t)sym_.ndof1 * res_.nev);
-  return P.empty() ? 0 : internal_to_host(d_->Phi.p, res_.nev, P.data());
+// The host's column-major n x nc array into rows map[0..n) (null: 0..n-1) of
+// the row-major out, the other way through the same pieces.
+int DeviceReducer::host_to_rows(int n, int nc, const int* map, const double* in, double* out, int ldo,
+                                std::string& err) const {
+  Stage& s = d_->stage;
+  HIPCHK(s.open());
+  return Pieces(n, nc).each([&](int h, int q0, int m, int c0, int k) -> int {
+    HIPCHK(s.wait(h));
+    runs(s.piece(h), const_cast<double*>(in), n, q0, m, c0, k,
+         [](double* p, const double* a, size_t count) { std::memcpy(p, a, count * sizeof(double)); });
+    launch_rows_in(st_, m, k, map ? map + q0 : nullptr, reinterpret_cast<const double*>(s.piece(h)), m,
+                   out + c0 + (map ? 0 : (size_t)q0 * ldo), ldo);
+    HIPCHK(hipGetLastError());
+    HIPCHK(s.mark(h, st_));
+    return 0;
+  });
+}
+
+int DeviceReducer::get_B(double* B) const {
+  std::string err;
+  return rows_to_host(sym_.ndof1, sym_.ndof2, d_->p1.p, d_->X.p, sym_.ndof2, nullptr, 0, B, err);
+}
+
+int DeviceReducer::get_phi(double* P) const {
+  std::string err;
+  return rows_to_host(sym_.ndof1, res_.nev, d_->p1.p, d_->Phi.p, res_.nev, nullptr, 0, P, err);
 }
 
 int DeviceReducer::get_schur(std::vector<double>& S) {
@@ -2140,8 +2210,7 @@ int DeviceReducer::get_element_matrices(std::vector<double>& Kp, std::vector<dou
 }
 
 // K_ii^-1 R into row-major x = d.sk_x (rows in elimination order), R as the
-// caller's column-major n1 x nrhs.  The caller's array is read by an
-// asynchronous copy: the stream has to pass it before the call returns.
+// caller's column-major n1 x nrhs, which has been read when the call returns.
 int DeviceReducer::solve_rows(int nrhs, const double* R_eq, std::string& err) {
   Impl& d = *d_;
   const Symbolic& y = sym_;
@@ -2153,9 +2222,7 @@ int DeviceReducer::solve_rows(int nrhs, const double* R_eq, std::string& err) {
   HIPCHK(d.sk_r.alloc(n));
   HIPCHK(d.sk_t.alloc(n));
   HIPCHK(d.sk_x.alloc(n));
-  // the caller's order arrives in the solve's work array
-  HIPCHK(hipMemcpyAsync(d.sk_t.p, R_eq, sizeof(double) * (size_t)n1 * nrhs, hipMemcpyHostToDevice, st_));
-  launch_rows_in(st_, n1, nrhs, d.p1.p, d.sk_t.p, n1, d.sk_r.p, nrhs);
+  if (int rc = host_to_rows(n1, nrhs, d.p1.p, R_eq, d.sk_r.p, nrhs, err)) return rc;
   launch_fill(st_, d.sk_r.p + (size_t)n1 * nrhs, (int64_t)(neq - n1) * nrhs, 0.0);
   return solve_int(st_, d, y, opt_, *p, d.sk_r.p, d.sk_t.p, d.sk_x.p, nullptr, err);
 }
@@ -2165,26 +2232,19 @@ int DeviceReducer::solve_kii(int nrhs, const double* R_eq, double* X_eq, std::st
   Impl& d = *d_;
   const int n1 = sym_.ndof1;
   if (n1 == 0) return 0;
-  if (int rc = solve_rows(nrhs, R_eq, err)) {
-    (void)hipStreamSynchronize(st_);
-    return rc;
-  }
-  launch_rows_out(st_, n1, nrhs, d.p1.p, d.sk_x.p, nrhs, nullptr, 0, d.sk_t.p, n1);
-  HIPCHK(d2h(X_eq, d.sk_t.p, sizeof(double) * (size_t)n1 * nrhs));
-  return 0;
+  if (int rc = solve_rows(nrhs, R_eq, err)) return rc;
+  return rows_to_host(n1, nrhs, d.p1.p, d.sk_x.p, nrhs, nullptr, 0, X_eq, err);
 }
 
-int DeviceReducer::gravity_internal(std::vector<double>& gi, std::string& err) {
+int DeviceReducer::gravity_internal(double* gi, std::string& err) {
   StreamScope scope(st_);
   Impl& d = *d_;
   const Symbolic& y = sym_;
-  const int neq = y.neq, n1 = y.ndof1;
   if (opt_.no_mass) { err = "gravity forces need the mass matrix"; return -1; }
   DBuf<double>& g = d.gi_g;
-  HIPCHK(g.alloc((size_t)neq * 3));
-  mass_mm(st_, neq, d, 3, d.grav.p, 3, g.p, 3);
-  gi.resize((size_t)n1 * 3);
-  return gi.empty() ? 0 : internal_to_host(g.p, 3, gi.data());
+  HIPCHK(g.alloc((size_t)y.neq * 3));
+  mass_mm(st_, y.neq, d, 3, d.grav.p, 3, g.p, 3);
+  return rows_to_host(y.ndof1, 3, d.p1.p, g.p, 3, nullptr, 0, gi, err);
 }
 
 int DeviceReducer::reduce_loads(int nrhs, const double* F_eq, std::vector<double>& out, std::string& err) {
@@ -2195,23 +2255,29 @@ int DeviceReducer::reduce_loads(int nrhs, const double* F_eq, std::vector<double
   out.assign((size_t)nd * std::max(nrhs, 0), 0.0);
   if (nrhs <= 0) return 0;
   if (out.empty()) return 0;
-  // the same launches as reduce_loads_noalloc, on buffers of the handle: the
-  // load vectors cross the bus in the caller's order, the result once
-  const size_t nF = (size_t)neq * nrhs, maxa = (size_t)std::max(n2, ngen);
+  // the products of reduce_loads_noalloc on buffers of the handle; the load
+  // vectors cross the bus in the caller's order, the result once
+  const size_t nF = (size_t)neq * nrhs, maxa = (size_t)std::max(n2, ngen), nout = out.size() * sizeof(double);
   HIPCHK(d.rl_f.alloc(nF));
-  HIPCHK(d.sk_t.alloc(nF));
   HIPCHK(d.part.alloc((size_t)xty_chunks(neq) * maxa * nrhs));
   HIPCHK(d.acc.alloc((size_t)(n2 + ngen + nd) * nrhs));
   double *const f = d.rl_f.p, *const r2 = d.acc.p, *const r1 = r2 + (size_t)n2 * nrhs;
-  double* const red = r1 + (size_t)ngen * nrhs;
-  HIPCHK(hipMemcpyAsync(d.sk_t.p, F_eq, sizeof(double) * nF, hipMemcpyHostToDevice, st_));
-  launch_perm_rows(st_, neq, nrhs, d.p2e.p, d.sk_t.p, f);
+  if (int rc = host_to_rows(neq, nrhs, d.e2p.p, F_eq, f, nrhs, err)) return rc;
   // rhs2 = f_e + B^T f_i = [B; I]^T f, rhs1 = Phi^T f_i
   if (n2 > 0) launch_xty(st_, neq, n2, nrhs, d.X.p, n2, f, nrhs, d.part.p, r2);
   if (ngen > 0) launch_xty(st_, neq, ngen, nrhs, d.Phi.p, nev, f, nrhs, d.part.p, r1);
+  // written straight into pinned memory where it fits
+  const bool small = nout <= Stage::PIECE;
+  if (small) HIPCHK(d.stage.wait(0));
+  double* const red = small ? reinterpret_cast<double*>(d.stage.piece(0)) : r1 + (size_t)ngen * nrhs;
   launch_scatter_reduced(st_, nd, n2, ngen, nrhs, d.pos2.p, r2, r1, red);
-  HIPCHK(d2h(out.data(), red, sizeof(double) * out.size()));
-  (void)err;
+  HIPCHK(hipGetLastError());
+  if (small) {
+    HIPCHK(hipStreamSynchronize(st_));
+    std::memcpy(out.data(), red, nout);
+  } else {
+    HIPCHK(d2h(out.data(), red, nout));
+  }
   return 0;
 }
 
@@ -2238,7 +2304,7 @@ int DeviceReducer::reduce_loads_noalloc(int nrhs, const double* F, double* Fred,
   double* part = Fp + nF;
   double* r2 = part + npart;
   double* r1 = r2 + (size_t)n2 * nrhs;
-  launch_perm_rows(st_, neq, nrhs, d.p2e.p, F, Fp);
+  launch_rows_in(st_, neq, nrhs, d.e2p.p, F, neq, Fp, nrhs);
   if (n2 > 0) launch_xty(st_, neq, n2, nrhs, d.X.p, n2, Fp, nrhs, part, r2);
   if (ngen > 0) launch_xty(st_, neq, ngen, nrhs, d.Phi.p, nev, Fp, nrhs, part, r1);
   launch_scatter_reduced(st_, nd, n2, ngen, nrhs, d.pos2.p, r2, r1, Fred);
@@ -2261,29 +2327,23 @@ int DeviceReducer::recover(int nrhs, const double* Ub, const double* Fi, double*
   }
   // x = K_ii^-1 F_i first, then per column chunk Y = [B; I] U_b and the sum of
   // both in the caller's order
-  int rc = 0;
-  if (Fi && (rc = solve_rows(nrhs, Fi, err))) {
-    (void)hipStreamSynchronize(st_);
-    return rc;
-  }
+  if (Fi)
+    if (int rc = solve_rows(nrhs, Fi, err)) return rc;
   const int cj = bound ? std::min(nrhs, 64) : nrhs;
-  HIPCHK(d.sk_t.alloc((size_t)n1 * nrhs));  // free again once x is there
   if (bound) {
-    HIPCHK(d.rc_s.alloc(2 * (size_t)n2 * nrhs));
+    HIPCHK(d.rc_s.alloc((size_t)n2 * cj));
     HIPCHK(d.rc_y.alloc((size_t)neq * cj));
-    HIPCHK(hipMemcpyAsync(d.rc_s.p, Ub, sizeof(double) * (size_t)n2 * nrhs, hipMemcpyHostToDevice, st_));
   }
   for (int j0 = 0; j0 < nrhs; j0 += cj) {
     const int nj = std::min(cj, nrhs - j0);
     if (bound) {
-      double* const S = d.rc_s.p + (size_t)n2 * nrhs;  // this chunk of U_b, row-major
-      launch_rows_in(st_, n2, nj, nullptr, d.rc_s.p + (size_t)j0 * n2, n2, S, nj);
-      launch_gemm_small(st_, neq, n2, nj, d.X.p, n2, S, d.rc_y.p, nj, 0.0, 1.0);
+      if (int rc = host_to_rows(n2, nj, nullptr, Ub + (size_t)j0 * n2, d.rc_s.p, nj, err)) return rc;
+      launch_gemm_small(st_, neq, n2, nj, d.X.p, n2, d.rc_s.p, d.rc_y.p, nj, 0.0, 1.0);
     }
-    launch_rows_out(st_, n1, nj, d.p1.p, bound ? d.rc_y.p : nullptr, nj, Fi ? d.sk_x.p + j0 : nullptr, nrhs,
-                    d.sk_t.p + (size_t)j0 * n1, n1);
+    if (int rc = rows_to_host(n1, nj, d.p1.p, bound ? d.rc_y.p : nullptr, nj, Fi ? d.sk_x.p + j0 : nullptr, nrhs,
+                              Ui + (size_t)j0 * n1, err))
+      return rc;
   }
-  HIPCHK(d2h(Ui, d.sk_t.p, sizeof(double) * (size_t)n1 * nrhs));
   return 0;
 }
 

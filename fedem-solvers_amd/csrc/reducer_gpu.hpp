@@ -91,8 +91,8 @@ class DeviceReducer {
   // One full numeric reduction on the device from the resident part data.
   int reduce(std::string& err);
   // Copies of device results in the reference layout (on demand).
-  int get_B(std::vector<double>& B);     // ndof1 x ndof2, MEQN1 rows, MEQN2 columns
-  int get_phi(std::vector<double>& P);   // ndof1 x nev, MEQN1 rows
+  int get_B(double* B) const;            // ndof1 x ndof2, MEQN1 rows, MEQN2 columns
+  int get_phi(double* P) const;          // ndof1 x nev, MEQN1 rows
   int get_schur(std::vector<double>& S); // ndof2 x ndof2 (MEQN2 order)
   int get_csr(std::vector<int>& rowptr, std::vector<int>& colind, std::vector<double>& K,
               std::vector<double>& M);     // perm-space CSR
@@ -100,7 +100,7 @@ class DeviceReducer {
   // Extra solves on the resident factor (load cases / recovery)
   int solve_kii(int nrhs, const double* R_eq, double* X_eq, std::string& err);  // MEQN1 rows
   // g_i = (M a) on the internal equations for unit accelerations along x, y, z
-  int gravity_internal(std::vector<double>& gi, std::string& err);  // ndof1 x 3, MEQN1 rows
+  int gravity_internal(double* gi, std::string& err);  // ndof1 x 3, MEQN1 rows
   // reduced load vectors [f_e + B^T f_i (dofPosIn2 order); Phi^T f_i], ndim x nrhs,
   // from full load vectors F_eq (neq x nrhs, equation order)
   int reduce_loads(int nrhs, const double* F_eq, std::vector<double>& out, std::string& err);
@@ -140,7 +140,10 @@ class DeviceReducer {
   hipStream_t st_ = nullptr;
   // device-to-host copy ordered after the handle's stream work
   hipError_t d2h(void* dst, const void* src, size_t bytes) const;
-  int internal_to_host(const double* A, int nc, double* out) const;
+  // callers' column-major arrays to and from row-major ones on the device
+  int rows_to_host(int n, int nc, const int* map, const double* A, int lda, const double* B, int ldb, double* out,
+                   std::string& err) const;
+  int host_to_rows(int n, int nc, const int* map, const double* in, double* out, int ldo, std::string& err) const;
   int solve_rows(int nrhs, const double* R_eq, std::string& err);
   bool uploaded_ = false;
   double upd_flops_ = 0;
