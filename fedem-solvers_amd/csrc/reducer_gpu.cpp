@@ -1072,6 +1072,7 @@ int DeviceReducer::upload(std::string& err) {
   HIPCHK(d.kids.upload(kids));
   for (size_t i = 0; i < sps.size(); i++)
     if (int rc = plan_upload(*sps[i], phs[i], err)) return rc;
+    else sps[i]->valid = true;
   HIPCHK(ensure_side(d));
   HIPCHK(d.ftasks.upload(ft));
   mark("factor schedule built");
@@ -1154,7 +1155,6 @@ static void plan_host(const Symbolic& y, const DeviceReducer::Impl& d, SolvePlan
 static int plan_upload(SolvePlan& sp, const PlanHost& h, std::string& err) {
   HIPCHK(sp.tasks.upload(h.tasks));
   HIPCHK(sp.inits.upload(h.inits));
-  sp.valid = true;
   return 0;
 }
 
@@ -1164,7 +1164,15 @@ static int get_plan(const Symbolic& y, DeviceReducer::Impl& d, int nrhs, SolvePl
   SolvePlan* sp = plan_slot(d, nrhs);
   PlanHost h;
   plan_host(y, d, *sp, h);
-  if (int rc = plan_upload(*sp, h, err)) return rc;
+  if (tl_batch) {
+    if (int rc = plan_upload(*sp, h, err)) return rc;
+  } else {  // a plan made for a call after the upload
+    HIPCHK(d.batch.open(tl_stream));
+    BatchScope gather(d.batch);
+    if (int rc = plan_upload(*sp, h, err)) return rc;
+    HIPCHK(d.batch.flush());
+  }
+  sp->valid = true;
   out = sp;
   return 0;
 }
