@@ -1115,7 +1115,9 @@ __global__ __launch_bounds__(256) void k_inv_mul(const FTask* __restrict__ tasks
 // 32 quarter with both operands straight from memory (rows of L contiguous;
 // X along k: each lane takes the VK neighbouring k of 16 bytes, step m of a
 // 4 VK-chunk multiplies k = VK (lane / 16) + m), one chunk ahead of its
-// products.  The tasks come with the longest sums first and are dealt out one by
+// products.  Both storage types add in FP64, so that a mixed-precision panel is
+// rounded once (with FP32 sums a reduction takes as long, 102.9 ms of a 200x200
+// plate).  The tasks come with the longest sums first and are dealt out one by
 // one: in contiguous ranges per XCD the first XCD got all long ones (45x41x43
 // block 2236 -> 890 us, 117x109 plate 265 -> 131, 17x13x11 block 52 -> 38).
 template <class T>
@@ -1153,7 +1155,7 @@ __global__ __launch_bounds__(256) void k_panel(const FTask* __restrict__ tasks, 
       for (int s = 0; s < 4; s++) g.a[s][x] = Fr[x][(int64_t)min(kof(kc, s), nc - 1) * ld];
     }
   };
-  typename MF<T>::acc acc[2][2];
+  MF<double>::acc acc[2][2];
   zero_acc(acc);
   auto multiply = [&](int kc, const Stage& g) {
 #pragma unroll
@@ -1162,7 +1164,7 @@ __global__ __launch_bounds__(256) void k_panel(const FTask* __restrict__ tasks, 
 #pragma unroll
       for (int x = 0; x < 2; x++)
 #pragma unroll
-        for (int y = 0; y < 2; y++) acc[x][y] = MF<T>::op(in ? g.b[s][y] : (T)0, in ? g.a[s][x] : (T)0, acc[x][y]);
+        for (int y = 0; y < 2; y++) acc[x][y] = MF<double>::op(in ? (double)g.b[s][y] : 0.0, in ? (double)g.a[s][x] : 0.0, acc[x][y]);
     }
   };
   Stage g0, g1;
@@ -1181,8 +1183,8 @@ __global__ __launch_bounds__(256) void k_panel(const FTask* __restrict__ tasks, 
     for (int y = 0; y < 2; y++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = i0 + 16 * x + lr, j = j0 + 16 * y + MF<T>::col(lk, r);
-        if (i < nu && j < nc) Z[(int64_t)nc + i + (int64_t)j * ld] = -acc[x][y][r];
+        const int i = i0 + 16 * x + lr, j = j0 + 16 * y + MF<double>::col(lk, r);
+        if (i < nu && j < nc) Z[(int64_t)nc + i + (int64_t)j * ld] = (T)-acc[x][y][r];
       }
 }
 

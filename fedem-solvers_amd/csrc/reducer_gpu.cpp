@@ -1054,7 +1054,9 @@ int DeviceReducer::upload(std::string& err) {
   d.fops.clear();
   std::vector<int> xr;
   int64_t inv_tmp = 0;
-  const int panel = std::min(256, std::max(64, (opt_.factor_panel / 64) * 64));
+  const int panel = opt_.factor_panel == ReduceOptions::PANEL_DEFAULT
+                        ? (opt_.mixed ? 64 : 256)
+                        : std::min(256, std::max(64, (opt_.factor_panel / 64) * 64));
   std::vector<int> gptr, gsrc;
   std::vector<int2> kids;
   HostJobs host_jobs;  // (after all that the jobs write)
@@ -2383,7 +2385,7 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
   // warm-up (allocations, first captures), then one timed reduction per candidate
   if (int rc = reduce(err)) return rc;
   double best = INFINITY;
-  int bestP = opt_.factor_panel;
+  int bestP = 256;
   for (int P : {64, 128, 192, 256}) {
     if (set_panel(P)) return -3;
     if (int rc = reduce(err)) return rc;

@@ -28,7 +28,14 @@ struct ReduceOptions {
   // and Schur updates, FP64 diagonal-block factorisation), every solve with
   // K_ii refined against the FP64 matrix until the correction falls below
   // ir_tol relative (at most ir_maxit steps; no convergence is an error).
-  int factor_panel = 256;   // most pivot columns per trailing update (64..256, multiple of 64)
+  // most pivot columns per trailing update (64..256, multiple of 64); by
+  // default 256, and 64 in mixed precision, whose FP32 update is a sum of as
+  // many products: with 256, 128 and 64 columns the first correction of a solve
+  // is off by 6.1e-5, 4.1e-5 and 2.4e-5 for a 30x22x20 block (geometric means of
+  // 8), 3.7e-3, 3.6e-3 and 4.1e-3 for a 100x100 plate of random thickness, and
+  // the reductions take the same time (102.9, 102.8, 102.7 ms of a 200x200 plate)
+  static constexpr int PANEL_DEFAULT = -0x7fffffff;
+  int factor_panel = PANEL_DEFAULT;
   // top levels: trailing tiles past the next panel on a side stream (off by
   // default: on the 48x24x24 block the side updates take the CUs that the
   // critical-path diagonal launches need, 12.8 -> 13.1 ms)

@@ -111,7 +111,7 @@ int fgpu_analyze(fgpu_reducer* h, int ngen, int neval, int flags);
  * "seed" (Lanczos start block), "leafNodes" (nested-dissection leaf size),
  * "timeUpdates" (1: time every trailing-update launch with HIP events),
  * "factorPanel" (most pivot columns per trailing update: 64, 128, 192 or
- * 256, default 256), "solveSplitK" (contraction range above which a wave of a
+ * 256, default 256, in mixed precision 64), "solveSplitK" (contraction range above which a wave of a
  * solve task shares it with more waves where tasks are few, a multiple of
  * 64, default 128; the parts are summed in order),
  * "factorLookahead" (1: on the levels of few large fronts, the trailing
