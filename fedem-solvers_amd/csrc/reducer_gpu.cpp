@@ -466,9 +466,29 @@ static SolveLayout solve_layout(const Symbolic& y, const ReduceOptions& o) {
   return q;
 }
 
+// Elements of the products that the pivot-block inverses of all fronts are
+// joined from, pairs of h tiles at a time (k_inv_mul): the most of any h, in
+// units of the 16 elements that a task counts by.
+static int64_t inverse_products(const Symbolic& y, int h, int s) {
+  int64_t units = 0;
+  for (int m = h; 64 * m < y.ncol[s]; m += 2 * h) units += 4 * h * (std::min(64 * (m + h), y.ncol[s]) - 64 * m);
+  return units;
+}
+static int64_t inverse_workspace(const Symbolic& y) {
+  int64_t most = 0;
+  int maxc = 0;
+  for (int s = 0; s < y.nsup; s++) maxc = std::max(maxc, y.ncol[s]);
+  for (int h = 1; 64 * h < maxc; h *= 2) {
+    int64_t all = 0;
+    for (int s = 0; s < y.nsup; s++) all += inverse_products(y, h, s);
+    most = std::max(most, 16 * all);
+  }
+  return most;
+}
+
 static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std::vector<FTask>& tasks,
                                   std::vector<Op>& ops, std::vector<int>& xrange, double& flops, int panel,
-                                  int64_t& inv_tmp, bool lookahead) {
+                                  bool lookahead) {
   xrange.clear();
   std::vector<int> at;
   flops = 0;
@@ -630,7 +650,6 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
   // after the whole factorisation, over all fronts at once, long sums first.
   int maxT = 0;
   for (int s = 0; s < y.nsup; s++) maxT = std::max(maxT, (y.ncol[s] + 63) / 64);
-  inv_tmp = 0;
   for (int h = 1; h < maxT; h *= 2) {
     std::vector<FTask> join[2];
     int at = 0;  // in 16-element units
@@ -641,10 +660,9 @@ static void build_factor_schedule(const Symbolic& y, const SolveLayout& lay, std
         for (int i = m; i < end; i++)
           for (int j = m - h; j < m; j++)
             for (int f = 0; f < 2; f++) join[f].push_back({s, j, i, 64 * m, f, at});
-        at += 4 * h * (std::min(64 * (m + h), y.ncol[s]) - 64 * m);
+        at += 4 * h * (std::min(64 * (m + h), y.ncol[s]) - 64 * m);  // as inverse_products counts
       }
     }
-    inv_tmp = std::max(inv_tmp, (int64_t)16 * at);
     auto terms = [](const FTask& t) { return t.kb ? t.b - t.k0 / 64 + 1 : t.k0 / 64 - t.a; };
     for (auto& q : join) {
       std::stable_sort(q.begin(), q.end(), [&](const FTask& a, const FTask& b) { return terms(a) > terms(b); });
@@ -1053,7 +1071,6 @@ int DeviceReducer::upload(std::string& err) {
   std::vector<FTask> ft;
   d.fops.clear();
   std::vector<int> xr;
-  int64_t inv_tmp = 0;
   const int panel = opt_.factor_panel == ReduceOptions::PANEL_DEFAULT
                         ? (opt_.mixed ? 64 : 256)
                         : std::min(256, std::max(64, (opt_.factor_panel / 64) * 64));
@@ -1061,7 +1078,7 @@ int DeviceReducer::upload(std::string& err) {
   std::vector<int2> kids;
   HostJobs host_jobs;  // (after all that the jobs write)
   host_jobs.start([&]() {
-    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, inv_tmp, opt_.factor_lookahead);
+    build_factor_schedule(y, d.lay, ft, d.fops, xr, upd_flops_, panel, opt_.factor_lookahead);
   });
   host_jobs.start([&]() { build_gather(y, gptr, gsrc, kids); });
   for (size_t i = 0; i < sps.size(); i++) host_jobs.start([&, i]() { plan_host(y, d, *sps[i], phs[i]); });
@@ -1079,7 +1096,7 @@ int DeviceReducer::upload(std::string& err) {
   HIPCHK(d.ftasks.upload(ft));
   mark("factor schedule built");
   HIPCHK(d.xrange.upload(xr));
-  HIPCHK(d.itmp.alloc((size_t)inv_tmp + PANEL_PAD));
+  HIPCHK(d.itmp.alloc((size_t)inverse_workspace(y) + PANEL_PAD));
   upd_launches_ = 0;
   for (auto& op : d.fops)
     if (op.kind == UPDATE || op.kind == UPDATE_SIDE) upd_launches_++;
@@ -2364,10 +2381,8 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
     std::vector<FTask> ft;
     std::vector<int> xr;
     d.fops.clear();
-    int64_t inv_tmp = 0;
-    build_factor_schedule(sym_, d.lay, ft, d.fops, xr, upd_flops_, P, inv_tmp, opt_.factor_lookahead);
+    build_factor_schedule(sym_, d.lay, ft, d.fops, xr, upd_flops_, P, opt_.factor_lookahead);
     HIPCHK(ensure_side(d));
-    HIPCHK(d.itmp.alloc((size_t)inv_tmp + PANEL_PAD));
     HIPCHK(d.ftasks.upload(ft));
     HIPCHK(d.xrange.upload(xr));
     upd_launches_ = 0;
@@ -2408,25 +2423,52 @@ int DeviceReducer::autotune(int& panel, int& split, std::string& err) {
   return 0;
 }
 
-size_t DeviceReducer::footprint_bytes() const {
+// The buffers of upload(), reduce() and, for nlc load cases, reduce_loads() and
+// recover(), in that order; task lists and index arrays of a few bytes per
+// front row or node are taken as a whole.
+size_t DeviceReducer::footprint_bytes(int nlc) const {
   const Symbolic& y = sym_;
+  const size_t neq = y.neq, n1 = y.ndof1, n2 = y.ndof2, nel = part_.nel, nnod = part_.nnod;
   const size_t nnz = y.rowptr.empty() ? 0 : (size_t)y.rowptr.back();
-  size_t wrows = 0;
-  for (int s = 0; s < y.nsup; s++) wrows += y.nrow[s];
-  const size_t ipool = y.nsup > 0 ? (size_t)solve_layout(y, opt_).ioff[y.nsup] : 0;
-  const int nev = opt_.ngen > 0 ? std::max(opt_.neval, opt_.ngen) : 0;
-  const int bs = opt_.lanczos_block;
-  const size_t mcap = nev > 0 ? (size_t)std::max(10 * nev + 40, 16 * bs) : 0;
-  const size_t rhs = (size_t)std::max(std::max(y.ndof2, bs), 3);
-  const size_t fb = opt_.mixed ? 4 : 8;  // bytes per factor entry
-  size_t b = fb * ((size_t)y.fpool + ipool) + 8 * (2 * nnz + 2 * (size_t)y.elem_pool);  // fronts, inverses, K, M, elements
-  b += (y.has_rigid ? 12 : 4) * (size_t)y.ncontrib + 4 * (nnz + 1) + 8 * nnz + 4 * nnz;  // contributions, fmap, colind
-  b += 4 * (2 * (size_t)y.neq + 1);  // node rows and diagonal places
-  b += 8 * nnz;                                                                     // structure-build counts
-  b += 20 * sam_.ceq_dof.size() + 4 * sam_.ceq_ptr.size();                          // constraint equations
-  b += 8 * (size_t)y.neq * (3 * (size_t)y.ndof2 + 2 * mcap + 8 * (size_t)bs);     // B solves and Lanczos basis
-  b += 8 * 2 * wrows * rhs;                                                        // solve work rows
-  if (opt_.mixed) b += 8 * 5 * (size_t)y.neq * rhs;                                // refinement work
+  const size_t ngen = opt_.ngen, lb = opt_.lanczos_block, ncases = std::max(nlc, 0);
+  const size_t nev = ngen > 0 ? std::max(opt_.neval, opt_.ngen) : 0;
+  int bs = 0, cap = 0;
+  if (nev > 0 && n1 > 0) lanczos_sizes(y.ndof1, (int)nev, opt_, bs, cap);
+  const size_t nb = bs, mcap = cap, chunks = xty_chunks(y.neq), f8 = sizeof(double), fb = opt_.mixed ? 4 : 8;
+  const SolveLayout lay = solve_layout(y, opt_);
+  size_t wrows = 0, tasks = 0;
+  for (int s = 0; s < y.nsup; s++) {
+    const size_t T = (y.nrow[s] + 63) / 64, C = (y.ncol[s] + 63) / 64;
+    wrows += y.nrow[s];
+    tasks += y.nrow[s] / 8 + C * (2 * T + C);  // cleared and gathered columns, inverse and panel tiles
+    for (size_t c = 0; c < C; c++) tasks += 5 * (T - c) + (c % 4 == 0 ? (T - c) * (T - c) / 2 : 0);  // factor
+  }
+  // part, structure, schedules
+  size_t b = nnod * 48 + nel * (f8 * NPROP + 32) + 4 * part_.enodes.size() + 40 * neq + 8 * y.nbl.size();
+  b += 8 * sam_.msc.size() + 20 * sam_.ceq_dof.size() + 4 * sam_.ceq_ptr.size();
+  b += 60 * (size_t)y.nsup + 4 * (y.rows.size() + 2 * y.rel.size()) + 12 * wrows;
+  b += (y.has_rigid ? 12 : 4) * (size_t)y.ncontrib + nnz * (4 + 4 + 8 + 4);
+  b += sizeof(FTask) * tasks + 12 * (wrows / 8 + y.rel.size() / 16) + 3 * 24 * wrows;
+  // factor, matrices
+  b += fb * ((size_t)y.fpool + (size_t)lay.ioff[y.nsup]) + f8 * inverse_workspace(y);
+  b += f8 * (2 * (size_t)y.elem_pool + 2 * nnz + 2 * n1);
+  // solves: the widest of B, the Lanczos block, the gravity displacements and the load cases
+  const size_t wide = std::max({n2, ncases > 0 ? std::max(ncases, lb) : (size_t)0, nev > 0 ? std::max(nb, n2) : (size_t)0,
+                                opt_.want_vgi ? std::max<size_t>(3, lb) : (size_t)0});
+  b += f8 * wrows * wide * (lay.unfused ? 2 : 1);
+  b += f8 * neq * 3 * n2;
+  if (nev > 0) {
+    b += f8 * neq * (2 * mcap + nb + std::max(nb, opt_.want_vgi ? std::max<size_t>(3, lb) : 0) + std::max(nb, std::max(ngen, lb)) + nev);
+    b += f8 * (mcap * std::max(nb, nev) + mcap * mcap + mcap * nb + nev * (1 + 3 * MODE_SIGN_GROUPS));
+  }
+  if (opt_.want_vgi) b += f8 * neq * 2 * std::max<size_t>(3, lb);
+  if (!opt_.no_mass) b += f8 * neq * std::max<size_t>(3, std::max(lb, nev));
+  // products: the partial sums of the largest
+  const size_t ab = std::max(std::max<size_t>(n2, 3), std::max<size_t>(nev, 1));
+  b += f8 * chunks * std::max({ab * ab, mcap * std::max(nb, nev), std::max(n2, ngen) * ncases});
+  b += f8 * (3 * (n2 + ngen + 6) * (n2 + ngen + 6) + (2 * (n2 + ngen) + 6) * ncases);
+  if (opt_.mixed) b += f8 * neq * (1 + 5 * wide);
+  if (ncases > 0) b += f8 * (neq * (4 * ncases + std::min<size_t>(ncases, 64)) + n2 * std::min<size_t>(ncases, 64));
   return b;
 }
 

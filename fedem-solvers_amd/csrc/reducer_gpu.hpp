@@ -118,8 +118,9 @@ class DeviceReducer {
   // U_i = B U_b (+ K_ii^{-1} F_i); U_b ndof2 x nrhs (MEQN2 rows), F_i and U_i
   // ndof1 x nrhs (MEQN1 rows), F_i may be null
   int recover(int nrhs, const double* Ub, const double* Fi, double* Ui, std::string& err);
-  // device memory one reduction of the analysed part needs (bytes, estimate)
-  size_t footprint_bytes() const;
+  // device memory that a reduction of the analysed part and nlc load cases need
+  // (bytes, estimate)
+  size_t footprint_bytes(int nlc = 0) const;
   // Times this part's reduction for every candidate factor panel width and
   // solve split and keeps the fastest pair (results then differ from the
   // defaults' at rounding level only); call after analyze.

@@ -197,7 +197,7 @@ class Server {
 
   int run(int slot, Request& r, std::string& err) {
     int rc = reducers_[slot]->analyze(r.part, r.opt, err);  // host only
-    const size_t fp = rc == 0 ? reducers_[slot]->footprint_bytes() : 0;
+    const size_t fp = rc == 0 ? reducers_[slot]->footprint_bytes(r.nlc) : 0;
     if (rc == 0) {
       std::unique_lock<std::mutex> g(mu_);
       cv_mem_.wait(g, [&] {
