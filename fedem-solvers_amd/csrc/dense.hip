@@ -5,26 +5,9 @@
 // dimensions.  All products run on FP64 MFMA with operands straight from
 // memory; every sum has a fixed order.
 #include <algorithm>
-#include "kernels.hpp"
+#include "kern_device.hpp"
 
 namespace fgpu {
-
-using f64x4 = __attribute__((__vector_size__(4 * sizeof(double)))) double;
-
-static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
-
-// Workgroup b's task: every XCD (workgroup b runs on XCD b mod 8) takes one
-// contiguous range of the list, so neighbouring tasks share its L2.
-__device__ __forceinline__ int xcd_task(int b, int n) {
-  const int q = n >> 3, r = n & 7, c = b & 7, m = b >> 3;
-  return c < r ? c * (q + 1) + m : r * (q + 1) + (c - r) * q + m;
-}
-
-__device__ __forceinline__ double lane_bcast(double v, int src) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
-  return __hiloint2double(hi, lo);
-}
 
 // ---------------------------------------------------------------- X^T Y
 // One workgroup: 16 XA columns of X by 16 YB columns of Y over crows rows,
@@ -53,7 +36,7 @@ __global__ __launch_bounds__(64 * WV) void k_xty(int n, int crows, int na, int n
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
   // the tiles of a chunk of rows are neighbours on one XCD and read them
   // through its L2; lower: tile q of the lower triangle in row order
-  const int id = xcd_task(blockIdx.x, gridDim.x), chunk = id / ntile;
+  const int id = xcd_ranges(blockIdx.x, gridDim.x), chunk = id / ntile;
   int ta = id % ntile, tb = 0;
   if (lower) {
     int row = 0;
@@ -173,8 +156,9 @@ int xty_chunks(int n) { return (n + 127) / 128; }
 template <int XA, int YB, int WV>
 static int xty_go(hipStream_t st, int n, int na, int nb, const double* X, int ldx, const double* Y, int ldy,
                   double* part, double* C, double* acc, int acc_add, int lower) {
-  // chunks: at least 32 rows a wave, and no more workgroups than fill the
-  // 256 CUs a few times over (each chunk costs a partial matrix)
+  // chunks of about 32 rows a wave at most, more where that would make more
+  // workgroups than fill the 256 CUs a few times over (each chunk costs a
+  // partial matrix)
   const int ta = (int)nblk(na, 16 * XA), tb = (int)nblk(nb, 16 * YB);
   if (XA != YB || na != nb) lower = 0;
   const int tiles = lower ? ta * (ta + 1) / 2 : ta * tb;
@@ -465,11 +449,7 @@ __global__ __launch_bounds__(1024) void k_chol16(int n, int nch, const double* _
   // a non-positive pivot goes on as 1 (a select per pivot on its own lane)
   bool nonpos = lane == 0 && !(a[0] > 0.0);
   auto pivot = [&](double v, int j) { return lane_bcast(v > 0.0 ? v : 1.0, j); };
-  auto recip = [](double dd) {
-    const double r = __builtin_amdgcn_rcp(dd), e = __builtin_fma(-dd, r, 1.0);
-    return __builtin_fma(__builtin_fma(e, e, e), r, r);
-  };
-  double dj = pivot(a[0], 0), rj = recip(dj);
+  double dj = pivot(a[0], 0), rj = recip64(dj);
 #pragma unroll
   for (int j = 0; j < 16; j++) {
     u[j] = a[j];
@@ -483,7 +463,7 @@ __global__ __launch_bounds__(1024) void k_chol16(int n, int nch, const double* _
     a[j + 1] = __builtin_fma(-l, ub[j + 1], a[j + 1]);
     nonpos = nonpos || (lane == j + 1 && !(a[j + 1] > 0.0));
     dj = pivot(a[j + 1], j + 1);
-    rj = recip(dj);
+    rj = recip64(dj);
 #pragma unroll
     for (int m = j + 2; m < 16; m++) a[m] = __builtin_fma(-l, ub[m], a[m]);
     __builtin_amdgcn_sched_barrier(0);

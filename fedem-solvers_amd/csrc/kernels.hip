@@ -1,7 +1,7 @@
 // gfx950 kernels of the part reducer: element matrices, pull assembly,
-// multifrontal LDL^T (panel factorisation on VALU, trailing updates on FP64
-// MFMA) and sparse products; the triangular solves are in solve.hip, the
-// tall-skinny products in dense.hip.
+// multifrontal LDL^T (pivot sweeps in registers, everything else of a diagonal
+// block, the panels and the trailing updates on MFMA) and sparse products; the
+// triangular solves are in solve.hip, the tall-skinny products in dense.hip.
 //
 // Front storage: the front of supernode s is an nrow x nrow column-major
 // FP64 block at pool + foff[s]; only its lower triangle is meaningful.  After
@@ -11,21 +11,9 @@
 #include <algorithm>
 #include <climits>
 #include <type_traits>
-#include "kernels.hpp"
+#include "kern_device.hpp"
 
 namespace fgpu {
-
-using f64x4 = __attribute__((__vector_size__(4 * sizeof(double)))) double;
-
-// Workgroups of a launch are dispatched round-robin over the eight XCDs of
-// the MI355X (workgroup b on XCD b mod 8), each with its own L2.  xcd_task
-// maps workgroup b to a task index so that every XCD takes one contiguous
-// range of the task list: neighbouring tasks, which share panel columns or
-// source rows, then share an L2.  A bijection of [0, n).
-__device__ __forceinline__ int xcd_task(int b, int n) {
-  const int q = n >> 3, r = n & 7, c = b & 7, m = b >> 3;
-  return c < r ? c * (q + 1) + m : r * (q + 1) + (c - r) * q + m;
-}
 
 // ---------------------------------------------------------------- HEX8
 // One 64-lane workgroup per element.  Lanes 0..26 evaluate the 27 Gauss
@@ -333,7 +321,7 @@ template <class T>
 __global__ __launch_bounds__(256) void k_extend_add(const FTask* __restrict__ tasks, DevSym S,
                                                     const int* __restrict__ xrange, T* __restrict__ pool) {
   __shared__ int srow[2][XADD_ROWS], scol[2][16];
-  const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const FTask t = tasks[xcd_ranges(blockIdx.x, gridDim.x)];
   const int sn = t.sn, ld = S.nrow[sn], own = t.k0, c0 = t.a, tid = threadIdx.x, lane = tid & 63;
   const int r0 = c0 + XADD_ROWS * blockIdx.y;
   if (r0 >= ld || (t.kb == 0 && c0 + 16 <= own)) return;
@@ -445,20 +433,6 @@ __device__ __forceinline__ void zero_acc(A (&acc)[2][2]) {
 }
 
 // ---------------------------------------------------------------- panel
-// Value of v in lane src (uniform src), through the scalar unit: no LDS
-// round trip and no memory wait between the broadcasts of a sweep.
-__device__ __forceinline__ double lane_bcast(double v, int src) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
-  return __hiloint2double(hi, lo);
-}
-
-// 1/d to rounding: the hardware estimate r0 (relative error e below 2^-20)
-// and r0 (1 + e + e^2).
-__device__ __forceinline__ double recip64(double d) {
-  const double r = __builtin_amdgcn_rcp(d), e = __builtin_fma(-d, r, 1.0);
-  return __builtin_fma(__builtin_fma(e, e, e), r, r);
-}
 // a/d from r = recip64(d): the product corrected by its own residual (the
 // quotient's rounding), three dependent operations instead of a division's
 // scaling sequence.
@@ -489,9 +463,10 @@ __device__ __forceinline__ float div_pivot(float a, double d) { return a / (floa
 // are carried as identity rows.
 // Bound by the dependent chain over the pivots (a reciprocal, a quotient and
 // a broadcast each): it sets the pace of every panel of the top separators.
-// 64 pivots take 25,400 cycles in one workgroup: 2500 of loads, four sweeps of
-// 2800 (issue bound: 15 broadcasts by two readlanes and a product per pivot),
-// 2000 around each (panel to and from LDS, its tiles), 1700 of stores.  A
+// 64 pivots take about 25,000 cycles in one workgroup, nearly half of them in
+// the four sweeps (2800 each, issue bound: 15 broadcasts by two readlanes and a
+// product per pivot), most of the others in loads, stores and the panels' way to
+// and from LDS.  A
 // k_diag_trsm launch of the 117 x 109 plate takes 14.7 us (18.2 with LDS reads
 // and stores under conditions, one wait each, and selects in the sweep that
 // kept the unread upper entries; 37-39 with 16-row sweeps, a division per pivot
@@ -713,14 +688,12 @@ __device__ __forceinline__ void trsm_product(const T (*sF)[65], const T (*sL)[65
 }
 
 // X = L^-1 into the diagonal tile of the pivot-block inverse pool and D into
-// the pivot array, plus the positive-definiteness check of the pivots.  The
-// front's diagonal block itself is left alone (later kernels read D from the
+// the pivot array.  The front's diagonal block itself is left alone (later kernels read D from the
 // pivot array, the solves L^-1 from the inverse pool), so that other
 // workgroups of the same launch can still read it.
 template <class T>
 __device__ __forceinline__ void diag_store(T* __restrict__ Xg, double* __restrict__ dpiv, int xld, int k0, int kb,
-                                           int col0, const double (&sD)[64], const double (&sX)[64][65],
-                                           int* __restrict__ piv) {
+                                           int col0, const double (&sD)[64], const double (&sX)[64][65]) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (tid < kb) dpiv[col0 + k0 + tid] = sD[tid];
   double x[16];
@@ -730,13 +703,12 @@ __device__ __forceinline__ void diag_store(T* __restrict__ Xg, double* __restric
 #pragma unroll
   for (int q = 0; q < 16; q++)
     if (lane < kb && wv + 4 * q < kb) out[(int64_t)(wv + 4 * q) * xld] = (T)x[q];
-  (void)piv;
 }
 
 template <class T>
 __global__ __launch_bounds__(256) void k_diag(const FTask* __restrict__ tasks, DevSym S,
                                               T* __restrict__ pool, const int64_t* __restrict__ ioff,
-                                              T* __restrict__ ipool, int* __restrict__ piv) {
+                                              T* __restrict__ ipool) {
   __shared__ double sA[64][65], sX[64][65], sD[64], sT[4][16][17];
   const FTask t = tasks[blockIdx.x];
   const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn], nc = S.ncol[sn];
@@ -744,7 +716,7 @@ __global__ __launch_bounds__(256) void k_diag(const FTask* __restrict__ tasks, D
   T* F = pool + S.foff[sn];
   T* Xg = ipool + ioff[sn];
   diag_block<T>(F, ld, k0, kb, sA, sX, sD, sT, S, S.col0[sn] + k0);
-  diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX, piv);
+  diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX);
 }
 
 // Diagonal block and triangular solve in one launch, for panels with few
@@ -759,9 +731,9 @@ __global__ __launch_bounds__(256) void k_diag(const FTask* __restrict__ tasks, D
 template <class T>
 __global__ __launch_bounds__(256) void k_diag_trsm(const FTask* __restrict__ tasks, DevSym S,
                                                    T* __restrict__ pool, const int64_t* __restrict__ ioff,
-                                                   T* __restrict__ ipool, int* __restrict__ piv) {
+                                                   T* __restrict__ ipool) {
   __shared__ double sA[64][65], sX[64][65], sD[64], sT[4][16][17];
-  const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const FTask t = tasks[xcd_ranges(blockIdx.x, gridDim.x)];
   const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn], nc = S.ncol[sn];
   const int kb = min(64, nc - k0);
   T* F = pool + S.foff[sn];
@@ -778,7 +750,7 @@ __global__ __launch_bounds__(256) void k_diag_trsm(const FTask* __restrict__ tas
   }
   diag_block<T>(F, ld, k0, kb, sA, sX, sD, sT, S, S.col0[sn] + k0);
   if (t.a < 0) {
-    diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX, piv);
+    diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX);
     return;
   }
   // operand tiles in the storage type: the row tile in sA's space (every
@@ -794,7 +766,7 @@ __global__ __launch_bounds__(256) void k_diag_trsm(const FTask* __restrict__ tas
   }
   __syncthreads();
   trsm_product<T>(sF, sL, F + (int64_t)k0 * ld, ld, R0, kb, [&](int j) { return sD[j]; });
-  if (t.a == 0) diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX, piv);
+  if (t.a == 0) diag_store<T>(Xg, S.dpiv, S.ild[sn], k0, kb, S.col0[sn], sD, sX);
 }
 
 // k_trsm task: sn, a = 64-row tile below the diagonal block, k0 = panel.
@@ -806,7 +778,7 @@ __global__ __launch_bounds__(256) void k_trsm(const FTask* __restrict__ tasks, D
                                               const T* __restrict__ ipool) {
   __shared__ T sA[64][65];
   __shared__ T sB[64][65];
-  const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const FTask t = tasks[xcd_ranges(blockIdx.x, gridDim.x)];
   const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn], nc = S.ncol[sn];
   const int kb = min(64, nc - k0);
   const int R0 = k0 + kb + 64 * t.a;
@@ -869,7 +841,7 @@ template <int XA, int YB, class T>
 __global__ __launch_bounds__(XA == 4 ? 128 : 256, XA == 4 ? 3 : 4) void k_update(const FTask* __restrict__ tasks, DevSym S,
                                                                 T* __restrict__ pool) {
   constexpr int CH = 8, ST = CH / 4;
-  const FTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const FTask t = tasks[xcd_ranges(blockIdx.x, gridDim.x)];
   const int sn = t.sn, k0 = t.k0, ld = S.nrow[sn], kb = t.kb;
   T* F = pool + S.foff[sn];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
@@ -1212,7 +1184,7 @@ __global__ __launch_bounds__(256) void k_spmm(int nnode, int nrhs, const int* __
   __shared__ double sv[4][RB][64];
   __shared__ int sc[4][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, j = lane % W, ph = lane / W;
-  const int node = 4 * xcd_task(blockIdx.x, gridDim.x) + wv;
+  const int node = 4 * xcd_ranges(blockIdx.x, gridDim.x) + wv;
   if (node >= nnode) return;
   const int r0 = nrow0[node], dn = nrow0[node + 1] - r0;
   const int kb = rowptr[r0], len = rowptr[r0 + 1] - kb;
@@ -1467,15 +1439,15 @@ __global__ void k_recip(int n, const double* __restrict__ x, double* __restrict_
   if (i < n) y[i] = 1.0 / x[i];
 }
 
-// Y[g] = a * X[g] + b * Y[g] over the first n entries
-// Y = a X + b Y (Y not read when b = 0; X and Y may be the same array)
+// Y = a X + b Y over the first n entries (Y not read when b = 0; X and Y may be
+// the same array)
 __global__ void k_axpby(int64_t n, double a, const double* X, double b, double* Y) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g < n) Y[g] = b == 0.0 ? a * X[g] : a * X[g] + b * Y[g];
 }
 
 // part[blk] = (sum x^2, sum y^2) over the block's slice of the first n
-// entries; k_sumsq_fin adds the blocks in order (deterministic norms)
+// entries; the host adds the blocks in order (deterministic norms)
 __global__ __launch_bounds__(256) void k_sumsq2(int64_t n, const double* __restrict__ x,
                                                 const double* __restrict__ y, double* __restrict__ part) {
   __shared__ double r0[256], r1[256];
@@ -1592,8 +1564,6 @@ __global__ __launch_bounds__(256) void k_col_axpby(int64_t n, int nr, const doub
 }
 
 // ---------------------------------------------------------------- launchers
-static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
-
 void launch_hex8(hipStream_t st, int nhex, const int* elist, const int* eptr, const int* enodes,
                  const double* xyz, const double* eprop, const int64_t* eoff, double* Kp, double* Mp,
                  int* ebad) {
@@ -1627,38 +1597,38 @@ void launch_reduced(hipStream_t st, int nd, int n2, int ngen, const int* pos2, c
 void launch_fill(hipStream_t st, double* p, int64_t n, double v) {
   if (n > 0) k_fill<<<(unsigned)std::min<int64_t>(nblk(n, 256), 16384), 256, 0, st>>>(p, n, v);
 }
-#define FGPU_FACTOR_LAUNCHERS(T)                                                                           \
-  void launch_front_zero(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {                \
-    if (n > 0) k_front_zero<T><<<n, 256, 0, st>>>(t, S, pool);                                               \
-  }                                                                                                        \
-  void launch_extend_add(hipStream_t st, const FTask* t, int n, int rows, const DevSym& S,                 \
-                         const int* xrange, T* pool) {                                                     \
-    if (n > 0) k_extend_add<T><<<dim3(n, nblk(rows, XADD_ROWS)), 256, 0, st>>>(t, S, xrange, pool);          \
-  }                                                                                                        \
-  void launch_diag(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,   \
-                   T* ipool, int* piv) {                                                                   \
-    if (n > 0) k_diag<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, piv);                                   \
-  }                                                                                                        \
-  void launch_diag_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool,                   \
-                        const int64_t* ioff, T* ipool, int* piv) {                                          \
-    if (n > 0) k_diag_trsm<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, piv);                             \
-  }                                                                                                        \
-  void launch_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,   \
-                   const T* ipool) {                                                                       \
-    if (n > 0) k_trsm<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                        \
-  }                                                                                                        \
-  void launch_update(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {                    \
-    if (n >= UPD_WIDE) k_update<4, 2, T><<<n, 128, 0, st>>>(t, S, pool);                                     \
-    else if (n > UPD_NARROW) k_update<2, 2, T><<<n, 256, 0, st>>>(t, S, pool);                               \
-    else if (n > 0) k_update<1, 1, T><<<dim3(n, 4), 256, 0, st>>>(t, S, pool);                               \
-  }                                                                                                        \
-  void launch_inv_mul(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,               \
-                      const int64_t* ioff, T* ipool, T* tmp) {                                             \
-    if (n > 0) k_inv_mul<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, tmp);                                \
-  }                                                                                                        \
-  void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                 \
-                    const int64_t* ioff, T* ipool) {                                                       \
-    if (n > 0) k_panel<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                       \
+#define FGPU_FACTOR_LAUNCHERS(T)                                                                          \
+  void launch_front_zero(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {               \
+    if (n > 0) k_front_zero<T><<<n, 256, 0, st>>>(t, S, pool);                                            \
+  }                                                                                                       \
+  void launch_extend_add(hipStream_t st, const FTask* t, int n, int rows, const DevSym& S,                \
+                         const int* xrange, T* pool) {                                                    \
+    if (n > 0) k_extend_add<T><<<dim3(n, nblk(rows, XADD_ROWS)), 256, 0, st>>>(t, S, xrange, pool);       \
+  }                                                                                                       \
+  void launch_diag(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,  \
+                   T* ipool) {                                                                            \
+    if (n > 0) k_diag<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                     \
+  }                                                                                                       \
+  void launch_diag_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool,                  \
+                        const int64_t* ioff, T* ipool) {                                                  \
+    if (n > 0) k_diag_trsm<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                \
+  }                                                                                                       \
+  void launch_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,  \
+                   const T* ipool) {                                                                      \
+    if (n > 0) k_trsm<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                     \
+  }                                                                                                       \
+  void launch_update(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool) {                   \
+    if (n >= UPD_WIDE) k_update<4, 2, T><<<n, 128, 0, st>>>(t, S, pool);                                  \
+    else if (n > UPD_NARROW) k_update<2, 2, T><<<n, 256, 0, st>>>(t, S, pool);                            \
+    else if (n > 0) k_update<1, 1, T><<<dim3(n, 4), 256, 0, st>>>(t, S, pool);                            \
+  }                                                                                                       \
+  void launch_inv_mul(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,              \
+                      const int64_t* ioff, T* ipool, T* tmp) {                                            \
+    if (n > 0) k_inv_mul<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool, tmp);                             \
+  }                                                                                                       \
+  void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                \
+                    const int64_t* ioff, T* ipool) {                                                      \
+    if (n > 0) k_panel<T><<<n, 256, 0, st>>>(t, S, pool, ioff, ipool);                                    \
   }
 FGPU_FACTOR_LAUNCHERS(double)
 FGPU_FACTOR_LAUNCHERS(float)

@@ -89,19 +89,19 @@ void launch_reduced(hipStream_t st, int nd, int n2, int ngen, const int* pos2, c
   void launch_extend_add(hipStream_t st, const FTask* t, int n, int rows, const DevSym& S,                \
                          const int* xrange, T* pool);                                                     \
   void launch_diag(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,  \
-                   T* ipool, int* piv);                                                                   \
+                   T* ipool);                                                                             \
   void launch_diag_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool,                  \
-                        const int64_t* ioff, T* ipool, int* piv);                                          \
+                        const int64_t* ioff, T* ipool);                                                   \
   void launch_trsm(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool, const int64_t* ioff,  \
                    const T* ipool);                                                                       \
   void launch_update(hipStream_t st, const FTask* t, int n, const DevSym& S, T* pool);                    \
   /* pivot-block inverses (tmp: the products that the pairs of blocks are joined by) */                   \
   void launch_inv_mul(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,              \
                       const int64_t* ioff, T* ipool, T* tmp);                                             \
-  /* Y21 = -L21 L11^-1 of the fused levels below L11^-1 (solve panels) */                               \
+  /* Y21 = -L21 L11^-1 of the fused levels below L11^-1 (solve panels) */                                 \
   void launch_panel(hipStream_t st, const FTask* t, int n, const DevSym& S, const T* pool,                \
                     const int64_t* ioff, T* ipool);                                                       \
-  /* solve products (solve.hip): nt 16-column groups of right-hand sides per task, kw K parts */         \
+  /* solve products (solve.hip): nt 16-column groups of right-hand sides per task, kw K parts */          \
   void launch_mv(hipStream_t st, const MvTask* t, int n, int kind, int nt, int kw, const T* pool,         \
                  const T* panel, const int* rows, const double* dpiv, const int2* kids, double* W,        \
                  double* V, const double* R, double* Y, double* X, int nrhs);

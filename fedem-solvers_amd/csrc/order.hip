@@ -1,12 +1,10 @@
 // Change of order between the callers' vectors (column-major, equations in
 // SAM order) and the reducer's (row-major, rows in elimination order), on the
 // device, so that a vector crosses the bus once and the host does not touch
-// it; and the gathered upload of small arrays.
-#include "kernels.hpp"
+// it; and the gathered upload of arrays.
+#include "kern_device.hpp"
 
 namespace fgpu {
-
-static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 // A workgroup takes 64 source rows by 16 columns through an LDS tile: the
 // column-major side in runs of 64 rows, the row-major side in runs of 16

@@ -1265,7 +1265,6 @@ static void run_mv(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, 
               sp.nrhs);
 }
 
-// Y = D^{-1} L^{-1} R on the internal rows
 // Z = M X
 static void mass_mm(hipStream_t st, int neq, const DeviceReducer::Impl& d, int nrhs, const double* X, int ldx, double* Z,
                     int ldz) {
@@ -1273,6 +1272,7 @@ static void mass_mm(hipStream_t st, int neq, const DeviceReducer::Impl& d, int n
   else launch_spmm(st, d.node_rows(neq), nrhs, d.rowptr.p, d.colind.p, d.Mv.p, X, ldx, Z, ldz);
 }
 
+// Y = D^{-1} L^{-1} R on the internal rows
 static void run_forward(hipStream_t st, DeviceReducer::Impl& d, const SolvePlan& sp, const double* R, double* Y) {
   for (const Op& op : sp.fw) {
     if (op.kind == FW_INIT)
@@ -1547,9 +1547,9 @@ int DeviceReducer::reduce(std::string& err) {
     for (const Op& op : d.fops) {
       switch (op.kind) {
         case EXTADD: launch_extend_add(st, d.ftasks.p + op.off, op.n, op.kw, d.S, d.xrange.p, pool); break;
-        case DIAG: launch_diag(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool, d.piv.p); break;
+        case DIAG: launch_diag(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
         case TRSM: launch_trsm(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
-        case DIAG_TRSM: launch_diag_trsm(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool, d.piv.p); break;
+        case DIAG_TRSM: launch_diag_trsm(st, d.ftasks.p + op.off, op.n, d.S, pool, d.ioff.p, ipool); break;
         case UPDATE:
         case UPDATE_SIDE: {
           // with per-launch timing everything stays on the main stream
@@ -1592,7 +1592,7 @@ int DeviceReducer::reduce(std::string& err) {
     // the factor schedule is fixed per symbolic structure: one graph
     HIPCHK(run_graph(st, d.g_factor,
                      {d.ftasks.p, d.xrange.p, d.itmp.p, d.pool.p, d.ipool.p, d.pool32.p, d.ipool32.p, d.ioff.p,
-                      d.piv.p, d.S.foff, d.S.rows, d.S.dpiv},
+                      d.S.foff, d.S.rows, d.S.dpiv},
                      factor_ops));
   }
   HIPCHK(fork_err);
@@ -1692,7 +1692,6 @@ int DeviceReducer::reduce(std::string& err) {
     }
   }
   // ---- component modes (block Lanczos, shift-invert on the resident factor)
-  std::vector<double> Sres;
   if (nev > 0) {
     int rc = 0;
     int bs = 0, mcap = 0;
@@ -1764,7 +1763,6 @@ int DeviceReducer::reduce(std::string& err) {
     HIPCHK(hipStreamSynchronize(st));
     if ((rc = orth_finish(0, R0))) return rc;
     int nb = 0;  // number of completed blocks in H
-    std::vector<double> theta, Svec, Rlast;
     bool conv = false;
     // symmetrised block-tridiagonal projection of the first mj Lanczos vectors
     auto projected = [&](int mj) {

@@ -10,23 +10,15 @@
 // An unfused level (large fronts, where forming Y21 costs more than the
 // launches it saves) multiplies by X11 and by L21 of the front in turn.
 #include <algorithm>
-#include "kernels.hpp"
+#include "kern_device.hpp"
 
 namespace fgpu {
 
-using f64x4 = __attribute__((__vector_size__(4 * sizeof(double)))) double;
-
-// Workgroup b's task: neighbouring tasks, which share source rows and the
-// lines between their target rows, go to one XCD (workgroup b runs on XCD b mod
-// 8) by fours, the fours round the XCDs.  Whole ranges per XCD gave one the
-// short and another the long sums of a triangular block: the products of a
-// Lanczos step of the 45x41x43 block 2074 -> 1950 us, 48x24x24 642 -> 610.
-__device__ __forceinline__ int xcd_task(int b, int n) {
-  constexpr int G = 4;
-  if (b >= n / (8 * G) * (8 * G)) return b;
-  const int c = b & 7, m = b >> 3;
-  return ((m / G) * 8 + c) * G + m % G;
-}
+// The tasks of a launch go to the XCDs by fours (xcd_fours): neighbours share
+// source rows and the lines between their target rows.  Whole ranges per XCD
+// gave one the short and another the long sums of a triangular block: the
+// products of a Lanczos step of the 45x41x43 block 2074 -> 1950 us, 48x24x24
+// 642 -> 610.
 
 // Result v of target row r, right-hand side j of task t.  GM > 0: base is what
 // the children add to a row of W, which the row itself does not hold.
@@ -103,7 +95,7 @@ __global__ __launch_bounds__(64 * RT * KW) void k_fw(const MvTask* __restrict__ 
   static_assert(KW == 1 || RT == 1, "the K split works on 16-row tasks");
   constexpr int CH = NT == 1 && GM < 2 ? 32 : 16, ST = CH / 4;
   constexpr int NB = KW == 1 ? 4 * NT : NT;  // results of a thread
-  const MvTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const MvTask t = tasks[xcd_fours(blockIdx.x, gridDim.x)];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
   const int r0 = 16 * (wv % RT), kw = wv / RT;
   if (KW == 1 && r0 >= t.rn) return;
@@ -235,7 +227,7 @@ __global__ __launch_bounds__(64 * KW) void k_bw(const MvTask* __restrict__ tasks
   // reads by (lane mod 16, lane / 16)
   constexpr int LT = CH + 2, TILE = 16 * LT * (int)sizeof(T) / 8;
   __shared__ double lds[KW * (TILE > 272 ? TILE : 272)];
-  const MvTask t = tasks[xcd_task(blockIdx.x, gridDim.x)];
+  const MvTask t = tasks[xcd_fours(blockIdx.x, gridDim.x)];
   const int lane = threadIdx.x & 63, kw = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
   T* tile = reinterpret_cast<T*>(lds + kw * TILE);
   const int part = KW == 1 ? t.kn : (((t.kn + KW - 1) / KW + CH - 1) / CH) * CH;
@@ -356,19 +348,19 @@ static void mv_launch(hipStream_t st, const MvTask* t, int n, int kind, int kw, 
   }
 }
 
-#define FGPU_MV(T)                                                                                                  \
-  void launch_mv(hipStream_t st, const MvTask* t, int n, int kind, int nt, int kw, const T* pool, const T* panel,   \
-                 const int* rows, const double* dpiv, const int2* kids, double* W, double* V, const double* R,      \
-                 double* Y, double* X, int nrhs) {                                                                                        \
-    if (n <= 0) return;                                                                                             \
-    switch (nt) {                                                                                                   \
-      case 1: mv_launch<1, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
-      case 2: mv_launch<2, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
-      case 3: mv_launch<3, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
-      case 4: mv_launch<4, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
-      case 5: mv_launch<5, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;              \
-      default: mv_launch<6, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;             \
-    }                                                                                                               \
+#define FGPU_MV(T)                                                                                                 \
+  void launch_mv(hipStream_t st, const MvTask* t, int n, int kind, int nt, int kw, const T* pool, const T* panel,  \
+                 const int* rows, const double* dpiv, const int2* kids, double* W, double* V, const double* R,     \
+                 double* Y, double* X, int nrhs) {                                                                 \
+    if (n <= 0) return;                                                                                            \
+    switch (nt) {                                                                                                  \
+      case 1: mv_launch<1, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;      \
+      case 2: mv_launch<2, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;      \
+      case 3: mv_launch<3, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;      \
+      case 4: mv_launch<4, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;      \
+      case 5: mv_launch<5, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;      \
+      default: mv_launch<6, T>(st, t, n, kind, kw, pool, panel, rows, dpiv, kids, W, V, R, Y, X, nrhs); break;     \
+    }                                                                                                              \
   }
 FGPU_MV(double)
 FGPU_MV(float)
