@@ -142,32 +142,39 @@ struct HBuf {
 struct Stage {
   static constexpr size_t PIECE = 512 << 10;
   HBuf<char> mem;
-  hipEvent_t passed[2]{};
-  bool in_use[2]{};
+  hipEvent_t event[2]{};
+  enum { FREE, EVENT, STREAM } until[2]{};  // what the device's work on a piece ends with
+  hipStream_t stream = nullptr;
 
   ~Stage() {
-    for (hipEvent_t& e : passed)
+    for (hipEvent_t& e : event)
       if (e) (void)hipEventDestroy(e);
   }
   hipError_t open() {
     if (mem.p) return hipSuccess;
-    for (hipEvent_t& ev : passed)
+    for (hipEvent_t& ev : event)
       if (!ev)
         if (hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) return e;
     return mem.alloc(2 * PIECE);
   }
   char* piece(int h) { return mem.p + h * PIECE; }
-  // the device's work on piece h is what the stream has been given so far
-  hipError_t mark(int h, hipStream_t st) {
-    in_use[h] = true;
-    return hipEventRecord(passed[h], st);
+  // The device's work on piece h is what the stream has been given so far.
+  // Without an event of its own (which costs the stream some 5 us) where the
+  // stream is waited for anyway before the piece is wanted again.
+  hipError_t mark(int h, hipStream_t st, bool own_event = true) {
+    stream = st;
+    until[h] = own_event ? EVENT : STREAM;
+    return own_event ? hipEventRecord(event[h], st) : hipSuccess;
   }
   // piece h is the host's again
   hipError_t wait(int h) {
-    if (!in_use[h]) return hipSuccess;
-    in_use[h] = false;
-    return hipEventSynchronize(passed[h]);
+    const auto u = until[h];
+    until[h] = FREE;
+    if (u == STREAM) return hipStreamSynchronize(stream);
+    return u == EVENT ? hipEventSynchronize(event[h]) : hipSuccess;
   }
+  // the stream has been waited for
+  void passed() { until[0] = until[1] = FREE; }
 };
 
 // Arrays on their way to the device.  While a batch is open on the thread its
@@ -192,15 +199,16 @@ struct UploadBatch {
     st = s;
     err = stage.open();
     used = blocks = 0;
-    return err == hipSuccess ? err = stage.wait(h) : err;
+    return err;
   }
   hipError_t put(void* dst, const void* src, size_t bytes) {
     for (size_t o = 0; o < bytes && err == hipSuccess;) {
       const size_t n = std::min({bytes - o, DATA - used, (MOST - blocks) * COPY_BLOCK});
       if (n == 0) {
-        (void)flush();  // (err)
+        (void)flush(true);  // (err)
         continue;
       }
+      if (blocks == 0 && (err = stage.wait(h)) != hipSuccess) break;
       CopyBlock* t = reinterpret_cast<CopyBlock*>(stage.piece(h));
       std::memcpy(stage.piece(h) + TABLE + used, static_cast<const char*>(src) + o, n);
       for (size_t q = 0; q < n; q += COPY_BLOCK)
@@ -211,14 +219,14 @@ struct UploadBatch {
     }
     return err;
   }
-  hipError_t flush() {
+  hipError_t flush(bool full = false) {
     if (blocks == 0 || err != hipSuccess) return err;
     launch_copy_blocks(st, (int)blocks, reinterpret_cast<const CopyBlock*>(stage.piece(h)), stage.piece(h));
     used = blocks = 0;
     err = hipGetLastError();
-    if (err == hipSuccess) err = stage.mark(h, st);
+    if (err == hipSuccess) err = stage.mark(h, st, full);
     h ^= 1;
-    return err == hipSuccess ? err = stage.wait(h) : err;
+    return err;
   }
 };
 static thread_local UploadBatch* tl_batch = nullptr;
@@ -966,6 +974,7 @@ int DeviceReducer::build_structure(std::string& err) {
   HIPCHK(hipMemcpyAsync(d.hpiv.p, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
   HIPCHK(hipMemcpyAsync(d.hpiv.p + 1, d.cptr.p + nnz, sizeof(int), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  d.stage.passed();
   const int hb = d.hpiv.p[0], total = d.hpiv.p[1];
   if (hb || total != y.ncontrib) {
     err = "device structure build: " + std::string(hb & 1 ? "element contribution outside the CSR pattern" :
@@ -1661,6 +1670,7 @@ int DeviceReducer::reduce(std::string& err) {
   HIPCHK(d.hpiv.alloc(PIVOT_STATS));
   HIPCHK(hipMemcpyAsync(d.hpiv.p, d.piv.p, sizeof(int) * PIVOT_STATS, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  d.stage.passed();
   int hbad[PIVOT_STATS];
   std::copy(d.hpiv.p, d.hpiv.p + PIVOT_STATS, hbad);
   if (const int e = hbad[6]; e != INT_MAX) {
