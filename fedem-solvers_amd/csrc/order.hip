@@ -10,7 +10,7 @@ namespace fgpu {
 // column-major side in runs of 64 rows, the row-major side in runs of 16
 // columns.  Bound by HBM, far below the copy over the bus.  With the order on
 // the host a solve of 40,404 equations by 33 columns took 3.6 ms, now 1.5, and
-// 7 load cases with their recovery on 38,000 equations 1.9, now 0.73.
+// 7 load cases with their recovery on 38,000 equations 1.9, now 0.67.
 constexpr int OT_ROWS = 64, OT_COLS = 16;
 
 // out[map[q]][c] = in[q + c ldi] (map null: row q itself)

@@ -183,7 +183,7 @@ struct Stage {
 // the other, flush() sends what is there.  Each array is uploaded once and
 // kept until the batch ends.  An array by itself costs a staged copy and a
 // wait, 15 us each (0.8 of the 1.46 ms in which a 20x10 plate was analysed,
-// uploaded and reduced; 0.74 in all with its 45 small arrays gathered), and a
+// uploaded and reduced; 0.69 in all with its 45 small arrays gathered), and a
 // large one goes through staging memory of the runtime's own, whose pages are
 // new with most handles: 2.4 GB/s, until 16 MB have passed.
 struct UploadBatch {
@@ -2144,7 +2144,7 @@ static void runs(char* piece, double* array, int n, int q0, int m, int c0, int k
 // the host copies one piece out while the device fills the other: no device
 // buffer, and the data crosses the bus once.  (With copies behind an ordering
 // kernel into a buffer of its own, through the runtime's staging memory, B of a
-// 16x12x10 block took 0.98 ms where the order on the host took 0.53.)
+// 16x12x10 block took 0.98 ms where the order on the host took 0.53; 0.2 now.)
 int DeviceReducer::rows_to_host(int n, int nc, const int* map, const double* A, int lda, const double* B, int ldb,
                                 double* out, std::string& err) const {
   Stage& s = d_->stage;
